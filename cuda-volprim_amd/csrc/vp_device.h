@@ -64,6 +64,28 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
+// Exclusive prefix sum over the wavefront's 64 lanes of v < 2^16, from one
+// ballot per bit; total receives the sum.
+__device__ __forceinline__ uint32_t wave_prefix16(uint32_t v, uint32_t& total) {
+    uint32_t pre = 0;
+    total = 0;
+    for (uint32_t bit = 0; bit < 16u; ++bit) {
+        const unsigned long long bm = __builtin_amdgcn_ballot_w64(((v >> bit) & 1u) != 0u);
+        pre += lanes_below(bm) << bit;
+        total += static_cast<uint32_t>(__popcll(bm)) << bit;
+    }
+    return pre;
+}
+// The lane that item g of a wavefront's flattened lists belongs to: the last
+// one whose prefix (pre[64], ascending) is at most g.
+__device__ __forceinline__ uint32_t prefix_owner(const uint32_t* pre, uint32_t g) {
+    uint32_t lo = 0;
+#pragma unroll
+    for (uint32_t s = 32u; s > 0u; s >>= 1)
+        if (pre[lo + s] <= g) lo += s;
+    return lo;
+}
+
 // ---- walk-tree traversal (tree layout and Walk4 in vp_walk.h) ----
 
 // Children of node n that the ray crosses within [0, tmax], as a 4-bit mask.
@@ -633,24 +655,26 @@ __device__ __forceinline__ bool wave_steal(const WaveQueue& wq, bool idle, bool 
     return got;
 }
 
-// The MIS shadow rays of the calling lanes, with the wave-shared leaf queue
-// and a wave-wide ray pool: every lane starts on one ray of the wavefront's
-// list (all rays a, then all rays b) and, when its ray is done, takes the
-// next one from the list, whichever lane the ray belongs to.  The node
-// phases then stay full however the walk lengths are spread, until the list
-// runs out.  Each ray's chords are summed in fixed point in LDS (a ray is
-// saturated once its sum reaches the tau = 88 limit, in whatever order the
-// chords arrive), so Ta and Tb equal two transmittance() calls bit for bit.
-// Every lane of the calling wavefront that is active here takes part.
-// With two = false only ray a is walked (the one shadow ray of RIS).  Each
-// ray's walk may stop once its depth reaches its limit (lim_a, lim_b: the
-// tau = 88 saturation, or a shadow-roulette threshold; multiples of 2^16);
-// acc_a and acc_b receive the fixed-point depths.
+// The shadow rays of a wavefront's lanes, up to two each (the MIS rays a and
+// b, or the one of RIS), with the wave-shared leaf queue and a wave-wide ray
+// pool.  All 64 lanes of the wavefront call it, those without a ray as
+// helpers: every lane starts on one ray of the wavefront's list (all rays a,
+// then all rays b) and, when its ray is done, takes the next one from the
+// list, whichever lane the ray belongs to.  The node phases then stay full
+// however the walk lengths are spread, until the list runs out; from there on
+// lanes without a ray share the running walks.  Each ray's chords are summed
+// in fixed point in LDS (a ray is saturated once its sum reaches the tau = 88
+// limit, in whatever order the chords arrive), so Ta and Tb equal two
+// transmittance() calls bit for bit.
+// Each ray's walk may stop once its depth reaches its limit (lim_a, lim_b:
+// the tau = 88 saturation, or a shadow-roulette threshold; multiples of
+// 2^16); a limit of 0 is a ray that is not walked.  acc_a and acc_b receive
+// the fixed-point depths.
 __device__ __forceinline__ void transmittance_pool(const SceneView& s, f3 o, f3 da, f3 db, const uint32_t* act,
-                                                   uint32_t na, uint32_t stride, const WaveQueue& wq,
-                                                   uint64_t lim_a, uint64_t lim_b, uint64_t& acc_a,
-                                                   uint64_t& acc_b, bool two = true) {
+                                                   uint32_t na_path, const WaveQueue& wq, uint64_t lim_a,
+                                                   uint64_t lim_b, uint64_t& acc_a, uint64_t& acc_b) {
     const uint32_t lane = __lane_id();
+    const uint32_t na = (lim_a | lim_b) != 0ull ? na_path : 0u;
     lds_store3(wq.ro + 3 * lane, o);
     wq.prims[lane] = s.prims;
     wq.nodes[lane] = s.w4;
@@ -658,56 +682,41 @@ __device__ __forceinline__ void transmittance_pool(const SceneView& s, f3 o, f3 
     lds_store3(wq.rd + 3 * (2 * lane), da);
     lds_store3(wq.rd + 3 * (2 * lane + 1), db);
     wq.acc[2 * lane] = 0ull;
-    wq.acc[2 * lane + 1] = two ? 0ull : kTauLimitFixed;
+    wq.acc[2 * lane + 1] = 0ull;
     wq.lim[2 * lane] = static_cast<uint32_t>(lim_a >> 16);
-    wq.lim[2 * lane + 1] = two ? static_cast<uint32_t>(lim_b >> 16) : 0u;
+    wq.lim[2 * lane + 1] = static_cast<uint32_t>(lim_b >> 16);
     // a ray is done once its depth reaches its limit
     auto reached = [&](uint32_t r) -> bool {
         return wq.acc[r] >= (static_cast<unsigned long long>(wq.lim[r]) << 16);
     };
-    wave_sync();
     // Chords of the origin set (every member's optical depth from the origin
     // to its exit), for all lanes' rays together: the wavefront's (member,
     // lane) pairs are numbered through a prefix sum of the set sizes and
-    // shared out over the lanes, so the loop runs sum(na) / lanes times
+    // shared out over the lanes, so the loop runs sum(na) / 64 times
     // instead of max(na).  Each chord goes into its ray's fixed-point sum; a
     // sum that passes the tau = 88 limit gives T = 0 however far it passes,
     // as in transmittance().  The owners' set pointers and prefix sums sit in
-    // wq.tj and their lane ids in wq.list, both free until the walks start.
+    // wq.tj, free until the walks start.
     {
-        const unsigned long long m0 = __builtin_amdgcn_ballot_w64(true);
-        const uint32_t rk = lanes_below(m0), nl = static_cast<uint32_t>(__popcll(m0));
-        uint32_t pre = 0, total = 0;
-        for (uint32_t bit = 0; bit < 16u; ++bit) {
-            const unsigned long long bm = __builtin_amdgcn_ballot_w64(((na >> bit) & 1u) != 0u);
-            pre += lanes_below(bm) << bit;
-            total += static_cast<uint32_t>(__popcll(bm)) << bit;
-        }
         static_assert(kWaveQ * sizeof(float) >= 64 * (sizeof(void*) + sizeof(uint32_t)),
                       "the shared queue must hold the origin-set tables");
-        const uint32_t** set_of = reinterpret_cast<const uint32_t**>(wq.tj);  // [64] by rank
-        uint32_t* pre_of = reinterpret_cast<uint32_t*>(wq.tj) + 2 * 64;     // [64] by rank
-        set_of[rk] = act;
-        pre_of[rk] = pre;
-        wq.list[rk] = static_cast<uint8_t>(lane);
+        const uint32_t** set_of = reinterpret_cast<const uint32_t**>(wq.tj);  // [64]
+        uint32_t* pre_of = reinterpret_cast<uint32_t*>(wq.tj) + 2 * 64;     // [64]
+        uint32_t total;
+        const uint32_t pre = wave_prefix16(na, total);
+        set_of[lane] = act;
+        pre_of[lane] = pre;
         wave_sync();
-        for (uint32_t g = rk; g < total; g += nl) {
-            // the owner: the last rank whose prefix is at most g
-            uint32_t lo = 0, hi = nl - 1u;
-            while (lo < hi) {
-                const uint32_t mid = (lo + hi + 1u) >> 1;
-                if (pre_of[mid] <= g) lo = mid;
-                else hi = mid - 1u;
-            }
-            const uint32_t ol = wq.list[lo];
-            const PrimRecord pr = load_prim(wq.prims[ol], set_of[lo][(g - pre_of[lo]) * stride]);
+        for (uint32_t g = lane; g < total; g += 64u) {
+            const uint32_t ol = prefix_owner(pre_of, g);
+            const PrimRecord pr = load_prim(wq.prims[ol], set_of[ol][g - pre_of[ol]]);
             const f3 xo = lds_load3(wq.ro + 3 * ol);
-            const f3 dra = lds_load3(wq.rd + 3 * (2 * ol));
-            const float ta = inside_chord(pr, xo, dra).tau;
-            if (ta > 0.0f) atomicAdd(&wq.acc[2 * ol], tau_fixed(ta));
-            if (two) {
-                const f3 drb = lds_load3(wq.rd + 3 * (2 * ol + 1));
-                const float tb = inside_chord(pr, xo, drb).tau;
+            if (wq.lim[2 * ol] != 0u) {
+                const float ta = inside_chord(pr, xo, lds_load3(wq.rd + 3 * (2 * ol))).tau;
+                if (ta > 0.0f) atomicAdd(&wq.acc[2 * ol], tau_fixed(ta));
+            }
+            if (wq.lim[2 * ol + 1] != 0u) {
+                const float tb = inside_chord(pr, xo, lds_load3(wq.rd + 3 * (2 * ol + 1))).tau;
                 if (tb > 0.0f) atomicAdd(&wq.acc[2 * ol + 1], tau_fixed(tb));
             }
         }
@@ -717,7 +726,6 @@ __device__ __forceinline__ void transmittance_pool(const SceneView& s, f3 o, f3 
     const bool full_b = reached(2 * lane + 1);
     // the rays still to walk: every ray a, then every ray b (a saturated ray
     // is done already)
-    const unsigned long long am = __builtin_amdgcn_ballot_w64(true);
     const unsigned long long pa = __builtin_amdgcn_ballot_w64(!full_a);
     const unsigned long long pb = __builtin_amdgcn_ballot_w64(!full_b);
     const uint32_t npa = static_cast<uint32_t>(__popcll(pa));
@@ -725,12 +733,10 @@ __device__ __forceinline__ void transmittance_pool(const SceneView& s, f3 o, f3 
     if (!full_a) wq.list[lanes_below(pa)] = static_cast<uint8_t>(2 * lane);
     if (!full_b) wq.list[npa + lanes_below(pb)] = static_cast<uint8_t>(2 * lane + 1);
     wave_sync();
-    const uint32_t nact = static_cast<uint32_t>(__popcll(am));
-    uint32_t next = nact < nr ? nact : nr;  // list entries handed out
+    uint32_t next = nr < 64u ? nr : 64u;  // list entries handed out
     constexpr uint32_t kNoRay = 0xffu;
     // the ray this lane walks, and its walk state
-    const uint32_t rank = lanes_below(am);
-    uint32_t ray = rank < nr ? wq.list[rank] : kNoRay;
+    uint32_t ray = lane < nr ? wq.list[lane] : kNoRay;
     const float4* w4 = nullptr;
     uint32_t levels = 0, half = 0;
     Walk4 w = walk4_begin();
@@ -762,7 +768,7 @@ __device__ __forceinline__ void transmittance_pool(const SceneView& s, f3 o, f3 
             // the list is used up and many lanes are idle: end the phase so
             // the running walks can be shared out (after at least one step,
             // so every phase progresses)
-            if (nsteps >= VP_STEAL_GAP && next >= nr && ns + VP_STEAL_IDLE <= nact &&
+            if (nsteps >= VP_STEAL_GAP && next >= nr && ns + VP_STEAL_IDLE <= 64u &&
                 __builtin_amdgcn_ballot_w64(step && walk4_pending(w) != 0ull) != 0ull)
                 break;
             ++nsteps;
@@ -779,8 +785,8 @@ __device__ __forceinline__ void transmittance_pool(const SceneView& s, f3 o, f3 
         // fixed-point sum
         // (two leaves per lane and round, both records loaded before either
         // crossing, so each lane has two loads in flight)
-        for (uint32_t g = rank; g < count; g += 2u * nact) {
-            const uint32_t g2 = g + nact;
+        for (uint32_t g = lane; g < count; g += 128u) {
+            const uint32_t g2 = g + 64u;
             const bool two_leaves = g2 < count;
             const uint32_t own = wq.owner[g], own2 = two_leaves ? wq.owner[g2] : own;
             const PrimRecord pr = load_prim(wq.prims[own >> 1], wq.prim[g]);

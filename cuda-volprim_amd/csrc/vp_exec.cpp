@@ -158,6 +158,7 @@ RenderLaunch vp_resolve_launch(vp_context* ctx, const vp_launch_config* cfg, uin
     // a wavefront claims paths once 8 of its lanes are idle (measured best on
     // the scattering workload: 15.9 against 15.5 Msamples/s at 1)
     L.regen_min = std::max<uint32_t>(1u, std::min<uint32_t>(64u, c.regen_min ? c.regen_min : 8u));
+    L.lane_max = 64u;
     L.count_events = count;
     L.measure = measure;
     // the wavefront pipeline has no event-counting or measuring variant
@@ -177,6 +178,23 @@ RenderLaunch vp_resolve_launch(vp_context* ctx, const vp_launch_config* cfg, uin
         L.wf.grid_scatter = cus * static_cast<uint32_t>(os);
         L.wf.grid_shadow = cus * static_cast<uint32_t>(osh);
     }
+    return L;
+}
+
+// A launch below one path per lane is bound by latency: a path is a serial
+// chain of walks, set rebuilds and roulettes, so its paths are spread over as
+// many wavefronts as there are, whose other lanes help with the walks.  From
+// one path per lane on (262144 on 256 CUs) lane_max is 64, as before.  With at
+// least 1, 2, 4, 8 and 16 paths per wavefront: 64x64x2 scattering image 3.7,
+// 3.8, 4.1, 4.1, 5.2 ms (22.5 ms when every wavefront took 64), 157x83x3 of 97
+// Gaussians 0.84, 0.82, 0.78, 0.88, 0.97 (2.7), 192x128x2 cloud 51, 49, 45, 50,
+// 70 (290), so one path is enough.
+RenderLaunch vp_size_launch(RenderLaunch L, uint64_t paths) {
+    const uint64_t waves_per_block = L.block / 64u;
+    L.grid = static_cast<uint32_t>(
+        std::max<uint64_t>(1u, std::min<uint64_t>(L.grid, (paths + waves_per_block - 1) / waves_per_block)));
+    const uint64_t waves = L.grid * waves_per_block;
+    L.lane_max = static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>(64u, (paths + waves - 1) / waves)));
     return L;
 }
 
@@ -224,7 +242,7 @@ static vp_status vp_run_step_wf(vp_context* ctx, const RenderLaunch& L, uint64_t
     VP_HIP_TRY(hipMemcpyAsync(ctx->job_begin_dev, ctx->begin_pinned, sizeof(uint64_t) * max_jobs,
                               hipMemcpyHostToDevice, s));
     VP_HIP_TRY(hipMemcpyAsync(ctx->launch_desc, ctx->desc_pinned, sizeof(uint64_t) * 3, hipMemcpyHostToDevice, s));
-    VP_HIP_TRY(vp_launch_fill_u64(ctx->path_counter, vp::kClaimParts, 0ull, s));
+    VP_HIP_TRY(vp_launch_fill_u64(ctx->path_counter, vp::kClaimWords, 0ull, s));
     VP_HIP_TRY(vp_launch_fill_u64(ctx->job_done_dev, max_jobs, 0ull, s));
     VP_HIP_TRY(vp_wf_launch_init(ctx->wf, s));
     // Every replay advances each live path by two bounces or retires it, and
@@ -267,7 +285,7 @@ vp_status vp_run_step(vp_context* ctx, const RenderLaunch& L, uint32_t nslices, 
         VP_HIP_TRY(enqueue());
         return VP_OK;
     }
-    const uint64_t key[6] = {L.block, L.grid, (uint64_t(L.active_cap) << 8) | L.regen_min,
+    const uint64_t key[6] = {L.block, L.grid, (uint64_t(L.active_cap) << 16) | (L.lane_max << 8) | L.regen_min,
                              uint64_t(L.count_events) << 1 | uint64_t(L.measure), (uint64_t(max_jobs) << 32) | max_npix,
                              reinterpret_cast<uint64_t>(s)};
     if (!ctx->graph_exec || !std::equal(key, key + 6, ctx->graph_key)) {
@@ -417,7 +435,7 @@ vp_status vp_run_jobs(vp_context* ctx, std::vector<JobRun>& runs, const vp_launc
         }
         if (k == 0) break;
         VP_HIP_TRY(hipEventRecord(ctx->ev0, s));
-        st = vp_run_step(ctx, L, k, total, max_jobs, max_npix, false, s);
+        st = vp_run_step(ctx, vp_size_launch(L, total), k, total, max_jobs, max_npix, false, s);
         if (st != VP_OK) return st;
         VP_HIP_TRY(hipEventRecord(ctx->ev1, s));
         // the pinned staging is rewritten next round (and the accumulators

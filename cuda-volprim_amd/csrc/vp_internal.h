@@ -133,6 +133,10 @@ VP_HD uint32_t mega_slab_stride(uint32_t cap) { return (cap + 3u) & ~3u; }
 // own XCD's part first (so each XCD's L2 serves a narrower band of the
 // image), then from the others once its part is used up.
 constexpr uint32_t kClaimParts = 8;
+// Words between two parts' counters: a 128-byte line each, so the atomics of
+// different parts do not queue behind each other.
+constexpr uint32_t kClaimStride = 16;
+constexpr uint32_t kClaimWords = kClaimParts * kClaimStride;
 // Largest active-set capacity: the walks count set sizes in 16 bits.
 constexpr uint32_t kMaxActiveCap = 65535;
 
@@ -293,6 +297,7 @@ struct RenderLaunch {
     uint32_t grid;
     uint32_t active_cap;
     uint32_t regen_min;
+    uint32_t lane_max;  // megakernel: lanes of a wavefront that hold a path (vp_size_launch)
     int count_events;
     int measure;
     uint32_t pipeline;  // VP_PIPELINE_MEGAKERNEL or VP_PIPELINE_WAVEFRONT
@@ -324,6 +329,9 @@ vp_status vp_ensure_jobs(vp_context* ctx, uint32_t n);
 void vp_drop_graph(vp_context* ctx);
 RenderLaunch vp_resolve_launch(vp_context* ctx, const vp_launch_config* cfg, uint32_t active_cap, int count,
                                int measure);
+// L for a megakernel launch over `paths` paths: no more workgroups than have a
+// path for each wavefront, and the paths spread over all wavefronts.
+RenderLaunch vp_size_launch(RenderLaunch L, uint64_t paths);
 // One step over the first nslices entries of the pinned job table (capacity max_jobs).
 vp_status vp_run_step(vp_context* ctx, const RenderLaunch& L, uint32_t nslices, uint64_t total_paths,
                       uint32_t max_jobs, uint32_t max_npix, bool use_graph, hipStream_t s);

@@ -33,7 +33,7 @@ constexpr size_t kNoAllocAccumBytes = size_t(kNoAllocMaxPixels) * kAccumWords * 
 constexpr size_t kNoAllocTableBytes = 4096;
 constexpr size_t kNoAllocSlabBytes = size_t(112) << 20;
 constexpr size_t kNoAllocScratchBytes = kNoAllocAccumBytes + kNoAllocTableBytes + kNoAllocSlabBytes;
-static_assert(sizeof(JobDesc) + 4 * 8 + kClaimParts * 8 + kNumCounters * 8 <= kNoAllocTableBytes,
+static_assert(sizeof(JobDesc) + 4 * 8 + kClaimWords * 8 + kNumCounters * 8 <= kNoAllocTableBytes,
               "tables fit their block");
 
 __device__ __align__(256) unsigned char scratch[kNoAllocScratchBytes];
@@ -44,7 +44,7 @@ struct NoAllocLayout {
     JobDesc* job;
     uint64_t* job_begin;     // [1]
     uint64_t* launch_desc;   // [3]: job count, end and start of the path range
-    unsigned long long* path_counter;  // [kClaimParts]
+    unsigned long long* path_counter;  // [kClaimWords]
     unsigned long long* counters;  // [kNumCounters]
     uint32_t* slab;
 };
@@ -57,7 +57,7 @@ NoAllocLayout layout(void* base) {
     l.job_begin = reinterpret_cast<uint64_t*>(t + sizeof(JobDesc));
     l.launch_desc = l.job_begin + 1;
     l.path_counter = reinterpret_cast<unsigned long long*>(l.job_begin + 4);
-    l.counters = l.path_counter + kClaimParts;
+    l.counters = l.path_counter + kClaimWords;
     l.slab = reinterpret_cast<uint32_t*>(b + kNoAllocAccumBytes + kNoAllocTableBytes);
     return l;
 }
@@ -74,7 +74,7 @@ __global__ void k_noalloc_install(JobDesc J, JobDesc* job, uint64_t* job_begin, 
         launch_desc[1] = J.path_count;
         launch_desc[2] = 0;
     }
-    if (i < kClaimParts) path_counter[i] = 0ull;
+    for (uint32_t c = i; c < kClaimWords; c += blockDim.x) path_counter[c] = 0ull;
     if (i < static_cast<uint32_t>(kNumCounters)) counters[i] = 0ull;
 }
 
@@ -143,7 +143,7 @@ extern "C" vp_status vp_render_device_noalloc(vp_context* ctx, vp_scene* sc, vp_
     hipLaunchKernelGGL(k_noalloc_install, dim3(1), dim3(64), 0, s, J, lay.job, lay.job_begin, lay.launch_desc,
                        lay.path_counter, lay.counters);
     VP_HIP_TRY(hipGetLastError());
-    VP_HIP_TRY(vp_launch_render(L, lay.job, lay.job_begin, lay.launch_desc, lay.path_counter, lay.slab, lay.counters,
+    VP_HIP_TRY(vp_launch_render(vp_size_launch(L, J.path_count), lay.job, lay.job_begin, lay.launch_desc, lay.path_counter, lay.slab, lay.counters,
                                 s));
     VP_HIP_TRY(vp_launch_resolve_job(lay.job, 0, static_cast<uint32_t>(npix), s));
     if (stats) {

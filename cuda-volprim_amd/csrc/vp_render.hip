@@ -65,8 +65,10 @@ struct PathState {
 #endif
 
 // Argmin free flight over the entered primitives (sampling.cuh:372-412) with
-// the wave-shared leaf queue: every active lane of the wavefront walks its
-// own ray, and the queued leaves of all rays are shared out among the lanes.
+// the wave-shared leaf queue.  All 64 lanes of the wavefront call it: a lane
+// with a path (alive) walks its own ray, and the origin-set members and queued
+// leaves of all rays are shared out among all lanes, so a wavefront with few
+// paths left still evaluates them 64 at a time.
 // Each ray's running minimum is an LDS atomic minimum over float bits (all
 // candidates are >= 0), so the result does not depend on which lane handles
 // which leaf.  Candidates for the rebuild are recorded while t_entry is at
@@ -78,11 +80,13 @@ struct PathState {
 // 0); from there on it prunes at the running minimum like any other ray.
 // ts_origin is the minimum over the origin set; the result keeps it unless a
 // walk candidate is strictly smaller.
-__device__ __forceinline__ void argmin_walk_shared(const SceneView& sc, f3 o, f3 d, uint64_t key, uint32_t b,
-                                                   bool direct, const uint32_t* act, uint32_t na, float* act_exit,
-                                                   uint32_t* __restrict__ slab, uint32_t cap, const WaveQueue& wq,
-                                                   float& ts, uint32_t& nc, uint64_t dlimit, uint64_t& dacc) {
+__device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& sc, f3 o, f3 d, uint64_t key,
+                                                   uint32_t b, bool direct, const uint32_t* act, uint32_t na_path,
+                                                   float* act_exit, uint32_t* __restrict__ slab, uint32_t cap,
+                                                   const WaveQueue& wq, float& ts, uint32_t& nc, uint64_t dlimit,
+                                                   uint64_t& dacc) {
     const uint32_t lane = __lane_id();
+    const uint32_t na = alive ? na_path : 0u;
     lds_store3(wq.ro + 3 * lane, o);
     lds_store3(wq.rd + 3 * lane, d);
     wq.key[lane] = key;
@@ -91,7 +95,6 @@ __device__ __forceinline__ void argmin_walk_shared(const SceneView& sc, f3 o, f3
     wq.acc[lane] = 0ull;
     wq.ts[lane] = __float_as_uint(kTMax);
     wq.nc[lane] = 0u;
-    wave_sync();
     // The origin set first (sampling.cuh:356-370), for all lanes' rays
     // together: the wavefront's (member, lane) pairs are numbered through a
     // prefix sum of the set sizes and shared out over the lanes.  Per member:
@@ -99,39 +102,25 @@ __device__ __forceinline__ void argmin_walk_shared(const SceneView& sc, f3 o, f3
     // into the owner's running minimum, and at bounce 0 its chord into the
     // owner's direct-term optical depth; minima and fixed-point sums do not
     // depend on which lane adds what.  The owners' pointers and prefix sums
-    // sit in wq.tj and their lane ids in wq.list, both free here.  (Active
-    // sets of the megakernel are contiguous.)
+    // sit in wq.tj, free here.  (Active sets of the megakernel are
+    // contiguous.)
     {
-        const unsigned long long m0 = __builtin_amdgcn_ballot_w64(true);
-        const uint32_t rk = lanes_below(m0), nl = static_cast<uint32_t>(__popcll(m0));
-        uint32_t pre = 0, total = 0;
-        for (uint32_t bit = 0; bit < 16u; ++bit) {
-            const unsigned long long bm = __builtin_amdgcn_ballot_w64(((na >> bit) & 1u) != 0u);
-            pre += lanes_below(bm) << bit;
-            total += static_cast<uint32_t>(__popcll(bm)) << bit;
-        }
-        const uint32_t** set_of = reinterpret_cast<const uint32_t**>(wq.tj);  // [64] by rank
-        float** exit_of = reinterpret_cast<float**>(wq.tj) + 64;               // [64] by rank
-        uint32_t* pre_of = reinterpret_cast<uint32_t*>(wq.tj) + 4 * 64;       // [64] by rank
-        set_of[rk] = act;
-        exit_of[rk] = act_exit;
-        pre_of[rk] = pre;
-        wq.list[rk] = static_cast<uint8_t>(lane);
+        const uint32_t** set_of = reinterpret_cast<const uint32_t**>(wq.tj);  // [64]
+        float** exit_of = reinterpret_cast<float**>(wq.tj) + 64;               // [64]
+        uint32_t* pre_of = reinterpret_cast<uint32_t*>(wq.tj) + 4 * 64;       // [64]
+        uint32_t total;
+        const uint32_t pre = wave_prefix16(na, total);
+        set_of[lane] = act;
+        exit_of[lane] = act_exit;
+        pre_of[lane] = pre;
         wave_sync();
-        for (uint32_t g = rk; g < total; g += nl) {
-            // the owner: the last rank whose prefix is at most g
-            uint32_t lo = 0, hi = nl - 1u;
-            while (lo < hi) {
-                const uint32_t mid = (lo + hi + 1u) >> 1;
-                if (pre_of[mid] <= g) lo = mid;
-                else hi = mid - 1u;
-            }
-            const uint32_t ol = wq.list[lo], k = g - pre_of[lo];
-            const uint32_t i = set_of[lo][k];
+        for (uint32_t g = lane; g < total; g += 64u) {
+            const uint32_t ol = prefix_owner(pre_of, g), k = g - pre_of[ol];
+            const uint32_t i = set_of[ol][k];
             const PrimRecord pr = load_prim(wq.prims[ol], i);
             const f3 ro = lds_load3(wq.ro + 3 * ol), rd = lds_load3(wq.rd + 3 * ol);
             const InsideChord x = inside_chord(pr, ro, rd);
-            exit_of[lo][k] = x.t1;
+            exit_of[ol][k] = x.t1;
             const uint32_t mo = wq.meta[ol];
             const float tau = free_flight_tau(prim_uniform(wq.key[ol], mo & 0x7fffffffu, 0u, i));
             if (tau <= x.tau) {
@@ -146,9 +135,10 @@ __device__ __forceinline__ void argmin_walk_shared(const SceneView& sc, f3 o, f3
     const f3 inv = safe_inv(d), oi = o * inv;
     float tmax = direct && wq.acc[lane] < dlimit ? kTMax : ts_origin;
     Walk4 w = walk4_begin();
+    if (!alive) w.n = kWalkEnd;
     // the first thread of this wavefront, for the owners' candidate buffers
     const uint32_t gbase = blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
-    while (__ballot(w.n != kWalkEnd) != 0) {
+    while (__builtin_amdgcn_ballot_w64(w.n != kWalkEnd) != 0) {
         uint32_t count = 0;
         while (true) {
             const bool step = w.n != kWalkEnd;
@@ -165,8 +155,6 @@ __device__ __forceinline__ void argmin_walk_shared(const SceneView& sc, f3 o, f3
             if (__builtin_amdgcn_ballot_w64(!fits) != 0) break;
         }
         wave_sync();
-        const unsigned long long am = __builtin_amdgcn_ballot_w64(true);
-        const uint32_t nact = static_cast<uint32_t>(__popcll(am));
         // leaf phase in three passes, each at full width.  First the entry
         // tests' early rejects (crossing_setup): the leaves a ray may enter
         // move down to the front of the queue (an entry is only overwritten
@@ -177,10 +165,9 @@ __device__ __forceinline__ void argmin_walk_shared(const SceneView& sc, f3 o, f3
         // sampled, which ends inside the chord when the sampled depth is at
         // most the chord's.  Those leaves move down again with their sampled
         // depth, and the third pass inverts their flights into distances.
-        const uint32_t rk = lanes_below(am);
         uint32_t ne = 0;
-        for (uint32_t base = 0; base < count; base += nact) {
-            const uint32_t g = base + rk;
+        for (uint32_t base = 0; base < count; base += 64u) {
+            const uint32_t g = base + lane;
             bool may = false;
             uint32_t own = 0, prim = 0;
             if (g < count) {
@@ -201,8 +188,8 @@ __device__ __forceinline__ void argmin_walk_shared(const SceneView& sc, f3 o, f3
         }
         wave_sync();
         uint32_t nk = 0;
-        for (uint32_t base = 0; base < ne; base += nact) {
-            const uint32_t g = base + rk;
+        for (uint32_t base = 0; base < ne; base += 64u) {
+            const uint32_t g = base + lane;
             bool keep = false;
             uint32_t own = 0, prim = 0;
             float tau = 0.0f;
@@ -241,7 +228,7 @@ __device__ __forceinline__ void argmin_walk_shared(const SceneView& sc, f3 o, f3
             nk += static_cast<uint32_t>(__popcll(km));
         }
         wave_sync();
-        for (uint32_t g = rk; g < nk; g += nact) {
+        for (uint32_t g = lane; g < nk; g += 64u) {
             const uint32_t own = wq.owner[g];
             const f3 ro = lds_load3(wq.ro + 3 * own), rd = lds_load3(wq.rd + 3 * own);
             const PrimRecord pr = load_prim(wq.prims[own], wq.prim[g]);
@@ -269,12 +256,22 @@ __device__ __forceinline__ void argmin_walk_shared(const SceneView& sc, f3 o, f3
 // longer job table adds while the earlier ones drain) hand out every path
 // exactly once, without the retries a compare-and-swap on one shared counter
 // costs when paths are short.
-template <bool kCount>
+//
+// At most lane_max lanes of a wavefront hold a path (the host sets it so that
+// a launch with fewer paths than lanes spreads them over all its wavefronts).
+// The argmin and shadow walks are run by all 64 lanes of a wavefront together,
+// so lanes without a path (past lane_max, or at the end of a launch) work on
+// the rays of those that have one: a wavefront with two paths left evaluates
+// their members and leaves 64 at a time and shares out their walks.  Only the
+// timed build does so (kShared); the counting and the measuring build walk
+// each ray by its own lane.
+template <bool kCount, bool kMeasure>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VP_RENDER_WAVES_PER_EU)))
 k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begin,
          const uint64_t* __restrict__ launch_desc, unsigned long long* __restrict__ path_counter,
-         uint32_t* __restrict__ slab, uint32_t cap, uint32_t regen_min,
-         unsigned long long* __restrict__ counters, int measure) {
+         uint32_t* __restrict__ slab, uint32_t cap, uint32_t regen_min, uint32_t lane_max,
+         unsigned long long* __restrict__ counters) {
+    constexpr bool kShared = !kCount && !kMeasure;
     extern __shared__ __align__(16) uint32_t s_leafq[];  // [blockDim.x][kLeafRow]
     const uint32_t njobs = static_cast<uint32_t>(launch_desc[0]);
     const uint64_t total_paths = launch_desc[1];
@@ -289,103 +286,127 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
     const uint32_t bs = mega_slab_stride(cap);
     uint32_t* my = slab + static_cast<size_t>(gl) * kMegaSlabBuffers * bs;  // entry k of buffer b at my[b * bs + k]
     const LeafQueue lq = leaf_queue(s_leafq);
-    const WaveQueue wq = wave_queue(s_leafq);  // the same LDS, used by the MIS shadow walks
-    PathState st;
+    const WaveQueue wq = wave_queue(s_leafq);  // the same LDS, used by the wave-shared walks
+    PathState st{};
     bool alive = false;
-    bool exhausted = false;
+    bool exhausted = false;  // every part of the path range is used up (the same in all lanes)
     Ev<kCount> ev;
     ev.reset();
     uint32_t overflow = 0;
-    // The launch's paths in kClaimParts parts, part k claimed through
-    // path_counter[k]; a wavefront starts with the part of the XCD it runs on
-    // (the XCC_ID hardware register, bits 3:0), so each XCD's waves trace a
-    // narrower band of the image and its L2 holds more of what they read.
-    // Which lane traces which path changes no result.  parts_done: the parts
-    // this wavefront has found used up.
+    // The launch's paths in kClaimParts parts.  The first paths of part k are
+    // handed out without a counter: wavefront i of the workgroups with
+    // blockIdx % kClaimParts = k starts on its lane_max paths from i * lane_max
+    // (workgroups are dealt out to the XCDs in turn), so a launch with no more
+    // paths than that needs no atomics (each wavefront's 8 on the way out took
+    // 430 us of a 4096-path launch).  The rest of part k is claimed through
+    // path_counter[k * kClaimStride]; a wavefront starts with the part of the
+    // XCD it runs on (the XCC_ID hardware register, bits 3:0), so each XCD's
+    // waves trace a narrower band of the image and its L2 holds more of what
+    // they read.  Which lane traces which path changes no result.
+    // parts_done: the parts this wavefront has found used up.
     const uint32_t xcd = __builtin_amdgcn_s_getreg((3u << 11) | (0u << 6) | 20u) % kClaimParts;
     const uint64_t part = (total_paths - path_lo + kClaimParts - 1u) / kClaimParts;
+    const uint32_t waves_per_block = blockDim.x / 64u;
+    // paths of part k handed out at the start
+    auto part_static = [&](uint32_t k) -> uint64_t {
+        return static_cast<uint64_t>((gridDim.x + kClaimParts - 1u - k) / kClaimParts) * waves_per_block * lane_max;
+    };
     uint32_t parts_done = 0;
+    bool first = true;
+    const uint32_t claim_min = regen_min < lane_max ? regen_min : lane_max;
 
     while (true) {
         // ---- claim new paths for idle lanes: one atomic per wavefront and part tried ----
-        const bool want = !alive && !exhausted;
-        unsigned long long wmask = __ballot(want);
-        if (wmask && __popcll(wmask) < regen_min && __ballot(alive) != 0) wmask = 0;
-        if (wmask) {
-            const uint32_t leader = __ffsll(static_cast<long long>(wmask)) - 1;
-            unsigned long long base = 0, got = 0;
-            if (lane == leader) {
-                const unsigned long long n_want = static_cast<unsigned long long>(__popcll(wmask));
-                for (uint32_t t = 0; t < kClaimParts; ++t) {
-                    const uint32_t k = (xcd + t) % kClaimParts;
-                    if ((parts_done >> k) & 1u) continue;
-                    const uint64_t lo_k = path_lo + k * part;
-                    const uint64_t hi_k = lo_k + part < total_paths ? lo_k + part : total_paths;
-                    if (lo_k < hi_k) {
-                        const unsigned long long c =
-                            __hip_atomic_fetch_add(path_counter + k, n_want, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                        const uint64_t b = lo_k + c;
-                        if (b < hi_k) {
-                            base = b;
-                            got = hi_k - b < n_want ? hi_k - b : n_want;
-                            break;
-                        }
-                    }
-                    parts_done |= 1u << k;
-                }
+        const unsigned long long idle = __builtin_amdgcn_ballot_w64(!alive);
+        const uint32_t busy = 64u - static_cast<uint32_t>(__popcll(idle));
+        const uint32_t room = lane_max > busy ? lane_max - busy : 0u;
+        if (!exhausted && room != 0u && (room >= claim_min || busy == 0u)) {
+            const uint32_t leader = static_cast<uint32_t>(__builtin_ctzll(idle));
+            unsigned long long base = 0;
+            uint32_t got = 0;
+            if (first) {
+                const uint32_t k = blockIdx.x % kClaimParts;
+                const uint64_t lo_k = path_lo + k * part;
+                const uint64_t hi_k = lo_k + part < total_paths ? lo_k + part : total_paths;
+                base = lo_k + (static_cast<uint64_t>(blockIdx.x / kClaimParts) * waves_per_block +
+                               __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * lane_max;
+                if (base < hi_k) got = hi_k - base < lane_max ? static_cast<uint32_t>(hi_k - base) : lane_max;
+                first = false;
             }
-            base = __shfl(base, leader);
-            got = __shfl(got, leader);
-            parts_done = __builtin_amdgcn_readfirstlane(__shfl(parts_done, leader));
-            if (want) {
-                const unsigned long long lt = lane == 0 ? 0ull : (~0ull >> (64 - lane));
-                const uint64_t rank = static_cast<uint64_t>(__popcll(wmask & lt));
-                const uint64_t p = base + rank;
-                if (rank >= got) {
-                    // every part used up; a lane beyond a part's last paths
-                    // claims again next round
-                    if (got == 0) exhausted = true;
-                } else {
-                    // ---- path setup (raygen.cuh:72-113) ----
-                    const uint32_t j = find_job(job_begin, njobs, p);
-                    const JobDesc& J = jobs[j];
-                    if (path_begin(J, p - J.path_begin, st.o, st.d, st.rng, st.key, st.pix, st.sl)) {
-                        st.beta = mk(1.0f);
-                        st.L = mk(0.0f);
-                        st.bounce = 0;
-                        st.job = j;
-                        st.cur = 0;
-                        // origin-inside set (sampling.cuh:322-341) by point query
-                        uint32_t na = 0, ov = 0, visits = 0, tests = 0;
-                        const SceneView sc = J.scene;
-                        const f3 o = st.o;
-                        walk_point(sc, o, visits, [&](uint32_t prim) {
-                            ++tests;
-                            if (point_inside(load_prim(sc.prims, prim), o)) {
-                                // counters updated without a branch keep them in registers
-                                const bool fits = na < cap;
-                                if (fits) my[na * stride] = prim;
-                                na += fits ? 1u : 0u;
-                                overflow += fits ? 0u : 1u;
-                                ++ov;
+            if (got == 0u) {
+                const uint32_t leader = static_cast<uint32_t>(__builtin_ctzll(idle));
+                if (lane == leader) {
+                    for (uint32_t t = 0; t < kClaimParts; ++t) {
+                        const uint32_t k = (xcd + t) % kClaimParts;
+                        if ((parts_done >> k) & 1u) continue;
+                        const uint64_t lo_k = path_lo + k * part + part_static(k);
+                        const uint64_t end_k = path_lo + (k + 1u) * part;
+                        const uint64_t hi_k = end_k < total_paths ? end_k : total_paths;
+                        if (lo_k < hi_k) {
+                            const unsigned long long c =
+                                __hip_atomic_fetch_add(path_counter + k * kClaimStride,
+                                                       static_cast<unsigned long long>(room), __ATOMIC_RELAXED,
+                                                       __HIP_MEMORY_SCOPE_AGENT);
+                            const uint64_t b = lo_k + c;
+                            if (b < hi_k) {
+                                base = b;
+                                got = hi_k - b < room ? static_cast<uint32_t>(hi_k - b) : room;
+                                break;
                             }
-                        });
-                        st.na = na;
-                        ev.add(kCntNodeVisits, visits);
-                        ev.add(kCntVisitsPoint, visits);
-                        ev.add(kCntContain, tests);
-                        ev.add(kCntPaths);
-                        if (measure) atomicMax(&counters[kCntMaxOverlap], static_cast<unsigned long long>(ov));
-                        alive = true;
+                        }
+                        parts_done |= 1u << k;
                     }
+                }
+                base = __shfl(base, leader);
+                got = __builtin_amdgcn_readfirstlane(__shfl(got, leader));
+                parts_done = __builtin_amdgcn_readfirstlane(__shfl(parts_done, leader));
+            }
+            // every part used up: this wavefront claims no more
+            if (got == 0u) exhausted = true;
+            const uint32_t rank = lanes_below(idle);
+            if (!alive && rank < got) {
+                const uint64_t p = base + rank;
+                // ---- path setup (raygen.cuh:72-113) ----
+                const uint32_t j = find_job(job_begin, njobs, p);
+                const JobDesc& J = jobs[j];
+                if (path_begin(J, p - J.path_begin, st.o, st.d, st.rng, st.key, st.pix, st.sl)) {
+                    st.beta = mk(1.0f);
+                    st.L = mk(0.0f);
+                    st.bounce = 0;
+                    st.job = j;
+                    st.cur = 0;
+                    // origin-inside set (sampling.cuh:322-341) by point query
+                    uint32_t na = 0, ov = 0, visits = 0, tests = 0;
+                    const SceneView sc = J.scene;
+                    const f3 o = st.o;
+                    walk_point(sc, o, visits, [&](uint32_t prim) {
+                        ++tests;
+                        if (point_inside(load_prim(sc.prims, prim), o)) {
+                            // counters updated without a branch keep them in registers
+                            const bool fits = na < cap;
+                            if (fits) my[na * stride] = prim;
+                            na += fits ? 1u : 0u;
+                            overflow += fits ? 0u : 1u;
+                            ++ov;
+                        }
+                    });
+                    st.na = na;
+                    ev.add(kCntNodeVisits, visits);
+                    ev.add(kCntVisitsPoint, visits);
+                    ev.add(kCntContain, tests);
+                    ev.add(kCntPaths);
+                    if constexpr (kMeasure)
+                        atomicMax(&counters[kCntMaxOverlap], static_cast<unsigned long long>(ov));
+                    alive = true;
                 }
             }
         }
-        if (__ballot(alive) == 0) {
-            if (__ballot(!exhausted) == 0) break;
+        if (__builtin_amdgcn_ballot_w64(alive) == 0) {
+            if (exhausted) break;
             continue;
         }
-        if (!alive) continue;
+        if constexpr (!kShared)
+            if (!alive) continue;
 
         // ---- one bounce (raygen.cuh:115-208) ----
         const JobDesc& J = jobs[st.job];
@@ -398,37 +419,25 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         bool finish = false;
 
         // At bounce 0 the analytic direct term needs the transmittance of the
-        // camera ray itself, so the timed kernel integrates it during the
-        // argmin loops below (the walk then runs over the whole ray instead
+        // camera ray itself, so the timed and the measuring kernel integrate
+        // it during the argmin (the walk then runs over the whole ray instead
         // of stopping at the running minimum): the same chords, summed in the
         // same fixed point as transmittance() does.  The counting build
         // keeps the separate shadow walk, so its counts are per-ray work.
-        const bool direct = !kCount && b == 0;
+        const bool direct = !kCount && alive && b == 0;
         uint64_t dacc = 0;
         bool dfull = false;
 
-        // argmin over the origin set (sampling.cuh:356-370); the members'
-        // exits are kept for the rebuild.  The timed kernel does this for the
-        // whole wavefront inside argmin_walk_shared.
         float ts = kTMax;
+        // the origin-set members' exits, kept for the rebuild
         float* act_exit = reinterpret_cast<float*>(my + 5 * bs * stride);
-        if (kCount || measure) {
-            for (uint32_t k = 0; k < na; ++k) {
-                const uint32_t i = act[k * stride];
-                const PrimRecord pr = load_prim(sc.prims, i);
-                const InsideChord x = inside_chord(pr, o, d);
-                act_exit[k * stride] = x.t1;
-                const float tau = free_flight_tau(prim_uniform(st.key, b, 0u, i));
-                if (tau <= x.tau) ts = minf(ts, origin_flight(pr, o, d, x, tau));
-                if (direct && !dfull) dfull = tau_add(dacc, x.tau);
-            }
-        }
         ev.add(kCntArgActive, na);
         ev.add(kCntTrace);
-        // argmin over entered primitives (sampling.cuh:372-412) in one walk;
-        // primitives entered before the running minimum are kept as rebuild
-        // candidates (every primitive entered before the final minimum is
-        // among them, because the walk only prunes beyond the running one)
+        // argmin over the origin set (sampling.cuh:356-370) and over entered
+        // primitives (sampling.cuh:372-412) in one walk; primitives entered
+        // before the running minimum are kept as rebuild candidates (every
+        // primitive entered before the final minimum is among them, because
+        // the walk only prunes beyond the running one)
         uint32_t* cnd = my + 2 * bs * stride;
         uint32_t nc = 0;
         // the analytic direct term's factor and its roulette (a no-op unless
@@ -440,16 +449,26 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
             return shadow_rr(max3(kd), J.shadow_rr, st.key, 0u, 2u);
         };
         uint64_t dwalk = 0;
-        if (!kCount && !measure) {
+        if constexpr (kShared) {
             uint64_t dlimit = kTauLimitFixed;
             if (direct) {
                 f3 kd;
                 dlimit = direct_rr(kd).limit();
             }
-            argmin_walk_shared(sc, o, d, st.key, b, direct, act, na, act_exit, slab, cap, wq, ts, nc, dlimit, dwalk);
+            argmin_walk_shared(alive, sc, o, d, st.key, b, direct, act, na, act_exit, slab, cap, wq, ts, nc, dlimit,
+                               dwalk);
         } else {
+            for (uint32_t k = 0; k < na; ++k) {
+                const uint32_t i = act[k * stride];
+                const PrimRecord pr = load_prim(sc.prims, i);
+                const InsideChord x = inside_chord(pr, o, d);
+                act_exit[k * stride] = x.t1;
+                const float tau = free_flight_tau(prim_uniform(st.key, b, 0u, i));
+                if (tau <= x.tau) ts = minf(ts, origin_flight(pr, o, d, x, tau));
+                if (direct && !dfull) dfull = tau_add(dacc, x.tau);
+            }
             const f3 inv = safe_inv(d);
-            const bool prune = !measure && !direct;
+            const bool prune = !kMeasure;
             float tmax = prune ? ts : kTMax;
             uint32_t hits = 0, visits = 0, leaves = 0, accept = 0;
             walk_ray_q(sc, o, inv, tmax, visits, lq, [&](uint32_t prim) -> bool {
@@ -483,28 +502,40 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
             ev.add(kCntArgAccept, accept);
             ev.add(kCntNodeVisits, visits);
             ev.add(kCntLeafTests, leaves);
-            if (measure) atomicMax(&counters[kCntMaxHits], static_cast<unsigned long long>(hits));
+            if constexpr (kMeasure) atomicMax(&counters[kCntMaxHits], static_cast<unsigned long long>(hits));
         }
 
         const EnvView env = env_view(J.env);
         // analytic direct term at bounce 0 (raygen.cuh:148-160)
-        if (b == 0) {
+        if (alive && b == 0) {
             ev.add(kCntShadowRays);
             f3 kd;
             const ShadowRr drr = direct_rr(kd);
             uint64_t a;
             if constexpr (kCount) a = shadow_depth(sc, o, d, act, na, stride, lq, ev, drr.limit());
-            else a = measure ? (dfull ? kTauLimitFixed : dacc) : dwalk;
+            else if constexpr (kMeasure) a = dfull ? kTauLimitFixed : dacc;
+            else a = dwalk;
             const float T = shadow_rr_T(a, drr, depth_T(a));
             st.L = st.L + kd * T;
         }
 
-        if (ts >= kTMax) {
-            finish = true;  // escape: with NEE + analytic direct nothing more is added
-        } else {
+        // The vertex of a path that scatters: its active set, the next
+        // direction and the NEE shadow rays (rays a and b of MIS, or ray a of
+        // RIS; a limit of 0 is no ray), whose depths are summed below.
+        const bool vertex = alive && ts < kTMax;
+        if (alive && !vertex) finish = true;  // escape: with NEE + analytic direct nothing more is added
+        f3 x = mk(0.0f), wo = mk(0.0f), da = mk(0.0f), db = mk(0.0f), ka = mk(0.0f), kb = mk(0.0f);
+        uint32_t nn = 0;
+        uint64_t lim_a = 0, lim_b = 0;
+        bool has_a = false, has_b = false;
+        // the shadow rays' roulettes (a no-op unless J.shadow_rr > 0) are
+        // drawn before and again after the walks (the same values), so they
+        // hold no registers during them
+        auto nee_rr = [&](f3 k, uint32_t ray) { return shadow_rr(max3(k), J.shadow_rr, st.key, b, ray); };
+        if (vertex) {
             // rebuild the active set at the scatter point (sampling.cuh:422-458)
-            const f3 x = o + ts * d;
-            uint32_t nn = 0, ia = 0, visits = 0, rb_a = 0, rb_h = 0;
+            x = o + ts * d;
+            uint32_t ia = 0, visits = 0, rb_a = 0, rb_h = 0;
             auto push = [&](uint32_t v) {
                 const bool fits = nn < cap;
                 if (fits) nxt[nn * stride] = v;
@@ -544,7 +575,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
                 }
                 if (keep) push(c);
             };
-            if (nc <= cap && !measure) {
+            if (nc <= cap && !kMeasure) {
                 // candidates from the argmin walk, in ascending index order
                 float* ctj = reinterpret_cast<float*>(my + 3 * bs * stride);
                 float* cte = reinterpret_cast<float*>(my + 4 * bs * stride);
@@ -632,14 +663,14 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
             st.cur ^= 1u;
             st.na = nn;
             act = nxt;
-            if (measure) {
+            if constexpr (kMeasure) {
                 uint32_t ovl = 0, v2 = 0;
                 walk_point(sc, x, v2, [&](uint32_t c) { ovl += point_inside(load_prim(sc.prims, c), x) ? 1u : 0u; });
                 atomicMax(&counters[kCntMaxOverlap], static_cast<unsigned long long>(ovl));
             }
 
             float phase_pdf;
-            const f3 wo = phase_sample(J.hg, d, st.rng, &phase_pdf);
+            wo = phase_sample(J.hg, d, st.rng, &phase_pdf);
             ev.add(kCntScatter);
 
             // evaluate_albedo (sampling.cuh:257-283)
@@ -682,60 +713,49 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
                     if (lumy > 0.0f) {
                         ev.add(kCntShadowRays);
                         const float Wr = wsum * rcpf(static_cast<float>(J.ris_candidates));
-                        // the factor T multiplies; the roulette is drawn again
-                        // after the walk (the same values), so it holds no
-                        // registers during it
-                        const f3 ky = (base * (yenv * rcpf(lumy))) * Wr;
-                        uint64_t acc, acc_unused;
-                        {
-                            const uint64_t lim = shadow_rr(max3(ky), J.shadow_rr, st.key, b, 0u).limit();
-                            if constexpr (kCount) acc = shadow_depth(sc, x, ydir, act, nn, stride, lq, ev, lim);
-                            else transmittance_pool(sc, x, ydir, ydir, act, nn, stride, wq, lim, 0ull, acc, acc_unused,
-                                                    false);
-                        }
-                        const ShadowRr rr = shadow_rr(max3(ky), J.shadow_rr, st.key, b, 0u);
-                        st.L = st.L + ky * shadow_rr_T(acc, rr, depth_T(acc));
+                        // the factor T multiplies
+                        ka = (base * (yenv * rcpf(lumy))) * Wr;
+                        da = ydir;
+                        has_a = true;
                     }
                 }
             } else {
                 float apdf;
-                const f3 awo = phase_sample(J.hg, d, st.rng, &apdf);
-                const float pb_a = env_pdf(env, awo);
+                da = phase_sample(J.hg, d, st.rng, &apdf);
+                const float pb_a = env_pdf(env, da);
                 const float sa = apdf + pb_a;
                 const float wa = sa > 0.0f ? apdf / sa : 0.0f;
-                const f3 enva = env_lookup(env, awo);
+                const f3 enva = env_lookup(env, da);
 
                 float bpdf;
-                const f3 bwo = env_sample(env, st.rng, &bpdf);
-                const float ph_b = phase_eval(J.hg, d, bwo);
+                db = env_sample(env, st.rng, &bpdf);
+                const float ph_b = phase_eval(J.hg, d, db);
                 const float sb = bpdf + ph_b;
                 const float wb = sb > 0.0f ? bpdf / sb : 0.0f;
-                const f3 envb = env_lookup(env, bwo);
+                const f3 envb = env_lookup(env, db);
                 ev.add(kCntShadowRays, 2);
-                // the factors the two transmittances multiply, and each ray's
-                // roulette (a no-op unless J.shadow_rr > 0); the roulettes
-                // are drawn again after the walks (the same values), so they
-                // hold no registers during them
-                const f3 ka = (base * enva) * wa;
-                const f3 kb = (((base * envb) * wb) * ph_b) * rcpf(bpdf);
-                // the counting build walks the two rays with separate calls,
-                // so its counts are per-ray work
-                uint64_t acc_a, acc_b;
-                {
-                    const uint64_t lim_a = shadow_rr(max3(ka), J.shadow_rr, st.key, b, 0u).limit();
-                    const uint64_t lim_b = shadow_rr(max3(kb), J.shadow_rr, st.key, b, 1u).limit();
-                    if constexpr (kCount) {
-                        acc_a = shadow_depth(sc, x, awo, act, nn, stride, lq, ev, lim_a);
-                        acc_b = shadow_depth(sc, x, bwo, act, nn, stride, lq, ev, lim_b);
-                    } else {
-                        transmittance_pool(sc, x, awo, bwo, act, nn, stride, wq, lim_a, lim_b, acc_a, acc_b);
-                    }
-                }
-                const float Ta = shadow_rr_T(acc_a, shadow_rr(max3(ka), J.shadow_rr, st.key, b, 0u), depth_T(acc_a));
-                const float Tb = shadow_rr_T(acc_b, shadow_rr(max3(kb), J.shadow_rr, st.key, b, 1u), depth_T(acc_b));
-                st.L = st.L + ka * Ta;
-                st.L = st.L + kb * Tb;
+                // the factors the two transmittances multiply
+                ka = (base * enva) * wa;
+                kb = (((base * envb) * wb) * ph_b) * rcpf(bpdf);
+                has_a = has_b = true;
             }
+            if (has_a) lim_a = nee_rr(ka, 0u).limit();
+            if (has_b) lim_b = nee_rr(kb, 1u).limit();
+        }
+
+        // the shadow rays' depths (the counting and the measuring build walk
+        // them one by one, so the former's counts are per-ray work)
+        uint64_t acc_a = 0, acc_b = 0;
+        if constexpr (kShared) {
+            transmittance_pool(sc, x, da, db, act, nn, wq, lim_a, lim_b, acc_a, acc_b);
+        } else {
+            if (has_a) acc_a = shadow_depth(sc, x, da, act, nn, stride, lq, ev, lim_a);
+            if (has_b) acc_b = shadow_depth(sc, x, db, act, nn, stride, lq, ev, lim_b);
+        }
+
+        if (vertex) {
+            if (has_a) st.L = st.L + ka * shadow_rr_T(acc_a, nee_rr(ka, 0u), depth_T(acc_a));
+            if (has_b) st.L = st.L + kb * shadow_rr_T(acc_b, nee_rr(kb, 1u), depth_T(acc_b));
 
             // russian_roulette (path_stages.cuh:25-37) and guards (raygen.cuh:191-204)
             if (b >= J.rr_depth) {
@@ -970,6 +990,13 @@ __global__ void k_prim(int fn, const PrimRecord* __restrict__ rec, const float* 
     out[i] = r;
 }
 
+using RenderKernel = void (*)(const JobDesc*, const uint64_t*, const uint64_t*, unsigned long long*, uint32_t*,
+                              uint32_t, uint32_t, uint32_t, unsigned long long*);
+RenderKernel render_kernel(int count_events, int measure) {
+    if (count_events) return measure ? k_render<true, true> : k_render<true, false>;
+    return measure ? k_render<false, true> : k_render<false, false>;
+}
+
 inline uint32_t cdiv(uint64_t a, uint32_t b) { return static_cast<uint32_t>((a + b - 1) / b); }
 
 }  // namespace
@@ -979,18 +1006,15 @@ using namespace vp;
 
 // One persistent render launch over a job table (device pointers): the
 // kernel claims the paths from launch_desc[2] below launch_desc[1], in
-// kClaimParts parts with one counter each (counter[0 .. kClaimParts), zero at
+// kClaimParts parts with one counter each (counter[0 .. kClaimWords), zero at
 // the start).
 hipError_t vp_launch_render(const RenderLaunch& L, const JobDesc* jobs, const uint64_t* job_begin,
                             const uint64_t* launch_desc, unsigned long long* counter, uint32_t* slab,
                             unsigned long long* counters, hipStream_t s) {
     const size_t lds = leaf_queue_bytes(L.block);
-    if (L.count_events)
-        hipLaunchKernelGGL(k_render<true>, dim3(L.grid), dim3(L.block), lds, s, jobs, job_begin, launch_desc, counter,
-                           slab, L.active_cap, L.regen_min, counters, L.measure);
-    else
-        hipLaunchKernelGGL(k_render<false>, dim3(L.grid), dim3(L.block), lds, s, jobs, job_begin, launch_desc, counter,
-                           slab, L.active_cap, L.regen_min, counters, L.measure);
+    const auto k = render_kernel(L.count_events, L.measure);
+    hipLaunchKernelGGL(k, dim3(L.grid), dim3(L.block), lds, s, jobs, job_begin, launch_desc, counter, slab,
+                       L.active_cap, L.regen_min, L.lane_max, counters);
     return hipGetLastError();
 }
 
@@ -1000,7 +1024,7 @@ hipError_t vp_launch_render(const RenderLaunch& L, const JobDesc* jobs, const ui
 // and path total come from ctx->launch_desc.
 hipError_t vp_launch_step(vp_context* ctx, const RenderLaunch& L, uint32_t max_jobs, uint32_t max_npix,
                           hipStream_t s) {
-    hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, s, ctx->path_counter, kClaimParts, 0ull);
+    hipLaunchKernelGGL(k_fill_u64, dim3(cdiv(kClaimWords, 64)), dim3(64), 0, s, ctx->path_counter, kClaimWords, 0ull);
     const hipError_t e = vp_launch_render(L, ctx->jobs_dev, ctx->job_begin_dev, ctx->launch_desc, ctx->path_counter,
                                           ctx->slab, ctx->counters, s);
     if (e != hipSuccess) return e;
@@ -1032,10 +1056,8 @@ int vp_render_occupancy(uint32_t block, uint32_t, int count_events, int* blocks_
     int nb = 0;
     hipError_t e;
     const size_t lds = leaf_queue_bytes(block);
-    if (count_events)
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(k_render<true>), block, lds);
-    else
-        e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, reinterpret_cast<const void*>(k_render<false>), block, lds);
+    e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
+        &nb, reinterpret_cast<const void*>(render_kernel(count_events, 0)), block, lds);
     *blocks_per_cu = nb > 0 ? nb : 1;
     return e == hipSuccess ? 0 : -1;
 }

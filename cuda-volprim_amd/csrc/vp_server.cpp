@@ -289,10 +289,10 @@ void server_loop(vp_server* S) {
                 if (hipStreamWaitEvent(S->ks[i], S->install_ev, 0) != hipSuccess ||
                     hipMemcpyAsync(S->desc_dev + 4 * i, d, 4 * sizeof(uint64_t), hipMemcpyHostToDevice, S->ks[i]) !=
                         hipSuccess ||
-                    hipMemcpyAsync(S->counter + vp::kClaimParts * i, S->zeros,
-                                   vp::kClaimParts * sizeof(unsigned long long), hipMemcpyHostToDevice,
+                    hipMemcpyAsync(S->counter + vp::kClaimWords * i, S->zeros,
+                                   vp::kClaimWords * sizeof(unsigned long long), hipMemcpyHostToDevice,
                                    S->ks[i]) != hipSuccess ||
-                    vp_launch_render(S->L, S->jobs_dev, S->begin_dev, S->desc_dev + 4 * i, S->counter + vp::kClaimParts * i,
+                    vp_launch_render(vp_size_launch(S->L, S->total - S->snap), S->jobs_dev, S->begin_dev, S->desc_dev + 4 * i, S->counter + vp::kClaimWords * i,
                                      S->slab[i],
                                      ctx->counters, S->ks[i]) != hipSuccess ||
                     hipEventRecord(S->kev[i], S->ks[i]) != hipSuccess) {
@@ -456,7 +456,7 @@ vp_status vp_server_create(vp_context* ctx, const vp_server_config* cfg, vp_serv
     bool ok = hipMalloc(&S->jobs_dev, sizeof(vp::JobDesc) * kServerTable) == hipSuccess &&
               hipMalloc(&S->begin_dev, sizeof(uint64_t) * kServerTable) == hipSuccess &&
               hipMalloc(&S->done_dev, sizeof(unsigned long long) * kServerTable) == hipSuccess &&
-              hipMalloc(&S->counter, 2 * vp::kClaimParts * sizeof(unsigned long long)) == hipSuccess &&
+              hipMalloc(&S->counter, 2 * vp::kClaimWords * sizeof(unsigned long long)) == hipSuccess &&
               hipMalloc(&S->desc_dev, 8 * sizeof(uint64_t)) == hipSuccess &&
               hipMalloc(&S->slab[0], slab_words * sizeof(uint32_t)) == hipSuccess &&
               hipMalloc(&S->slab[1], slab_words * sizeof(uint32_t)) == hipSuccess;
