@@ -280,12 +280,13 @@ constexpr float kExpHalfExtent2 = 0x1.6c0504p-7f;
 struct InsideChord {
     float t1, tau;
 };
-VP_HD InsideChord inside_chord(const PrimRecord& pr, f3 o, f3 d) {
+// With p the origin in the primitive's frame, pp = |p|^2 and e() = e^(-pp/2),
+// which a caller that tests several directions from one origin evaluates once.
+template <typename Exp>
+VP_HD InsideChord inside_chord_from(const PrimRecord& pr, f3 p, float pp, f3 d, Exp&& e) {
     const f3 w = to_local_dir(pr, d);
-    const f3 p = to_local_pos(pr, o);
     const float a = length2(w);
     const float b = dot(p, w);
-    const float pp = length2(p);
     const float c = pp - kExtent2;
     const float disc = fmaf_(-a, c, b * b);
     const float sq = sqrtf_(disc);
@@ -295,10 +296,15 @@ VP_HD InsideChord inside_chord(const PrimRecord& pr, f3 o, f3 d) {
     r.tau = 0.0f;
     if (r.t1 > kSegMin && r.t1 < kTMax) {
         const float far = (kExpHalfExtent2 * (sq * a_inv)) * chord_poly_(minf(disc * a_inv, kExtent2));
-        const float near = (expf_(-0.5f * pp) * (b * a_inv)) * chord_poly_(minf((b * b) * a_inv, kExtent2));
+        const float near = (e() * (b * a_inv)) * chord_poly_(minf((b * b) * a_inv, kExtent2));
         r.tau = maxf((pr.mass * pr.dnf) * (far - near), 0.0f);
     }
     return r;
+}
+VP_HD InsideChord inside_chord(const PrimRecord& pr, f3 o, f3 d) {
+    const f3 p = to_local_pos(pr, o);
+    const float pp = length2(p);
+    return inside_chord_from(pr, p, pp, d, [&]() { return expf_(-0.5f * pp); });
 }
 
 // Free flight from an origin inside a primitive (argmin over the origin set,

@@ -64,12 +64,12 @@ __device__ __forceinline__ void wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
-// Exclusive prefix sum over the wavefront's 64 lanes of v < 2^16, from one
-// ballot per bit; total receives the sum.
-__device__ __forceinline__ uint32_t wave_prefix16(uint32_t v, uint32_t& total) {
+// Exclusive prefix sum over the wavefront's 64 lanes of v (every lane active),
+// from one ballot per bit in use; total receives the sum.
+__device__ __forceinline__ uint32_t wave_prefix(uint32_t v, uint32_t& total) {
     uint32_t pre = 0;
     total = 0;
-    for (uint32_t bit = 0; bit < 16u; ++bit) {
+    for (uint32_t bit = 0; __builtin_amdgcn_ballot_w64((v >> bit) != 0u) != 0ull; ++bit) {
         const unsigned long long bm = __builtin_amdgcn_ballot_w64(((v >> bit) & 1u) != 0u);
         pre += lanes_below(bm) << bit;
         total += static_cast<uint32_t>(__popcll(bm)) << bit;
@@ -670,57 +670,19 @@ __device__ __forceinline__ bool wave_steal(const WaveQueue& wq, bool idle, bool 
 // the tau = 88 saturation, or a shadow-roulette threshold; multiples of
 // 2^16); a limit of 0 is a ray that is not walked.  acc_a and acc_b receive
 // the fixed-point depths.
-__device__ __forceinline__ void transmittance_pool(const SceneView& s, f3 o, f3 da, f3 db, const uint32_t* act,
-                                                   uint32_t na_path, const WaveQueue& wq, uint64_t lim_a,
-                                                   uint64_t lim_b, uint64_t& acc_a, uint64_t& acc_b) {
+// wq.ro, wq.prims, wq.rd and wq.acc hold the rays' origins, primitive arrays,
+// directions and the depths of their origin sets.
+__device__ __forceinline__ void shadow_walks(const SceneView& s, const WaveQueue& wq, uint64_t lim_a, uint64_t lim_b,
+                                             uint64_t& acc_a, uint64_t& acc_b) {
     const uint32_t lane = __lane_id();
-    const uint32_t na = (lim_a | lim_b) != 0ull ? na_path : 0u;
-    lds_store3(wq.ro + 3 * lane, o);
-    wq.prims[lane] = s.prims;
     wq.nodes[lane] = s.w4;
     wq.nn[lane] = s.w4_levels | (s.w4_half << 8);
-    lds_store3(wq.rd + 3 * (2 * lane), da);
-    lds_store3(wq.rd + 3 * (2 * lane + 1), db);
-    wq.acc[2 * lane] = 0ull;
-    wq.acc[2 * lane + 1] = 0ull;
     wq.lim[2 * lane] = static_cast<uint32_t>(lim_a >> 16);
     wq.lim[2 * lane + 1] = static_cast<uint32_t>(lim_b >> 16);
     // a ray is done once its depth reaches its limit
     auto reached = [&](uint32_t r) -> bool {
         return wq.acc[r] >= (static_cast<unsigned long long>(wq.lim[r]) << 16);
     };
-    // Chords of the origin set (every member's optical depth from the origin
-    // to its exit), for all lanes' rays together: the wavefront's (member,
-    // lane) pairs are numbered through a prefix sum of the set sizes and
-    // shared out over the lanes, so the loop runs sum(na) / 64 times
-    // instead of max(na).  Each chord goes into its ray's fixed-point sum; a
-    // sum that passes the tau = 88 limit gives T = 0 however far it passes,
-    // as in transmittance().  The owners' set pointers and prefix sums sit in
-    // wq.tj, free until the walks start.
-    {
-        static_assert(kWaveQ * sizeof(float) >= 64 * (sizeof(void*) + sizeof(uint32_t)),
-                      "the shared queue must hold the origin-set tables");
-        const uint32_t** set_of = reinterpret_cast<const uint32_t**>(wq.tj);  // [64]
-        uint32_t* pre_of = reinterpret_cast<uint32_t*>(wq.tj) + 2 * 64;     // [64]
-        uint32_t total;
-        const uint32_t pre = wave_prefix16(na, total);
-        set_of[lane] = act;
-        pre_of[lane] = pre;
-        wave_sync();
-        for (uint32_t g = lane; g < total; g += 64u) {
-            const uint32_t ol = prefix_owner(pre_of, g);
-            const PrimRecord pr = load_prim(wq.prims[ol], set_of[ol][g - pre_of[ol]]);
-            const f3 xo = lds_load3(wq.ro + 3 * ol);
-            if (wq.lim[2 * ol] != 0u) {
-                const float ta = inside_chord(pr, xo, lds_load3(wq.rd + 3 * (2 * ol))).tau;
-                if (ta > 0.0f) atomicAdd(&wq.acc[2 * ol], tau_fixed(ta));
-            }
-            if (wq.lim[2 * ol + 1] != 0u) {
-                const float tb = inside_chord(pr, xo, lds_load3(wq.rd + 3 * (2 * ol + 1))).tau;
-                if (tb > 0.0f) atomicAdd(&wq.acc[2 * ol + 1], tau_fixed(tb));
-            }
-        }
-    }
     wave_sync();
     const bool full_a = reached(2 * lane);
     const bool full_b = reached(2 * lane + 1);

@@ -116,13 +116,16 @@ static_assert(sizeof(JobDesc) % 128 == 0, "job-table entries fill whole cache li
 // buffer of rebuild candidates, each of the active-set capacity.
 constexpr uint32_t kSlabBuffers = 3;
 // Per-lane slab of the megakernel, buffers of the active-set capacity:
-//   0, 1  active sets (ping-pong)
+//   0, 1  the active set, and (timed kernel) its members' exit distances along
+//         the current ray in the other one; the rebuild swaps their roles
 //   2     rebuild candidates (stored primitive index)
 //   3, 4  their entry and exit distances along the ray (float bits)
-//   5     exit distance of each member of the current active set along the
-//         current ray
-// The argmin computes the values of 3, 4 and 5 anyway, so the rebuild only
-// compares them with the scatter distance.
+//   5     exit distances of the active set's members in the counting and the
+//         measuring kernel, whose rebuild writes the other set buffer while it
+//         reads them
+// The argmin computes the values of 3, 4 and the exits anyway, so the rebuild
+// only compares them with the scatter distance.  Between two argmins the timed
+// kernel keeps the members' albedo terms (a float4 each) in 2 to 5.
 constexpr uint32_t kMegaSlabBuffers = 6;
 // Words between the megakernel's slab buffers: the capacity rounded up to a
 // multiple of 4, so every buffer starts 16-byte aligned and can be read four

@@ -57,6 +57,7 @@ struct PathState {
     Pcg32 rng;
     uint64_t key;
     uint32_t bounce, job, na, cur, pix, sl;
+    float ts_set;  // minimum free flight over the active set (timed kernel, bounces > 0)
 };
 
 // Minimum waves per SIMD the register allocator targets for the megakernel.
@@ -82,34 +83,35 @@ struct PathState {
 // walk candidate is strictly smaller.
 __device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& sc, f3 o, f3 d, uint64_t key,
                                                    uint32_t b, bool direct, const uint32_t* act, uint32_t na_path,
-                                                   float* act_exit, uint32_t* __restrict__ slab, uint32_t cap,
-                                                   const WaveQueue& wq, float& ts, uint32_t& nc, uint64_t dlimit,
-                                                   uint64_t& dacc) {
+                                                   float* act_exit, float ts_set, uint32_t* __restrict__ slab,
+                                                   uint32_t cap, const WaveQueue& wq, float& ts, uint32_t& nc,
+                                                   uint64_t dlimit, uint64_t& dacc) {
     const uint32_t lane = __lane_id();
-    const uint32_t na = alive ? na_path : 0u;
+    const uint32_t na = direct ? na_path : 0u;
     lds_store3(wq.ro + 3 * lane, o);
     lds_store3(wq.rd + 3 * lane, d);
     wq.key[lane] = key;
     wq.prims[lane] = sc.prims;
     wq.meta[lane] = b | (direct ? 0x80000000u : 0u);
     wq.acc[lane] = 0ull;
-    wq.ts[lane] = __float_as_uint(kTMax);
+    wq.ts[lane] = __float_as_uint(direct ? kTMax : ts_set);
     wq.nc[lane] = 0u;
-    // The origin set first (sampling.cuh:356-370), for all lanes' rays
-    // together: the wavefront's (member, lane) pairs are numbered through a
-    // prefix sum of the set sizes and shared out over the lanes.  Per member:
-    // its exit (kept in the owner's slab for the rebuild), its free flight
-    // into the owner's running minimum, and at bounce 0 its chord into the
+    // The origin set (sampling.cuh:356-370) of a path at bounce 0; from then
+    // on the last vertex's pass over the set has evaluated it (vertex_members)
+    // and ts_set is its minimum.  The wavefront's (member, lane) pairs are
+    // numbered through a prefix sum of the set sizes and shared out over the
+    // lanes.  Per member: its exit (kept in the owner's slab for the rebuild),
+    // its free flight into the owner's running minimum, and its chord into the
     // owner's direct-term optical depth; minima and fixed-point sums do not
     // depend on which lane adds what.  The owners' pointers and prefix sums
     // sit in wq.tj, free here.  (Active sets of the megakernel are
     // contiguous.)
-    {
+    if (__builtin_amdgcn_ballot_w64(na != 0u) != 0ull) {
         const uint32_t** set_of = reinterpret_cast<const uint32_t**>(wq.tj);  // [64]
         float** exit_of = reinterpret_cast<float**>(wq.tj) + 64;               // [64]
         uint32_t* pre_of = reinterpret_cast<uint32_t*>(wq.tj) + 4 * 64;       // [64]
         uint32_t total;
-        const uint32_t pre = wave_prefix16(na, total);
+        const uint32_t pre = wave_prefix(na, total);
         set_of[lane] = act;
         exit_of[lane] = act_exit;
         pre_of[lane] = pre;
@@ -121,13 +123,12 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& 
             const f3 ro = lds_load3(wq.ro + 3 * ol), rd = lds_load3(wq.rd + 3 * ol);
             const InsideChord x = inside_chord(pr, ro, rd);
             exit_of[ol][k] = x.t1;
-            const uint32_t mo = wq.meta[ol];
-            const float tau = free_flight_tau(prim_uniform(wq.key[ol], mo & 0x7fffffffu, 0u, i));
+            const float tau = free_flight_tau(prim_uniform(wq.key[ol], wq.meta[ol] & 0x7fffffffu, 0u, i));
             if (tau <= x.tau) {
                 const float t = origin_flight(pr, ro, rd, x, tau);
                 atomicMin(&wq.ts[ol], t == 0.0f ? 0u : __float_as_uint(t));
             }
-            if ((mo >> 31) != 0u && x.tau > 0.0f) atomicAdd(&wq.acc[ol], tau_fixed(x.tau));
+            if (x.tau > 0.0f) atomicAdd(&wq.acc[ol], tau_fixed(x.tau));
         }
     }
     wave_sync();
@@ -243,6 +244,245 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& 
     ts = wmin < ts_origin ? wmin : ts_origin;
     nc = wq.nc[lane];
     dacc = wq.acc[lane];
+}
+
+// ---- the vertex stage of the timed kernel, all lanes of a wavefront together ----
+//
+// Slab buffers of a path at a vertex (kMegaSlabBuffers of bs words each): its
+// active set in buffer cur, the members' exits along the ray in the other set
+// buffer, cur ^ 1, and the ray's candidates in 2 (index), 3 and 4 (entry and
+// exit).  The rebuild compacts the members and candidates that contain the
+// vertex in place (buffers cur and 2) and merges them into buffer cur ^ 1,
+// which becomes the active set; the pass over its members then writes their
+// albedo terms over buffers 2 to 5 and their exits along the next ray into the
+// old set's buffer.
+
+// Words of the slab before lane own's buffers (gbase: the wavefront's first thread).
+__device__ __forceinline__ uint32_t* slab_of(uint32_t* slab, uint32_t gbase, uint32_t own, uint32_t bs) {
+    return slab + static_cast<size_t>(gbase + own) * kMegaSlabBuffers * bs;
+}
+
+// Lists longer than this are merged by their own lane: the merge below scans
+// a path's kept candidates once per item.
+constexpr uint32_t kRebuildScanMax = 1024;
+
+// The active sets at the scatter points (sampling.cuh:422-458) of the lanes
+// with a vertex (part): a member stays while ts <= its exit; an entered
+// candidate joins if its entry <= ts <= its exit; the set keeps ascending
+// stored index, and the first cap of it are kept.  Both steps run over the
+// wavefront's flattened items (members, then candidates, of every lane), 64
+// at a time: first the tests, compacting what is kept within each path's
+// buffers, then each kept item's position in the merged set, which is the
+// number of kept members and candidates below it: a member's rank or a binary
+// search among the members (ascending), plus a scan of the candidates (in the
+// order the walk found them).  A per-lane loop over its own lists waited on a
+// load per entry and ran as long as the wavefront's longest list: 7 to 13 % of
+// the dense scenes' and 11 % of a preview's time.
+__device__ __forceinline__ uint32_t rebuild_shared(bool part, uint32_t na, uint32_t nc, uint32_t cur, float ts,
+                                                   uint32_t* __restrict__ slab, uint32_t cap, const WaveQueue& wq,
+                                                   uint32_t& overflow) {
+    const uint32_t lane = __lane_id();
+    const uint32_t gbase = blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
+    const uint32_t bs = mega_slab_stride(cap);
+    // tables in wq.tj, 64 words each
+    uint32_t* pre_of = reinterpret_cast<uint32_t*>(wq.tj);
+    uint32_t* na_of = pre_of + 64;        // members of the list being flattened | set buffer << 31
+    uint32_t* kept_of = pre_of + 128;     // [2][64] kept members, kept candidates
+    float* ts_of = reinterpret_cast<float*>(pre_of + 256);
+    static_assert(kWaveQ >= 320, "the rebuild's tables must fit in wq.tj");
+    uint32_t total;
+    pre_of[lane] = wave_prefix(part ? na + nc : 0u, total);
+    na_of[lane] = na | (cur << 31);
+    kept_of[lane] = 0u;
+    kept_of[64 + lane] = 0u;
+    ts_of[lane] = ts;
+    wave_sync();
+    for (uint32_t base = 0; base < total; base += 64u) {
+        const uint32_t g = base + lane;
+        const uint32_t own = prefix_owner(pre_of, g), p0 = pre_of[own], k = g - p0;
+        const uint32_t meta = na_of[own], n = meta & 0x7fffffffu, set = (meta >> 31) * bs;
+        uint32_t* mine = slab_of(slab, gbase, own, bs);
+        const bool member = k < n;
+        const uint32_t kc = k - n;
+        bool keep = false;
+        uint32_t id = 0;
+        if (g < total) {
+            const float t = ts_of[own];
+            id = mine[member ? set + k : 2u * bs + kc];
+            const float t1 = __uint_as_float(mine[member ? bs - set + k : 4u * bs + kc]);
+            const float t0 = member ? 0.0f : __uint_as_float(mine[3u * bs + kc]);
+            keep = t0 >= 0.0f && (member || t0 <= t) && t <= t1;
+        }
+        const unsigned long long km = __builtin_amdgcn_ballot_w64(keep && member);
+        const unsigned long long kc_m = __builtin_amdgcn_ballot_w64(keep && !member);
+        // the lanes of this round with the same owner start at p0 - base
+        const unsigned long long seg = p0 > base ? ~0ull << (p0 - base) : ~0ull;
+        if (keep) {
+            uint32_t* kept = kept_of + (member ? own : 64u + own);
+            const uint32_t pos = *kept + lanes_below((member ? km : kc_m) & seg);
+            atomicAdd(kept, 1u);
+            mine[(member ? set : 2u * bs) + pos] = id;
+        }
+        wave_sync();
+    }
+    const uint32_t mm = kept_of[lane], mc = kept_of[64 + lane];
+    wave_sync();
+    pre_of[lane] = wave_prefix(mm + mc, total);
+    wave_sync();
+    // a candidate that is also a member (an origin the rounding puts outside
+    // a member's bound can enter it again) would be counted twice
+    bool serial = mc > kRebuildScanMax;
+    if (__builtin_amdgcn_ballot_w64(serial) == 0ull) {
+        for (uint32_t g = lane; g < total; g += 64u) {
+            const uint32_t own = prefix_owner(pre_of, g), k = g - pre_of[own];
+            const uint32_t set = (na_of[own] >> 31) * bs, nm = kept_of[own], nk = kept_of[64 + own];
+            uint32_t* mine = slab_of(slab, gbase, own, bs);
+            const uint32_t* cand = mine + 2u * bs;
+            const bool member = k < nm;
+            const uint32_t id = member ? mine[set + k] : cand[k - nm];
+            uint32_t below = 0;
+            for (uint32_t j = 0; j < nk; j += 4u) {
+                const uint4 c = *reinterpret_cast<const uint4*>(cand + j);
+                below += (c.x < id ? 1u : 0u) + (j + 1u < nk && c.y < id ? 1u : 0u) +
+                         (j + 2u < nk && c.z < id ? 1u : 0u) + (j + 3u < nk && c.w < id ? 1u : 0u);
+            }
+            uint32_t lo = k;
+            if (!member) {
+                lo = 0;
+                uint32_t hi = nm;
+                while (lo < hi) {
+                    const uint32_t mid = (lo + hi) >> 1;
+                    if (mine[set + mid] < id) lo = mid + 1u;
+                    else hi = mid;
+                }
+                if (lo < nm && mine[set + lo] == id) serial = true;
+            }
+            const uint32_t pos = lo + below;
+            if (pos < cap) mine[bs - set + pos] = id;
+        }
+    }
+    uint32_t nn = mm + mc;
+    if (__builtin_amdgcn_ballot_w64(serial) != 0ull) {
+        // each lane sorts its kept candidates and merges them with its kept
+        // members, an index that is in both once
+        wave_sync();
+        uint32_t* mine = slab_of(slab, gbase, lane, bs);
+        const uint32_t* set = mine + cur * bs;
+        uint32_t* out = mine + (cur ^ 1u) * bs;
+        uint32_t* cand = mine + 2u * bs;
+        for (uint32_t i = 1; i < mc; ++i) {
+            const uint32_t v = cand[i];
+            uint32_t j = i;
+            for (; j > 0 && cand[j - 1] > v; --j) cand[j] = cand[j - 1];
+            cand[j] = v;
+        }
+        nn = 0;
+        for (uint32_t i = 0, j = 0; i < mm || j < mc; ++nn) {
+            const uint32_t a = i < mm ? set[i] : 0xffffffffu, c = j < mc ? cand[j] : 0xffffffffu;
+            const uint32_t v = a < c ? a : c;
+            if (a == v) ++i;
+            if (c == v) ++j;
+            if (nn < cap) out[nn] = v;
+        }
+    }
+    wave_sync();
+    if (nn > cap) {
+        overflow += nn - cap;
+        nn = cap;
+    }
+    return nn;
+}
+
+// One pass over the members of the wavefront's new active sets (nn members in
+// buffer cur of the lanes with a vertex), flattened over the lanes: a
+// member's record and its frame's origin serve its albedo term
+// (evaluate_albedo, sampling.cuh:257-283), the chords of both shadow rays
+// (has_a, has_b) and the next ray's exit and free flight (sampling.cuh:356-370
+// at bounce b1), which were three passes with a load of the record each, the
+// albedo's a loop per lane (11 to 22 % of the dense scenes' time).
+// The albedo terms {albedo w, w} go to the owner's slab, to be summed in set
+// order; the shadow rays' fixed-point depths stay in wq.acc; ts_next receives
+// the minimum free flight of the next ray over the set, kTMax if none.
+// da, db and wo are the two shadow rays' and the next ray's directions from x.
+__device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has_a, bool has_b, const SceneView& sc,
+                                             f3 x, f3 da, f3 db, f3 wo, uint64_t key, uint32_t b1,
+                                             uint32_t* __restrict__ slab, uint32_t cap, const WaveQueue& wq,
+                                             float& ts_next) {
+    const uint32_t lane = __lane_id();
+    const uint32_t gbase = blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
+    const uint32_t bs = mega_slab_stride(cap);
+    uint32_t* pre_of = reinterpret_cast<uint32_t*>(wq.tj);  // [64]
+    uint32_t* meta_of = pre_of + 64;                          // [64] set buffer | has_a << 1 | has_b << 2
+    float* wo_of = reinterpret_cast<float*>(wq.prim);         // [64 * 3]
+    unsigned long long* key_of = reinterpret_cast<unsigned long long*>(wq.prim + 192);  // [64]
+    uint32_t* ts_of = wq.prim + 320;                          // [64]
+    uint32_t* b_of = wq.prim + 384;                           // [64]
+    static_assert(kWaveQ >= 448, "the member pass's tables must fit in wq.prim");
+    uint32_t total;
+    pre_of[lane] = wave_prefix(nn, total);
+    meta_of[lane] = cur | (has_a ? 2u : 0u) | (has_b ? 4u : 0u);
+    lds_store3(wq.ro + 3 * lane, x);
+    wq.prims[lane] = sc.prims;
+    lds_store3(wq.rd + 3 * (2 * lane), da);
+    lds_store3(wq.rd + 3 * (2 * lane + 1), db);
+    wq.acc[2 * lane] = 0ull;
+    wq.acc[2 * lane + 1] = 0ull;
+    lds_store3(wo_of + 3 * lane, wo);
+    key_of[lane] = key;
+    ts_of[lane] = __float_as_uint(kTMax);
+    b_of[lane] = b1;
+    wave_sync();
+    for (uint32_t g = lane; g < total; g += 64u) {
+        const uint32_t own = prefix_owner(pre_of, g), k = g - pre_of[own];
+        const uint32_t meta = meta_of[own], set = (meta & 1u) * bs;
+        uint32_t* mine = slab_of(slab, gbase, own, bs);
+        const uint32_t i = mine[set + k];
+        const PrimRecord pr = load_prim(wq.prims[own], i);
+        const f3 ro = lds_load3(wq.ro + 3 * own);
+        const f3 p = to_local_pos(pr, ro);
+        const float pp = length2(p);
+        const float ex = expf_(-0.5f * pp);
+        auto e = [&]() { return ex; };
+        const float wgt = pr.mass * (ex * pr.dnf);  // mass * prim_pdf
+        *reinterpret_cast<float4*>(mine + 2u * bs + 4u * k) =
+            make_float4(pr.ar * wgt, pr.ag * wgt, pr.ab * wgt, wgt);
+        if ((meta & 2u) != 0u) {
+            const float ta = inside_chord_from(pr, p, pp, lds_load3(wq.rd + 3 * (2 * own)), e).tau;
+            if (ta > 0.0f) atomicAdd(&wq.acc[2 * own], tau_fixed(ta));
+        }
+        if ((meta & 4u) != 0u) {
+            const float tb = inside_chord_from(pr, p, pp, lds_load3(wq.rd + 3 * (2 * own + 1)), e).tau;
+            if (tb > 0.0f) atomicAdd(&wq.acc[2 * own + 1], tau_fixed(tb));
+        }
+        const f3 rw = lds_load3(wo_of + 3 * own);
+        const InsideChord c = inside_chord_from(pr, p, pp, rw, e);
+        mine[bs - set + k] = __float_as_uint(c.t1);
+        const float tau = free_flight_tau(prim_uniform(key_of[own], b_of[own], 0u, i));
+        if (tau <= c.tau) {
+            const float t = origin_flight(pr, ro, rw, c, tau);
+            atomicMin(&ts_of[own], t == 0.0f ? 0u : __float_as_uint(t));
+        }
+    }
+    wave_sync();
+    ts_next = __uint_as_float(ts_of[lane]);
+    // the owner's terms in set order, read four at a time
+    const float4* terms = reinterpret_cast<const float4*>(slab_of(slab, gbase, lane, bs) + 2u * bs);
+    f3 aa = mk(0.0f);
+    float aw = 0.0f;
+    for (uint32_t k = 0; k < nn; k += 4u) {
+        float4 t[4];
+#pragma unroll
+        for (uint32_t q = 0; q < 4u; ++q) t[q] = terms[k + q];  // (entries past nn lie in the slab and are not used)
+#pragma unroll
+        for (uint32_t q = 0; q < 4u; ++q) {
+            if (k + q < nn) {
+                aa = aa + f3{t[q].x, t[q].y, t[q].z};
+                aw += t[q].w;
+            }
+        }
+    }
+    wave_sync();
+    return aw <= 0.0f ? mk(0.0f) : aa * rcpf(aw);
 }
 
 // launch_desc[0] = number of job slices, launch_desc[1] = end of the
@@ -430,7 +670,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
 
         float ts = kTMax;
         // the origin-set members' exits, kept for the rebuild
-        float* act_exit = reinterpret_cast<float*>(my + 5 * bs * stride);
+        float* act_exit = kShared ? reinterpret_cast<float*>(nxt) : reinterpret_cast<float*>(my + 5 * bs * stride);
         ev.add(kCntArgActive, na);
         ev.add(kCntTrace);
         // argmin over the origin set (sampling.cuh:356-370) and over entered
@@ -455,8 +695,8 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
                 f3 kd;
                 dlimit = direct_rr(kd).limit();
             }
-            argmin_walk_shared(alive, sc, o, d, st.key, b, direct, act, na, act_exit, slab, cap, wq, ts, nc, dlimit,
-                               dwalk);
+            argmin_walk_shared(alive, sc, o, d, st.key, b, direct, act, na, act_exit, st.ts_set, slab, cap, wq, ts, nc,
+                               dlimit, dwalk);
         } else {
             for (uint32_t k = 0; k < na; ++k) {
                 const uint32_t i = act[k * stride];
@@ -528,138 +768,108 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         uint32_t nn = 0;
         uint64_t lim_a = 0, lim_b = 0;
         bool has_a = false, has_b = false;
+        // the sampled directions' densities (MIS); pdf_a is RIS's weight sum
+        // and ka its candidate's radiance until the albedo is known
+        float pdf_a = 0.0f, pdf_b = 0.0f;
+        const f3 luma = f3{kLumR, kLumG, kLumB};
         // the shadow rays' roulettes (a no-op unless J.shadow_rr > 0) are
         // drawn before and again after the walks (the same values), so they
         // hold no registers during them
         auto nee_rr = [&](f3 k, uint32_t ray) { return shadow_rr(max3(k), J.shadow_rr, st.key, b, ray); };
+        // rebuild the active set at the scatter point (sampling.cuh:422-458):
+        // from the candidates of the argmin walk, or, if they were more than
+        // fit (and in the other builds), by a point query
+        const bool listed = kShared && nc <= cap;
+        if constexpr (kShared)
+            nn = rebuild_shared(vertex && listed, na, nc, st.cur, ts, slab, cap, wq, overflow);
         if (vertex) {
-            // rebuild the active set at the scatter point (sampling.cuh:422-458)
             x = o + ts * d;
-            uint32_t ia = 0, visits = 0, rb_a = 0, rb_h = 0;
-            auto push = [&](uint32_t v) {
-                const bool fits = nn < cap;
-                if (fits) nxt[nn * stride] = v;
-                nn += fits ? 1u : 0u;
-                overflow += fits ? 0u : 1u;
-            };
-            // old member ia stays while the vertex is before its exit (kept
-            // from the argmin's origin loop)
-            auto keep_member = [&]() {
-                ++rb_a;
-                const bool k = ts <= act_exit[ia * stride];
-                ++ia;
-                return k;
-            };
-            auto drain_below = [&](uint32_t c) {
+            if (!listed) {
+                uint32_t ia = 0, visits = 0, rb_a = 0, rb_h = 0;
+                // (the timed kernel's exits are in nxt: its set is built in
+                // buffer 5 and copied)
+                uint32_t* out = kShared ? my + 5 * bs * stride : nxt;
+                nn = 0;
+                auto push = [&](uint32_t v) {
+                    const bool fits = nn < cap;
+                    if (fits) out[nn * stride] = v;
+                    nn += fits ? 1u : 0u;
+                    overflow += fits ? 0u : 1u;
+                };
+                // old member ia stays while the vertex is before its exit (kept
+                // from the argmin's origin loop)
+                auto keep_member = [&]() {
+                    ++rb_a;
+                    const bool k = ts <= act_exit[ia * stride];
+                    ++ia;
+                    return k;
+                };
+                auto drain_below = [&](uint32_t c) {
+                    while (ia < na) {
+                        const uint32_t a = act[ia * stride];
+                        if (a >= c) break;
+                        if (keep_member()) push(a);
+                    }
+                };
+                // a candidate: an old member kept while the vertex is inside
+                // it, else an entered primitive kept if the vertex lies on its
+                // chord (entry and exit as the argmin recorded them, or
+                // computed here for the point query)
+                auto visit = [&](uint32_t c, bool stored, float tj, float te) {
+                    bool keep = false;
+                    if (ia < na && act[ia * stride] == c) keep = keep_member();
+                    if (!keep) {
+                        ++rb_h;
+                        if (!stored) {
+                            const Crossing cx = crossing(load_prim(sc.prims, c), o, d);
+                            tj = cx.t0;
+                            te = cx.t1;
+                        }
+                        keep = tj >= 0.0f && tj <= ts && ts <= te;
+                    }
+                    if (keep) push(c);
+                };
+                if (!kShared && !kMeasure && nc <= cap) {
+                    // candidates from the argmin walk, in ascending index order
+                    float* ctj = reinterpret_cast<float*>(my + 3 * bs * stride);
+                    float* cte = reinterpret_cast<float*>(my + 4 * bs * stride);
+                    for (uint32_t i = 1; i < nc; ++i) {
+                        const uint32_t v = cnd[i * stride];
+                        const float vt = ctj[i * stride], ve = cte[i * stride];
+                        uint32_t j = i;
+                        while (j > 0 && cnd[(j - 1) * stride] > v) {
+                            cnd[j * stride] = cnd[(j - 1) * stride];
+                            ctj[j * stride] = ctj[(j - 1) * stride];
+                            cte[j * stride] = cte[(j - 1) * stride];
+                            --j;
+                        }
+                        cnd[j * stride] = v;
+                        ctj[j * stride] = vt;
+                        cte[j * stride] = ve;
+                    }
+                    for (uint32_t k = 0; k < nc; ++k) {
+                        const uint32_t c = cnd[k * stride];
+                        drain_below(c);
+                        visit(c, true, ctj[k * stride], cte[k * stride]);
+                    }
+                } else {
+                    // one BVH point query at the vertex
+                    walk_point_q(sc, x, visits, lq, [&](uint32_t c) {
+                        drain_below(c);
+                        visit(c, false, 0.0f, 0.0f);
+                    });
+                }
                 while (ia < na) {
                     const uint32_t a = act[ia * stride];
-                    if (a >= c) break;
                     if (keep_member()) push(a);
                 }
-            };
-            // a candidate: an old member kept while the vertex is inside it,
-            // else an entered primitive kept if the vertex lies on its chord
-            // (entry and exit as the argmin recorded them, or computed here
-            // for the point query)
-            auto visit = [&](uint32_t c, bool stored, float tj, float te) {
-                bool keep = false;
-                if (ia < na && act[ia * stride] == c) keep = keep_member();
-                if (!keep) {
-                    ++rb_h;
-                    if (!stored) {
-                        const Crossing cx = crossing(load_prim(sc.prims, c), o, d);
-                        tj = cx.t0;
-                        te = cx.t1;
-                    }
-                    keep = tj >= 0.0f && tj <= ts && ts <= te;
-                }
-                if (keep) push(c);
-            };
-            if (nc <= cap && !kMeasure) {
-                // candidates from the argmin walk, in ascending index order
-                float* ctj = reinterpret_cast<float*>(my + 3 * bs * stride);
-                float* cte = reinterpret_cast<float*>(my + 4 * bs * stride);
-                for (uint32_t i = 1; i < nc; ++i) {
-                    const uint32_t v = cnd[i * stride];
-                    const float vt = ctj[i * stride], ve = cte[i * stride];
-                    uint32_t j = i;
-                    while (j > 0 && cnd[(j - 1) * stride] > v) {
-                        cnd[j * stride] = cnd[(j - 1) * stride];
-                        ctj[j * stride] = ctj[(j - 1) * stride];
-                        cte[j * stride] = cte[(j - 1) * stride];
-                        --j;
-                    }
-                    cnd[j * stride] = v;
-                    ctj[j * stride] = vt;
-                    cte[j * stride] = ve;
-                }
-                // Merge with the old members, read four at a time (ids and
-                // exits: the buffers are 16-byte aligned and the reads stay
-                // inside them) so the loop does not wait on a load per
-                // member.  Same tests and the same ascending order as
-                // drain_below/visit: an old member stays while the vertex is
-                // before its exit; a candidate that is also an old member is
-                // tested as a candidate only if the member test fails.
-                static_assert(stride == 1, "the merge reads the slab buffers four entries at a time");
-                // the next candidate is held in registers (id ~0 once none is left)
-                uint32_t ic = 0, c_id = 0xffffffffu;
-                float c_tj = 0.0f, c_te = 0.0f;
-                auto next_candidate = [&]() {
-                    c_id = ic < nc ? cnd[ic] : 0xffffffffu;
-                    if (ic < nc) {
-                        c_tj = ctj[ic];
-                        c_te = cte[ic];
-                    }
-                    ++ic;
-                };
-                auto candidate = [&]() {
-                    ++rb_h;
-                    if (c_tj >= 0.0f && c_tj <= ts && ts <= c_te) push(c_id);
-                };
-                next_candidate();
-                for (uint32_t base = 0; base < na; base += 4u) {
-                    const uint4 id4 = *reinterpret_cast<const uint4*>(act + base);
-                    const float4 ex4 = *reinterpret_cast<const float4*>(act_exit + base);
-                    const uint32_t id[4] = {id4.x, id4.y, id4.z, id4.w};
-                    const float ex[4] = {ex4.x, ex4.y, ex4.z, ex4.w};
-                    const uint32_t nk = na - base < 4u ? na - base : 4u;
-                    for (uint32_t k = 0; k < nk; ++k) {
-                        const uint32_t a = id[k];
-                        while (c_id < a) {
-                            candidate();
-                            next_candidate();
-                        }
-                        ++rb_a;
-                        const bool stay = ts <= ex[k];
-                        if (c_id == a) {
-                            if (stay) push(a);
-                            else candidate();
-                            next_candidate();
-                        } else if (stay) {
-                            push(a);
-                        }
-                    }
-                }
-                ia = na;
-                while (c_id != 0xffffffffu) {
-                    candidate();
-                    next_candidate();
-                }
-            } else {
-                // more candidates than fit: one BVH point query at the vertex
-                walk_point_q(sc, x, visits, lq, [&](uint32_t c) {
-                    drain_below(c);
-                    visit(c, false, 0.0f, 0.0f);
-                });
+                if constexpr (kShared)
+                    for (uint32_t k = 0; k < nn; ++k) nxt[k * stride] = out[k * stride];
+                ev.add(kCntNodeVisits, visits);
+                ev.add(kCntVisitsPoint, visits);
+                ev.add(kCntRbActive, rb_a);
+                ev.add(kCntRbHit, rb_h);
             }
-            while (ia < na) {
-                const uint32_t a = act[ia * stride];
-                if (keep_member()) push(a);
-            }
-            ev.add(kCntNodeVisits, visits);
-            ev.add(kCntVisitsPoint, visits);
-            ev.add(kCntRbActive, rb_a);
-            ev.add(kCntRbHit, rb_h);
             st.cur ^= 1u;
             st.na = nn;
             act = nxt;
@@ -669,11 +879,42 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
                 atomicMax(&counters[kCntMaxOverlap], static_cast<unsigned long long>(ovl));
             }
 
+            // the next direction, then NEE's (accumulate_nee_direct,
+            // path_stages.cuh:148-226): RIS picks one environment candidate,
+            // MIS draws one direction from the phase function and one from
+            // the environment
             float phase_pdf;
             wo = phase_sample(J.hg, d, st.rng, &phase_pdf);
             ev.add(kCntScatter);
+            if (J.use_ris) {
+                for (uint32_t c = 0; c < J.ris_candidates; ++c) {
+                    float cpdf;
+                    const f3 cwo = env_sample(env, st.rng, &cpdf);
+                    if (cpdf <= 0.0f) continue;
+                    const f3 envc = env_lookup(env, cwo);
+                    const float lumc = dot(envc, luma);
+                    const float wgt = phase_eval(J.hg, d, cwo) * lumc * rcpf(cpdf);
+                    if (!(wgt > 0.0f)) continue;
+                    pdf_a += wgt;
+                    if (next_uniform(st.rng) * pdf_a < wgt) {
+                        da = cwo;
+                        ka = envc;
+                    }
+                }
+                has_a = pdf_a > 0.0f && dot(ka, luma) > 0.0f;
+            } else {
+                da = phase_sample(J.hg, d, st.rng, &pdf_a);
+                db = env_sample(env, st.rng, &pdf_b);
+                has_a = has_b = true;
+            }
+        }
 
-            // evaluate_albedo (sampling.cuh:257-283)
+        // evaluate_albedo (sampling.cuh:257-283)
+        f3 albedo;
+        if constexpr (kShared) {
+            albedo = vertex_members(nn, st.cur, has_a, has_b, sc, x, da, db, wo, st.key, b + 1u, slab, cap, wq,
+                                    st.ts_set);
+        } else {
             f3 aa = mk(0.0f);
             float aw = 0.0f;
             for (uint32_t k = 0; k < nn; ++k) {
@@ -683,61 +924,36 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
                 aw += wgt;
             }
             ev.add(kCntAlb, nn);
-            const f3 albedo = aw <= 0.0f ? mk(0.0f) : aa * rcpf(aw);
-
-            // accumulate_nee_direct (path_stages.cuh:148-226); base is also
-            // the next bounce's throughput (raygen.cuh:189), set here so the
-            // albedo holds no registers during the shadow walks
+            albedo = aw <= 0.0f ? mk(0.0f) : aa * rcpf(aw);
+        }
+        if (vertex) {
+            // the factors the shadow rays' transmittances multiply; base is
+            // also the next bounce's throughput (raygen.cuh:189), set here so
+            // the albedo holds no registers during the shadow walks
             const f3 base = st.beta * albedo;
             st.beta = base;
-            const f3 luma = f3{kLumR, kLumG, kLumB};
             if (J.use_ris) {
-                float wsum = 0.0f;
-                f3 ydir = mk(0.0f), yenv = mk(0.0f);
-                for (uint32_t c = 0; c < J.ris_candidates; ++c) {
-                    float cpdf;
-                    const f3 cwo = env_sample(env, st.rng, &cpdf);
-                    if (cpdf <= 0.0f) continue;
-                    const f3 envc = env_lookup(env, cwo);
-                    const float lumc = dot(envc, luma);
-                    const float wgt = phase_eval(J.hg, d, cwo) * lumc * rcpf(cpdf);
-                    if (!(wgt > 0.0f)) continue;
-                    wsum += wgt;
-                    if (next_uniform(st.rng) * wsum < wgt) {
-                        ydir = cwo;
-                        yenv = envc;
-                    }
-                }
-                if (wsum > 0.0f) {
-                    const float lumy = dot(yenv, luma);
-                    if (lumy > 0.0f) {
-                        ev.add(kCntShadowRays);
-                        const float Wr = wsum * rcpf(static_cast<float>(J.ris_candidates));
-                        // the factor T multiplies
-                        ka = (base * (yenv * rcpf(lumy))) * Wr;
-                        da = ydir;
-                        has_a = true;
-                    }
+                if (has_a) {
+                    ev.add(kCntShadowRays);
+                    const float Wr = pdf_a * rcpf(static_cast<float>(J.ris_candidates));
+                    ka = (base * (ka * rcpf(dot(ka, luma)))) * Wr;
                 }
             } else {
-                float apdf;
-                da = phase_sample(J.hg, d, st.rng, &apdf);
+                if constexpr (kShared) {
+                    da = lds_load3(wq.rd + 3 * (2 * lane));
+                    db = lds_load3(wq.rd + 3 * (2 * lane + 1));
+                }
                 const float pb_a = env_pdf(env, da);
-                const float sa = apdf + pb_a;
-                const float wa = sa > 0.0f ? apdf / sa : 0.0f;
+                const float sa = pdf_a + pb_a;
+                const float wa = sa > 0.0f ? pdf_a / sa : 0.0f;
                 const f3 enva = env_lookup(env, da);
-
-                float bpdf;
-                db = env_sample(env, st.rng, &bpdf);
                 const float ph_b = phase_eval(J.hg, d, db);
-                const float sb = bpdf + ph_b;
-                const float wb = sb > 0.0f ? bpdf / sb : 0.0f;
+                const float sb = pdf_b + ph_b;
+                const float wb = sb > 0.0f ? pdf_b / sb : 0.0f;
                 const f3 envb = env_lookup(env, db);
                 ev.add(kCntShadowRays, 2);
-                // the factors the two transmittances multiply
                 ka = (base * enva) * wa;
-                kb = (((base * envb) * wb) * ph_b) * rcpf(bpdf);
-                has_a = has_b = true;
+                kb = (((base * envb) * wb) * ph_b) * rcpf(pdf_b);
             }
             if (has_a) lim_a = nee_rr(ka, 0u).limit();
             if (has_b) lim_b = nee_rr(kb, 1u).limit();
@@ -747,7 +963,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         // them one by one, so the former's counts are per-ray work)
         uint64_t acc_a = 0, acc_b = 0;
         if constexpr (kShared) {
-            transmittance_pool(sc, x, da, db, act, nn, wq, lim_a, lim_b, acc_a, acc_b);
+            shadow_walks(sc, wq, lim_a, lim_b, acc_a, acc_b);
         } else {
             if (has_a) acc_a = shadow_depth(sc, x, da, act, nn, stride, lq, ev, lim_a);
             if (has_b) acc_b = shadow_depth(sc, x, db, act, nn, stride, lq, ev, lim_b);
