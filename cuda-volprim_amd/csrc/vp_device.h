@@ -604,185 +604,236 @@ __device__ __forceinline__ unsigned long long tau_fixed(float od) {
     return c >= kMaxTau ? kTauLimitFixed : static_cast<unsigned long long>(c * kTauScaleF);
 }
 
-// Work sharing between the walks of one wavefront, for queries whose result
-// does not depend on visiting order.  Lanes without a walk (idle) each take
-// the shallowest pending subtree of a running walk (can_give): the donor
-// clears that child from its trail and the thief starts a walk at the child
-// with an empty trail, which ends once the subtree is done, so every subtree
-// is still walked exactly once.  The handoff uses the first 128 words of
-// wq.tj, which are free between leaf phases.  Returns true for a lane that
-// received a subtree; its ray and walk are set.
-// A node phase ends to share out the running walks once at least
-// VP_STEAL_IDLE lanes have nothing to step (scattering workload: 8, 16 and 32
-// measured 27.7, 28.3 and 28.5 Msamples/s).
-#ifndef VP_STEAL_IDLE
-#define VP_STEAL_IDLE 32
+// ---- wave-wide walks of the megakernel ----
+//
+// The rays of a wavefront are walked together by its 64 lanes from one stack
+// of (node, ray) items in LDS: every lane takes an item from the top, tests
+// its node's four children against its ray, and appends the crossed ones; the
+// crossed children of a last-level node are leaves and go to a leaf queue,
+// from which 64 at a time are evaluated.  Which lane tests which node is of no
+// account: all results are fixed-point sums and minima.  Node steps and leaf
+// tests then run at full width however few rays are left and however uneven
+// their walks are, and no lane holds a walk in registers.  (With a walk per
+// lane, the argmin's node steps ran at 19 to 28 % of the lanes, and a walk's
+// nodes were a serial chain.)
+// Node k of the implicit 4-ary tree has the children 4k + 1 .. 4k + 4 in heap
+// order; a node is on the last level from index w4_level_base(levels - 1) on.
+#ifndef VP_NODE_Q
+#define VP_NODE_Q 448
 #endif
-// ... and only after at least VP_STEAL_GAP node steps in the phase, so each
-// handoff (a leaf phase, the handoff and the lanes' ray setup) is paid for by
-// that many steps of the lanes it feeds.
-#ifndef VP_STEAL_GAP
-#define VP_STEAL_GAP 1u
+#ifndef VP_LEAF_ITEMS
+#define VP_LEAF_ITEMS 240
 #endif
-__device__ __forceinline__ bool wave_steal(const WaveQueue& wq, bool idle, bool can_give, uint32_t& ray, Walk4& w) {
-    const uint64_t pend = can_give ? walk4_pending(w) : 0ull;
-    const unsigned long long im = __builtin_amdgcn_ballot_w64(idle);
-    const unsigned long long dm = __builtin_amdgcn_ballot_w64(pend != 0ull);
-    const uint32_t ni = static_cast<uint32_t>(__popcll(im)), nd = static_cast<uint32_t>(__popcll(dm));
-    const uint32_t pairs = ni < nd ? ni : nd;
-    if (pairs == 0u) return false;
-    uint32_t* slot = reinterpret_cast<uint32_t*>(wq.tj);
-    if (pend != 0ull) {
-        const uint32_t r = lanes_below(dm);
-        if (r < pairs) {
-            Walk4 part;
-            walk4_split(w, part);
-            slot[r] = part.n;
-            slot[64 + r] = ray | (part.lvl << 8);
+constexpr uint32_t kNodeQ = VP_NODE_Q;       // stack items
+constexpr uint32_t kLeafItems = VP_LEAF_ITEMS;  // leaf queue items
+// Items of the stack held back from wide steps: one item at a time adds at
+// most 3 per level, so a walk always finishes.
+constexpr uint32_t kNodeReserve = 3 * kW4MaxLevels + 3;
+static_assert(kNodeQ > kNodeReserve + 3 * 64 + 64 && kLeafItems >= 64 + 4, "room for a step of every lane");
+
+// The rays are numbered 2 l and 2 l + 1 for lane l: its two shadow rays, or
+// for the argmin ray 2 l alone, with the argmin's state in the other's place.
+struct MegaQueue {
+    uint32_t* node;          // [kNodeQ] stack: nodes still to be tested
+    uint32_t* leaf;          // [kLeafItems] stored primitives still to be tested
+    uint8_t* node_ray;       // [kNodeQ] their rays
+    uint8_t* leaf_ray;       // [kLeafItems]
+    float* ro;               // [64 * 3] ray origin of each lane
+    float* rd;               // [128 * 3] ray directions
+    float* inv;              // [128 * 3] their reciprocals (safe_inv)
+    unsigned long long* acc;   // [128] fixed-point optical depth of each ray
+    const PrimRecord** prims;  // [64] primitive array of each lane's scene (lanes of one
+                               //      wavefront may run jobs over different scenes)
+    const float4** nodes;    // [64] walk-tree records of each lane's scene
+    uint32_t* lim;           // [128] depth at which each ray's walk may stop, >> 16
+    uint32_t* tree;          // [64] level count | w4_half << 8 of each lane's scene
+    uint8_t* list;           // [128] the rays still to be walked
+    uint32_t* scratch;       // [kScratch] words over node and leaf, free outside the walks
+
+    // argmin state of lane l
+    __device__ __forceinline__ uint32_t& ts(uint32_t l) const {  // running minimum, float bits
+        return reinterpret_cast<uint32_t*>(acc + 2 * l + 1)[0];
+    }
+    __device__ __forceinline__ uint32_t& nc(uint32_t l) const {  // candidates recorded
+        return reinterpret_cast<uint32_t*>(acc + 2 * l + 1)[1];
+    }
+    __device__ __forceinline__ uint32_t* draw(uint32_t l) const {  // [3] path key (2 words), bounce | direct << 31
+        return reinterpret_cast<uint32_t*>(rd + 3 * (2 * l + 1));
+    }
+    // depth of ray r has reached its limit
+    __device__ __forceinline__ bool full(uint32_t r) const {
+        return acc[r] >= (static_cast<unsigned long long>(lim[r]) << 16);
+    }
+};
+constexpr uint32_t kScratch = kNodeQ + kLeafItems;
+constexpr uint32_t kMegaQueueBytes = 5 * (kNodeQ + kLeafItems) + 64 * 12 + 128 * 24 + 128 * 8 + 64 * 16 + 128 * 4 +
+                                     64 * 4 + 128;
+static_assert((5 * (kNodeQ + kLeafItems)) % 8 == 0, "the 8-byte arrays stay aligned");
+constexpr uint32_t kMegaBytes =
+    ((64 * kLeafRow * 4 > kMegaQueueBytes ? 64 * kLeafRow * 4 : kMegaQueueBytes) + 15) / 16 * 16;
+inline size_t mega_queue_bytes(uint32_t block) { return static_cast<size_t>(kMegaBytes) * ((block + 63) / 64); }
+
+// the calling wavefront's queue
+__device__ __forceinline__ MegaQueue mega_queue(uint32_t* lds) {
+    uint8_t* base = reinterpret_cast<uint8_t*>(lds) + (threadIdx.x >> 6) * kMegaBytes;
+    MegaQueue q;
+    q.scratch = q.node = reinterpret_cast<uint32_t*>(base);
+    q.leaf = q.node + kNodeQ;
+    q.node_ray = reinterpret_cast<uint8_t*>(q.leaf + kLeafItems);
+    q.leaf_ray = q.node_ray + kNodeQ;
+    q.ro = reinterpret_cast<float*>(q.leaf_ray + kLeafItems);
+    q.rd = q.ro + 64 * 3;
+    q.inv = q.rd + 128 * 3;
+    q.acc = reinterpret_cast<unsigned long long*>(q.inv + 128 * 3);
+    q.prims = reinterpret_cast<const PrimRecord**>(q.acc + 128);
+    q.nodes = reinterpret_cast<const float4**>(q.prims + 64);
+    q.lim = reinterpret_cast<uint32_t*>(q.nodes + 64);
+    q.tree = q.lim + 128;
+    q.list = reinterpret_cast<uint8_t*>(q.tree + 64);
+    return q;
+}
+// the calling thread's point-query queue over the same LDS
+__device__ __forceinline__ LeafQueue mega_leaf_queue(uint32_t* lds) {
+    return LeafQueue{lds + (threadIdx.x >> 6) * (kMegaBytes / 4) + (threadIdx.x & 63u) * kLeafRow};
+}
+
+// Exclusive prefix sum over the wavefront of v <= 7 (every lane active).
+__device__ __forceinline__ uint32_t wave_prefix3(uint32_t v, uint32_t& total) {
+    const unsigned long long b0 = __builtin_amdgcn_ballot_w64((v & 1u) != 0u);
+    const unsigned long long b1 = __builtin_amdgcn_ballot_w64((v & 2u) != 0u);
+    const unsigned long long b2 = __builtin_amdgcn_ballot_w64((v & 4u) != 0u);
+    total = static_cast<uint32_t>(__popcll(b0) + 2 * __popcll(b1) + 4 * __popcll(b2));
+    return lanes_below(b0) + 2u * lanes_below(b1) + 4u * lanes_below(b2);
+}
+
+// One node step of the wavefront: the top items of the stack (nn of them in
+// all, at least one), as many as the lanes and the room left allow, are
+// replaced by their crossed children, and crossed leaves are appended to the
+// leaf queue (nl items, leaf_cap at most).  kArgmin: a ray is tested over
+// [0, its running minimum], or over its whole length until its direct-term
+// depth reaches the limit; else (shadow rays) over its whole length, and not
+// at all once its depth has reached the limit.
+template <bool kArgmin>
+__device__ __forceinline__ void walk_nodes(const MegaQueue& q, uint32_t& nn, uint32_t& nl, uint32_t leaf_cap) {
+    const uint32_t lane = __lane_id();
+    const uint32_t room = nn + kNodeReserve + 3u < kNodeQ ? (kNodeQ - kNodeReserve - nn) / 3u : 1u;
+    uint32_t n = nn < 64u ? nn : 64u;
+    n = n < room ? n : room;
+    uint32_t node = 0, ray = 0, m = 0, child = 0;
+    bool last = false;
+    if (lane < n) {
+        node = q.node[nn - n + lane];
+        ray = q.node_ray[nn - n + lane];
+        const uint32_t own = ray >> 1;
+        const bool full = q.full(ray);
+        if (kArgmin || !full) {
+            const f3 inv = lds_load3(q.inv + 3 * ray), oi = lds_load3(q.ro + 3 * own) * inv;
+            const float tmax = kArgmin && full ? __uint_as_float(q.ts(own)) : kTMax;
+            const uint32_t tree = q.tree[own], base = w4_level_base((tree & 0xffu) - 1u);
+            m = mega_ray_mask(q.nodes[own], tree >> 8, node, inv, oi, tmax);
+            last = node >= base;
+            child = last ? 4u * (node - base) : 4u * node + 1u;
         }
+    }
+    nn -= n;
+    wave_sync();
+    uint32_t push = last ? 0u : m;
+    if (__builtin_amdgcn_ballot_w64(last && m != 0u) != 0ull) {
+        const uint32_t c = last ? static_cast<uint32_t>(__popc(m)) : 0u;
+        uint32_t total;
+        uint32_t at = nl + wave_prefix3(c, total);
+        // the lanes whose leaves fit come first; the others' nodes go back
+        const bool fits = c == 0u || at + c <= leaf_cap;
+        if (nl + total > leaf_cap) {
+            (void)wave_prefix3(fits ? c : 0u, total);
+            if (!fits) {
+                push = 1u;
+                child = node;
+            }
+        }
+        if (last && fits)
+            for (uint32_t b = m; b != 0u; b &= b - 1u, ++at) {
+                q.leaf[at] = child + static_cast<uint32_t>(__builtin_ctz(b));
+                q.leaf_ray[at] = static_cast<uint8_t>(ray);
+            }
+        nl += total;
+    }
+    if (__builtin_amdgcn_ballot_w64(push != 0u) != 0ull) {
+        uint32_t total;
+        uint32_t at = nn + wave_prefix3(static_cast<uint32_t>(__popc(push)), total);
+        for (uint32_t b = push; b != 0u; b &= b - 1u, ++at) {
+            q.node[at] = child + static_cast<uint32_t>(__builtin_ctz(b));
+            q.node_ray[at] = static_cast<uint8_t>(ray);
+        }
+        nn += total;
     }
     wave_sync();
-    bool got = false;
-    if (idle) {
-        const uint32_t r = lanes_below(im);
-        if (r < pairs) {
-            const uint32_t meta = slot[64 + r];
-            ray = meta & 0xffu;
-            w = Walk4{slot[r], meta >> 8, 0ull};
-            got = true;
-        }
-    }
-    return got;
 }
 
 // The shadow rays of a wavefront's lanes, up to two each (the MIS rays a and
-// b, or the one of RIS), with the wave-shared leaf queue and a wave-wide ray
-// pool.  All 64 lanes of the wavefront call it, those without a ray as
-// helpers: every lane starts on one ray of the wavefront's list (all rays a,
-// then all rays b) and, when its ray is done, takes the next one from the
-// list, whichever lane the ray belongs to.  The node phases then stay full
-// however the walk lengths are spread, until the list runs out; from there on
-// lanes without a ray share the running walks.  Each ray's chords are summed
-// in fixed point in LDS (a ray is saturated once its sum reaches the tau = 88
-// limit, in whatever order the chords arrive), so Ta and Tb equal two
+// b, or the one of RIS).  All 64 lanes of the wavefront call it.  q.ro,
+// q.prims, q.rd and q.acc hold the rays' origins, primitive arrays,
+// directions and the depths of their origin sets.  Each ray's chords are
+// summed in fixed point in LDS (a ray is saturated once its sum reaches the
+// tau = 88 limit, in whatever order the chords arrive), so Ta and Tb equal two
 // transmittance() calls bit for bit.
 // Each ray's walk may stop once its depth reaches its limit (lim_a, lim_b:
 // the tau = 88 saturation, or a shadow-roulette threshold; multiples of
 // 2^16); a limit of 0 is a ray that is not walked.  acc_a and acc_b receive
 // the fixed-point depths.
-// wq.ro, wq.prims, wq.rd and wq.acc hold the rays' origins, primitive arrays,
-// directions and the depths of their origin sets.
-__device__ __forceinline__ void shadow_walks(const SceneView& s, const WaveQueue& wq, uint64_t lim_a, uint64_t lim_b,
+__device__ __forceinline__ void shadow_walks(const SceneView& s, const MegaQueue& q, uint64_t lim_a, uint64_t lim_b,
                                              uint64_t& acc_a, uint64_t& acc_b) {
     const uint32_t lane = __lane_id();
-    wq.nodes[lane] = s.w4;
-    wq.nn[lane] = s.w4_levels | (s.w4_half << 8);
-    wq.lim[2 * lane] = static_cast<uint32_t>(lim_a >> 16);
-    wq.lim[2 * lane + 1] = static_cast<uint32_t>(lim_b >> 16);
-    // a ray is done once its depth reaches its limit
-    auto reached = [&](uint32_t r) -> bool {
-        return wq.acc[r] >= (static_cast<unsigned long long>(wq.lim[r]) << 16);
-    };
-    wave_sync();
-    const bool full_a = reached(2 * lane);
-    const bool full_b = reached(2 * lane + 1);
-    // the rays still to walk: every ray a, then every ray b (a saturated ray
-    // is done already)
-    const unsigned long long pa = __builtin_amdgcn_ballot_w64(!full_a);
-    const unsigned long long pb = __builtin_amdgcn_ballot_w64(!full_b);
+    q.nodes[lane] = s.w4;
+    q.tree[lane] = s.w4_levels | (s.w4_half << 8);
+    q.lim[2 * lane] = static_cast<uint32_t>(lim_a >> 16);
+    q.lim[2 * lane + 1] = static_cast<uint32_t>(lim_b >> 16);
+    lds_store3(q.inv + 3 * (2 * lane), safe_inv(lds_load3(q.rd + 3 * (2 * lane))));
+    lds_store3(q.inv + 3 * (2 * lane + 1), safe_inv(lds_load3(q.rd + 3 * (2 * lane + 1))));
+    // the rays to walk: every ray a, then every ray b, that is not done already
+    const bool walk_a = !q.full(2 * lane), walk_b = !q.full(2 * lane + 1);
+    const unsigned long long pa = __builtin_amdgcn_ballot_w64(walk_a);
+    const unsigned long long pb = __builtin_amdgcn_ballot_w64(walk_b);
     const uint32_t npa = static_cast<uint32_t>(__popcll(pa));
     const uint32_t nr = npa + static_cast<uint32_t>(__popcll(pb));
-    if (!full_a) wq.list[lanes_below(pa)] = static_cast<uint8_t>(2 * lane);
-    if (!full_b) wq.list[npa + lanes_below(pb)] = static_cast<uint8_t>(2 * lane + 1);
+    if (walk_a) q.list[lanes_below(pa)] = static_cast<uint8_t>(2 * lane);
+    if (walk_b) q.list[npa + lanes_below(pb)] = static_cast<uint8_t>(2 * lane + 1);
     wave_sync();
-    uint32_t next = nr < 64u ? nr : 64u;  // list entries handed out
-    constexpr uint32_t kNoRay = 0xffu;
-    // the ray this lane walks, and its walk state
-    uint32_t ray = lane < nr ? wq.list[lane] : kNoRay;
-    const float4* w4 = nullptr;
-    uint32_t levels = 0, half = 0;
-    Walk4 w = walk4_begin();
-    f3 inv = mk(0.0f), oi = mk(0.0f);
-    // the walk setup of the lane's ray (any lane may run it: an idle lane
-    // reads ray 127's data and does not use it)
-    auto setup = [&]() {
-        const uint32_t r = ray & 127u, own = r >> 1;
-        const f3 ro = lds_load3(wq.ro + 3 * own), rd = lds_load3(wq.rd + 3 * r);
-        inv = safe_inv(rd);
-        oi = ro * inv;
-        w4 = wq.nodes[own];
-        levels = walk4_block_levels(wq.nn[own] & 0xffu);
-        half = wq.nn[own] >> 8;
-    };
-    setup();
-    while (__builtin_amdgcn_ballot_w64(ray != kNoRay) != 0) {
-        // node phase: every lane with a ray steps; crossed leaves are queued
-        // for the wavefront.  It ends when no lane steps, when the queue
-        // could not take some lane's leaves, or, once a quarter of the queue
-        // is filled, when fewer than VP_SHARED_STEP_MIN lanes still step.
-        uint32_t count = 0, nsteps = 0;
-        while (true) {
-            const bool step = ray != kNoRay && w.n != kWalkEnd;
-            const unsigned long long sm = __builtin_amdgcn_ballot_w64(step);
-            if (sm == 0) break;
-            const uint32_t ns = static_cast<uint32_t>(__popcll(sm));
-            if (count >= kWaveQ / VP_SHARED_END_DIV && ns < VP_SHARED_STEP_MIN) break;
-            // the list is used up and many lanes are idle: end the phase so
-            // the running walks can be shared out (after at least one step,
-            // so every phase progresses)
-            if (nsteps >= VP_STEAL_GAP && next >= nr && ns + VP_STEAL_IDLE <= 64u &&
-                __builtin_amdgcn_ballot_w64(step && walk4_pending(w) != 0ull) != 0ull)
-                break;
-            ++nsteps;
-            uint32_t lm = 0, first = 0;
-            Walk4 nw = w;
-            if (step) lm = walk4_advance(nw, levels, mega_ray_mask(w4, half, w.n, inv, oi, kTMax), first);
-            const bool fits = wave_push_blocks(wq, count, lm, first, ray);
-            if (step && fits) w = nw;
-            if (__builtin_amdgcn_ballot_w64(!fits) != 0) break;
+    uint32_t next = 0, nn = 0, nl = 0;
+    while (true) {
+        if (nn < 64u && next < nr) {
+            // the next rays start at the root, up to an item per lane
+            const uint32_t k = nr - next < 64u - nn ? nr - next : 64u - nn;
+            if (lane < k) {
+                q.node[nn + lane] = 0u;
+                q.node_ray[nn + lane] = q.list[next + lane];
+            }
+            nn += k;
+            next += k;
+            wave_sync();
         }
-        wave_sync();
-        // leaf phase, shared by all lanes: each queued leaf's crossing (entry
-        // test and whole-chord depth from one transform) goes into its ray's
-        // fixed-point sum
-        // (two leaves per lane and round, both records loaded before either
-        // crossing, so each lane has two loads in flight)
-        for (uint32_t g = lane; g < count; g += 128u) {
-            const uint32_t g2 = g + 64u;
-            const bool two_leaves = g2 < count;
-            const uint32_t own = wq.owner[g], own2 = two_leaves ? wq.owner[g2] : own;
-            const PrimRecord pr = load_prim(wq.prims[own >> 1], wq.prim[g]);
-            const PrimRecord pr2 = load_prim(wq.prims[own2 >> 1], two_leaves ? wq.prim[g2] : wq.prim[g]);
-            const Crossing x = crossing(pr, lds_load3(wq.ro + 3 * (own >> 1)), lds_load3(wq.rd + 3 * own));
-            if (x.tau > 0.0f) atomicAdd(&wq.acc[own], tau_fixed(x.tau));
-            if (two_leaves) {
-                const Crossing x2 = crossing(pr2, lds_load3(wq.ro + 3 * (own2 >> 1)), lds_load3(wq.rd + 3 * own2));
-                if (x2.tau > 0.0f) atomicAdd(&wq.acc[own2], tau_fixed(x2.tau));
+        if (nl < 64u && nn != 0u) {
+            walk_nodes<false>(q, nn, nl, kLeafItems);
+            continue;
+        }
+        if (nl == 0u) break;
+        // 64 leaves (or the last ones): each one's crossing (entry test and
+        // whole-chord depth from one transform) goes into its ray's sum
+        const uint32_t n = nl < 64u ? nl : 64u;
+        nl -= n;
+        if (lane < n) {
+            const uint32_t ray = q.leaf_ray[nl + lane], own = ray >> 1;
+            if (!q.full(ray)) {
+                const PrimRecord pr = load_prim(q.prims[own], q.leaf[nl + lane]);
+                const Crossing x = crossing(pr, lds_load3(q.ro + 3 * own), lds_load3(q.rd + 3 * ray));
+                if (x.tau > 0.0f) atomicAdd(&q.acc[ray], tau_fixed(x.tau));
             }
         }
         wave_sync();
-        // lanes whose ray is done (walked to the end, or saturated) take the
-        // next ray of the list
-        const bool fin = ray != kNoRay && (w.n == kWalkEnd || reached(ray & 127u));
-        const unsigned long long fm = __builtin_amdgcn_ballot_w64(fin);
-        const uint32_t k = next + lanes_below(fm);
-        const uint32_t listed = k < nr ? wq.list[k < 128u ? k : 0u] : kNoRay;
-        ray = fin ? listed : ray;
-        if (fin) w = walk4_begin();
-        next += static_cast<uint32_t>(__popcll(fm));
-        // once the list is used up, idle lanes take over subtrees of running
-        // walks.  Every lane then redoes its ray setup (the same values for a
-        // lane that kept its ray): the refill and the handoff stay free of
-        // branches around the setup, so every lane of the wavefront stays in
-        // the loop and takes part in its ballots and leaf passes.
-        const bool can_give = ray != kNoRay && w.n != kWalkEnd && !reached(ray & 127u);
-        if (next >= nr) wave_steal(wq, ray == kNoRay, can_give, ray, w);
-        setup();
-        wave_sync();
     }
+    acc_a = q.acc[2 * lane];
+    acc_b = q.acc[2 * lane + 1];
     wave_sync();
-    acc_a = wq.acc[2 * lane];
-    acc_b = wq.acc[2 * lane + 1];
 }
 
 __device__ __forceinline__ EnvView env_view(const EnvDev& e) {

@@ -47,11 +47,6 @@
 namespace vp {
 namespace {
 
-// The argmin's origin-set tables (64 set pointers, 64 exit pointers, 64
-// prefix sums) borrow wq.tj between leaf phases.
-static_assert(kWaveQ * sizeof(float) >= 64 * (2 * sizeof(void*) + sizeof(uint32_t)),
-              "the shared queue must hold the argmin's origin-set tables");
-
 struct PathState {
     f3 o, d, beta, L;
     Pcg32 rng;
@@ -81,21 +76,37 @@ struct PathState {
 // 0); from there on it prunes at the running minimum like any other ray.
 // ts_origin is the minimum over the origin set; the result keeps it unless a
 // walk candidate is strictly smaller.
+// Flights waiting to be inverted are taken up once there are VP_FLIGHT_MIN of
+// them (few leaves have one, and the inversion's erf and erfinv cost as much
+// as the leaf round), or at the end of a run of leaves.
+#ifndef VP_FLIGHT_MIN
+#define VP_FLIGHT_MIN 16u
+#endif
 __device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& sc, f3 o, f3 d, uint64_t key,
                                                    uint32_t b, bool direct, const uint32_t* act, uint32_t na_path,
                                                    float* act_exit, float ts_set, uint32_t* __restrict__ slab,
-                                                   uint32_t cap, const WaveQueue& wq, float& ts, uint32_t& nc,
+                                                   uint32_t cap, const MegaQueue& q, float& ts, uint32_t& nc,
                                                    uint64_t dlimit, uint64_t& dacc) {
     const uint32_t lane = __lane_id();
     const uint32_t na = direct ? na_path : 0u;
-    lds_store3(wq.ro + 3 * lane, o);
-    lds_store3(wq.rd + 3 * lane, d);
-    wq.key[lane] = key;
-    wq.prims[lane] = sc.prims;
-    wq.meta[lane] = b | (direct ? 0x80000000u : 0u);
-    wq.acc[lane] = 0ull;
-    wq.ts[lane] = __float_as_uint(direct ? kTMax : ts_set);
-    wq.nc[lane] = 0u;
+    lds_store3(q.ro + 3 * lane, o);
+    lds_store3(q.rd + 3 * (2 * lane), d);
+    lds_store3(q.inv + 3 * (2 * lane), safe_inv(d));
+    q.draw(lane)[0] = static_cast<uint32_t>(key);
+    q.draw(lane)[1] = static_cast<uint32_t>(key >> 32);
+    q.draw(lane)[2] = b | (direct ? 0x80000000u : 0u);
+    q.prims[lane] = sc.prims;
+    q.nodes[lane] = sc.w4;
+    q.tree[lane] = sc.w4_levels | (sc.w4_half << 8);
+    q.acc[2 * lane] = 0ull;
+    q.lim[2 * lane] = direct ? static_cast<uint32_t>(dlimit >> 16) : 0u;
+    q.ts(lane) = __float_as_uint(direct ? kTMax : ts_set);
+    q.nc(lane) = 0u;
+    // the path key and bounce of lane l's draws
+    auto key_of = [&](uint32_t l) {
+        return (static_cast<uint64_t>(q.draw(l)[1]) << 32) | q.draw(l)[0];
+    };
+    auto bounce_of = [&](uint32_t l) { return q.draw(l)[2] & 0x7fffffffu; };
     // The origin set (sampling.cuh:356-370) of a path at bounce 0; from then
     // on the last vertex's pass over the set has evaluated it (vertex_members)
     // and ts_set is its minimum.  The wavefront's (member, lane) pairs are
@@ -103,147 +114,121 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& 
     // lanes.  Per member: its exit (kept in the owner's slab for the rebuild),
     // its free flight into the owner's running minimum, and its chord into the
     // owner's direct-term optical depth; minima and fixed-point sums do not
-    // depend on which lane adds what.  The owners' pointers and prefix sums
-    // sit in wq.tj, free here.  (Active sets of the megakernel are
+    // depend on which lane adds what.  (Active sets of the megakernel are
     // contiguous.)
     if (__builtin_amdgcn_ballot_w64(na != 0u) != 0ull) {
-        const uint32_t** set_of = reinterpret_cast<const uint32_t**>(wq.tj);  // [64]
-        float** exit_of = reinterpret_cast<float**>(wq.tj) + 64;               // [64]
-        uint32_t* pre_of = reinterpret_cast<uint32_t*>(wq.tj) + 4 * 64;       // [64]
+        const uint32_t** set_of = reinterpret_cast<const uint32_t**>(q.scratch);  // [64]
+        float** exit_of = reinterpret_cast<float**>(q.scratch) + 64;               // [64]
+        uint32_t* pre_of = q.scratch + 4 * 64;                                    // [64]
+        static_assert(kScratch >= 5 * 64, "the origin-set tables must fit in the queue");
         uint32_t total;
-        const uint32_t pre = wave_prefix(na, total);
+        pre_of[lane] = wave_prefix(na, total);
         set_of[lane] = act;
         exit_of[lane] = act_exit;
-        pre_of[lane] = pre;
         wave_sync();
         for (uint32_t g = lane; g < total; g += 64u) {
             const uint32_t ol = prefix_owner(pre_of, g), k = g - pre_of[ol];
             const uint32_t i = set_of[ol][k];
-            const PrimRecord pr = load_prim(wq.prims[ol], i);
-            const f3 ro = lds_load3(wq.ro + 3 * ol), rd = lds_load3(wq.rd + 3 * ol);
+            const PrimRecord pr = load_prim(q.prims[ol], i);
+            const f3 ro = lds_load3(q.ro + 3 * ol), rd = lds_load3(q.rd + 3 * (2 * ol));
             const InsideChord x = inside_chord(pr, ro, rd);
             exit_of[ol][k] = x.t1;
-            const float tau = free_flight_tau(prim_uniform(wq.key[ol], wq.meta[ol] & 0x7fffffffu, 0u, i));
+            const float tau = free_flight_tau(prim_uniform(key_of(ol), bounce_of(ol), 0u, i));
             if (tau <= x.tau) {
                 const float t = origin_flight(pr, ro, rd, x, tau);
-                atomicMin(&wq.ts[ol], t == 0.0f ? 0u : __float_as_uint(t));
+                atomicMin(&q.ts(ol), t == 0.0f ? 0u : __float_as_uint(t));
             }
-            if (x.tau > 0.0f) atomicAdd(&wq.acc[ol], tau_fixed(x.tau));
+            if (x.tau > 0.0f) atomicAdd(&q.acc[2 * ol], tau_fixed(x.tau));
         }
     }
     wave_sync();
-    const float ts_origin = __uint_as_float(wq.ts[lane]);
-    const f3 inv = safe_inv(d), oi = o * inv;
-    float tmax = direct && wq.acc[lane] < dlimit ? kTMax : ts_origin;
-    Walk4 w = walk4_begin();
-    if (!alive) w.n = kWalkEnd;
+    const float ts_origin = __uint_as_float(q.ts(lane));
     // the first thread of this wavefront, for the owners' candidate buffers
     const uint32_t gbase = blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
-    while (__builtin_amdgcn_ballot_w64(w.n != kWalkEnd) != 0) {
-        uint32_t count = 0;
-        while (true) {
-            const bool step = w.n != kWalkEnd;
-            const unsigned long long sm = __builtin_amdgcn_ballot_w64(step);
-            if (sm == 0) break;
-            if (count >= kWaveQ / VP_SHARED_END_DIV && static_cast<uint32_t>(__popcll(sm)) < VP_SHARED_STEP_MIN) break;
-            uint32_t lm = 0, first = 0;
-            Walk4 nw = w;
-            if (step)
-                lm = walk4_advance(nw, walk4_block_levels(sc.w4_levels),
-                                   mega_ray_mask(sc.w4, sc.w4_half, w.n, inv, oi, tmax), first);
-            const bool fits = wave_push_blocks(wq, count, lm, first, lane);
-            if (step && fits) w = nw;
-            if (__builtin_amdgcn_ballot_w64(!fits) != 0) break;
+    const uint32_t bs = mega_slab_stride(cap);
+    // every ray starts at the root
+    uint32_t nn, nl = 0, nf = 0;
+    {
+        const unsigned long long am = __builtin_amdgcn_ballot_w64(alive);
+        if (alive) {
+            q.node[lanes_below(am)] = 0u;
+            q.node_ray[lanes_below(am)] = static_cast<uint8_t>(2 * lane);
         }
-        wave_sync();
-        // leaf phase in three passes, each at full width.  First the entry
-        // tests' early rejects (crossing_setup): the leaves a ray may enter
-        // move down to the front of the queue (an entry is only overwritten
-        // after it has been read).  Then those leaves' crossings (entry, exit
-        // and whole-chord depth from one transform): on a direct ray the
-        // depth joins the ray's sum; if the leaf is entered before the
-        // running minimum it is a rebuild candidate and its free flight is
-        // sampled, which ends inside the chord when the sampled depth is at
-        // most the chord's.  Those leaves move down again with their sampled
-        // depth, and the third pass inverts their flights into distances.
-        uint32_t ne = 0;
-        for (uint32_t base = 0; base < count; base += 64u) {
-            const uint32_t g = base + lane;
-            bool may = false;
-            uint32_t own = 0, prim = 0;
-            if (g < count) {
-                own = wq.owner[g];
-                prim = wq.prim[g];
-                CrossingSetup cs;
-                may = crossing_setup(load_prim(wq.prims[own], prim), lds_load3(wq.ro + 3 * own),
-                                     lds_load3(wq.rd + 3 * own), cs);
-            }
-            const unsigned long long mm = __builtin_amdgcn_ballot_w64(may);
-            wave_sync();
-            if (may) {
-                const uint32_t h = ne + lanes_below(mm);
-                wq.prim[h] = prim;
-                wq.owner[h] = static_cast<uint8_t>(own);
-            }
-            ne += static_cast<uint32_t>(__popcll(mm));
+        nn = static_cast<uint32_t>(__popcll(am));
+    }
+    wave_sync();
+    while (true) {
+        if (nl < 64u && nn != 0u) {
+            walk_nodes<true>(q, nn, nl, kLeafItems - nf);
+            continue;
         }
-        wave_sync();
-        uint32_t nk = 0;
-        for (uint32_t base = 0; base < ne; base += 64u) {
-            const uint32_t g = base + lane;
+        if (nl != 0u) {
+            // 64 leaves (or the last ones): their crossings (entry, exit and
+            // whole-chord depth from one transform).  On a direct ray the
+            // depth joins the ray's sum; a leaf entered before the running
+            // minimum is a rebuild candidate (beyond it nothing can change,
+            // t >= entry > minimum) and its free flight is sampled, which
+            // ends inside the chord when the sampled depth is at most the
+            // chord's.
+            const uint32_t n = nl < 64u ? nl : 64u;
+            nl -= n;
             bool keep = false;
-            uint32_t own = 0, prim = 0;
-            float tau = 0.0f;
-            if (g < ne) {
-                own = wq.owner[g];
-                prim = wq.prim[g];
-                const PrimRecord pr = load_prim(wq.prims[own], prim);
-                const Crossing x = crossing(pr, lds_load3(wq.ro + 3 * own), lds_load3(wq.rd + 3 * own));
+            uint32_t ray = 0, prim = 0;
+            if (lane < n) {
+                ray = q.leaf_ray[nl + lane];
+                prim = q.leaf[nl + lane];
+                const uint32_t own = ray >> 1;
+                const PrimRecord pr = load_prim(q.prims[own], prim);
+                const Crossing x = crossing(pr, lds_load3(q.ro + 3 * own), lds_load3(q.rd + 3 * ray));
                 if (x.t0 >= 0.0f) {
-                    const uint32_t meta = wq.meta[own];
-                    if ((meta >> 31) != 0u && x.tau > 0.0f) atomicAdd(&wq.acc[own], tau_fixed(x.tau));
-                    // entered before the running minimum: a rebuild candidate.
-                    // Beyond it nothing can change (t >= entry > minimum).
-                    if (x.t0 <= __uint_as_float(wq.ts[own])) {
-                        const uint32_t pos = atomicAdd(&wq.nc[own], 1u);
+                    const uint32_t meta = q.draw(own)[2];
+                    if ((meta >> 31) != 0u && x.tau > 0.0f) atomicAdd(&q.acc[ray], tau_fixed(x.tau));
+                    if (x.t0 <= __uint_as_float(q.ts(own))) {
+                        const uint32_t pos = atomicAdd(&q.nc(own), 1u);
                         if (pos < cap) {
-                            const uint32_t bs = mega_slab_stride(cap);
                             uint32_t* mine = slab + static_cast<size_t>(gbase + own) * kMegaSlabBuffers * bs;
                             mine[2 * bs + pos] = prim;
                             mine[3 * bs + pos] = __float_as_uint(x.t0);
                             mine[4 * bs + pos] = __float_as_uint(x.t1);
                         }
-                        tau = free_flight_tau(prim_uniform(wq.key[own], meta & 0x7fffffffu, 1u, prim));
+                        const float tau = free_flight_tau(prim_uniform(key_of(own), meta & 0x7fffffffu, 1u, prim));
                         keep = tau <= x.tau;
                     }
                 }
             }
             const unsigned long long km = __builtin_amdgcn_ballot_w64(keep);
             wave_sync();
+            // the flights to invert wait at the end of the leaf queue (the
+            // slots of the leaves just taken are free)
             if (keep) {
-                const uint32_t h = nk + lanes_below(km);
-                wq.prim[h] = prim;
-                wq.owner[h] = static_cast<uint8_t>(own);
-                wq.tj[h] = tau;
+                const uint32_t at = kLeafItems - 1u - nf - lanes_below(km);
+                q.leaf[at] = prim;
+                q.leaf_ray[at] = static_cast<uint8_t>(ray);
             }
-            nk += static_cast<uint32_t>(__popcll(km));
+            nf += static_cast<uint32_t>(__popcll(km));
+            wave_sync();
         }
-        wave_sync();
-        for (uint32_t g = lane; g < nk; g += 64u) {
-            const uint32_t own = wq.owner[g];
-            const f3 ro = lds_load3(wq.ro + 3 * own), rd = lds_load3(wq.rd + 3 * own);
-            const PrimRecord pr = load_prim(wq.prims[own], wq.prim[g]);
-            const float t = entered_flight(pr, ro, rd, crossing(pr, ro, rd), wq.tj[g]);
-            atomicMin(&wq.ts[own], t == 0.0f ? 0u : __float_as_uint(t));
+        if (nf >= VP_FLIGHT_MIN || (nl == 0u && nf != 0u)) {
+            // invert the waiting flights into distances
+            for (uint32_t f = lane; f < nf; f += 64u) {
+                const uint32_t ray = q.leaf_ray[kLeafItems - 1u - f], prim = q.leaf[kLeafItems - 1u - f];
+                const uint32_t own = ray >> 1;
+                const f3 ro = lds_load3(q.ro + 3 * own), rd = lds_load3(q.rd + 3 * ray);
+                const PrimRecord pr = load_prim(q.prims[own], prim);
+                const float tau = free_flight_tau(prim_uniform(key_of(own), bounce_of(own), 1u, prim));
+                const float t = entered_flight(pr, ro, rd, crossing(pr, ro, rd), tau);
+                atomicMin(&q.ts(own), t == 0.0f ? 0u : __float_as_uint(t));
+            }
+            nf = 0;
+            wave_sync();
         }
-        wave_sync();
-        if (!direct || wq.acc[lane] >= dlimit) tmax = __uint_as_float(wq.ts[lane]);
+        if (nl == 0u && nn == 0u) break;
     }
-    wave_sync();
-    const float wmin = __uint_as_float(wq.ts[lane]);
+    const float wmin = __uint_as_float(q.ts(lane));
     ts = wmin < ts_origin ? wmin : ts_origin;
-    nc = wq.nc[lane];
-    dacc = wq.acc[lane];
+    nc = q.nc(lane);
+    dacc = q.acc[2 * lane];
+    wave_sync();
 }
 
 // ---- the vertex stage of the timed kernel, all lanes of a wavefront together ----
@@ -279,17 +264,17 @@ constexpr uint32_t kRebuildScanMax = 1024;
 // load per entry and ran as long as the wavefront's longest list: 7 to 13 % of
 // the dense scenes' and 11 % of a preview's time.
 __device__ __forceinline__ uint32_t rebuild_shared(bool part, uint32_t na, uint32_t nc, uint32_t cur, float ts,
-                                                   uint32_t* __restrict__ slab, uint32_t cap, const WaveQueue& wq,
+                                                   uint32_t* __restrict__ slab, uint32_t cap, const MegaQueue& q,
                                                    uint32_t& overflow) {
     const uint32_t lane = __lane_id();
     const uint32_t gbase = blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
     const uint32_t bs = mega_slab_stride(cap);
-    // tables in wq.tj, 64 words each
-    uint32_t* pre_of = reinterpret_cast<uint32_t*>(wq.tj);
+    // tables in the queue's space, 64 words each
+    uint32_t* pre_of = q.scratch;
     uint32_t* na_of = pre_of + 64;        // members of the list being flattened | set buffer << 31
     uint32_t* kept_of = pre_of + 128;     // [2][64] kept members, kept candidates
     float* ts_of = reinterpret_cast<float*>(pre_of + 256);
-    static_assert(kWaveQ >= 320, "the rebuild's tables must fit in wq.tj");
+    static_assert(kScratch >= 5 * 64, "the rebuild's tables must fit in the queue");
     uint32_t total;
     pre_of[lane] = wave_prefix(part ? na + nc : 0u, total);
     na_of[lane] = na | (cur << 31);
@@ -401,32 +386,33 @@ __device__ __forceinline__ uint32_t rebuild_shared(bool part, uint32_t na, uint3
 // at bounce b1), which were three passes with a load of the record each, the
 // albedo's a loop per lane (11 to 22 % of the dense scenes' time).
 // The albedo terms {albedo w, w} go to the owner's slab, to be summed in set
-// order; the shadow rays' fixed-point depths stay in wq.acc; ts_next receives
+// order; the shadow rays' fixed-point depths stay in q.acc; ts_next receives
 // the minimum free flight of the next ray over the set, kTMax if none.
 // da, db and wo are the two shadow rays' and the next ray's directions from x.
 __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has_a, bool has_b, const SceneView& sc,
                                              f3 x, f3 da, f3 db, f3 wo, uint64_t key, uint32_t b1,
-                                             uint32_t* __restrict__ slab, uint32_t cap, const WaveQueue& wq,
+                                             uint32_t* __restrict__ slab, uint32_t cap, const MegaQueue& q,
                                              float& ts_next) {
     const uint32_t lane = __lane_id();
     const uint32_t gbase = blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
     const uint32_t bs = mega_slab_stride(cap);
-    uint32_t* pre_of = reinterpret_cast<uint32_t*>(wq.tj);  // [64]
-    uint32_t* meta_of = pre_of + 64;                          // [64] set buffer | has_a << 1 | has_b << 2
-    float* wo_of = reinterpret_cast<float*>(wq.prim);         // [64 * 3]
-    unsigned long long* key_of = reinterpret_cast<unsigned long long*>(wq.prim + 192);  // [64]
-    uint32_t* ts_of = wq.prim + 320;                          // [64]
-    uint32_t* b_of = wq.prim + 384;                           // [64]
-    static_assert(kWaveQ >= 448, "the member pass's tables must fit in wq.prim");
+    // tables in the queue's space
+    unsigned long long* key_of = reinterpret_cast<unsigned long long*>(q.scratch);  // [64]
+    uint32_t* pre_of = q.scratch + 2 * 64;                           // [64]
+    uint32_t* meta_of = pre_of + 64;                                 // [64] set buffer | has_a << 1 | has_b << 2
+    uint32_t* ts_of = meta_of + 64;                                  // [64]
+    uint32_t* b_of = ts_of + 64;                                     // [64]
+    float* wo_of = reinterpret_cast<float*>(b_of + 64);              // [64 * 3]
+    static_assert(kScratch >= 9 * 64, "the member pass's tables must fit in the queue");
     uint32_t total;
     pre_of[lane] = wave_prefix(nn, total);
     meta_of[lane] = cur | (has_a ? 2u : 0u) | (has_b ? 4u : 0u);
-    lds_store3(wq.ro + 3 * lane, x);
-    wq.prims[lane] = sc.prims;
-    lds_store3(wq.rd + 3 * (2 * lane), da);
-    lds_store3(wq.rd + 3 * (2 * lane + 1), db);
-    wq.acc[2 * lane] = 0ull;
-    wq.acc[2 * lane + 1] = 0ull;
+    lds_store3(q.ro + 3 * lane, x);
+    q.prims[lane] = sc.prims;
+    lds_store3(q.rd + 3 * (2 * lane), da);
+    lds_store3(q.rd + 3 * (2 * lane + 1), db);
+    q.acc[2 * lane] = 0ull;
+    q.acc[2 * lane + 1] = 0ull;
     lds_store3(wo_of + 3 * lane, wo);
     key_of[lane] = key;
     ts_of[lane] = __float_as_uint(kTMax);
@@ -437,8 +423,8 @@ __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has
         const uint32_t meta = meta_of[own], set = (meta & 1u) * bs;
         uint32_t* mine = slab_of(slab, gbase, own, bs);
         const uint32_t i = mine[set + k];
-        const PrimRecord pr = load_prim(wq.prims[own], i);
-        const f3 ro = lds_load3(wq.ro + 3 * own);
+        const PrimRecord pr = load_prim(q.prims[own], i);
+        const f3 ro = lds_load3(q.ro + 3 * own);
         const f3 p = to_local_pos(pr, ro);
         const float pp = length2(p);
         const float ex = expf_(-0.5f * pp);
@@ -447,12 +433,12 @@ __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has
         *reinterpret_cast<float4*>(mine + 2u * bs + 4u * k) =
             make_float4(pr.ar * wgt, pr.ag * wgt, pr.ab * wgt, wgt);
         if ((meta & 2u) != 0u) {
-            const float ta = inside_chord_from(pr, p, pp, lds_load3(wq.rd + 3 * (2 * own)), e).tau;
-            if (ta > 0.0f) atomicAdd(&wq.acc[2 * own], tau_fixed(ta));
+            const float ta = inside_chord_from(pr, p, pp, lds_load3(q.rd + 3 * (2 * own)), e).tau;
+            if (ta > 0.0f) atomicAdd(&q.acc[2 * own], tau_fixed(ta));
         }
         if ((meta & 4u) != 0u) {
-            const float tb = inside_chord_from(pr, p, pp, lds_load3(wq.rd + 3 * (2 * own + 1)), e).tau;
-            if (tb > 0.0f) atomicAdd(&wq.acc[2 * own + 1], tau_fixed(tb));
+            const float tb = inside_chord_from(pr, p, pp, lds_load3(q.rd + 3 * (2 * own + 1)), e).tau;
+            if (tb > 0.0f) atomicAdd(&q.acc[2 * own + 1], tau_fixed(tb));
         }
         const f3 rw = lds_load3(wo_of + 3 * own);
         const InsideChord c = inside_chord_from(pr, p, pp, rw, e);
@@ -525,8 +511,8 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
     // argmin walk entered before the running minimum (rebuild candidates)
     const uint32_t bs = mega_slab_stride(cap);
     uint32_t* my = slab + static_cast<size_t>(gl) * kMegaSlabBuffers * bs;  // entry k of buffer b at my[b * bs + k]
-    const LeafQueue lq = leaf_queue(s_leafq);
-    const WaveQueue wq = wave_queue(s_leafq);  // the same LDS, used by the wave-shared walks
+    const LeafQueue lq = mega_leaf_queue(s_leafq);
+    const MegaQueue q = mega_queue(s_leafq);  // the same LDS, used by the wave-wide walks
     PathState st{};
     bool alive = false;
     bool exhausted = false;  // every part of the path range is used up (the same in all lanes)
@@ -695,7 +681,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
                 f3 kd;
                 dlimit = direct_rr(kd).limit();
             }
-            argmin_walk_shared(alive, sc, o, d, st.key, b, direct, act, na, act_exit, st.ts_set, slab, cap, wq, ts, nc,
+            argmin_walk_shared(alive, sc, o, d, st.key, b, direct, act, na, act_exit, st.ts_set, slab, cap, q, ts, nc,
                                dlimit, dwalk);
         } else {
             for (uint32_t k = 0; k < na; ++k) {
@@ -781,7 +767,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         // fit (and in the other builds), by a point query
         const bool listed = kShared && nc <= cap;
         if constexpr (kShared)
-            nn = rebuild_shared(vertex && listed, na, nc, st.cur, ts, slab, cap, wq, overflow);
+            nn = rebuild_shared(vertex && listed, na, nc, st.cur, ts, slab, cap, q, overflow);
         if (vertex) {
             x = o + ts * d;
             if (!listed) {
@@ -912,7 +898,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         // evaluate_albedo (sampling.cuh:257-283)
         f3 albedo;
         if constexpr (kShared) {
-            albedo = vertex_members(nn, st.cur, has_a, has_b, sc, x, da, db, wo, st.key, b + 1u, slab, cap, wq,
+            albedo = vertex_members(nn, st.cur, has_a, has_b, sc, x, da, db, wo, st.key, b + 1u, slab, cap, q,
                                     st.ts_set);
         } else {
             f3 aa = mk(0.0f);
@@ -940,8 +926,8 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
                 }
             } else {
                 if constexpr (kShared) {
-                    da = lds_load3(wq.rd + 3 * (2 * lane));
-                    db = lds_load3(wq.rd + 3 * (2 * lane + 1));
+                    da = lds_load3(q.rd + 3 * (2 * lane));
+                    db = lds_load3(q.rd + 3 * (2 * lane + 1));
                 }
                 const float pb_a = env_pdf(env, da);
                 const float sa = pdf_a + pb_a;
@@ -963,7 +949,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         // them one by one, so the former's counts are per-ray work)
         uint64_t acc_a = 0, acc_b = 0;
         if constexpr (kShared) {
-            shadow_walks(sc, wq, lim_a, lim_b, acc_a, acc_b);
+            shadow_walks(sc, q, lim_a, lim_b, acc_a, acc_b);
         } else {
             if (has_a) acc_a = shadow_depth(sc, x, da, act, nn, stride, lq, ev, lim_a);
             if (has_b) acc_b = shadow_depth(sc, x, db, act, nn, stride, lq, ev, lim_b);
@@ -1227,7 +1213,7 @@ using namespace vp;
 hipError_t vp_launch_render(const RenderLaunch& L, const JobDesc* jobs, const uint64_t* job_begin,
                             const uint64_t* launch_desc, unsigned long long* counter, uint32_t* slab,
                             unsigned long long* counters, hipStream_t s) {
-    const size_t lds = leaf_queue_bytes(L.block);
+    const size_t lds = mega_queue_bytes(L.block);
     const auto k = render_kernel(L.count_events, L.measure);
     hipLaunchKernelGGL(k, dim3(L.grid), dim3(L.block), lds, s, jobs, job_begin, launch_desc, counter, slab,
                        L.active_cap, L.regen_min, L.lane_max, counters);
@@ -1271,7 +1257,7 @@ hipError_t vp_launch_fill_u32(uint32_t* p, uint32_t n, uint32_t v, hipStream_t s
 int vp_render_occupancy(uint32_t block, uint32_t, int count_events, int* blocks_per_cu) {
     int nb = 0;
     hipError_t e;
-    const size_t lds = leaf_queue_bytes(block);
+    const size_t lds = mega_queue_bytes(block);
     e = hipOccupancyMaxActiveBlocksPerMultiprocessor(
         &nb, reinterpret_cast<const void*>(render_kernel(count_events, 0)), block, lds);
     *blocks_per_cu = nb > 0 ? nb : 1;
