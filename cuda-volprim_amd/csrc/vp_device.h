@@ -206,18 +206,44 @@ __device__ __forceinline__ uint32_t ray_mask_nf(const float4* w4, uint32_t half,
     return half ? w4h_ray_mask_nf(w4, n, inv, oi, tmax) : w4_ray_mask_nf(w4, n, inv, oi, tmax);
 }
 
-// The node test of the megakernel's shared-queue walks: 1 selects the
-// near/far form (vp_render.hip sets it).
-#ifndef VP_MEGA_NEAR_FAR
-#define VP_MEGA_NEAR_FAR 0
-#endif
-__device__ __forceinline__ uint32_t mega_ray_mask(const float4* w4, uint32_t half, uint32_t n, f3 inv, f3 oi,
-                                                  float tmax) {
-#if VP_MEGA_NEAR_FAR
-    return ray_mask_nf(w4, half, n, inv, oi, tmax);
-#else
-    return ray_mask(w4, half, n, inv, oi, tmax);
-#endif
+// The megakernel's node test: the near and far form on whole 16-byte words,
+// the sides picked by selects after the load, since a load costs the L1 a
+// cycle per lane whatever its size (three for a 16-bit record, where the form
+// above makes six).  n: the node's index, 32 bits wide where the tree lies
+// within 2^32 bytes (the address is then a scalar and an offset), else 64.
+template <typename Index>
+__device__ __forceinline__ uint32_t mega_ray_mask(const float4* w4, uint32_t half, Index n, f3 inv, f3 oi,
+                                                  float tmax, float (&tn4)[4]) {
+    const bool sx = inv.x < 0.0f, sy = inv.y < 0.0f, sz = inv.z < 0.0f;
+    auto hit = [&](int c, float ax, float ay, float az, float bx, float by, float bz) {
+        const float tn = fmaxf(fmaxf(fmaf_(ax, inv.x, -oi.x), fmaf_(ay, inv.y, -oi.y)),
+                               fmaxf(fmaf_(az, inv.z, -oi.z), 0.0f));
+        const float tf = fminf(fminf(fmaf_(bx, inv.x, -oi.x), fmaf_(by, inv.y, -oi.y)),
+                               fminf(fmaf_(bz, inv.z, -oi.z), tmax));
+        tn4[c] = tn <= tf ? tn : kTMax;
+        return tn <= tf;
+    };
+    if (half) {
+        const auto* r = reinterpret_cast<const VP_GLOBAL_AS uint4*>(
+            reinterpret_cast<const VP_GLOBAL_AS char*>(as_global(w4)) + n * static_cast<Index>(kW4hRecordB));
+        // a = min.x (children 0,1 | 2,3), min.y; b = min.z, max.x; c = max.y, max.z
+        const uint4 a = r[0], b = r[1], c = r[2];
+        auto pair = [&](int c, uint32_t lx, uint32_t ly, uint32_t lz, uint32_t hx, uint32_t hy, uint32_t hz) {
+            const uint32_t ax = sx ? hx : lx, ay = sy ? hy : ly, az = sz ? hz : lz;
+            const uint32_t bx = sx ? lx : hx, by = sy ? ly : hy, bz = sz ? lz : hz;
+            return (hit(c, h16lo(ax), h16lo(ay), h16lo(az), h16lo(bx), h16lo(by), h16lo(bz)) ? 1u : 0u) |
+                   (hit(c + 1, h16hi(ax), h16hi(ay), h16hi(az), h16hi(bx), h16hi(by), h16hi(bz)) ? 2u : 0u);
+        };
+        return pair(0, a.x, a.z, b.x, b.z, c.x, c.z) | pair(2, a.y, a.w, b.y, b.w, c.y, c.w) << 2;
+    }
+    const auto* r = reinterpret_cast<const VP_GLOBAL_AS float4*>(
+        reinterpret_cast<const VP_GLOBAL_AS char*>(as_global(w4)) + n * static_cast<Index>(16u * kW4RecordF4));
+    const float4 lx = r[0], ly = r[1], lz = r[2], hx = r[3], hy = r[4], hz = r[5];
+    auto one = [&](int c, float l0, float l1, float l2, float h0, float h1, float h2) {
+        return hit(c, sx ? h0 : l0, sy ? h1 : l1, sz ? h2 : l2, sx ? l0 : h0, sy ? l1 : h1, sz ? l2 : h2);
+    };
+    return (one(0, lx.x, ly.x, lz.x, hx.x, hy.x, hz.x) ? 1u : 0u) | (one(1, lx.y, ly.y, lz.y, hx.y, hy.y, hz.y) ? 2u : 0u) |
+           (one(2, lx.z, ly.z, lz.z, hx.z, hy.z, hz.z) ? 4u : 0u) | (one(3, lx.w, ly.w, lz.w, hx.w, hy.w, hz.w) ? 8u : 0u);
 }
 
 // children of node n whose box contains x
@@ -616,16 +642,19 @@ __device__ __forceinline__ unsigned long long tau_fixed(float od) {
 // their walks are, and no lane holds a walk in registers.  (With a walk per
 // lane, the argmin's node steps ran at 19 to 28 % of the lanes, and a walk's
 // nodes were a serial chain.)
+// The walks are bound by VALU issue and the L1's data return, which takes a
+// cycle per lane of each load whatever its size: with six 8-byte loads a node
+// it was busy 91 % of the scattering workload's time (VALU 85 %); whole 16-byte
+// words, one scene's pointers in scalar registers and the ray's end in one
+// word took 10 % off it, 14 % off the torus and 23 % off the 10^6 cloud.
+// Measured and not taken: four lanes to a node (16 nodes a step, a record read
+// as 64 contiguous bytes: 38 ms against 27), a leaf's record read by four lanes
+// and transposed by lane swaps (+3 to +7 %: 60 more VALU a round), two leaves
+// per lane and round (0).
 // Node k of the implicit 4-ary tree has the children 4k + 1 .. 4k + 4 in heap
 // order; a node is on the last level from index w4_level_base(levels - 1) on.
-#ifndef VP_NODE_Q
-#define VP_NODE_Q 448
-#endif
-#ifndef VP_LEAF_ITEMS
-#define VP_LEAF_ITEMS 240
-#endif
-constexpr uint32_t kNodeQ = VP_NODE_Q;       // stack items
-constexpr uint32_t kLeafItems = VP_LEAF_ITEMS;  // leaf queue items
+constexpr uint32_t kNodeQ = 656;      // stack items
+constexpr uint32_t kLeafItems = 240;  // leaf queue items
 // Items of the stack held back from wide steps: one item at a time adds at
 // most 3 per level, so a walk always finishes.
 constexpr uint32_t kNodeReserve = 3 * kW4MaxLevels + 3;
@@ -642,11 +671,8 @@ struct MegaQueue {
     float* rd;               // [128 * 3] ray directions
     float* inv;              // [128 * 3] their reciprocals (safe_inv)
     unsigned long long* acc;   // [128] fixed-point optical depth of each ray
-    const PrimRecord** prims;  // [64] primitive array of each lane's scene (lanes of one
-                               //      wavefront may run jobs over different scenes)
-    const float4** nodes;    // [64] walk-tree records of each lane's scene
-    uint32_t* lim;           // [128] depth at which each ray's walk may stop, >> 16
-    uint32_t* tree;          // [64] level count | w4_half << 8 of each lane's scene
+    float* tmax;             // [128] the rays' ends; negative once a ray is done
+    uint32_t* job;           // [64] job-table entry of each lane's path
     uint8_t* list;           // [128] the rays still to be walked
     uint32_t* scratch;       // [kScratch] words over node and leaf, free outside the walks
 
@@ -654,20 +680,18 @@ struct MegaQueue {
     __device__ __forceinline__ uint32_t& ts(uint32_t l) const {  // running minimum, float bits
         return reinterpret_cast<uint32_t*>(acc + 2 * l + 1)[0];
     }
+    __device__ __forceinline__ uint32_t& bound(uint32_t l) const {  // an upper bound of the final minimum, float bits
+        return reinterpret_cast<uint32_t*>(tmax)[2 * l + 1];
+    }
     __device__ __forceinline__ uint32_t& nc(uint32_t l) const {  // candidates recorded
         return reinterpret_cast<uint32_t*>(acc + 2 * l + 1)[1];
     }
     __device__ __forceinline__ uint32_t* draw(uint32_t l) const {  // [3] path key (2 words), bounce | direct << 31
         return reinterpret_cast<uint32_t*>(rd + 3 * (2 * l + 1));
     }
-    // depth of ray r has reached its limit
-    __device__ __forceinline__ bool full(uint32_t r) const {
-        return acc[r] >= (static_cast<unsigned long long>(lim[r]) << 16);
-    }
 };
 constexpr uint32_t kScratch = kNodeQ + kLeafItems;
-constexpr uint32_t kMegaQueueBytes = 5 * (kNodeQ + kLeafItems) + 64 * 12 + 128 * 24 + 128 * 8 + 64 * 16 + 128 * 4 +
-                                     64 * 4 + 128;
+constexpr uint32_t kMegaQueueBytes = 5 * (kNodeQ + kLeafItems) + 64 * 12 + 128 * 24 + 128 * 8 + 128 * 4 + 64 * 4 + 128;
 static_assert((5 * (kNodeQ + kLeafItems)) % 8 == 0, "the 8-byte arrays stay aligned");
 constexpr uint32_t kMegaBytes =
     ((64 * kLeafRow * 4 > kMegaQueueBytes ? 64 * kLeafRow * 4 : kMegaQueueBytes) + 15) / 16 * 16;
@@ -685,16 +709,62 @@ __device__ __forceinline__ MegaQueue mega_queue(uint32_t* lds) {
     q.rd = q.ro + 64 * 3;
     q.inv = q.rd + 128 * 3;
     q.acc = reinterpret_cast<unsigned long long*>(q.inv + 128 * 3);
-    q.prims = reinterpret_cast<const PrimRecord**>(q.acc + 128);
-    q.nodes = reinterpret_cast<const float4**>(q.prims + 64);
-    q.lim = reinterpret_cast<uint32_t*>(q.nodes + 64);
-    q.tree = q.lim + 128;
-    q.list = reinterpret_cast<uint8_t*>(q.tree + 64);
+    q.tmax = reinterpret_cast<float*>(q.acc + 128);
+    q.job = reinterpret_cast<uint32_t*>(q.tmax + 128);
+    q.list = reinterpret_cast<uint8_t*>(q.job + 64);
     return q;
 }
 // the calling thread's point-query queue over the same LDS
 __device__ __forceinline__ LeafQueue mega_leaf_queue(uint32_t* lds) {
     return LeafQueue{lds + (threadIdx.x >> 6) * (kMegaBytes / 4) + (threadIdx.x & 63u) * kLeafRow};
+}
+
+// The scene of a wavefront's paths.  Lanes may run jobs over different scenes
+// (batches, the server); when all paths of the wavefront share one (one, as
+// nearly always) its pointers are held in scalar registers and records are
+// read through 32-bit offsets from them, else each item's scene is looked up
+// through its lane's job.  A scene too large for the offsets takes the second
+// way as well.
+struct WaveScene {
+    bool one;
+    const PrimRecord* prims;
+    const float4* w4;
+    uint32_t half, leaf_base;
+    const JobDesc* jobs;
+};
+template <typename T>
+__device__ __forceinline__ const T* read_lane_ptr(const T* p, uint32_t l) {
+    const uint64_t v = reinterpret_cast<uint64_t>(p);
+    const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v), static_cast<int>(l)));
+    const uint32_t hi =
+        static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(v >> 32), static_cast<int>(l)));
+    return reinterpret_cast<const T*>((static_cast<uint64_t>(hi) << 32) | lo);
+}
+// on: the lanes with a path (at least one)
+__device__ __forceinline__ WaveScene wave_scene(const SceneView& sc, bool on, const JobDesc* jobs) {
+    const uint32_t lead = static_cast<uint32_t>(__builtin_ctzll(__builtin_amdgcn_ballot_w64(on)));
+    WaveScene ws;
+    ws.prims = read_lane_ptr(sc.prims, lead);
+    ws.w4 = read_lane_ptr(sc.w4, lead);
+    const uint32_t tree = static_cast<uint32_t>(
+        __builtin_amdgcn_readlane(static_cast<int>(sc.w4_levels | (sc.w4_half << 8)), static_cast<int>(lead)));
+    const uint32_t levels = tree & 0xffu;
+    ws.half = tree >> 8;
+    ws.leaf_base = w4_level_base(levels - 1u);
+    ws.jobs = jobs;
+    // records of 64 bytes (primitives) and at most 128 (nodes) within 2^32
+    ws.one = levels <= 13u && __builtin_amdgcn_ballot_w64(on && (sc.prims != ws.prims || sc.w4 != ws.w4)) == 0ull;
+    return ws;
+}
+// Record `prim` of the scene of lane own's path.
+__device__ __forceinline__ PrimRecord load_wave_prim(const MegaQueue& q, const WaveScene& ws, uint32_t own,
+                                                     uint32_t prim) {
+    if (ws.one) {
+        const auto* p = reinterpret_cast<const VP_GLOBAL_AS char*>(as_global(ws.prims)) +
+                        prim * static_cast<uint32_t>(sizeof(PrimRecord));
+        return load_prim((const PrimRecord*)p, 0u);
+    }
+    return load_prim(ws.jobs[q.job[own]].scene.prims, prim);
 }
 
 // Exclusive prefix sum over the wavefront of v <= 7 (every lane active).
@@ -709,33 +779,43 @@ __device__ __forceinline__ uint32_t wave_prefix3(uint32_t v, uint32_t& total) {
 // One node step of the wavefront: the top items of the stack (nn of them in
 // all, at least one), as many as the lanes and the room left allow, are
 // replaced by their crossed children, and crossed leaves are appended to the
-// leaf queue (nl items, leaf_cap at most).  kArgmin: a ray is tested over
-// [0, its running minimum], or over its whole length until its direct-term
-// depth reaches the limit; else (shadow rays) over its whole length, and not
-// at all once its depth has reached the limit.
-template <bool kArgmin>
-__device__ __forceinline__ void walk_nodes(const MegaQueue& q, uint32_t& nn, uint32_t& nl, uint32_t leaf_cap) {
+// leaf queue (nl items, leaf_cap at most).  A ray is tested over [0, its
+// tmax], and not at all once that is negative.
+// The order of the children on the stack: for the argmin, nearest first and
+// lane by lane, so a few rays at a time reach their nearest leaves and the
+// bounds they prune by; for shadow rays, first children of all lanes first, so
+// the step's rays descend together and one that reaches its limit leaves few
+// items behind.  (Lane by lane in index order for both, an argmin flight kept
+// waiting: 10^6 cloud 310 ms, torus 49, scattering 26.9; nearest first: 281,
+// 42.6, 27.0; first children first for the shadow rays as well: 266, 41.7,
+// 26.7; for both: 258, 46, 25.0.)
+template <bool kNearFirst>
+__device__ __forceinline__ void walk_nodes(const MegaQueue& q, const WaveScene& ws, uint32_t& nn, uint32_t& nl,
+                                           uint32_t leaf_cap) {
     const uint32_t lane = __lane_id();
     const uint32_t room = nn + kNodeReserve + 3u < kNodeQ ? (kNodeQ - kNodeReserve - nn) / 3u : 1u;
     uint32_t n = nn < 64u ? nn : 64u;
     n = n < room ? n : room;
-    uint32_t node = 0, ray = 0, m = 0, child = 0;
-    bool last = false;
+    nn -= n;
+    uint32_t node = 0, ray = 0, m = 0, base = ws.leaf_base;
+    float tn[4] = {0.0f, 0.0f, 0.0f, 0.0f};
     if (lane < n) {
-        node = q.node[nn - n + lane];
-        ray = q.node_ray[nn - n + lane];
-        const uint32_t own = ray >> 1;
-        const bool full = q.full(ray);
-        if (kArgmin || !full) {
-            const f3 inv = lds_load3(q.inv + 3 * ray), oi = lds_load3(q.ro + 3 * own) * inv;
-            const float tmax = kArgmin && full ? __uint_as_float(q.ts(own)) : kTMax;
-            const uint32_t tree = q.tree[own], base = w4_level_base((tree & 0xffu) - 1u);
-            m = mega_ray_mask(q.nodes[own], tree >> 8, node, inv, oi, tmax);
-            last = node >= base;
-            child = last ? 4u * (node - base) : 4u * node + 1u;
+        node = q.node[nn + lane];
+        ray = q.node_ray[nn + lane];
+        const float tmax = q.tmax[ray];
+        const f3 inv = lds_load3(q.inv + 3 * ray), oi = lds_load3(q.ro + 3 * (ray >> 1)) * inv;
+        if (tmax >= 0.0f) {
+            if (ws.one) {
+                m = mega_ray_mask(ws.w4, ws.half, node, inv, oi, tmax, tn);
+            } else {
+                const SceneView& sc = ws.jobs[q.job[ray >> 1]].scene;
+                m = mega_ray_mask(sc.w4, sc.w4_half, static_cast<size_t>(node), inv, oi, tmax, tn);
+                base = w4_level_base(sc.w4_levels - 1u);
+            }
         }
     }
-    nn -= n;
+    const bool last = node >= base;
+    uint32_t child = last ? 4u * (node - base) : 4u * node + 1u;
     wave_sync();
     uint32_t push = last ? 0u : m;
     if (__builtin_amdgcn_ballot_w64(last && m != 0u) != 0ull) {
@@ -759,39 +839,73 @@ __device__ __forceinline__ void walk_nodes(const MegaQueue& q, uint32_t& nn, uin
         nl += total;
     }
     if (__builtin_amdgcn_ballot_w64(push != 0u) != 0ull) {
-        uint32_t total;
-        uint32_t at = nn + wave_prefix3(static_cast<uint32_t>(__popc(push)), total);
-        for (uint32_t b = push; b != 0u; b &= b - 1u, ++at) {
-            q.node[at] = child + static_cast<uint32_t>(__builtin_ctz(b));
+        auto put = [&](uint32_t at, uint32_t c) {
+            q.node[at] = child + c;
             q.node_ray[at] = static_cast<uint8_t>(ray);
+        };
+        if constexpr (kNearFirst) {
+            // the nearest child on top, its sibling below it, then the others
+            // (children c ^ s, c descending)
+            const float a = fminf(tn[0], tn[1]), b = fminf(tn[2], tn[3]);
+            uint32_t s = b < a ? (tn[3] < tn[2] ? 3u : 2u) : (tn[1] < tn[0] ? 1u : 0u);
+            if (last) s = 0u;
+            push = (s & 1u) != 0u ? ((push & 5u) << 1) | ((push >> 1) & 5u) : push;
+            push = (s & 2u) != 0u ? ((push & 3u) << 2) | (push >> 2) : push;
+            const uint32_t c = static_cast<uint32_t>(__popc(push));
+            uint32_t total;
+            uint32_t at = nn + wave_prefix3(c, total) + c;
+            for (uint32_t b = push; b != 0u; b &= b - 1u) put(--at, static_cast<uint32_t>(__builtin_ctz(b)) ^ s);
+            nn += total;
+        } else {
+            // every lane's first child on top, below them the second ones, and
+            // so on: the next step goes on with all the rays of this one
+            const uint32_t c = static_cast<uint32_t>(__popc(push));
+            const unsigned long long b0 = __builtin_amdgcn_ballot_w64(c > 0u);
+            const unsigned long long b1 = __builtin_amdgcn_ballot_w64(c > 1u);
+            const unsigned long long b2 = __builtin_amdgcn_ballot_w64(c > 2u);
+            const unsigned long long b3 = __builtin_amdgcn_ballot_w64(c > 3u);
+            const uint32_t t2 = nn + static_cast<uint32_t>(__popcll(b3)), t1 = t2 + static_cast<uint32_t>(__popcll(b2));
+            const uint32_t t0 = t1 + static_cast<uint32_t>(__popcll(b1));
+            auto put_next = [&](uint32_t at) {
+                put(at, static_cast<uint32_t>(__builtin_ctz(push)));
+                push &= push - 1u;
+            };
+            if (c > 0u) {
+                put_next(t0 + lanes_below(b0));
+                if (c > 1u) {
+                    put_next(t1 + lanes_below(b1));
+                    if (c > 2u) {
+                        put_next(t2 + lanes_below(b2));
+                        if (c > 3u) put_next(nn + lanes_below(b3));
+                    }
+                }
+            }
+            nn = t0 + static_cast<uint32_t>(__popcll(b0));
         }
-        nn += total;
     }
     wave_sync();
 }
 
 // The shadow rays of a wavefront's lanes, up to two each (the MIS rays a and
-// b, or the one of RIS).  All 64 lanes of the wavefront call it.  q.ro,
-// q.prims, q.rd and q.acc hold the rays' origins, primitive arrays,
-// directions and the depths of their origin sets.  Each ray's chords are
-// summed in fixed point in LDS (a ray is saturated once its sum reaches the
-// tau = 88 limit, in whatever order the chords arrive), so Ta and Tb equal two
-// transmittance() calls bit for bit.
+// b, or the one of RIS).  All 64 lanes of the wavefront call it.  q.ro, q.job,
+// q.rd and q.acc hold the rays' origins, jobs, directions and the depths of
+// their origin sets.  Each ray's chords are summed in fixed point in LDS (a
+// ray is saturated once its sum reaches the tau = 88 limit, in whatever order
+// the chords arrive), so Ta and Tb equal two transmittance() calls bit for
+// bit.
 // Each ray's walk may stop once its depth reaches its limit (lim_a, lim_b:
-// the tau = 88 saturation, or a shadow-roulette threshold; multiples of
-// 2^16); a limit of 0 is a ray that is not walked.  acc_a and acc_b receive
-// the fixed-point depths.
-__device__ __forceinline__ void shadow_walks(const SceneView& s, const MegaQueue& q, uint64_t lim_a, uint64_t lim_b,
-                                             uint64_t& acc_a, uint64_t& acc_b) {
+// the tau = 88 saturation, or a shadow-roulette threshold); a limit of 0 is a
+// ray that is not walked.  acc_a and acc_b receive the fixed-point depths;
+// rounds counts the node steps and leaf rounds.
+__device__ __forceinline__ void shadow_walks(const WaveScene& ws, const MegaQueue& q, uint64_t lim_a, uint64_t lim_b,
+                                             uint64_t& acc_a, uint64_t& acc_b, uint32_t& rounds) {
     const uint32_t lane = __lane_id();
-    q.nodes[lane] = s.w4;
-    q.tree[lane] = s.w4_levels | (s.w4_half << 8);
-    q.lim[2 * lane] = static_cast<uint32_t>(lim_a >> 16);
-    q.lim[2 * lane + 1] = static_cast<uint32_t>(lim_b >> 16);
     lds_store3(q.inv + 3 * (2 * lane), safe_inv(lds_load3(q.rd + 3 * (2 * lane))));
     lds_store3(q.inv + 3 * (2 * lane + 1), safe_inv(lds_load3(q.rd + 3 * (2 * lane + 1))));
     // the rays to walk: every ray a, then every ray b, that is not done already
-    const bool walk_a = !q.full(2 * lane), walk_b = !q.full(2 * lane + 1);
+    const bool walk_a = q.acc[2 * lane] < lim_a, walk_b = q.acc[2 * lane + 1] < lim_b;
+    q.tmax[2 * lane] = walk_a ? kTMax : -1.0f;
+    q.tmax[2 * lane + 1] = walk_b ? kTMax : -1.0f;
     const unsigned long long pa = __builtin_amdgcn_ballot_w64(walk_a);
     const unsigned long long pb = __builtin_amdgcn_ballot_w64(walk_b);
     const uint32_t npa = static_cast<uint32_t>(__popcll(pa));
@@ -802,7 +916,7 @@ __device__ __forceinline__ void shadow_walks(const SceneView& s, const MegaQueue
     uint32_t next = 0, nn = 0, nl = 0;
     while (true) {
         if (nn < 64u && next < nr) {
-            // the next rays start at the root, up to an item per lane
+            // the next rays start at the root
             const uint32_t k = nr - next < 64u - nn ? nr - next : 64u - nn;
             if (lane < k) {
                 q.node[nn + lane] = 0u;
@@ -813,7 +927,8 @@ __device__ __forceinline__ void shadow_walks(const SceneView& s, const MegaQueue
             wave_sync();
         }
         if (nl < 64u && nn != 0u) {
-            walk_nodes<false>(q, nn, nl, kLeafItems);
+            walk_nodes<false>(q, ws, nn, nl, kLeafItems);
+            ++rounds;
             continue;
         }
         if (nl == 0u) break;
@@ -821,14 +936,20 @@ __device__ __forceinline__ void shadow_walks(const SceneView& s, const MegaQueue
         // whole-chord depth from one transform) goes into its ray's sum
         const uint32_t n = nl < 64u ? nl : 64u;
         nl -= n;
-        if (lane < n) {
-            const uint32_t ray = q.leaf_ray[nl + lane], own = ray >> 1;
-            if (!q.full(ray)) {
-                const PrimRecord pr = load_prim(q.prims[own], q.leaf[nl + lane]);
+        ++rounds;
+        {
+            const bool on = lane < n;
+            const uint32_t ray = on ? q.leaf_ray[nl + lane] : 0u, own = ray >> 1;
+            const bool live = on && q.tmax[ray] >= 0.0f;
+            const PrimRecord pr = load_wave_prim(q, ws, own, live ? q.leaf[nl + lane] : 0u);
+            if (live) {
                 const Crossing x = crossing(pr, lds_load3(q.ro + 3 * own), lds_load3(q.rd + 3 * ray));
                 if (x.tau > 0.0f) atomicAdd(&q.acc[ray], tau_fixed(x.tau));
             }
         }
+        wave_sync();
+        if (q.acc[2 * lane] >= lim_a) q.tmax[2 * lane] = -1.0f;
+        if (q.acc[2 * lane + 1] >= lim_b) q.tmax[2 * lane + 1] = -1.0f;
         wave_sync();
     }
     acc_a = q.acc[2 * lane];

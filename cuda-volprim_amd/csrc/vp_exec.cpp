@@ -158,7 +158,8 @@ RenderLaunch vp_resolve_launch(vp_context* ctx, const vp_launch_config* cfg, uin
     // a wavefront claims paths once 8 of its lanes are idle (measured best on
     // the scattering workload: 15.9 against 15.5 Msamples/s at 1)
     L.regen_min = std::max<uint32_t>(1u, std::min<uint32_t>(64u, c.regen_min ? c.regen_min : 8u));
-    L.lane_max = 64u;
+    L.first_paths = 4u;
+    L.claim_step = 8u;
     L.count_events = count;
     L.measure = measure;
     // the wavefront pipeline has no event-counting or measuring variant
@@ -183,18 +184,21 @@ RenderLaunch vp_resolve_launch(vp_context* ctx, const vp_launch_config* cfg, uin
 
 // A launch below one path per lane is bound by latency: a path is a serial
 // chain of walks, set rebuilds and roulettes, so its paths are spread over as
-// many wavefronts as there are, whose other lanes help with the walks.  From
-// one path per lane on (262144 on 256 CUs) lane_max is 64, as before.  With at
-// least 1, 2, 4, 8 and 16 paths per wavefront: 64x64x2 scattering image 3.7,
-// 3.8, 4.1, 4.1, 5.2 ms (22.5 ms when every wavefront took 64), 157x83x3 of 97
-// Gaussians 0.84, 0.82, 0.78, 0.88, 0.97 (2.7), 192x128x2 cloud 51, 49, 45, 50,
-// 70 (290), so one path is enough.
+// many wavefronts as there are, whose other lanes help with the walks (a
+// 64x64x2 scattering image took 22.5 ms when every wavefront took 64 paths).
+// A wavefront starts on up to 4 paths and then claims up to 8 at a time, or a
+// third of its share of a small launch, which leaves the paths of the costly
+// wavefronts to the others.  Starting on 4 and claiming 4, 8 and 16: 192x128x2
+// cloud (12 paths per wavefront) 17, 24, 38 ms, 512x512x1 torus (64) 19.9, 20.2,
+// 21.9, 256x256x24 scattering (384) 27.0, 26.4, 26.1.
 RenderLaunch vp_size_launch(RenderLaunch L, uint64_t paths) {
     const uint64_t waves_per_block = L.block / 64u;
     L.grid = static_cast<uint32_t>(
         std::max<uint64_t>(1u, std::min<uint64_t>(L.grid, (paths + waves_per_block - 1) / waves_per_block)));
     const uint64_t waves = L.grid * waves_per_block;
-    L.lane_max = static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>(64u, (paths + waves - 1) / waves)));
+    const uint64_t share = (paths + waves - 1) / waves;
+    L.first_paths = static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>(4u, share)));
+    L.claim_step = static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>(8u, (share + 2u) / 3u)));
     return L;
 }
 
@@ -285,7 +289,7 @@ vp_status vp_run_step(vp_context* ctx, const RenderLaunch& L, uint32_t nslices, 
         VP_HIP_TRY(enqueue());
         return VP_OK;
     }
-    const uint64_t key[6] = {L.block, L.grid, (uint64_t(L.active_cap) << 16) | (L.lane_max << 8) | L.regen_min,
+    const uint64_t key[6] = {L.block, L.grid, (uint64_t(L.active_cap) << 32) | (L.first_paths << 16) | (L.claim_step << 8) | L.regen_min,
                              uint64_t(L.count_events) << 1 | uint64_t(L.measure), (uint64_t(max_jobs) << 32) | max_npix,
                              reinterpret_cast<uint64_t>(s)};
     if (!ctx->graph_exec || !std::equal(key, key + 6, ctx->graph_key)) {

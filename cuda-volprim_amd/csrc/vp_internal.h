@@ -300,7 +300,8 @@ struct RenderLaunch {
     uint32_t grid;
     uint32_t active_cap;
     uint32_t regen_min;
-    uint32_t lane_max;  // megakernel: lanes of a wavefront that hold a path (vp_size_launch)
+    uint32_t first_paths;  // megakernel: paths a wavefront starts on, and the most it claims at
+    uint32_t claim_step;   // a time from then on (vp_size_launch)
     int count_events;
     int measure;
     uint32_t pipeline;  // VP_PIPELINE_MEGAKERNEL or VP_PIPELINE_WAVEFRONT
@@ -333,7 +334,7 @@ void vp_drop_graph(vp_context* ctx);
 RenderLaunch vp_resolve_launch(vp_context* ctx, const vp_launch_config* cfg, uint32_t active_cap, int count,
                                int measure);
 // L for a megakernel launch over `paths` paths: no more workgroups than have a
-// path for each wavefront, and the paths spread over all wavefronts.
+// path for each wavefront, and the paths' hand-out.
 RenderLaunch vp_size_launch(RenderLaunch L, uint64_t paths);
 // One step over the first nslices entries of the pinned job table (capacity max_jobs).
 vp_status vp_run_step(vp_context* ctx, const RenderLaunch& L, uint32_t nslices, uint64_t total_paths,

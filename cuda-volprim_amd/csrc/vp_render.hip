@@ -17,31 +17,18 @@
 //      phase and environment sampling, or product RIS) with shadow rays whose
 //      optical depth is accumulated in fixed point;
 //   4. applies Russian roulette and the throughput guards.
-// The argmin and MIS shadow walks share one leaf queue per wavefront: every
-// lane walks a ray, and the leaves all rays cross are evaluated by whichever
-// lanes are free (see WaveQueue).
-// Each path writes its radiance to a per-sample slot; a second kernel folds
-// slots into the per-pixel Welford mean in sample order, so the image does
-// not depend on which lane ran which path or on what else shared the launch.
+// The argmin and shadow walks and the work on the active sets are done by the
+// 64 lanes of a wavefront together, for all its paths.
+// Each path adds its radiance to its pixel's exact fixed-point sums; a second
+// kernel divides them, so the image does not depend on which lane ran which
+// path or on what else shared the launch.
 //
 // Reference (kfernandez31/cuda-volprim): device/entry/raygen.cuh:21-243,
 // device/entry/path_stages.cuh:25-226, device/core/sampling.cuh:257-583,
 // device/entry/anyhit.cuh:53-86, device/kernels/normalize_accumulator.cu:16-35.
-// The megakernel holds a whole path and a walk per lane, so it is tuned for
-// registers over occupancy: 4 waves per SIMD (128 VGPRs), a 512-entry shared
-// leaf queue in the LDS this frees (16 waves x 9856 bytes of the CU's
-// 160 KiB), and the near/far node test.  On the scattering workload (4096
-// Gaussians, 512x512, 64 spp): 26.5 Msamples/s with 448 entries, against 23.6
-// at 6 waves with a 224-entry queue and the min/max test, 26.0 at 5 waves
-// (320 entries) and 24.5 at 3 waves (640 entries); with the leaf-block walks,
-// which fill the queue four leaves at a time, 512 entries gained 0.6-1.2 %
-// over 448.
-#ifndef VP_WAVE_Q
-#define VP_WAVE_Q 512
-#endif
-#ifndef VP_MEGA_NEAR_FAR
-#define VP_MEGA_NEAR_FAR 1
-#endif
+// The megakernel holds a whole path per lane at 4 waves per SIMD (128 VGPRs);
+// a wavefront's queues and ray tables take the 10 KiB of LDS that 16 waves
+// leave each other of a CU's 160 KiB.
 #include "vp_device.h"
 
 namespace vp {
@@ -76,17 +63,19 @@ struct PathState {
 // 0); from there on it prunes at the running minimum like any other ray.
 // ts_origin is the minimum over the origin set; the result keeps it unless a
 // walk candidate is strictly smaller.
-// Flights waiting to be inverted are taken up once there are VP_FLIGHT_MIN of
+// Flights waiting to be inverted are taken up once there are kFlightMin of
 // them (few leaves have one, and the inversion's erf and erfinv cost as much
-// as the leaf round), or at the end of a run of leaves.
-#ifndef VP_FLIGHT_MIN
-#define VP_FLIGHT_MIN 16u
-#endif
-__device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& sc, f3 o, f3 d, uint64_t key,
+// as the leaf round), or at the end of a run of leaves.  A flight ends inside
+// its chord, so until then its exit bounds the minimum (bound, which the walk
+// prunes by): without that bound, waiting for 16 flights cost the 10^6 cloud
+// 12 % and the 192x128 cloud 18 % against waiting for 4; with it, nothing.
+constexpr uint32_t kFlightMin = 16;
+__device__ __forceinline__ void argmin_walk_shared(bool alive, const WaveScene& ws, uint32_t job, f3 o, f3 d, uint64_t key,
                                                    uint32_t b, bool direct, const uint32_t* act, uint32_t na_path,
                                                    float* act_exit, float ts_set, uint32_t* __restrict__ slab,
                                                    uint32_t cap, const MegaQueue& q, float& ts, uint32_t& nc,
-                                                   uint64_t dlimit, uint64_t& dacc) {
+                                                   uint64_t dlimit, uint64_t& dacc,
+                                                   uint32_t& rounds) {
     const uint32_t lane = __lane_id();
     const uint32_t na = direct ? na_path : 0u;
     lds_store3(q.ro + 3 * lane, o);
@@ -95,11 +84,8 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& 
     q.draw(lane)[0] = static_cast<uint32_t>(key);
     q.draw(lane)[1] = static_cast<uint32_t>(key >> 32);
     q.draw(lane)[2] = b | (direct ? 0x80000000u : 0u);
-    q.prims[lane] = sc.prims;
-    q.nodes[lane] = sc.w4;
-    q.tree[lane] = sc.w4_levels | (sc.w4_half << 8);
+    q.job[lane] = job;
     q.acc[2 * lane] = 0ull;
-    q.lim[2 * lane] = direct ? static_cast<uint32_t>(dlimit >> 16) : 0u;
     q.ts(lane) = __float_as_uint(direct ? kTMax : ts_set);
     q.nc(lane) = 0u;
     // the path key and bounce of lane l's draws
@@ -129,7 +115,7 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& 
         for (uint32_t g = lane; g < total; g += 64u) {
             const uint32_t ol = prefix_owner(pre_of, g), k = g - pre_of[ol];
             const uint32_t i = set_of[ol][k];
-            const PrimRecord pr = load_prim(q.prims[ol], i);
+            const PrimRecord pr = load_prim(ws.jobs[q.job[ol]].scene.prims, i);
             const f3 ro = lds_load3(q.ro + 3 * ol), rd = lds_load3(q.rd + 3 * (2 * ol));
             const InsideChord x = inside_chord(pr, ro, rd);
             exit_of[ol][k] = x.t1;
@@ -143,6 +129,12 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& 
     }
     wave_sync();
     const float ts_origin = __uint_as_float(q.ts(lane));
+    // a ray is walked up to the bound of its minimum, a direct one whole until
+    // its depth reaches the limit
+    const uint64_t lim = direct ? dlimit : 0ull;
+    auto set_tmax = [&]() { q.tmax[2 * lane] = q.acc[2 * lane] < lim ? kTMax : __uint_as_float(q.bound(lane)); };
+    q.bound(lane) = q.ts(lane);
+    set_tmax();
     // the first thread of this wavefront, for the owners' candidate buffers
     const uint32_t gbase = blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
     const uint32_t bs = mega_slab_stride(cap);
@@ -156,10 +148,12 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& 
         }
         nn = static_cast<uint32_t>(__popcll(am));
     }
+    static_assert(kLeafItems >= 64u + kFlightMin + 64 + 4, "room for a step's leaves and the flights");
     wave_sync();
     while (true) {
         if (nl < 64u && nn != 0u) {
-            walk_nodes<true>(q, nn, nl, kLeafItems - nf);
+            walk_nodes<true>(q, ws, nn, nl, kLeafItems - nf);
+            ++rounds;
             continue;
         }
         if (nl != 0u) {
@@ -172,18 +166,18 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& 
             // chord's.
             const uint32_t n = nl < 64u ? nl : 64u;
             nl -= n;
+            ++rounds;
             bool keep = false;
-            uint32_t ray = 0, prim = 0;
-            if (lane < n) {
-                ray = q.leaf_ray[nl + lane];
-                prim = q.leaf[nl + lane];
-                const uint32_t own = ray >> 1;
-                const PrimRecord pr = load_prim(q.prims[own], prim);
+            const bool on = lane < n;
+            const uint32_t ray = on ? q.leaf_ray[nl + lane] : 0u, own = ray >> 1;
+            const uint32_t prim = on ? q.leaf[nl + lane] : 0u;
+            const PrimRecord pr = load_wave_prim(q, ws, own, prim);
+            if (on) {
                 const Crossing x = crossing(pr, lds_load3(q.ro + 3 * own), lds_load3(q.rd + 3 * ray));
                 if (x.t0 >= 0.0f) {
                     const uint32_t meta = q.draw(own)[2];
                     if ((meta >> 31) != 0u && x.tau > 0.0f) atomicAdd(&q.acc[ray], tau_fixed(x.tau));
-                    if (x.t0 <= __uint_as_float(q.ts(own))) {
+                    if (x.t0 <= __uint_as_float(q.bound(own))) {
                         const uint32_t pos = atomicAdd(&q.nc(own), 1u);
                         if (pos < cap) {
                             uint32_t* mine = slab + static_cast<size_t>(gbase + own) * kMegaSlabBuffers * bs;
@@ -193,6 +187,7 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& 
                         }
                         const float tau = free_flight_tau(prim_uniform(key_of(own), meta & 0x7fffffffu, 1u, prim));
                         keep = tau <= x.tau;
+                        if (keep) atomicMin(&q.bound(own), __float_as_uint(x.t1));
                     }
                 }
             }
@@ -207,19 +202,25 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const SceneView& 
             }
             nf += static_cast<uint32_t>(__popcll(km));
             wave_sync();
+            set_tmax();
+            wave_sync();
         }
-        if (nf >= VP_FLIGHT_MIN || (nl == 0u && nf != 0u)) {
+        if (nf >= kFlightMin || (nl == 0u && nf != 0u)) {
             // invert the waiting flights into distances
             for (uint32_t f = lane; f < nf; f += 64u) {
                 const uint32_t ray = q.leaf_ray[kLeafItems - 1u - f], prim = q.leaf[kLeafItems - 1u - f];
                 const uint32_t own = ray >> 1;
                 const f3 ro = lds_load3(q.ro + 3 * own), rd = lds_load3(q.rd + 3 * ray);
-                const PrimRecord pr = load_prim(q.prims[own], prim);
+                const PrimRecord pr = load_prim(ws.jobs[q.job[own]].scene.prims, prim);
                 const float tau = free_flight_tau(prim_uniform(key_of(own), bounce_of(own), 1u, prim));
                 const float t = entered_flight(pr, ro, rd, crossing(pr, ro, rd), tau);
-                atomicMin(&q.ts(own), t == 0.0f ? 0u : __float_as_uint(t));
+                const uint32_t tb = t == 0.0f ? 0u : __float_as_uint(t);
+                atomicMin(&q.ts(own), tb);
+                atomicMin(&q.bound(own), tb);
             }
             nf = 0;
+            wave_sync();
+            set_tmax();
             wave_sync();
         }
         if (nl == 0u && nn == 0u) break;
@@ -389,7 +390,7 @@ __device__ __forceinline__ uint32_t rebuild_shared(bool part, uint32_t na, uint3
 // order; the shadow rays' fixed-point depths stay in q.acc; ts_next receives
 // the minimum free flight of the next ray over the set, kTMax if none.
 // da, db and wo are the two shadow rays' and the next ray's directions from x.
-__device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has_a, bool has_b, const SceneView& sc,
+__device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has_a, bool has_b, const WaveScene& ws,
                                              f3 x, f3 da, f3 db, f3 wo, uint64_t key, uint32_t b1,
                                              uint32_t* __restrict__ slab, uint32_t cap, const MegaQueue& q,
                                              float& ts_next) {
@@ -408,7 +409,6 @@ __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has
     pre_of[lane] = wave_prefix(nn, total);
     meta_of[lane] = cur | (has_a ? 2u : 0u) | (has_b ? 4u : 0u);
     lds_store3(q.ro + 3 * lane, x);
-    q.prims[lane] = sc.prims;
     lds_store3(q.rd + 3 * (2 * lane), da);
     lds_store3(q.rd + 3 * (2 * lane + 1), db);
     q.acc[2 * lane] = 0ull;
@@ -418,12 +418,14 @@ __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has
     ts_of[lane] = __float_as_uint(kTMax);
     b_of[lane] = b1;
     wave_sync();
-    for (uint32_t g = lane; g < total; g += 64u) {
+    for (uint32_t base = 0; base < total; base += 64u) {
+        const uint32_t g = base + lane;
         const uint32_t own = prefix_owner(pre_of, g), k = g - pre_of[own];
         const uint32_t meta = meta_of[own], set = (meta & 1u) * bs;
         uint32_t* mine = slab_of(slab, gbase, own, bs);
-        const uint32_t i = mine[set + k];
-        const PrimRecord pr = load_prim(q.prims[own], i);
+        const uint32_t i = g < total ? mine[set + k] : 0u;
+        const PrimRecord pr = load_wave_prim(q, ws, own, i);
+        if (g >= total) continue;
         const f3 ro = lds_load3(q.ro + 3 * own);
         const f3 p = to_local_pos(pr, ro);
         const float pp = length2(p);
@@ -483,20 +485,32 @@ __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has
 // exactly once, without the retries a compare-and-swap on one shared counter
 // costs when paths are short.
 //
-// At most lane_max lanes of a wavefront hold a path (the host sets it so that
-// a launch with fewer paths than lanes spreads them over all its wavefronts).
+// How many of a wavefront's lanes hold a path: enough that a bounce's walks
+// take about kRoundsTarget rounds (node steps and leaf rounds), which its fixed
+// part (set-up, rebuild, sampling, the walks' ends) is small against, and not
+// more, since what a wavefront holds it has to finish by itself: a path of the
+// 10^6 cloud takes about 40 rounds a bounce and one of the scattering scene 5.
+// A wavefront starts on first_paths paths and claims at most claim_step at a
+// time, so it sees what its paths cost before it takes more (neighbouring
+// paths cost alike: with 64 paths to a wavefront, or a small launch's paths
+// handed out at once, the longest wavefront of the torus ran 3.1 times and of
+// the 192x128 cloud 9 times the mean).  At least 4 paths, target 128, 192 and
+// 256 rounds, scattering 27.3, 26.4, 25.9 ms, torus 19.9, 20.2, 20.6, 10^6 cloud
+// 202, 199, 197; 64 lanes always: 25.9, 41.3, 243.
 // The argmin and shadow walks are run by all 64 lanes of a wavefront together,
-// so lanes without a path (past lane_max, or at the end of a launch) work on
+// so lanes without a path work on
 // the rays of those that have one: a wavefront with two paths left evaluates
 // their members and leaves 64 at a time and shares out their walks.  Only the
 // timed build does so (kShared); the counting and the measuring build walk
 // each ray by its own lane.
+constexpr uint32_t kRoundsTarget = 256;
+constexpr uint32_t kPathsMin = 4;
 template <bool kCount, bool kMeasure>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VP_RENDER_WAVES_PER_EU)))
 k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begin,
          const uint64_t* __restrict__ launch_desc, unsigned long long* __restrict__ path_counter,
-         uint32_t* __restrict__ slab, uint32_t cap, uint32_t regen_min, uint32_t lane_max,
-         unsigned long long* __restrict__ counters) {
+         uint32_t* __restrict__ slab, uint32_t cap, uint32_t regen_min, uint32_t first_paths,
+         uint32_t claim_step, unsigned long long* __restrict__ counters) {
     constexpr bool kShared = !kCount && !kMeasure;
     extern __shared__ __align__(16) uint32_t s_leafq[];  // [blockDim.x][kLeafRow]
     const uint32_t njobs = static_cast<uint32_t>(launch_desc[0]);
@@ -521,7 +535,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
     uint32_t overflow = 0;
     // The launch's paths in kClaimParts parts.  The first paths of part k are
     // handed out without a counter: wavefront i of the workgroups with
-    // blockIdx % kClaimParts = k starts on its lane_max paths from i * lane_max
+    // blockIdx % kClaimParts = k starts on its first_paths paths from i * first_paths
     // (workgroups are dealt out to the XCDs in turn), so a launch with no more
     // paths than that needs no atomics (each wavefront's 8 on the way out took
     // 430 us of a 4096-path launch).  The rest of part k is claimed through
@@ -535,18 +549,21 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
     const uint32_t waves_per_block = blockDim.x / 64u;
     // paths of part k handed out at the start
     auto part_static = [&](uint32_t k) -> uint64_t {
-        return static_cast<uint64_t>((gridDim.x + kClaimParts - 1u - k) / kClaimParts) * waves_per_block * lane_max;
+        return static_cast<uint64_t>((gridDim.x + kClaimParts - 1u - k) / kClaimParts) * waves_per_block * first_paths;
     };
     uint32_t parts_done = 0;
     bool first = true;
-    const uint32_t claim_min = regen_min < lane_max ? regen_min : lane_max;
+    // paths this wavefront may hold, and the smoothed rounds of one per bounce
+    uint32_t limit = kShared ? first_paths : 64u, work = 0;
 
     while (true) {
         // ---- claim new paths for idle lanes: one atomic per wavefront and part tried ----
         const unsigned long long idle = __builtin_amdgcn_ballot_w64(!alive);
         const uint32_t busy = 64u - static_cast<uint32_t>(__popcll(idle));
-        const uint32_t room = lane_max > busy ? lane_max - busy : 0u;
+        uint32_t room = limit > busy ? limit - busy : 0u;
+        const uint32_t claim_min = regen_min < (limit + 1u) / 2u ? regen_min : (limit + 1u) / 2u;
         if (!exhausted && room != 0u && (room >= claim_min || busy == 0u)) {
+            if (kShared && room > claim_step) room = claim_step;
             const uint32_t leader = static_cast<uint32_t>(__builtin_ctzll(idle));
             unsigned long long base = 0;
             uint32_t got = 0;
@@ -555,8 +572,8 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
                 const uint64_t lo_k = path_lo + k * part;
                 const uint64_t hi_k = lo_k + part < total_paths ? lo_k + part : total_paths;
                 base = lo_k + (static_cast<uint64_t>(blockIdx.x / kClaimParts) * waves_per_block +
-                               __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * lane_max;
-                if (base < hi_k) got = hi_k - base < lane_max ? static_cast<uint32_t>(hi_k - base) : lane_max;
+                               __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * first_paths;
+                if (base < hi_k) got = hi_k - base < first_paths ? static_cast<uint32_t>(hi_k - base) : first_paths;
                 first = false;
             }
             if (got == 0u) {
@@ -675,14 +692,18 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
             return shadow_rr(max3(kd), J.shadow_rr, st.key, 0u, 2u);
         };
         uint64_t dwalk = 0;
+        WaveScene ws{};
+        uint32_t rounds = 0;
+        const uint32_t nalive = static_cast<uint32_t>(__popcll(__builtin_amdgcn_ballot_w64(alive)));
         if constexpr (kShared) {
+            ws = wave_scene(sc, alive, jobs);
             uint64_t dlimit = kTauLimitFixed;
             if (direct) {
                 f3 kd;
                 dlimit = direct_rr(kd).limit();
             }
-            argmin_walk_shared(alive, sc, o, d, st.key, b, direct, act, na, act_exit, st.ts_set, slab, cap, q, ts, nc,
-                               dlimit, dwalk);
+            argmin_walk_shared(alive, ws, st.job, o, d, st.key, b, direct, act, na, act_exit, st.ts_set, slab, cap, q, ts, nc,
+                               dlimit, dwalk, rounds);
         } else {
             for (uint32_t k = 0; k < na; ++k) {
                 const uint32_t i = act[k * stride];
@@ -898,7 +919,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         // evaluate_albedo (sampling.cuh:257-283)
         f3 albedo;
         if constexpr (kShared) {
-            albedo = vertex_members(nn, st.cur, has_a, has_b, sc, x, da, db, wo, st.key, b + 1u, slab, cap, q,
+            albedo = vertex_members(nn, st.cur, has_a, has_b, ws, x, da, db, wo, st.key, b + 1u, slab, cap, q,
                                     st.ts_set);
         } else {
             f3 aa = mk(0.0f);
@@ -949,7 +970,11 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         // them one by one, so the former's counts are per-ray work)
         uint64_t acc_a = 0, acc_b = 0;
         if constexpr (kShared) {
-            shadow_walks(sc, q, lim_a, lim_b, acc_a, acc_b);
+            shadow_walks(ws, q, lim_a, lim_b, acc_a, acc_b, rounds);
+            // the bounce's rounds per path, smoothed over bounces, in sixteenths
+            work = (3u * work + 16u * rounds / nalive) / 4u;
+            limit = 16u * kRoundsTarget / (work + 1u);
+            limit = limit < kPathsMin ? kPathsMin : (limit < 64u ? limit : 64u);
         } else {
             if (has_a) acc_a = shadow_depth(sc, x, da, act, nn, stride, lq, ev, lim_a);
             if (has_b) acc_b = shadow_depth(sc, x, db, act, nn, stride, lq, ev, lim_b);
@@ -1193,7 +1218,7 @@ __global__ void k_prim(int fn, const PrimRecord* __restrict__ rec, const float* 
 }
 
 using RenderKernel = void (*)(const JobDesc*, const uint64_t*, const uint64_t*, unsigned long long*, uint32_t*,
-                              uint32_t, uint32_t, uint32_t, unsigned long long*);
+                              uint32_t, uint32_t, uint32_t, uint32_t, unsigned long long*);
 RenderKernel render_kernel(int count_events, int measure) {
     if (count_events) return measure ? k_render<true, true> : k_render<true, false>;
     return measure ? k_render<false, true> : k_render<false, false>;
@@ -1216,7 +1241,7 @@ hipError_t vp_launch_render(const RenderLaunch& L, const JobDesc* jobs, const ui
     const size_t lds = mega_queue_bytes(L.block);
     const auto k = render_kernel(L.count_events, L.measure);
     hipLaunchKernelGGL(k, dim3(L.grid), dim3(L.block), lds, s, jobs, job_begin, launch_desc, counter, slab,
-                       L.active_cap, L.regen_min, L.lane_max, counters);
+                       L.active_cap, L.regen_min, L.first_paths, L.claim_step, counters);
     return hipGetLastError();
 }
 
