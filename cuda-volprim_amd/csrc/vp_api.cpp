@@ -261,8 +261,17 @@ vp_status vp_scene_export(vp_scene* sc, uint32_t* order, uint32_t* morton, float
     hipStream_t s = sc->ctx->stream;
     if (order) VP_HIP_TRY(hipMemcpyAsync(order, sc->order, sizeof(uint32_t) * sc->n, hipMemcpyDeviceToHost, s));
     if (morton) VP_HIP_TRY(hipMemcpyAsync(morton, sc->morton, sizeof(uint32_t) * sc->n, hipMemcpyDeviceToHost, s));
-    if (records16)
-        VP_HIP_TRY(hipMemcpyAsync(records16, sc->prims, sizeof(vp::PrimRecord) * sc->n, hipMemcpyDeviceToHost, s));
+    // the records in the exported field order, through a stream-ordered copy
+    void* rec = nullptr;
+    hipError_t e = hipSuccess;
+    if (records16) {
+        const size_t bytes = sizeof(vp::PrimRecord) * sc->n;
+        e = hipMallocAsync(&rec, bytes, s);
+        if (e == hipSuccess) e = vp_launch_export_records(sc->prims, sc->n, static_cast<float4*>(rec), s);
+        if (e == hipSuccess) e = hipMemcpyAsync(records16, rec, bytes, hipMemcpyDeviceToHost, s);
+        if (rec) (void)hipFreeAsync(rec, s);
+    }
+    VP_HIP_TRY(e);
     VP_HIP_TRY(hipStreamSynchronize(s));
     if (depth) *depth = sc->depth;
     return VP_OK;

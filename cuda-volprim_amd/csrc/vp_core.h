@@ -70,17 +70,20 @@ constexpr float kTauScaleF = 1099511627776.0f;
 constexpr uint64_t kTauLimitFixed = 96757023244288ull;  // 88 * 2^40
 
 // ---------------------------------------------------------------------------
-// Primitive record: 64 bytes, the reference's hot fields in its order.
+// Primitive record: 64 bytes.  The first 48 are what a ray's crossing needs,
+// so a leaf test is three 16-byte loads.
 // ---------------------------------------------------------------------------
 struct alignas(16) PrimRecord {
     float cx, cy, cz;     // centre
     float qw, qx, qy, qz; // CONJUGATE of the forward rotation (world -> local)
     float rsx, rsy, rsz;  // 1 / scale
     float dnf;            // density_norm_factor = (2 pi)^(-3/2) / prod(scale)
-    float icf;            // inv_cdf_factor = M * dnf * sqrt(pi/2)
+    float md;             // M * dnf
     float ar, ag, ab;     // albedo
     float mass;           // optical_thickness M (total mass)
 };
+// inv_cdf_factor = M * dnf * sqrt(pi/2)
+#define VP_ICF(pr) ((pr).md * kRootHalfPi)
 static_assert(sizeof(PrimRecord) == 64, "PrimRecord must stay 64 bytes");
 
 // Build a record from a forward rotation (w, x, y, z), per-axis scale, albedo
@@ -101,7 +104,7 @@ VP_HD PrimRecord make_prim(f3 c, float w, float x, float y, float z, f3 scale, f
     p.rsy = 1.0f / scale.y;
     p.rsz = 1.0f / scale.z;
     p.dnf = kOneOverTwoPiPow32 * (p.rsx * p.rsy * p.rsz);
-    p.icf = mass * p.dnf * kRootHalfPi;
+    p.md = mass * p.dnf;
     p.ar = albedo.x;
     p.ag = albedo.y;
     p.ab = albedo.z;
@@ -141,7 +144,7 @@ VP_HD float inv_cdf(const PrimRecord& pr, f3 o, f3 d, float tau) {
     const float wp = dot(w, p) * w_inv_len;
     const float pp = length2(p);
     const float diff = fmaf_(-wp, wp, pp);
-    const float K = w_inv_len * expf_(-0.5f * diff) * pr.icf;
+    const float K = w_inv_len * expf_(-0.5f * diff) * VP_ICF(pr);
     const float raw = erff_(wp * kOneOverRootTwo) + tau * rcpf(K);
     if (raw > 1.0f) return kTMax;
     const float v = erfinvf_(clampf(raw, -1.0f, 1.0f));
@@ -158,7 +161,7 @@ VP_HD float inv_cdf_span(const PrimRecord& pr, f3 o, f3 d, float t_off, float ta
     const float wp = dot(w, p) * w_inv_len;
     const float pp = length2(p);
     const float diff = fmaf_(-wp, wp, pp);
-    const float K = w_inv_len * expf_(-0.5f * diff) * pr.icf;
+    const float K = w_inv_len * expf_(-0.5f * diff) * VP_ICF(pr);
     const float wp_off = fmaf_(t_off, w_len, wp);
     const float raw = erff_(wp_off * kOneOverRootTwo) + tau * rcpf(K);
     if (raw > 1.0f) return kTMax;
@@ -223,40 +226,32 @@ constexpr float kChordScale = 0x1.6c0504p-6f;
 struct Crossing {
     float t0, t1, tau;
 };
-// The first part of crossing(): false where crossing() finds no entry
-// before solving for it (a direction too short, an origin inside or on the
-// bound, a ray moving away, a miss or a tangent).  The same operations, so a
-// leaf pass can sort out beforehand the leaves crossing() would reject.
-struct CrossingSetup {
-    float a, b, c, a_inv, delta;
-};
-VP_HD bool crossing_setup(const PrimRecord& pr, f3 o, f3 d, CrossingSetup& s) {
+// Written without branches: a wavefront nearly always has a lane that enters,
+// so early outs save it nothing and split the chain of dependent steps into
+// blocks that each wait (the early outs' conditions are the factors of
+// enters).
+VP_HD Crossing crossing(const PrimRecord& pr, f3 o, f3 d) {
     const f3 w = to_local_dir(pr, d);
     const f3 p = to_local_pos(pr, o);
-    s.a = length2(w);
-    if (s.a < kDirMin2) return false;
-    s.c = length2(p) - kExtent2;
-    if (!(s.c > 0.0f)) return false;
-    s.b = -dot(p, w);
-    if (!(s.b > 0.0f)) return false;  // moving away: both roots behind the origin
-    s.a_inv = rcpf(s.a);
-    const f3 q0 = fma3(s.b * s.a_inv, w, p);
-    s.delta = kExtent2 - length2(q0);
-    return !(s.delta < kDiscEps);
-}
-VP_HD Crossing crossing(const PrimRecord& pr, f3 o, f3 d) {
-    Crossing r{-1.0f, -1.0f, 0.0f};
-    CrossingSetup s;
-    if (!crossing_setup(pr, o, d, s)) return r;
-    const float a = s.a, b = s.b, c = s.c, a_inv = s.a_inv, delta = s.delta;
+    const float a = length2(w);
+    const float c = length2(p) - kExtent2;
+    const float b = -dot(p, w);
+    const float a_inv = rcpf(a);
+    const f3 q0 = fma3(b * a_inv, w, p);
+    const float delta = kExtent2 - length2(q0);
     const float sq = sqrtf_(a * delta);
     const float q = b + sq;
     const float t = c * rcpf(q);
-    if (!(t >= 0.0f && t < kTMax)) return r;
-    r.t0 = t;
-    r.t1 = q * a_inv;
-    if (r.t1 - t > kSegMin && r.t1 < kTMax)
-        r.tau = ((kChordScale * (pr.mass * pr.dnf)) * (sq * a_inv)) * chord_poly_(delta);
+    const float t1 = q * a_inv;
+    const float tau = ((kChordScale * pr.md) * (sq * a_inv)) * chord_poly_(delta);
+    // a direction long enough, an origin outside the bound, a ray moving
+    // towards it that neither misses nor grazes
+    const bool enters = !(a < kDirMin2) & (c > 0.0f) & (b > 0.0f) & !(delta < kDiscEps) & (t >= 0.0f) & (t < kTMax);
+    const bool chord = enters & (t1 - t > kSegMin) & (t1 < kTMax);
+    Crossing r;
+    r.t0 = enters ? t : -1.0f;
+    r.t1 = enters ? t1 : -1.0f;
+    r.tau = chord ? tau : 0.0f;
     return r;
 }
 
@@ -280,10 +275,9 @@ constexpr float kExpHalfExtent2 = 0x1.6c0504p-7f;
 struct InsideChord {
     float t1, tau;
 };
-// With p the origin in the primitive's frame, pp = |p|^2 and e() = e^(-pp/2),
+// With p the origin in the primitive's frame, pp = |p|^2 and e = e^(-pp/2),
 // which a caller that tests several directions from one origin evaluates once.
-template <typename Exp>
-VP_HD InsideChord inside_chord_from(const PrimRecord& pr, f3 p, float pp, f3 d, Exp&& e) {
+VP_HD InsideChord inside_chord_from(const PrimRecord& pr, f3 p, float pp, f3 d, float e) {
     const f3 w = to_local_dir(pr, d);
     const float a = length2(w);
     const float b = dot(p, w);
@@ -291,20 +285,18 @@ VP_HD InsideChord inside_chord_from(const PrimRecord& pr, f3 p, float pp, f3 d, 
     const float disc = fmaf_(-a, c, b * b);
     const float sq = sqrtf_(disc);
     const float a_inv = rcpf(a);
+    const float far = (kExpHalfExtent2 * (sq * a_inv)) * chord_poly_(minf(disc * a_inv, kExtent2));
+    const float near = (e * (b * a_inv)) * chord_poly_(minf((b * b) * a_inv, kExtent2));
+    const float tau = maxf(pr.md * (far - near), 0.0f);
     InsideChord r;
     r.t1 = (-b + sq) * a_inv;
-    r.tau = 0.0f;
-    if (r.t1 > kSegMin && r.t1 < kTMax) {
-        const float far = (kExpHalfExtent2 * (sq * a_inv)) * chord_poly_(minf(disc * a_inv, kExtent2));
-        const float near = (e() * (b * a_inv)) * chord_poly_(minf((b * b) * a_inv, kExtent2));
-        r.tau = maxf((pr.mass * pr.dnf) * (far - near), 0.0f);
-    }
+    r.tau = (r.t1 > kSegMin) & (r.t1 < kTMax) ? tau : 0.0f;
     return r;
 }
 VP_HD InsideChord inside_chord(const PrimRecord& pr, f3 o, f3 d) {
     const f3 p = to_local_pos(pr, o);
     const float pp = length2(p);
-    return inside_chord_from(pr, p, pp, d, [&]() { return expf_(-0.5f * pp); });
+    return inside_chord_from(pr, p, pp, d, expf_(-0.5f * pp));
 }
 
 // Free flight from an origin inside a primitive (argmin over the origin set,

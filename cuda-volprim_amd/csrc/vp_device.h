@@ -41,8 +41,25 @@ __device__ __forceinline__ PrimRecord load_prim(const PrimRecord* prims, uint32_
     PrimRecord r;
     r.cx = a.x; r.cy = a.y; r.cz = a.z; r.qw = a.w;
     r.qx = b.x; r.qy = b.y; r.qz = b.z; r.rsx = b.w;
-    r.rsy = c.x; r.rsz = c.y; r.dnf = c.z; r.icf = c.w;
+    r.rsy = c.x; r.rsz = c.y; r.dnf = c.z; r.md = c.w;
     r.ar = d.x; r.ag = d.y; r.ab = d.z; r.mass = d.w;
+    return r;
+}
+
+// The 48 bytes of record i that crossing() reads (albedo and mass are left at
+// 0), loaded here: left alone, the compiler moves the load of what is used
+// last to its use, behind the wait for the others.
+template <typename Index>
+__device__ __forceinline__ PrimRecord load_leaf(const PrimRecord* prims, Index i) {
+    const auto* p = reinterpret_cast<const VP_GLOBAL_AS float4*>(
+        reinterpret_cast<const VP_GLOBAL_AS char*>(as_global(prims)) + i * static_cast<Index>(sizeof(PrimRecord)));
+    float4 a = p[0], b = p[1], c = p[2];
+    asm volatile("" : "+v"(a.x), "+v"(a.y), "+v"(a.z), "+v"(a.w), "+v"(b.x), "+v"(b.y), "+v"(b.z), "+v"(b.w),
+                      "+v"(c.x), "+v"(c.y), "+v"(c.z), "+v"(c.w));
+    PrimRecord r{};
+    r.cx = a.x; r.cy = a.y; r.cz = a.z; r.qw = a.w;
+    r.qx = b.x; r.qy = b.y; r.qz = b.z; r.rsx = b.w;
+    r.rsy = c.x; r.rsz = c.y; r.dnf = c.z; r.md = c.w;
     return r;
 }
 
@@ -756,7 +773,13 @@ __device__ __forceinline__ WaveScene wave_scene(const SceneView& sc, bool on, co
     ws.one = levels <= 13u && __builtin_amdgcn_ballot_w64(on && (sc.prims != ws.prims || sc.w4 != ws.w4)) == 0ull;
     return ws;
 }
-// Record `prim` of the scene of lane own's path.
+// Record `prim` of the scene of lane own's path: what crossing() needs, or all
+// of it.
+__device__ __forceinline__ PrimRecord load_wave_leaf(const MegaQueue& q, const WaveScene& ws, uint32_t own,
+                                                     uint32_t prim) {
+    if (ws.one) return load_leaf(ws.prims, prim);
+    return load_leaf(ws.jobs[q.job[own]].scene.prims, static_cast<size_t>(prim));
+}
 __device__ __forceinline__ PrimRecord load_wave_prim(const MegaQueue& q, const WaveScene& ws, uint32_t own,
                                                      uint32_t prim) {
     if (ws.one) {
@@ -937,13 +960,11 @@ __device__ __forceinline__ void shadow_walks(const WaveScene& ws, const MegaQueu
         const uint32_t n = nl < 64u ? nl : 64u;
         nl -= n;
         ++rounds;
-        {
-            const bool on = lane < n;
-            const uint32_t ray = on ? q.leaf_ray[nl + lane] : 0u, own = ray >> 1;
-            const bool live = on && q.tmax[ray] >= 0.0f;
-            const PrimRecord pr = load_wave_prim(q, ws, own, live ? q.leaf[nl + lane] : 0u);
-            if (live) {
-                const Crossing x = crossing(pr, lds_load3(q.ro + 3 * own), lds_load3(q.rd + 3 * ray));
+        if (lane < n) {
+            const uint32_t ray = q.leaf_ray[nl + lane], own = ray >> 1, prim = q.leaf[nl + lane];
+            const f3 ro = lds_load3(q.ro + 3 * own), rd = lds_load3(q.rd + 3 * ray);
+            if (q.tmax[ray] >= 0.0f) {
+                const Crossing x = crossing(load_wave_leaf(q, ws, own, prim), ro, rd);
                 if (x.tau > 0.0f) atomicAdd(&q.acc[ray], tau_fixed(x.tau));
             }
         }

@@ -354,6 +354,7 @@ hipError_t vp_launch_transmittance(vp::SceneView sc, const float* rays, uint32_t
 hipError_t vp_launch_overlaps(vp::SceneView sc, const float* rays, uint32_t m, uint32_t cap, uint32_t* counts,
                               float* t, uint32_t* idx, hipStream_t s);
 hipError_t vp_launch_math(int fn, const float* x, const float* y, uint32_t n, float* out, hipStream_t s);
+hipError_t vp_launch_export_records(const vp::PrimRecord* prims, uint32_t n, float4* out, hipStream_t s);
 hipError_t vp_launch_prim(int fn, const vp::PrimRecord* rec, const float* args, uint32_t m, float* out,
                           hipStream_t s);
 int vp_render_occupancy(uint32_t block, uint32_t active_cap, int count_events, int* blocks_per_cu);

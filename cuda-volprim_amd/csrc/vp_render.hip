@@ -168,12 +168,13 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const WaveScene& 
             nl -= n;
             ++rounds;
             bool keep = false;
-            const bool on = lane < n;
-            const uint32_t ray = on ? q.leaf_ray[nl + lane] : 0u, own = ray >> 1;
-            const uint32_t prim = on ? q.leaf[nl + lane] : 0u;
-            const PrimRecord pr = load_wave_prim(q, ws, own, prim);
-            if (on) {
-                const Crossing x = crossing(pr, lds_load3(q.ro + 3 * own), lds_load3(q.rd + 3 * ray));
+            uint32_t ray = 0, prim = 0;
+            if (lane < n) {
+                ray = q.leaf_ray[nl + lane];
+                prim = q.leaf[nl + lane];
+                const uint32_t own = ray >> 1;
+                const f3 ro = lds_load3(q.ro + 3 * own), rd = lds_load3(q.rd + 3 * ray);
+                const Crossing x = crossing(load_wave_leaf(q, ws, own, prim), ro, rd);
                 if (x.t0 >= 0.0f) {
                     const uint32_t meta = q.draw(own)[2];
                     if ((meta >> 31) != 0u && x.tau > 0.0f) atomicAdd(&q.acc[ray], tau_fixed(x.tau));
@@ -430,20 +431,19 @@ __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has
         const f3 p = to_local_pos(pr, ro);
         const float pp = length2(p);
         const float ex = expf_(-0.5f * pp);
-        auto e = [&]() { return ex; };
         const float wgt = pr.mass * (ex * pr.dnf);  // mass * prim_pdf
         *reinterpret_cast<float4*>(mine + 2u * bs + 4u * k) =
             make_float4(pr.ar * wgt, pr.ag * wgt, pr.ab * wgt, wgt);
         if ((meta & 2u) != 0u) {
-            const float ta = inside_chord_from(pr, p, pp, lds_load3(q.rd + 3 * (2 * own)), e).tau;
+            const float ta = inside_chord_from(pr, p, pp, lds_load3(q.rd + 3 * (2 * own)), ex).tau;
             if (ta > 0.0f) atomicAdd(&q.acc[2 * own], tau_fixed(ta));
         }
         if ((meta & 4u) != 0u) {
-            const float tb = inside_chord_from(pr, p, pp, lds_load3(q.rd + 3 * (2 * own + 1)), e).tau;
+            const float tb = inside_chord_from(pr, p, pp, lds_load3(q.rd + 3 * (2 * own + 1)), ex).tau;
             if (tb > 0.0f) atomicAdd(&q.acc[2 * own + 1], tau_fixed(tb));
         }
         const f3 rw = lds_load3(wo_of + 3 * own);
-        const InsideChord c = inside_chord_from(pr, p, pp, rw, e);
+        const InsideChord c = inside_chord_from(pr, p, pp, rw, ex);
         mine[bs - set + k] = __float_as_uint(c.t1);
         const float tau = free_flight_tau(prim_uniform(key_of[own], b_of[own], 0u, i));
         if (tau <= c.tau) {
@@ -1188,11 +1188,22 @@ __global__ void k_math(int fn, const float* __restrict__ x, const float* __restr
     out[i] = r;
 }
 
+// The records as vp_scene_export gives them: the reference's fields in its
+// order, the inverse-CDF factor M dnf sqrt(pi/2) in word 11.
+__global__ void k_export_records(const PrimRecord* __restrict__ in, uint32_t n, float4* __restrict__ out) {
+    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i >= 4u * n) return;
+    float4 v = reinterpret_cast<const float4*>(in)[i];
+    if ((i & 3u) == 2u) v.w *= kRootHalfPi;
+    out[i] = v;
+}
+
 __global__ void k_prim(int fn, const PrimRecord* __restrict__ rec, const float* __restrict__ args, uint32_t m,
                        float* __restrict__ out) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= m) return;
-    const PrimRecord p = *rec;
+    PrimRecord p = *rec;
+    p.md = p.mass * p.dnf;  // (the exported record has the inverse-CDF factor there)
     const float* a = args + 9 * i;
     const f3 o = f3{a[0], a[1], a[2]}, d = f3{a[3], a[4], a[5]};
     float r;
@@ -1308,6 +1319,11 @@ hipError_t vp_launch_overlaps(SceneView sc, const float* rays, uint32_t m, uint3
 
 hipError_t vp_launch_math(int fn, const float* x, const float* y, uint32_t n, float* out, hipStream_t s) {
     hipLaunchKernelGGL(k_math, dim3(cdiv(n, 256)), dim3(256), 0, s, fn, x, y, n, out);
+    return hipGetLastError();
+}
+
+hipError_t vp_launch_export_records(const PrimRecord* prims, uint32_t n, float4* out, hipStream_t s) {
+    hipLaunchKernelGGL(k_export_records, dim3(cdiv(uint64_t(4) * n, 256)), dim3(256), 0, s, prims, n, out);
     return hipGetLastError();
 }
 
