@@ -239,14 +239,17 @@ VP_HD Crossing crossing(const PrimRecord& pr, f3 o, f3 d) {
     const float a_inv = rcpf(a);
     const f3 q0 = fma3(b * a_inv, w, p);
     const float delta = kExtent2 - length2(q0);
-    const float sq = sqrtf_(a * delta);
-    const float q = b + sq;
+    // a direction long enough, an origin outside the bound, a ray moving
+    // towards it that neither misses nor grazes
+    // (the root's argument and its reciprocal stay ordinary numbers for a ray
+    // that does not enter: nothing below is used then)
+    const bool meets = !(a < kDirMin2) & (c > 0.0f) & (b > 0.0f) & !(delta < kDiscEps);
+    const float sq = sqrtf_(meets ? a * delta : 1.0f);
+    const float q = meets ? b + sq : 1.0f;
     const float t = c * rcpf(q);
     const float t1 = q * a_inv;
     const float tau = ((kChordScale * pr.md) * (sq * a_inv)) * chord_poly_(delta);
-    // a direction long enough, an origin outside the bound, a ray moving
-    // towards it that neither misses nor grazes
-    const bool enters = !(a < kDirMin2) & (c > 0.0f) & (b > 0.0f) & !(delta < kDiscEps) & (t >= 0.0f) & (t < kTMax);
+    const bool enters = meets & (t >= 0.0f) & (t < kTMax);
     const bool chord = enters & (t1 - t > kSegMin) & (t1 < kTMax);
     Crossing r;
     r.t0 = enters ? t : -1.0f;

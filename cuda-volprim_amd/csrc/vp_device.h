@@ -16,7 +16,7 @@ __device__ __forceinline__ f3 safe_inv(f3 d) {
     const float x = fabsf_(d.x) < 1e-20f ? copysignf_(1e-20f, d.x) : d.x;
     const float y = fabsf_(d.y) < 1e-20f ? copysignf_(1e-20f, d.y) : d.y;
     const float z = fabsf_(d.z) < 1e-20f ? copysignf_(1e-20f, d.z) : d.z;
-    return f3{1.0f / x, 1.0f / y, 1.0f / z};
+    return f3{rcpf(x), rcpf(y), rcpf(z)};
 }
 
 // Scene arrays are reached through pointers stored in device memory (the job

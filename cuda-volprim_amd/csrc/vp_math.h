@@ -53,6 +53,16 @@ VP_HD float fmaf_(float a, float b, float c) { return __builtin_fmaf(a, b, c); }
 VP_HD float sqrtf_(float x) {
 #if VP_FAST_DEVICE
     return __builtin_amdgcn_sqrtf(x);
+#elif defined(__HIP_DEVICE_COMPILE__)
+    // The IEEE root in 5 instructions instead of the compiler's 16: the
+    // hardware's reciprocal root and one correction of x y, which is correctly
+    // rounded for every x in [2^-96, inf) (checked on gfx950 against the IEEE
+    // root over all of them); the rest takes the compiler's.
+    const float y = __builtin_amdgcn_rsqf(x);
+    const float g = x * y, h = 0.5f * y;
+    float r = __builtin_fmaf(__builtin_fmaf(-g, g, x), h, g);
+    if (__builtin_expect(!(x >= 0x1p-96f && x < __builtin_inff()), 0)) r = __builtin_sqrtf(x);
+    return r;
 #else
     return __builtin_sqrtf(x);
 #endif
@@ -76,8 +86,21 @@ VP_HD float clampf(float x, float lo, float hi) { return maxf(lo, minf(x, hi)); 
 VP_HD float rcpf(float x) { return __builtin_amdgcn_rcpf(x); }
 VP_HD float rsqrtf_(float x) { return __builtin_amdgcn_rsqf(x); }
 #else
-VP_HD float rcpf(float x) { return 1.0f / x; }
-VP_HD float rsqrtf_(float x) { return 1.0f / sqrtf_(x); }
+// 1 / x, IEEE.  On the device one Newton step on the hardware's reciprocal,
+// which is correctly rounded whenever that is a normal number (checked on
+// gfx950 against the division over all 2^32 inputs), 3 instructions and a test
+// instead of 10; else the division.
+VP_HD float rcpf(float x) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const float y = __builtin_amdgcn_rcpf(x);
+    float r = __builtin_fmaf(__builtin_fmaf(-x, y, 1.0f), y, y);
+    if (__builtin_expect(!__builtin_amdgcn_classf(y, 0x108), 0)) r = 1.0f / x;  // 0x108: normal
+    return r;
+#else
+    return 1.0f / x;
+#endif
+}
+VP_HD float rsqrtf_(float x) { return rcpf(sqrtf_(x)); }
 #endif
 
 constexpr float kInf = __builtin_huge_valf();

@@ -1183,6 +1183,7 @@ __global__ void k_math(int fn, const float* __restrict__ x, const float* __restr
         case 10: r = sqrtf_(a); break;
         case 11: r = a / b; break;
         case 12: r = chord_poly_(a); break;
+        case 13: r = rcpf(a); break;
         default: r = __builtin_nanf("");
     }
     out[i] = r;

@@ -284,7 +284,8 @@ vp_status vp_collect_overlaps(vp_context* ctx, vp_scene* scene, const float* ray
 vp_status vp_render_count_events(vp_context* ctx, vp_scene* scene, vp_env* env, const vp_camera* cam,
                                  const vp_render_params* params, uint64_t* events, uint32_t n_events);
 /* Evaluate math function fn (0 exp 1 log 2 sin 3 cos 4 atan2 5 acos 6 erf
- * 7 erfc 8 erfinv 9 erf_diff 10 sqrt 11 div 12 chord_poly) on the device. */
+ * 7 erfc 8 erfinv 9 erf_diff 10 sqrt 11 div 12 chord_poly
+ * 13 rcp) on the device. */
 vp_status vp_math_eval(vp_context* ctx, int fn, const float* x, const float* y, uint32_t n, float* out);
 /* Evaluate primitive function fn (0 inv_cdf 1 inv_cdf_span 2 optical_depth
  * 3 exit_inside 4 entry_t 5 exit_entry 6 point_inside 7 pdf 8 chord_tau (the
