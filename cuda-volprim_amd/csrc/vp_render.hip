@@ -405,7 +405,11 @@ __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has
     uint32_t* ts_of = meta_of + 64;                                  // [64]
     uint32_t* b_of = ts_of + 64;                                     // [64]
     float* wo_of = reinterpret_cast<float*>(b_of + 64);              // [64 * 3]
-    static_assert(kScratch >= 9 * 64, "the member pass's tables must fit in the queue");
+    constexpr uint32_t kFlightItems = 256;
+    uint32_t* flight = q.scratch + 9 * 64;                           // [kFlightItems] primitives
+    uint8_t* flight_of = q.node_ray;                                 // [kFlightItems] their lanes
+    static_assert(kScratch >= 9 * 64 + kFlightItems && kNodeQ >= kFlightItems,
+                  "the member pass's tables must fit in the queue");
     uint32_t total;
     pre_of[lane] = wave_prefix(nn, total);
     meta_of[lane] = cur | (has_a ? 2u : 0u) | (has_b ? 4u : 0u);
@@ -419,36 +423,58 @@ __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has
     ts_of[lane] = __float_as_uint(kTMax);
     b_of[lane] = b1;
     wave_sync();
+    uint32_t nf = 0;  // flights waiting
     for (uint32_t base = 0; base < total; base += 64u) {
         const uint32_t g = base + lane;
-        const uint32_t own = prefix_owner(pre_of, g), k = g - pre_of[own];
-        const uint32_t meta = meta_of[own], set = (meta & 1u) * bs;
-        uint32_t* mine = slab_of(slab, gbase, own, bs);
-        const uint32_t i = g < total ? mine[set + k] : 0u;
-        const PrimRecord pr = load_wave_prim(q, ws, own, i);
-        if (g >= total) continue;
-        const f3 ro = lds_load3(q.ro + 3 * own);
-        const f3 p = to_local_pos(pr, ro);
-        const float pp = length2(p);
-        const float ex = expf_(-0.5f * pp);
-        const float wgt = pr.mass * (ex * pr.dnf);  // mass * prim_pdf
-        *reinterpret_cast<float4*>(mine + 2u * bs + 4u * k) =
-            make_float4(pr.ar * wgt, pr.ag * wgt, pr.ab * wgt, wgt);
-        if ((meta & 2u) != 0u) {
-            const float ta = inside_chord_from(pr, p, pp, lds_load3(q.rd + 3 * (2 * own)), ex).tau;
-            if (ta > 0.0f) atomicAdd(&q.acc[2 * own], tau_fixed(ta));
+        bool flies = false;
+        uint32_t own = 0, i = 0;
+        if (g < total) {
+            own = prefix_owner(pre_of, g);
+            const uint32_t k = g - pre_of[own];
+            const uint32_t meta = meta_of[own], set = (meta & 1u) * bs;
+            uint32_t* mine = slab_of(slab, gbase, own, bs);
+            i = mine[set + k];
+            const PrimRecord pr = load_wave_prim(q, ws, own, i);
+            const f3 ro = lds_load3(q.ro + 3 * own);
+            const f3 p = to_local_pos(pr, ro);
+            const float pp = length2(p);
+            const float ex = expf_(-0.5f * pp);
+            const float wgt = pr.mass * (ex * pr.dnf);  // mass * prim_pdf
+            *reinterpret_cast<float4*>(mine + 2u * bs + 4u * k) =
+                make_float4(pr.ar * wgt, pr.ag * wgt, pr.ab * wgt, wgt);
+            if ((meta & 2u) != 0u) {
+                const float ta = inside_chord_from(pr, p, pp, lds_load3(q.rd + 3 * (2 * own)), ex).tau;
+                if (ta > 0.0f) atomicAdd(&q.acc[2 * own], tau_fixed(ta));
+            }
+            if ((meta & 4u) != 0u) {
+                const float tb = inside_chord_from(pr, p, pp, lds_load3(q.rd + 3 * (2 * own + 1)), ex).tau;
+                if (tb > 0.0f) atomicAdd(&q.acc[2 * own + 1], tau_fixed(tb));
+            }
+            const InsideChord c = inside_chord_from(pr, p, pp, lds_load3(wo_of + 3 * own), ex);
+            mine[bs - set + k] = __float_as_uint(c.t1);
+            flies = free_flight_tau(prim_uniform(key_of[own], b_of[own], 0u, i)) <= c.tau;
         }
-        if ((meta & 4u) != 0u) {
-            const float tb = inside_chord_from(pr, p, pp, lds_load3(q.rd + 3 * (2 * own + 1)), ex).tau;
-            if (tb > 0.0f) atomicAdd(&q.acc[2 * own + 1], tau_fixed(tb));
+        // the few flights that end inside their chords wait until there are
+        // enough to invert together (the inversion's erf, erfinv and exp took
+        // as long as half a round for one or two lanes in most rounds)
+        const unsigned long long fm = __builtin_amdgcn_ballot_w64(flies);
+        if (flies) {
+            flight[nf + lanes_below(fm)] = i;
+            flight_of[nf + lanes_below(fm)] = static_cast<uint8_t>(own);
         }
-        const f3 rw = lds_load3(wo_of + 3 * own);
-        const InsideChord c = inside_chord_from(pr, p, pp, rw, ex);
-        mine[bs - set + k] = __float_as_uint(c.t1);
-        const float tau = free_flight_tau(prim_uniform(key_of[own], b_of[own], 0u, i));
-        if (tau <= c.tau) {
-            const float t = origin_flight(pr, ro, rw, c, tau);
-            atomicMin(&ts_of[own], t == 0.0f ? 0u : __float_as_uint(t));
+        nf += static_cast<uint32_t>(__popcll(fm));
+        wave_sync();
+        if (nf + 64u > kFlightItems || base + 64u >= total) {
+            for (uint32_t f = lane; f < nf; f += 64u) {
+                const uint32_t fo = flight_of[f], fi = flight[f];
+                const PrimRecord pr = load_wave_leaf(q, ws, fo, fi);
+                const f3 ro = lds_load3(q.ro + 3 * fo), rw = lds_load3(wo_of + 3 * fo);
+                const float tau = free_flight_tau(prim_uniform(key_of[fo], b_of[fo], 0u, fi));
+                const float t = origin_flight(pr, ro, rw, inside_chord(pr, ro, rw), tau);
+                atomicMin(&ts_of[fo], t == 0.0f ? 0u : __float_as_uint(t));
+            }
+            nf = 0;
+            wave_sync();
         }
     }
     wave_sync();
