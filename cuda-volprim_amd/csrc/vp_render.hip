@@ -249,8 +249,10 @@ __device__ __forceinline__ uint32_t* slab_of(uint32_t* slab, uint32_t gbase, uin
     return slab + static_cast<size_t>(gbase + own) * kMegaSlabBuffers * bs;
 }
 
-// Lists longer than this are merged by their own lane: the merge below scans
-// a path's kept candidates once per item.
+// Kept candidates of a wavefront that the merge below holds in LDS; more than
+// these are read from the slab.  A path with more than kRebuildScanMax merges
+// them by its own lane (the merge scans them once per item).
+constexpr uint32_t kCandItems = 512;
 constexpr uint32_t kRebuildScanMax = 1024;
 
 // The active sets at the scatter points (sampling.cuh:422-458) of the lanes
@@ -276,8 +278,9 @@ __device__ __forceinline__ uint32_t rebuild_shared(bool part, uint32_t na, uint3
     uint32_t* na_of = pre_of + 64;        // members of the list being flattened | set buffer << 31
     uint32_t* kept_of = pre_of + 128;     // [2][64] kept members, kept candidates
     float* ts_of = reinterpret_cast<float*>(pre_of + 256);
-    static_assert(kScratch >= 5 * 64, "the rebuild's tables must fit in the queue");
-    uint32_t total;
+    uint32_t* cand = pre_of + 320;        // [kCandItems + 3] kept candidates
+    static_assert(kScratch >= 5 * 64 + kCandItems + 3, "the rebuild's tables must fit in the queue");
+    uint32_t total, total_c = 0;
     pre_of[lane] = wave_prefix(part ? na + nc : 0u, total);
     na_of[lane] = na | (cur << 31);
     kept_of[lane] = 0u;
@@ -309,42 +312,67 @@ __device__ __forceinline__ uint32_t rebuild_shared(bool part, uint32_t na, uint3
             const uint32_t pos = *kept + lanes_below((member ? km : kc_m) & seg);
             atomicAdd(kept, 1u);
             mine[(member ? set : 2u * bs) + pos] = id;
+            const uint32_t at = total_c + lanes_below(kc_m);
+            if (!member && at < kCandItems) cand[at] = id;
         }
+        total_c += static_cast<uint32_t>(__popcll(kc_m));
         wave_sync();
     }
     const uint32_t mm = kept_of[lane], mc = kept_of[64 + lane];
-    wave_sync();
-    pre_of[lane] = wave_prefix(mm + mc, total);
-    wave_sync();
-    // a candidate that is also a member (an origin the rounding puts outside
-    // a member's bound can enter it again) would be counted twice
     bool serial = mc > kRebuildScanMax;
     if (__builtin_amdgcn_ballot_w64(serial) == 0ull) {
-        for (uint32_t g = lane; g < total; g += 64u) {
-            const uint32_t own = prefix_owner(pre_of, g), k = g - pre_of[own];
-            const uint32_t set = (na_of[own] >> 31) * bs, nm = kept_of[own], nk = kept_of[64 + own];
-            uint32_t* mine = slab_of(slab, gbase, own, bs);
-            const uint32_t* cand = mine + 2u * bs;
-            const bool member = k < nm;
-            const uint32_t id = member ? mine[set + k] : cand[k - nm];
-            uint32_t below = 0;
-            for (uint32_t j = 0; j < nk; j += 4u) {
-                const uint4 c = *reinterpret_cast<const uint4*>(cand + j);
-                below += (c.x < id ? 1u : 0u) + (j + 1u < nk && c.y < id ? 1u : 0u) +
-                         (j + 2u < nk && c.z < id ? 1u : 0u) + (j + 3u < nk && c.w < id ? 1u : 0u);
-            }
-            uint32_t lo = k;
-            if (!member) {
-                lo = 0;
-                uint32_t hi = nm;
-                while (lo < hi) {
-                    const uint32_t mid = (lo + hi) >> 1;
-                    if (mine[set + mid] < id) lo = mid + 1u;
-                    else hi = mid;
+        // items were met path by path, so the kept candidates lie in LDS path
+        // by path, from c_of[path]
+        const bool in_lds = total_c <= kCandItems;
+        uint32_t* c_of = reinterpret_cast<uint32_t*>(ts_of);
+        uint32_t total_m;
+        wave_sync();
+        pre_of[lane] = wave_prefix(mm, total_m);
+        c_of[lane] = wave_prefix(mc, total_c);
+        wave_sync();
+        // kept candidates of path own below id
+        auto below = [&](uint32_t own, uint32_t id) {
+            const uint32_t nk = kept_of[64 + own];
+            uint32_t n = 0;
+            auto count = [&](uint32_t j, uint32_t v0, uint32_t v1, uint32_t v2, uint32_t v3) {
+                n += (v0 < id ? 1u : 0u) + (j + 1u < nk && v1 < id ? 1u : 0u) + (j + 2u < nk && v2 < id ? 1u : 0u) +
+                     (j + 3u < nk && v3 < id ? 1u : 0u);
+            };
+            if (in_lds) {
+                const uint32_t* c = cand + c_of[own];
+                for (uint32_t j = 0; j < nk; j += 4u) count(j, c[j], c[j + 1u], c[j + 2u], c[j + 3u]);
+            } else {
+                const uint32_t* c = slab_of(slab, gbase, own, bs) + 2u * bs;
+                for (uint32_t j = 0; j < nk; j += 4u) {
+                    const uint4 v = *reinterpret_cast<const uint4*>(c + j);
+                    count(j, v.x, v.y, v.z, v.w);
                 }
-                if (lo < nm && mine[set + lo] == id) serial = true;
             }
-            const uint32_t pos = lo + below;
+            return n;
+        };
+        for (uint32_t g = lane; g < total_m; g += 64u) {
+            const uint32_t own = prefix_owner(pre_of, g), k = g - pre_of[own];
+            const uint32_t set = (na_of[own] >> 31) * bs;
+            uint32_t* mine = slab_of(slab, gbase, own, bs);
+            const uint32_t id = mine[set + k];
+            const uint32_t pos = k + below(own, id);
+            if (pos < cap) mine[bs - set + pos] = id;
+        }
+        for (uint32_t g = lane; g < total_c; g += 64u) {
+            const uint32_t own = prefix_owner(c_of, g);
+            const uint32_t set = (na_of[own] >> 31) * bs, nm = kept_of[own];
+            uint32_t* mine = slab_of(slab, gbase, own, bs);
+            const uint32_t id = in_lds ? cand[g] : mine[2u * bs + g - c_of[own]];
+            uint32_t lo = 0, hi = nm;
+            while (lo < hi) {
+                const uint32_t mid = (lo + hi) >> 1;
+                if (mine[set + mid] < id) lo = mid + 1u;
+                else hi = mid;
+            }
+            // a candidate that is also a member (an origin the rounding puts
+            // outside a member's bound can enter it again) was counted twice
+            if (lo < nm && mine[set + lo] == id) serial = true;
+            const uint32_t pos = lo + below(own, id);
             if (pos < cap) mine[bs - set + pos] = id;
         }
     }
@@ -356,16 +384,16 @@ __device__ __forceinline__ uint32_t rebuild_shared(bool part, uint32_t na, uint3
         uint32_t* mine = slab_of(slab, gbase, lane, bs);
         const uint32_t* set = mine + cur * bs;
         uint32_t* out = mine + (cur ^ 1u) * bs;
-        uint32_t* cand = mine + 2u * bs;
+        uint32_t* own_cand = mine + 2u * bs;
         for (uint32_t i = 1; i < mc; ++i) {
-            const uint32_t v = cand[i];
+            const uint32_t v = own_cand[i];
             uint32_t j = i;
-            for (; j > 0 && cand[j - 1] > v; --j) cand[j] = cand[j - 1];
-            cand[j] = v;
+            for (; j > 0 && own_cand[j - 1] > v; --j) own_cand[j] = own_cand[j - 1];
+            own_cand[j] = v;
         }
         nn = 0;
         for (uint32_t i = 0, j = 0; i < mm || j < mc; ++nn) {
-            const uint32_t a = i < mm ? set[i] : 0xffffffffu, c = j < mc ? cand[j] : 0xffffffffu;
+            const uint32_t a = i < mm ? set[i] : 0xffffffffu, c = j < mc ? own_cand[j] : 0xffffffffu;
             const uint32_t v = a < c ? a : c;
             if (a == v) ++i;
             if (c == v) ++j;
