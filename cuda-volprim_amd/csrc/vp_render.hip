@@ -138,16 +138,11 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const WaveScene& 
     // the first thread of this wavefront, for the owners' candidate buffers
     const uint32_t gbase = blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
     const uint32_t bs = mega_slab_stride(cap);
-    // every ray starts at the root
-    uint32_t nn, nl = 0, nf = 0;
-    {
-        const unsigned long long am = __builtin_amdgcn_ballot_w64(alive);
-        if (alive) {
-            q.node[lanes_below(am)] = 0u;
-            q.node_ray[lanes_below(am)] = static_cast<uint8_t>(2 * lane);
-        }
-        nn = static_cast<uint32_t>(__popcll(am));
-    }
+    uint32_t nn = 0, nl = 0, nf = 0;
+    const unsigned long long am = __builtin_amdgcn_ballot_w64(alive);
+    if (alive) q.list[lanes_below(am)] = static_cast<uint8_t>(2 * lane);
+    wave_sync();
+    push_rays(q, ws, q.list, static_cast<uint32_t>(__popcll(am)), nn);
     static_assert(kLeafItems >= 64u + kFlightMin + 64 + 4, "room for a step's leaves and the flights");
     wave_sync();
     while (true) {
