@@ -232,10 +232,7 @@ vp_status vp_scene_create_ex(vp_context* ctx, const vp_primitive* prims, uint32_
     auto* sc = new vp_scene();
     sc->ctx = ctx;
     sc->n = n;
-    vp_status st = vp_build_scene_device(ctx, prims, n, sc);
-    if (st == VP_OK && (flags & (VP_SCENE_BVH_SAH | VP_SCENE_BVH_MEDIAN)))
-        st = vp_build_scene_sah(ctx, prims, n, sc, (flags & VP_SCENE_BVH_MEDIAN) != 0u);
-    if (st == VP_OK) st = vp_build_walk_tree(ctx, sc, flags & (VP_SCENE_WALK_F32 | VP_SCENE_WALK_F16));
+    const vp_status st = vp_build_scene(ctx, prims, n, flags, sc);
     if (st != VP_OK) {
         vp_scene_destroy(sc);
         return st;
@@ -247,11 +244,8 @@ vp_status vp_scene_create_ex(vp_context* ctx, const vp_primitive* prims, uint32_
 vp_status vp_scene_destroy(vp_scene* sc) {
     if (!sc) return VP_OK;
     if (sc->ctx && sc->ctx->stream) (void)hipStreamSynchronize(sc->ctx->stream);
-    if (sc->prims) (void)hipFree(sc->prims);
-    if (sc->nodes) (void)hipFree(sc->nodes);
+    if (sc->mem) (void)hipFree(sc->mem);
     if (sc->w4) (void)hipFree(sc->w4);
-    if (sc->order) (void)hipFree(sc->order);
-    if (sc->morton) (void)hipFree(sc->morton);
     delete sc;
     return VP_OK;
 }

@@ -1,7 +1,8 @@
 // vp_bvh.hip — GPU construction of the scene: primitive records, Morton
-// codes, a stable LDS radix sort, the Karras (2012) binary radix tree, a
-// bottom-up bounding-box refit and the depth-first "rope" node layout the
-// traversal kernels walk without a stack.
+// codes, a stable LDS radix sort, the depth of the Karras (2012) binary radix
+// tree over them, and the walk tree over the stored order (vp_walk.h).  The
+// radix tree orders the leaves as the sort does, and no walk uses its inner
+// nodes, so their boxes are not built.
 //
 // Replaces the reference's Morton sort (src/thesis/host/app/renderer.cpp:90-121,
 // include/thesis/host/utils/math.h:103-160) and its OptiX GAS/IAS build
@@ -74,15 +75,22 @@ __global__ void k_bounds_partial(const float* centers, uint32_t n, float* partia
         }
 }
 
-__global__ void k_bounds_final(const float* partial, uint32_t nb, float* bounds) {
-    if (threadIdx.x != 0 || blockIdx.x != 0) return;
+// One wavefront folds the partial bounds, a lane every 64th of them (a single
+// lane over all took 181 us for 250000 primitives, this 7).
+__global__ void __launch_bounds__(64) k_bounds_final(const float* partial, uint32_t nb, float* bounds) {
     float mn[3] = {3.402823466e38f, 3.402823466e38f, 3.402823466e38f};
     float mx[3] = {-3.402823466e38f, -3.402823466e38f, -3.402823466e38f};
-    for (uint32_t b = 0; b < nb; ++b)
+    for (uint32_t b = threadIdx.x; b < nb; b += 64u)
         for (int k = 0; k < 3; ++k) {
             mn[k] = minf(mn[k], partial[6 * b + k]);
             mx[k] = maxf(mx[k], partial[6 * b + 3 + k]);
         }
+    for (int off = 32; off > 0; off >>= 1)
+        for (int k = 0; k < 3; ++k) {
+            mn[k] = minf(mn[k], __shfl_xor(mn[k], off));
+            mx[k] = maxf(mx[k], __shfl_xor(mx[k], off));
+        }
+    if (threadIdx.x != 0) return;
     for (int k = 0; k < 3; ++k) {
         bounds[k] = mn[k];
         bounds[3 + k] = 1.0f / maxf(mx[k] + (-mn[k]), 1e-30f);  // inverse extent
@@ -120,28 +128,50 @@ __global__ void __launch_bounds__(kSortBlock) k_hist(const uint32_t* keys, uint3
     hist[t * nblocks + blockIdx.x] = h[t];
 }
 
-// Exclusive scan of hist (digit-major, block-minor) in one 1024-thread block.
+// Exclusive scan of hist (digit-major, block-minor; count is a multiple of
+// 256) in one 1024-thread block, 8192 entries a round, eight consecutive ones
+// a thread (each thread scanning one long run of its own, read with a stride
+// of its length, took 49 us for 250000 keys, this 6).
 __global__ void __launch_bounds__(1024) k_scan(uint32_t* hist, uint32_t count) {
-    __shared__ uint32_t part[1024];
-    const uint32_t t = threadIdx.x;
-    const uint32_t chunk = (count + 1023) / 1024;
-    const uint32_t b = t * chunk;
-    const uint32_t e = min(count, b + chunk);
-    uint32_t s = 0;
-    for (uint32_t i = b; i < e; ++i) s += hist[i];
-    part[t] = s;
-    __syncthreads();
-    for (uint32_t off = 1; off < 1024; off <<= 1) {
-        const uint32_t v = t >= off ? part[t - off] : 0u;
+    __shared__ uint32_t wave_sum[16];
+    const uint32_t t = threadIdx.x, lane = t & 63u, wave = t >> 6;
+    uint32_t carry = 0;
+    for (uint32_t base = 0; base < count; base += 8192u) {
+        const uint32_t i = base + 8u * t;
+        uint4* at = reinterpret_cast<uint4*>(hist + i);
+        uint4 a = make_uint4(0u, 0u, 0u, 0u), b = a;
+        if (i < count) {
+            a = at[0];
+            b = at[1];
+        }
+        const uint32_t s = a.x + a.y + a.z + a.w + b.x + b.y + b.z + b.w;
+        uint32_t incl = s;
+        for (uint32_t off = 1; off < 64u; off <<= 1) {
+            const uint32_t u = __shfl_up(incl, off);
+            if (lane >= off) incl += u;
+        }
+        if (lane == 63u) wave_sum[wave] = incl;
         __syncthreads();
-        part[t] += v;
+        uint32_t before = 0, all = 0;
+        for (uint32_t w = 0; w < 16u; ++w) {
+            before += w < wave ? wave_sum[w] : 0u;
+            all += wave_sum[w];
+        }
+        if (i < count) {
+            uint4 o;
+            o.x = carry + before + incl - s;
+            o.y = o.x + a.x;
+            o.z = o.y + a.y;
+            o.w = o.z + a.z;
+            at[0] = o;
+            o.x = o.w + a.w;
+            o.y = o.x + b.x;
+            o.z = o.y + b.y;
+            o.w = o.z + b.z;
+            at[1] = o;
+        }
+        carry += all;
         __syncthreads();
-    }
-    uint32_t run = part[t] - s;  // exclusive prefix of this chunk
-    for (uint32_t i = b; i < e; ++i) {
-        const uint32_t v = hist[i];
-        hist[i] = run;
-        run += v;
     }
 }
 
@@ -200,12 +230,11 @@ __device__ __forceinline__ int delta(const uint32_t* codes, int n, int i, int j)
     return __clzll(a ^ b);
 }
 
-constexpr uint32_t kLeafBit = 0x80000000u;
-
-__global__ void k_karras(const uint32_t* codes, int n, uint32_t* left, uint32_t* right, uint32_t* range_lo,
-                         uint32_t* range_hi, int* parent) {
+// Parents of the radix tree's nodes: inner node i is i, leaf k is n - 1 + k.
+__global__ void k_karras(const uint32_t* codes, int n, int* parent) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n - 1) return;
+    if (i == 0) parent[0] = -1;
     const int d = (delta(codes, n, i, i + 1) - delta(codes, n, i, i - 1)) >= 0 ? 1 : -1;
     const int dmin = delta(codes, n, i, i - d);
     int lmax = 2;
@@ -223,88 +252,22 @@ __global__ void k_karras(const uint32_t* codes, int n, uint32_t* left, uint32_t*
     }
     const int gamma = i + s * d + (d < 0 ? -1 : 0);
     const int lo = min(i, j), hi = max(i, j);
-    const uint32_t lc = (lo == gamma) ? (kLeafBit | (uint32_t)gamma) : (uint32_t)gamma;
-    const uint32_t rc = (hi == gamma + 1) ? (kLeafBit | (uint32_t)(gamma + 1)) : (uint32_t)(gamma + 1);
-    left[i] = lc;
-    right[i] = rc;
-    range_lo[i] = lo;
-    range_hi[i] = hi;
-    // parent array over the unified index space: inner i -> i, leaf k -> n-1+k
-    parent[(lc & kLeafBit) ? (n - 1 + (lc & ~kLeafBit)) : lc] = i;
-    parent[(rc & kLeafBit) ? (n - 1 + (rc & ~kLeafBit)) : rc] = i;
+    parent[lo == gamma ? n - 1 + gamma : gamma] = i;
+    parent[hi == gamma + 1 ? n - 1 + gamma + 1 : gamma + 1] = i;
 }
 
-// Inner boxes are written by other threads of the same launch: read them with
-// agent-scope atomic loads so no stale L1 line is used.
-__device__ __forceinline__ void box_of(uint32_t child, const float* leaf_box, const float* inner_box, float* b) {
-    if (child & kLeafBit) {
-        const float* src = leaf_box + 6 * (child & ~kLeafBit);
-        for (int k = 0; k < 6; ++k) b[k] = src[k];
-    } else {
-        const uint32_t* src = reinterpret_cast<const uint32_t*>(inner_box + 6 * child);
-        for (int k = 0; k < 6; ++k)
-            b[k] = __uint_as_float(__hip_atomic_load(src + k, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT));
-    }
-}
-
-// Bottom-up refit: the second thread to reach an inner node builds its box.
-__global__ void k_refit(int n, const int* parent, const uint32_t* left, const uint32_t* right, const float* leaf_box,
-                        float* inner_box, uint32_t* flags) {
+// The tree's depth: the longest way from a leaf to the root (one atomic per
+// wavefront).
+__global__ void k_depth(int n, const int* parent, uint32_t* max_depth) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= n) return;
-    int node = parent[n - 1 + k];
-    while (node >= 0) {
-        __threadfence();
-        const uint32_t old = atomicAdd(&flags[node], 1u);
-        if (old == 0) return;
-        __threadfence();
-        float a[6], b[6];
-        box_of(left[node], leaf_box, inner_box, a);
-        box_of(right[node], leaf_box, inner_box, b);
-        uint32_t* dst = reinterpret_cast<uint32_t*>(inner_box + 6 * node);
-        for (int q = 0; q < 3; ++q) {
-            __hip_atomic_store(dst + q, __float_as_uint(minf(a[q], b[q])), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-            __hip_atomic_store(dst + 3 + q, __float_as_uint(maxf(a[3 + q], b[3 + q])), __ATOMIC_RELAXED,
-                               __HIP_MEMORY_SCOPE_AGENT);
-        }
-        __threadfence();
-        node = parent[node];
-    }
+    uint32_t depth = 0;
+    if (k < n)
+        for (int u = parent[n - 1 + k]; u >= 0; u = parent[u]) ++depth;
+    for (int off = 32; off > 0; off >>= 1) depth = max(depth, static_cast<uint32_t>(__shfl_xor(depth, off)));
+    if ((threadIdx.x & 63u) == 0u) atomicMax(max_depth, depth);
 }
 
-__device__ __forceinline__ uint32_t subtree_size(uint32_t child, const uint32_t* range_lo, const uint32_t* range_hi) {
-    if (child & kLeafBit) return 1u;
-    return 2u * (range_hi[child] - range_lo[child] + 1u) - 1u;
-}
-
-// Depth-first position of every node (walk to the root) and the rope layout.
-__global__ void k_emit(int n, const int* parent, const uint32_t* left, const uint32_t* right, const uint32_t* range_lo,
-                       const uint32_t* range_hi, const float* leaf_box, const float* inner_box, float4* nodes,
-                       uint32_t* max_depth) {
-    const int v = blockIdx.x * blockDim.x + threadIdx.x;
-    if (v >= 2 * n - 1) return;
-    // unified index: v < n-1 inner node v; else leaf v-(n-1)
-    const bool leaf = v >= n - 1;
-    const uint32_t self = leaf ? (kLeafBit | (uint32_t)(v - (n - 1))) : (uint32_t)v;
-    uint32_t pos = 0, depth = 0;
-    int u = v;
-    uint32_t cu = self;
-    while (true) {
-        const int par = parent[u];
-        if (par < 0) break;
-        if (left[par] == cu) pos += 1u;
-        else pos += 1u + subtree_size(left[par], range_lo, range_hi);
-        ++depth;
-        u = par;
-        cu = (uint32_t)par;
-    }
-    const uint32_t size = subtree_size(self, range_lo, range_hi);
-    const float* b = leaf ? (leaf_box + 6 * (v - (n - 1))) : (inner_box + 6 * v);
-    nodes[2 * pos] = make_float4(b[0], b[1], b[2], __uint_as_float(pos + size));
-    nodes[2 * pos + 1] = make_float4(b[3], b[4], b[5], __uint_as_float(leaf ? (uint32_t)(v - (n - 1)) : kInnerNode));
-    atomicMax(max_depth, depth);
-}
-
+// Records and leaf boxes in stored order.
 __global__ void k_gather(const uint32_t* order, uint32_t n, const PrimRecord* rec, const float* box, PrimRecord* rec_out,
                          float* box_out) {
     const uint32_t k = blockIdx.x * blockDim.x + threadIdx.x;
@@ -314,33 +277,7 @@ __global__ void k_gather(const uint32_t* order, uint32_t n, const PrimRecord* re
     for (int q = 0; q < 6; ++q) box_out[6 * k + q] = box[6 * i + q];
 }
 
-__global__ void k_init_parent(int* parent, int count) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < count) parent[i] = -1;
-}
-
-__global__ void k_single_leaf(const float* box, float4* nodes) {
-    nodes[0] = make_float4(box[0], box[1], box[2], __uint_as_float(1u));
-    nodes[1] = make_float4(box[3], box[4], box[5], __uint_as_float(0u));
-}
-
-// ---- walk tree (implicit 4-ary, see vp_internal.h) ----
-
-// Leaf boxes in stored order, taken from the rope tree's leaves.
-__global__ void k_w4_leaf_boxes(const float4* nodes, uint32_t nn, float* box) {
-    const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nn) return;
-    const float4 a = nodes[2 * i], b = nodes[2 * i + 1];
-    const uint32_t prim = __float_as_uint(b.w);
-    if (prim == kInnerNode) return;
-    float* o = box + 6 * static_cast<size_t>(prim);
-    o[0] = a.x;
-    o[1] = a.y;
-    o[2] = a.z;
-    o[3] = b.x;
-    o[4] = b.y;
-    o[5] = b.z;
-}
+// ---- walk tree (implicit 4-ary, see vp_walk.h) ----
 
 __device__ __forceinline__ void w4_store(float4* w4, uint32_t idx, const float lo[3][4], const float hi[3][4]) {
     float4* r = w4 + static_cast<size_t>(kW4RecordF4) * idx;
@@ -447,162 +384,152 @@ __global__ void k_w4_half(const float4* w4, uint32_t records, uint32_t leaf_base
 
 inline uint32_t cdiv(uint32_t a, uint32_t b) { return (a + b - 1) / b; }
 
-struct DevBuf {
-    void* p = nullptr;
-    ~DevBuf() {
-        if (p) (void)hipFree(p);
+// Parts of one allocation, each 256-byte aligned; with base null it only
+// adds up the bytes.
+struct Arena {
+    char* base = nullptr;
+    size_t used = 0;
+    template <typename T>
+    T* take(size_t count) {
+        T* p = reinterpret_cast<T*>(base + used);
+        used += (count * sizeof(T) + 255) / 256 * 256;
+        return p;
+    }
+};
+
+// Device temporaries of a scene build.
+struct BuildTemps {
+    vp_primitive* in;
+    PrimRecord* rec;                // input order
+    float *centers, *box, *sorted_box, *partial, *bounds;
+    uint32_t *codes, *idx, *codes2, *idx2, *hist, *depth;
+    int* parent;
+    float4* w4;                     // 32-bit records
+    uint4* w4_half;
+    double* sums;
+    BuildTemps(Arena& a, uint32_t n, uint32_t nb_sort, uint32_t nbounds, size_t records) {
+        in = a.take<vp_primitive>(n);
+        rec = a.take<PrimRecord>(n);
+        centers = a.take<float>(3 * static_cast<size_t>(n));
+        box = a.take<float>(6 * static_cast<size_t>(n));
+        sorted_box = a.take<float>(6 * static_cast<size_t>(n));
+        partial = a.take<float>(6 * nbounds);
+        bounds = a.take<float>(6);
+        codes = a.take<uint32_t>(n);
+        idx = a.take<uint32_t>(n);
+        codes2 = a.take<uint32_t>(n);
+        idx2 = a.take<uint32_t>(n);
+        hist = a.take<uint32_t>(256 * static_cast<size_t>(nb_sort));
+        depth = a.take<uint32_t>(1);
+        parent = a.take<int>(2 * static_cast<size_t>(n));
+        w4 = a.take<float4>(kW4RecordF4 * records);
+        w4_half = a.take<uint4>(kW4hRecordB / sizeof(uint4) * records);
+        sums = a.take<double>(2);
     }
 };
 
 }  // namespace
 }  // namespace vp
 
-vp_status vp_build_scene_device(vp_context* ctx, const vp_primitive* host_prims, uint32_t n, vp_scene* sc) {
+// Builds scene sc (whose n is set): records, Morton codes and stored order,
+// the order from the radix sort or, with VP_SCENE_BVH_SAH / _MEDIAN in flags,
+// from the host tree, and the walk tree over it.  The temporaries are one
+// allocation and the scene owns two.
+vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32_t n, uint32_t flags, vp_scene* sc) {
     using namespace vp;
     hipStream_t s = ctx->stream;
     const uint32_t nb_sort = cdiv(n, kSortTile);
     const uint32_t nbounds = min(cdiv(n, 256u), 1024u);
-    DevBuf d_in, d_rec, d_centers, d_box, d_partial, d_bounds, d_codes, d_idx, d_codes2, d_idx2, d_hist, d_box_sorted;
-    DevBuf d_left, d_right, d_lo, d_hi, d_parent, d_inner, d_flags, d_depth;
-    VP_HIP_TRY(hipMalloc(&d_in.p, sizeof(vp_primitive) * n));
-    VP_HIP_TRY(hipMalloc(&d_rec.p, sizeof(PrimRecord) * n));
-    VP_HIP_TRY(hipMalloc(&d_centers.p, sizeof(float) * 3 * n));
-    VP_HIP_TRY(hipMalloc(&d_box.p, sizeof(float) * 6 * n));
-    VP_HIP_TRY(hipMalloc(&d_box_sorted.p, sizeof(float) * 6 * n));
-    VP_HIP_TRY(hipMalloc(&d_partial.p, sizeof(float) * 6 * nbounds));
-    VP_HIP_TRY(hipMalloc(&d_bounds.p, sizeof(float) * 6));
-    VP_HIP_TRY(hipMalloc(&d_codes.p, sizeof(uint32_t) * n));
-    VP_HIP_TRY(hipMalloc(&d_idx.p, sizeof(uint32_t) * n));
-    VP_HIP_TRY(hipMalloc(&d_codes2.p, sizeof(uint32_t) * n));
-    VP_HIP_TRY(hipMalloc(&d_idx2.p, sizeof(uint32_t) * n));
-    VP_HIP_TRY(hipMalloc(&d_hist.p, sizeof(uint32_t) * 256 * nb_sort));
-    VP_HIP_TRY(hipMalloc(&d_depth.p, sizeof(uint32_t)));
+    const uint32_t levels = w4_levels(n);
+    const size_t records = w4_records(levels);
+    Arena need;
+    BuildTemps(need, n, nb_sort, nbounds, records);
+    Arena arena;
+    struct Free {
+        char*& p;
+        ~Free() {
+            if (p) (void)hipFree(p);
+        }
+    } free_temps{arena.base};
+    VP_HIP_TRY(hipMalloc(reinterpret_cast<void**>(&arena.base), need.used));
+    const BuildTemps T(arena, n, nb_sort, nbounds, records);
     // the records are padded to a multiple of the leaf block with zero records
     // (zero inverse scales: no ray enters them), so a walk may hand every slot
     // of a leaf block to the leaf tests
     const size_t n_slots = (static_cast<size_t>(n) + kLeafBlock - 1u) / kLeafBlock * kLeafBlock;
-    VP_HIP_TRY(hipMalloc(&sc->prims, sizeof(PrimRecord) * n_slots));
+    for (int pass = 0; pass < 2; ++pass) {
+        Arena a;
+        a.base = static_cast<char*>(sc->mem);
+        sc->prims = a.take<PrimRecord>(n_slots);
+        sc->order = a.take<uint32_t>(n);
+        sc->morton = a.take<uint32_t>(n);
+        if (pass == 0) VP_HIP_TRY(hipMalloc(&sc->mem, a.used));
+    }
     if (n_slots > n) VP_HIP_TRY(hipMemsetAsync(sc->prims + n, 0, sizeof(PrimRecord) * (n_slots - n), s));
-    VP_HIP_TRY(hipMalloc(&sc->nodes, sizeof(float4) * 2 * (2 * n - 1)));
-    VP_HIP_TRY(hipMalloc(&sc->order, sizeof(uint32_t) * n));
-    VP_HIP_TRY(hipMalloc(&sc->morton, sizeof(uint32_t) * n));
-    VP_HIP_TRY(hipMemcpyAsync(d_in.p, host_prims, sizeof(vp_primitive) * n, hipMemcpyHostToDevice, s));
-    VP_HIP_TRY(hipMemsetAsync(d_depth.p, 0, sizeof(uint32_t), s));
+    VP_HIP_TRY(hipMemcpyAsync(T.in, host_prims, sizeof(vp_primitive) * n, hipMemcpyHostToDevice, s));
+    VP_HIP_TRY(hipMemsetAsync(T.depth, 0, sizeof(uint32_t), s));
+    VP_HIP_TRY(hipMemsetAsync(T.sums, 0, 2 * sizeof(double), s));
 
     const uint32_t g = cdiv(n, 256u);
-    hipLaunchKernelGGL(k_setup, dim3(g), dim3(256), 0, s, (const vp_primitive*)d_in.p, n, (PrimRecord*)d_rec.p,
-                       (float*)d_centers.p, (float*)d_box.p);
-    hipLaunchKernelGGL(k_bounds_partial, dim3(nbounds), dim3(256), 0, s, (const float*)d_centers.p, n,
-                       (float*)d_partial.p);
-    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(64), 0, s, (const float*)d_partial.p, nbounds,
-                       (float*)d_bounds.p);
-    hipLaunchKernelGGL(k_morton, dim3(g), dim3(256), 0, s, (const float*)d_centers.p, n, (const float*)d_bounds.p,
-                       (uint32_t*)d_codes.p, (uint32_t*)d_idx.p);
-    VP_HIP_TRY(hipMemcpyAsync(sc->morton, d_codes.p, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
+    hipLaunchKernelGGL(k_setup, dim3(g), dim3(256), 0, s, T.in, n, T.rec, T.centers, T.box);
+    hipLaunchKernelGGL(k_bounds_partial, dim3(nbounds), dim3(256), 0, s, T.centers, n, T.partial);
+    hipLaunchKernelGGL(k_bounds_final, dim3(1), dim3(64), 0, s, T.partial, nbounds, T.bounds);
+    hipLaunchKernelGGL(k_morton, dim3(g), dim3(256), 0, s, T.centers, n, T.bounds, T.codes, T.idx);
+    VP_HIP_TRY(hipGetLastError());
+    VP_HIP_TRY(hipMemcpyAsync(sc->morton, T.codes, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
 
-    uint32_t* kin = (uint32_t*)d_codes.p;
-    uint32_t* vin = (uint32_t*)d_idx.p;
-    uint32_t* kout = (uint32_t*)d_codes2.p;
-    uint32_t* vout = (uint32_t*)d_idx2.p;
-    for (uint32_t shift = 0; shift < 32; shift += 8) {
-        hipLaunchKernelGGL(k_hist, dim3(nb_sort), dim3(kSortBlock), 0, s, kin, n, shift, (uint32_t*)d_hist.p,
-                           nb_sort);
-        hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, (uint32_t*)d_hist.p, 256 * nb_sort);
-        hipLaunchKernelGGL(k_scatter, dim3(nb_sort), dim3(kSortBlock), 0, s, kin, vin, n, shift,
-                           (const uint32_t*)d_hist.p, nb_sort, kout, vout);
-        std::swap(kin, kout);
-        std::swap(vin, vout);
-    }
-    // after 4 passes the sorted data is back in kin/vin
-    VP_HIP_TRY(hipMemcpyAsync(sc->order, vin, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
-    hipLaunchKernelGGL(k_gather, dim3(g), dim3(256), 0, s, (const uint32_t*)vin, n, (const PrimRecord*)d_rec.p,
-                       (const float*)d_box.p, sc->prims, (float*)d_box_sorted.p);
-
-    if (n == 1) {
-        hipLaunchKernelGGL(k_single_leaf, dim3(1), dim3(1), 0, s, (const float*)d_box_sorted.p, sc->nodes);
-        sc->depth = 0;
+    uint32_t depth = 0;
+    std::vector<uint32_t> host_order;
+    const bool host_tree = (flags & (VP_SCENE_BVH_SAH | VP_SCENE_BVH_MEDIAN)) != 0u;
+    if (host_tree) {
+        vp_host_tree_order(host_prims, n, (flags & VP_SCENE_BVH_MEDIAN) != 0u, host_order, sc->depth);
+        VP_HIP_TRY(hipMemcpyAsync(sc->order, host_order.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice, s));
     } else {
-        VP_HIP_TRY(hipMalloc(&d_left.p, sizeof(uint32_t) * (n - 1)));
-        VP_HIP_TRY(hipMalloc(&d_right.p, sizeof(uint32_t) * (n - 1)));
-        VP_HIP_TRY(hipMalloc(&d_lo.p, sizeof(uint32_t) * (n - 1)));
-        VP_HIP_TRY(hipMalloc(&d_hi.p, sizeof(uint32_t) * (n - 1)));
-        VP_HIP_TRY(hipMalloc(&d_parent.p, sizeof(int) * (2 * n - 1)));
-        VP_HIP_TRY(hipMalloc(&d_inner.p, sizeof(float) * 6 * (n - 1)));
-        VP_HIP_TRY(hipMalloc(&d_flags.p, sizeof(uint32_t) * (n - 1)));
-        VP_HIP_TRY(hipMemsetAsync(d_flags.p, 0, sizeof(uint32_t) * (n - 1), s));
-        hipLaunchKernelGGL(k_init_parent, dim3(cdiv(2 * n - 1, 256u)), dim3(256), 0, s, (int*)d_parent.p,
-                           (int)(2 * n - 1));
-        hipLaunchKernelGGL(k_karras, dim3(cdiv(n - 1, 256u)), dim3(256), 0, s, (const uint32_t*)kin, (int)n,
-                           (uint32_t*)d_left.p, (uint32_t*)d_right.p, (uint32_t*)d_lo.p, (uint32_t*)d_hi.p,
-                           (int*)d_parent.p);
-        hipLaunchKernelGGL(k_refit, dim3(g), dim3(256), 0, s, (int)n, (const int*)d_parent.p,
-                           (const uint32_t*)d_left.p, (const uint32_t*)d_right.p, (const float*)d_box_sorted.p,
-                           (float*)d_inner.p, (uint32_t*)d_flags.p);
-        hipLaunchKernelGGL(k_emit, dim3(cdiv(2 * n - 1, 256u)), dim3(256), 0, s, (int)n, (const int*)d_parent.p,
-                           (const uint32_t*)d_left.p, (const uint32_t*)d_right.p, (const uint32_t*)d_lo.p,
-                           (const uint32_t*)d_hi.p, (const float*)d_box_sorted.p, (const float*)d_inner.p,
-                           sc->nodes, (uint32_t*)d_depth.p);
-        uint32_t depth = 0;
-        VP_HIP_TRY(hipMemcpyAsync(&depth, d_depth.p, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        VP_HIP_TRY(hipStreamSynchronize(s));
-        sc->depth = depth;
+        uint32_t *kin = T.codes, *vin = T.idx, *kout = T.codes2, *vout = T.idx2;
+        for (uint32_t shift = 0; shift < 32; shift += 8) {
+            hipLaunchKernelGGL(k_hist, dim3(nb_sort), dim3(kSortBlock), 0, s, kin, n, shift, T.hist, nb_sort);
+            hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, s, T.hist, 256 * nb_sort);
+            hipLaunchKernelGGL(k_scatter, dim3(nb_sort), dim3(kSortBlock), 0, s, kin, vin, n, shift, T.hist, nb_sort,
+                               kout, vout);
+            std::swap(kin, kout);
+            std::swap(vin, vout);
+        }
+        // after 4 passes the sorted data is back in kin/vin
+        VP_HIP_TRY(hipMemcpyAsync(sc->order, vin, sizeof(uint32_t) * n, hipMemcpyDeviceToDevice, s));
+        if (n > 1) {
+            hipLaunchKernelGGL(k_karras, dim3(cdiv(n - 1, 256u)), dim3(256), 0, s, kin, (int)n, T.parent);
+            hipLaunchKernelGGL(k_depth, dim3(g), dim3(256), 0, s, (int)n, T.parent, T.depth);
+        }
+        VP_HIP_TRY(hipGetLastError());
+        VP_HIP_TRY(hipMemcpyAsync(&depth, T.depth, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     }
-    VP_HIP_TRY(hipGetLastError());
-    VP_HIP_TRY(hipStreamSynchronize(s));
-    return VP_OK;
-}
+    hipLaunchKernelGGL(k_gather, dim3(g), dim3(256), 0, s, sc->order, n, T.rec, T.box, sc->prims, T.sorted_box);
 
-vp_status vp_build_walk_tree(vp_context* ctx, vp_scene* sc, uint32_t walk_format) {
-    using namespace vp;
-    hipStream_t s = ctx->stream;
-    const uint32_t n = sc->n;
-    const uint32_t levels = w4_levels(n);
-    const size_t records = w4_records(levels);
-    if (sc->w4) {
-        VP_HIP_TRY(hipStreamSynchronize(s));
-        VP_HIP_TRY(hipFree(sc->w4));
-        sc->w4 = nullptr;
-    }
-    DevBuf d_box;
-    VP_HIP_TRY(hipMalloc(&d_box.p, sizeof(float) * 6 * static_cast<size_t>(n)));
-    VP_HIP_TRY(hipMalloc(&sc->w4, sizeof(float4) * kW4RecordF4 * records));
-    const uint32_t nn = 2 * n - 1;
-    hipLaunchKernelGGL(k_w4_leaf_boxes, dim3(cdiv(nn, 256u)), dim3(256), 0, s, (const float4*)sc->nodes, nn,
-                       (float*)d_box.p);
+    // the walk tree in 32-bit records, bottom up
     const uint32_t bottom = 1u << (2u * (levels - 1u));
-    hipLaunchKernelGGL(k_w4_bottom, dim3(cdiv(bottom, 256u)), dim3(256), 0, s, (const float*)d_box.p, n, levels,
-                       sc->w4);
+    hipLaunchKernelGGL(k_w4_bottom, dim3(cdiv(bottom, 256u)), dim3(256), 0, s, T.sorted_box, n, levels, T.w4);
     for (uint32_t l = levels - 1u; l-- > 0;)
-        hipLaunchKernelGGL(k_w4_level, dim3(cdiv(1u << (2u * l), 256u)), dim3(256), 0, s, l, sc->w4);
-    VP_HIP_TRY(hipGetLastError());
+        hipLaunchKernelGGL(k_w4_level, dim3(cdiv(1u << (2u * l), 256u)), dim3(256), 0, s, l, T.w4);
     sc->w4_levels = levels;
-    sc->w4_half = 0u;
-    sc->w4_growth = 0.0;
-    if (walk_format == VP_SCENE_WALK_F32) {
-        VP_HIP_TRY(hipStreamSynchronize(s));
-        return VP_OK;
-    }
     // the 16-bit records, kept when forced or when the leaf boxes' summed
     // surface grows by at most 1/16 (more leaf tests and node visits, against
     // half the bytes per node visit)
-    DevBuf d_half, d_sums;
-    VP_HIP_TRY(hipMalloc(&d_half.p, static_cast<size_t>(kW4hRecordB) * records));
-    VP_HIP_TRY(hipMalloc(&d_sums.p, 2 * sizeof(double)));
-    VP_HIP_TRY(hipMemsetAsync(d_sums.p, 0, 2 * sizeof(double), s));
-    hipLaunchKernelGGL(k_w4_half, dim3(cdiv(static_cast<uint32_t>(records), 256u)), dim3(256), 0, s,
-                       (const float4*)sc->w4, static_cast<uint32_t>(records), w4_level_base(levels - 1u),
-                       (uint4*)d_half.p, (double*)d_sums.p);
-    VP_HIP_TRY(hipGetLastError());
     double sums[2] = {0.0, 0.0};
-    VP_HIP_TRY(hipMemcpyAsync(sums, d_sums.p, sizeof(sums), hipMemcpyDeviceToHost, s));
-    VP_HIP_TRY(hipStreamSynchronize(s));
-    const double growth = sums[0] > 0.0 ? sums[1] / sums[0] - 1.0 : 0.0;
-    sc->w4_growth = growth;
-    if (walk_format == VP_SCENE_WALK_F16 || (growth <= 1.0 / 16.0)) {
-        VP_HIP_TRY(hipFree(sc->w4));
-        sc->w4 = static_cast<float4*>(d_half.p);
-        d_half.p = nullptr;
-        sc->w4_half = 1u;
+    if (!(flags & VP_SCENE_WALK_F32)) {
+        hipLaunchKernelGGL(k_w4_half, dim3(cdiv(static_cast<uint32_t>(records), 256u)), dim3(256), 0, s, T.w4,
+                           static_cast<uint32_t>(records), w4_level_base(levels - 1u), T.w4_half, T.sums);
+        VP_HIP_TRY(hipMemcpyAsync(sums, T.sums, sizeof(sums), hipMemcpyDeviceToHost, s));
     }
+    VP_HIP_TRY(hipGetLastError());
+    VP_HIP_TRY(hipStreamSynchronize(s));
+    if (!host_tree) sc->depth = depth;
+    sc->w4_growth = sums[0] > 0.0 ? sums[1] / sums[0] - 1.0 : 0.0;
+    const bool half = !(flags & VP_SCENE_WALK_F32) && ((flags & VP_SCENE_WALK_F16) || sc->w4_growth <= 1.0 / 16.0);
+    const size_t w4_bytes = (half ? static_cast<size_t>(kW4hRecordB) : sizeof(float4) * kW4RecordF4) * records;
+    VP_HIP_TRY(hipMalloc(&sc->w4, w4_bytes));
+    VP_HIP_TRY(hipMemcpyAsync(sc->w4, half ? static_cast<const void*>(T.w4_half) : T.w4, w4_bytes,
+                              hipMemcpyDeviceToDevice, s));
+    sc->w4_half = half ? 1u : 0u;
+    VP_HIP_TRY(hipStreamSynchronize(s));
     return VP_OK;
 }

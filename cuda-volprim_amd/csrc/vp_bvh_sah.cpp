@@ -5,16 +5,13 @@
 // Morton-code bits, which leaves sibling boxes overlapping when primitive
 // sizes vary; shadow rays then visit more nodes.  This builder makes a binned
 // SAH tree over the same conservative leaf boxes (32 bins per axis, one
-// primitive per leaf) on the host and lays it out exactly like the LBVH:
-// depth-first nodes with skip links, primitives stored in leaf order.  It
-// replaces the LBVH's nodes, stored records and order; the Morton codes the
-// GPU build computed stay available for export.  Render results do not
-// depend on the tree (every query is consumed order-independently or in
-// stored-index order), so both builds give the same images for the same
-// stored order.
+// primitive per leaf) on the host and hands its leaf order to the GPU build,
+// which stores the primitives in it and lays the walk tree over them; the
+// Morton codes stay available for export.  Render results do not depend on
+// the tree (every query is consumed order-independently or in stored-index
+// order), so both builds give the same images for the same stored order.
 #include <algorithm>
 #include <cmath>
-#include <cstring>
 #include <vector>
 
 #include "vp_internal.h"
@@ -210,18 +207,18 @@ int32_t build_median(Tree& T, std::vector<uint32_t>& idx, uint32_t n, const std:
 
 }  // namespace
 
-vp_status vp_build_scene_sah(vp_context* ctx, const vp_primitive* in, uint32_t n, vp_scene* sc, bool median) {
-    // records and conservative boxes exactly as the GPU setup kernel makes them
-    std::vector<vp::PrimRecord> rec(n);
+void vp_host_tree_order(const vp_primitive* in, uint32_t n, bool median, std::vector<uint32_t>& order,
+                        uint32_t& depth_out) {
+    // conservative boxes exactly as the GPU setup kernel makes them
     std::vector<Box> boxes(n);
     std::vector<float> cen(3 * static_cast<size_t>(n));
     for (uint32_t i = 0; i < n; ++i) {
         const vp_primitive& p = in[i];
         const vp::f3 c = vp::f3{p.center[0], p.center[1], p.center[2]};
         const vp::f3 s = vp::f3{p.scale[0], p.scale[1], p.scale[2]};
-        rec[i] = vp::make_prim(c, p.quat_wxyz[0], p.quat_wxyz[1], p.quat_wxyz[2], p.quat_wxyz[3], s,
-                               vp::f3{p.albedo[0], p.albedo[1], p.albedo[2]}, p.mass);
-        vp::conservative_box(rec[i], p.scale, boxes[i].lo, boxes[i].hi);
+        const vp::PrimRecord rec = vp::make_prim(c, p.quat_wxyz[0], p.quat_wxyz[1], p.quat_wxyz[2], p.quat_wxyz[3], s,
+                                                 vp::f3{p.albedo[0], p.albedo[1], p.albedo[2]}, p.mass);
+        vp::conservative_box(rec, p.scale, boxes[i].lo, boxes[i].hi);
         for (int k = 0; k < 3; ++k) cen[3 * i + k] = p.center[k];
     }
     Tree T;
@@ -232,52 +229,25 @@ vp_status vp_build_scene_sah(vp_context* ctx, const vp_primitive* in, uint32_t n
         build_median(T, idx, n, boxes, cen);
     else
         build(T, idx, 0, n, boxes, cen);
-    // depth-first layout with skip links; leaves numbered in visiting order
-    const size_t nn = 2 * static_cast<size_t>(n) - 1;
-    std::vector<float4> nodes(2 * nn);
-    std::vector<uint32_t> order;
+    // leaves numbered in depth-first order
+    order.clear();
     order.reserve(n);
-    std::vector<vp::PrimRecord> stored;
-    stored.reserve(n);
     uint32_t depth = 0;
     struct Frame {
         int32_t node;
         uint32_t level;
     };
     std::vector<Frame> st{{0, 1}};
-    uint32_t pos = 0;
-    std::vector<uint32_t> size_of(T.nodes.size(), 1);
-    // subtree sizes (children are created after their parent)
-    for (size_t k = T.nodes.size(); k-- > 0;)
-        if (T.nodes[k].left >= 0) size_of[k] = 1 + size_of[T.nodes[k].left] + size_of[T.nodes[k].right];
     while (!st.empty()) {
         const Frame f = st.back();
         st.pop_back();
         const auto& N = T.nodes[f.node];
         depth = std::max(depth, f.level);
-        const uint32_t skip = pos + size_of[f.node];
-        uint32_t prim_field = vp::kInnerNode;
-        if (N.prim >= 0) {
-            prim_field = static_cast<uint32_t>(order.size());
-            order.push_back(static_cast<uint32_t>(N.prim));
-            stored.push_back(rec[N.prim]);
-        }
-        float sk, pf;
-        std::memcpy(&sk, &skip, 4);
-        std::memcpy(&pf, &prim_field, 4);
-        nodes[2 * pos] = make_float4(N.box.lo[0], N.box.lo[1], N.box.lo[2], sk);
-        nodes[2 * pos + 1] = make_float4(N.box.hi[0], N.box.hi[1], N.box.hi[2], pf);
-        ++pos;
+        if (N.prim >= 0) order.push_back(static_cast<uint32_t>(N.prim));
         if (N.left >= 0) {
             st.push_back({N.right, f.level + 1});
             st.push_back({N.left, f.level + 1});
         }
     }
-    hipStream_t s = ctx->stream;
-    VP_HIP_TRY(hipMemcpyAsync(sc->nodes, nodes.data(), sizeof(float4) * nodes.size(), hipMemcpyHostToDevice, s));
-    VP_HIP_TRY(hipMemcpyAsync(sc->prims, stored.data(), sizeof(vp::PrimRecord) * n, hipMemcpyHostToDevice, s));
-    VP_HIP_TRY(hipMemcpyAsync(sc->order, order.data(), sizeof(uint32_t) * n, hipMemcpyHostToDevice, s));
-    VP_HIP_TRY(hipStreamSynchronize(s));
-    sc->depth = depth;
-    return VP_OK;
+    depth_out = depth;
 }

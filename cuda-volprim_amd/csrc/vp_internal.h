@@ -15,20 +15,6 @@
 
 namespace vp {
 
-// ---------------------------------------------------------------------------
-// BVH: 2N-1 nodes in depth-first preorder, 32 bytes each (two float4):
-//   a = (min.x, min.y, min.z, skip)   skip = index of the next node when the
-//                                     subtree is skipped (2N-1 ends the walk)
-//   b = (max.x, max.y, max.z, prim)   prim = stored primitive index of a leaf,
-//                                     0xffffffff for an inner node
-// A hit inner node continues at i + 1 (its left child).  Leaves appear in
-// stored-primitive order, so a walk meets primitives in ascending index.
-// ---------------------------------------------------------------------------
-constexpr uint32_t kInnerNode = 0xffffffffu;
-
-// The walk tree the render kernels traverse is defined in vp_walk.h; its leaf
-// boxes are the rope tree's, so a walk of either meets the same leaves.
-
 // Conservative leaf box of record r (input scale s, centre c): the 3-sigma
 // ellipsoid with forward rotation R and scale s has half extent
 // 3 sqrt(sum_j (R_ij s_j)^2) along world axis i; the box is widened by a
@@ -56,9 +42,6 @@ VP_HD void conservative_box(const PrimRecord& r, const float s[3], float lo[3], 
 
 struct SceneView {
     const PrimRecord* prims;
-    const float4* nodes;
-    uint32_t n_prims;
-    uint32_t n_nodes;
     const float4* w4;    // walk-tree records (kW4RecordF4 float4 each, or 16-bit records)
     uint32_t w4_levels;  // its level count L
     uint32_t w4_half;    // 1: w4 holds 16-bit records (kW4hRecordB bytes each)
@@ -244,8 +227,8 @@ struct vp_scene {
     vp_context* ctx = nullptr;
     uint32_t n = 0;
     uint32_t depth = 0;
-    vp::PrimRecord* prims = nullptr;  // stored (Morton) order
-    float4* nodes = nullptr;           // 2 * (2n - 1)
+    void* mem = nullptr;               // prims, order and morton
+    vp::PrimRecord* prims = nullptr;  // stored order
     uint32_t* order = nullptr;         // order[k] = input index
     uint32_t* morton = nullptr;        // codes in input order
     float4* w4 = nullptr;              // walk tree, w4_records(w4_levels) records
@@ -253,7 +236,7 @@ struct vp_scene {
     uint32_t w4_half = 0;              // 1: 16-bit records
     double w4_growth = 0.0;            // summed leaf-box surface of the 16-bit records / 32-bit - 1
     vp::SceneView view() const {
-        return vp::SceneView{prims, nodes, n, n ? 2 * n - 1 : 0, w4, w4_levels, w4_half};
+        return vp::SceneView{prims, w4, w4_levels, w4_half};
     }
 };
 
@@ -282,17 +265,13 @@ void vp_set_error(const std::string& msg);
         }                                                                                  \
     } while (0)
 
-// launchers (vp_bvh.hip)
-vp_status vp_build_scene_device(vp_context* ctx, const vp_primitive* host_prims, uint32_t n, vp_scene* scene);
-// host tree replacing the device LBVH's nodes, records and order (vp_bvh_sah.cpp):
-// binned SAH, or (median) balanced median splits on the walk tree's record
-// boundaries
-vp_status vp_build_scene_sah(vp_context* ctx, const vp_primitive* host_prims, uint32_t n, vp_scene* scene,
-                             bool median);
-// walk tree over the scene's stored order, from its rope tree's leaf boxes (vp_bvh.hip)
-// walk_format: 0 (16-bit records when the leaf boxes grow little),
-// VP_SCENE_WALK_F32 or VP_SCENE_WALK_F16
-vp_status vp_build_walk_tree(vp_context* ctx, vp_scene* scene, uint32_t walk_format);
+// Scene build (vp_bvh.hip); flags as in vp_scene_create_ex, checked.
+vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32_t n, uint32_t flags, vp_scene* scene);
+// Leaf order and depth of a host tree over the input primitives
+// (vp_bvh_sah.cpp): binned SAH, or (median) balanced median splits on the walk
+// tree's record boundaries.
+void vp_host_tree_order(const vp_primitive* in, uint32_t n, bool median, std::vector<uint32_t>& order,
+                        uint32_t& depth);
 
 // launchers (vp_render.hip)
 struct RenderLaunch {
