@@ -128,7 +128,56 @@ void build_alias(const std::vector<float>& joint, std::vector<vp::AliasEntry>& o
     }
 }
 
+// One render, its image in device memory or for the host.
+vp_status render_one(vp_context* ctx, vp_scene* sc, vp_env* env, const vp_camera* cam, const vp_render_params* params,
+                     const vp_launch_config* launch, float* out_dev, float* out_host, float* out_samples_dev,
+                     hipStream_t s, vp_render_stats* stats) {
+    vp_status st = vp_check_params(params);
+    if (st != VP_OK) return st;
+    const auto t0 = std::chrono::steady_clock::now();
+    VP_HIP_TRY(hipSetDevice(ctx->device));
+    const uint32_t cap = params->active_cap ? params->active_cap : 128u;
+    std::vector<JobRun> runs(1);
+    runs[0].desc = vp_make_job(sc, env, cam, params);
+    runs[0].mean = reinterpret_cast<float4*>(out_dev);
+    runs[0].host_out = out_host;
+    runs[0].samples_all = reinterpret_cast<float4*>(out_samples_dev);
+    if (launch && launch->batch_spp) runs[0].slice_spp = launch->batch_spp;
+    double kms = 0.0;
+    unsigned long long c[vp::kNumCounters];
+    st = vp_run_jobs(ctx, runs, launch, cap, 0, params->measure_caps ? 1 : 0, s, &kms, nullptr, c);
+    if (st != VP_OK) return st;
+    vp_fill_stats(c, stats);
+    if (stats) {
+        stats->kernel_ms = kms;
+        stats->launches = ctx->last_launches;
+        stats->paths = runs[0].traced;
+        stats->wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
+    }
+    return VP_OK;
+}
+
+// The validation of loadPrimitivesFromPLY (ply.cpp:146-172): nullptr, or what
+// is wrong with p.
+const char* primitive_fault(const vp_primitive& p) {
+    if (!(p.scale[0] > 0.0f && p.scale[1] > 0.0f && p.scale[2] > 0.0f) || !finite3(p.scale))
+        return "scale must be finite and > 0";
+    if (!(p.mass > 0.0f) || !std::isfinite(p.mass)) return "mass must be finite and > 0";
+    if (!finite3(p.center)) return "non-finite centre";
+    const float q2 = p.quat_wxyz[0] * p.quat_wxyz[0] + p.quat_wxyz[1] * p.quat_wxyz[1] +
+                     p.quat_wxyz[2] * p.quat_wxyz[2] + p.quat_wxyz[3] * p.quat_wxyz[3];
+    if (!(q2 > 0.0f) || !std::isfinite(q2)) return "degenerate quaternion";
+    return nullptr;
+}
+
 }  // namespace
+
+bool vp_primitives_valid(const void* rows, size_t count) {
+    const auto* p = static_cast<const vp_primitive*>(rows);
+    for (size_t i = 0; i < count; ++i)
+        if (primitive_fault(p[i])) return false;
+    return true;
+}
 
 void vp_set_error(const std::string& msg) { g_error = msg; }
 vp_status vp_check_params(const vp_render_params* p) { return check_params_impl(p); }
@@ -172,6 +221,10 @@ vp_status vp_context_destroy(vp_context* ctx) {
     (void)hipSetDevice(ctx->device);
     if (ctx->stream) (void)hipStreamSynchronize(ctx->stream);
     if (ctx->slab) (void)hipFree(ctx->slab);
+    if (ctx->scratch) (void)hipFree(ctx->scratch);
+    if (ctx->stage) (void)hipHostFree(ctx->stage);
+    for (hipEvent_t e : ctx->stage_ev)
+        if (e) (void)hipEventDestroy(e);
     if (ctx->counters) (void)hipFree(ctx->counters);
     if (ctx->path_counter) (void)hipFree(ctx->path_counter);
     vp_drop_graph(ctx);
@@ -215,19 +268,6 @@ vp_status vp_scene_create_ex(vp_context* ctx, const vp_primitive* prims, uint32_
         return fail(VP_ERR_INVALID, "VP_SCENE_WALK_F32 and VP_SCENE_WALK_F16 exclude each other");
     if (n == 0) return fail(VP_ERR_INVALID, "scene has no primitives");
     if (n > (1u << 30)) return fail(VP_ERR_INVALID, "scene has more than 2^30 primitives");
-    // the validation of loadPrimitivesFromPLY (ply.cpp:146-172)
-    for (uint32_t i = 0; i < n; ++i) {
-        const vp_primitive& p = prims[i];
-        if (!(p.scale[0] > 0.0f && p.scale[1] > 0.0f && p.scale[2] > 0.0f) || !finite3(p.scale))
-            return fail(VP_ERR_INVALID, "primitive " + std::to_string(i) + ": scale must be finite and > 0");
-        if (!(p.mass > 0.0f) || !std::isfinite(p.mass))
-            return fail(VP_ERR_INVALID, "primitive " + std::to_string(i) + ": mass must be finite and > 0");
-        if (!finite3(p.center)) return fail(VP_ERR_INVALID, "primitive " + std::to_string(i) + ": non-finite centre");
-        const float q2 = p.quat_wxyz[0] * p.quat_wxyz[0] + p.quat_wxyz[1] * p.quat_wxyz[1] +
-                         p.quat_wxyz[2] * p.quat_wxyz[2] + p.quat_wxyz[3] * p.quat_wxyz[3];
-        if (!(q2 > 0.0f) || !std::isfinite(q2))
-            return fail(VP_ERR_INVALID, "primitive " + std::to_string(i) + ": degenerate quaternion");
-    }
     VP_HIP_TRY(hipSetDevice(ctx->device));
     auto* sc = new vp_scene();
     sc->ctx = ctx;
@@ -235,6 +275,10 @@ vp_status vp_scene_create_ex(vp_context* ctx, const vp_primitive* prims, uint32_
     const vp_status st = vp_build_scene(ctx, prims, n, flags, sc);
     if (st != VP_OK) {
         vp_scene_destroy(sc);
+        // a fault of the input is reported before any other
+        for (uint32_t i = 0; i < n; ++i)
+            if (const char* what = primitive_fault(prims[i]))
+                return fail(VP_ERR_INVALID, "primitive " + std::to_string(i) + ": " + what);
         return st;
     }
     *out = sc;
@@ -253,20 +297,21 @@ vp_status vp_scene_destroy(vp_scene* sc) {
 vp_status vp_scene_export(vp_scene* sc, uint32_t* order, uint32_t* morton, float* records16, uint32_t* depth) {
     if (!sc) return fail(VP_ERR_INVALID, "scene is null");
     hipStream_t s = sc->ctx->stream;
-    if (order) VP_HIP_TRY(hipMemcpyAsync(order, sc->order, sizeof(uint32_t) * sc->n, hipMemcpyDeviceToHost, s));
-    if (morton) VP_HIP_TRY(hipMemcpyAsync(morton, sc->morton, sizeof(uint32_t) * sc->n, hipMemcpyDeviceToHost, s));
-    // the records in the exported field order, through a stream-ordered copy
-    void* rec = nullptr;
-    hipError_t e = hipSuccess;
+    const size_t words = sizeof(uint32_t) * static_cast<size_t>(sc->n);
+    HostCopy outs[3];
+    size_t k = 0;
+    if (order) outs[k++] = {order, sc->order, words};
+    if (morton) outs[k++] = {morton, sc->morton, words};
+    ScratchLease rec;  // the records in the exported field order
     if (records16) {
-        const size_t bytes = sizeof(vp::PrimRecord) * sc->n;
-        e = hipMallocAsync(&rec, bytes, s);
-        if (e == hipSuccess) e = vp_launch_export_records(sc->prims, sc->n, static_cast<float4*>(rec), s);
-        if (e == hipSuccess) e = hipMemcpyAsync(records16, rec, bytes, hipMemcpyDeviceToHost, s);
-        if (rec) (void)hipFreeAsync(rec, s);
+        const vp_status st = vp_lease_scratch(sc->ctx, 16 * words, s, rec);
+        if (st != VP_OK) return st;
+        VP_HIP_TRY(vp_launch_export_records(sc->prims, sc->n, static_cast<float4*>(rec.p), s));
+        outs[k++] = {records16, rec.p, 16 * words};
     }
-    VP_HIP_TRY(e);
-    VP_HIP_TRY(hipStreamSynchronize(s));
+    const vp_status st = vp_copy_out(sc->ctx, outs, k, s);
+    if (st != VP_OK) return st;
+    rec.done = true;
     if (depth) *depth = sc->depth;
     return VP_OK;
 }
@@ -433,32 +478,8 @@ vp_status vp_render_device(vp_context* ctx, vp_scene* sc, vp_env* env, const vp_
                            const vp_render_params* params, const vp_launch_config* launch, float* out_rgba_dev,
                            float* out_samples_dev, void* stream, vp_render_stats* stats) {
     if (!ctx || !sc || !env || !cam || !out_rgba_dev) return fail(VP_ERR_INVALID, "null argument");
-    vp_status st = vp_check_params(params);
-    if (st != VP_OK) return st;
-    const auto t0 = std::chrono::steady_clock::now();
-    VP_HIP_TRY(hipSetDevice(ctx->device));
-    hipStream_t s = stream ? static_cast<hipStream_t>(stream) : ctx->stream;
-    const uint32_t cap = params->active_cap ? params->active_cap : 128u;
-    std::vector<JobRun> runs(1);
-    runs[0].desc = vp_make_job(sc, env, cam, params);
-    runs[0].mean = reinterpret_cast<float4*>(out_rgba_dev);
-    runs[0].samples_all = reinterpret_cast<float4*>(out_samples_dev);
-    if (launch && launch->batch_spp) runs[0].slice_spp = launch->batch_spp;
-    st = vp_reset_counters(ctx, s);
-    if (st != VP_OK) return st;
-    double kms = 0.0;
-    uint64_t paths = 0;
-    st = vp_run_jobs(ctx, runs, launch, cap, 0, params->measure_caps ? 1 : 0, s, &kms, &paths);
-    if (st != VP_OK) return st;
-    st = vp_read_stats(ctx, s, stats);
-    if (st != VP_OK) return st;
-    if (stats) {
-        stats->kernel_ms = kms;
-        stats->launches = ctx->last_launches;
-        stats->paths = runs[0].traced;
-        stats->wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-    }
-    return VP_OK;
+    return render_one(ctx, sc, env, cam, params, launch, out_rgba_dev, nullptr, out_samples_dev,
+                      stream ? static_cast<hipStream_t>(stream) : ctx->stream, stats);
 }
 
 vp_status vp_render_count_events(vp_context* ctx, vp_scene* sc, vp_env* env, const vp_camera* cam,
@@ -467,21 +488,12 @@ vp_status vp_render_count_events(vp_context* ctx, vp_scene* sc, vp_env* env, con
     vp_status st = vp_check_params(params);
     if (st != VP_OK) return st;
     VP_HIP_TRY(hipSetDevice(ctx->device));
-    hipStream_t s = ctx->stream;
-    const size_t bytes = static_cast<size_t>(params->width) * params->height * sizeof(float4);
-    Dev mean;
-    if (hipMalloc(&mean.p, bytes) != hipSuccess) return fail(VP_ERR_OOM, "cannot allocate the image");
     std::vector<JobRun> runs(1);
     runs[0].desc = vp_make_job(sc, env, cam, params);
-    runs[0].mean = static_cast<float4*>(mean.p);
-    st = vp_reset_counters(ctx, s);
-    if (st != VP_OK) return st;
-    st = vp_run_jobs(ctx, runs, nullptr, params->active_cap ? params->active_cap : 128u, 1,
-                  params->measure_caps ? 1 : 0, s, nullptr, nullptr);
-    if (st != VP_OK) return st;
     unsigned long long c[vp::kNumCounters];
-    VP_HIP_TRY(hipMemcpyAsync(c, ctx->counters, sizeof(c), hipMemcpyDeviceToHost, s));
-    VP_HIP_TRY(hipStreamSynchronize(s));
+    st = vp_run_jobs(ctx, runs, nullptr, params->active_cap ? params->active_cap : 128u, 1,
+                     params->measure_caps ? 1 : 0, ctx->stream, nullptr, nullptr, c);
+    if (st != VP_OK) return st;
     for (uint32_t i = 0; i < n_events && i < static_cast<uint32_t>(vp::kNumCounters); ++i) events[i] = c[i];
     return VP_OK;
 }
@@ -489,20 +501,10 @@ vp_status vp_render_count_events(vp_context* ctx, vp_scene* sc, vp_env* env, con
 vp_status vp_render(vp_context* ctx, vp_scene* sc, vp_env* env, const vp_camera* cam, const vp_render_params* params,
                     float* out_rgba, vp_render_stats* stats) {
     if (!ctx || !out_rgba) return fail(VP_ERR_INVALID, "null argument");
-    vp_status st = vp_check_params(params);
+    const vp_status st = vp_check_params(params);
     if (st != VP_OK) return st;
-    const auto t0 = std::chrono::steady_clock::now();
-    VP_HIP_TRY(hipSetDevice(ctx->device));
-    const size_t bytes = static_cast<size_t>(params->width) * params->height * sizeof(float4);
-    Dev mean;
-    if (hipMalloc(&mean.p, bytes) != hipSuccess) return fail(VP_ERR_OOM, "cannot allocate the image");
-    st = vp_render_device(ctx, sc, env, cam, params, nullptr, static_cast<float*>(mean.p), nullptr, nullptr, stats);
-    if (st != VP_OK) return st;
-    VP_HIP_TRY(hipMemcpyAsync(out_rgba, mean.p, bytes, hipMemcpyDeviceToHost, ctx->stream));
-    VP_HIP_TRY(hipStreamSynchronize(ctx->stream));
-    if (stats)
-        stats->wall_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();
-    return VP_OK;
+    if (!sc || !env || !cam) return fail(VP_ERR_INVALID, "null argument");
+    return render_one(ctx, sc, env, cam, params, nullptr, nullptr, out_rgba, nullptr, ctx->stream, stats);
 }
 
 vp_status vp_normalize_accumulator(float* out_rgba_dev, const float* mean_rgba_dev, size_t n, float scale,
@@ -521,9 +523,7 @@ vp_status vp_render_jobs(vp_context* ctx, vp_job* jobs, uint32_t njobs, const vp
     VP_HIP_TRY(hipSetDevice(ctx->device));
     uint32_t cap = 0;
     int measure = 0;
-    uint64_t samples = 0;
     std::vector<JobRun> runs(njobs);
-    std::vector<Dev> means(njobs);
     for (uint32_t i = 0; i < njobs; ++i) {
         const vp_job& j = jobs[i];
         if (!j.scene || !j.env || !j.out_rgba) return fail(VP_ERR_INVALID, "job " + std::to_string(i) + ": null field");
@@ -532,29 +532,20 @@ vp_status vp_render_jobs(vp_context* ctx, vp_job* jobs, uint32_t njobs, const vp
         cap = std::max(cap, j.params.active_cap ? j.params.active_cap : 128u);
         measure |= j.params.measure_caps ? 1 : 0;
         runs[i].desc = vp_make_job(j.scene, j.env, &j.camera, &j.params);
-        const size_t bytes = static_cast<size_t>(j.params.width) * j.params.height * sizeof(float4);
-        if (hipMalloc(&means[i].p, bytes) != hipSuccess) return fail(VP_ERR_OOM, "cannot allocate job images");
-        runs[i].mean = static_cast<float4*>(means[i].p);
+        runs[i].host_out = j.out_rgba;
         if (launch && launch->batch_spp) runs[i].slice_spp = launch->batch_spp;
-        samples += static_cast<uint64_t>(j.params.width) * j.params.height * j.params.spp;
     }
     // one capacity serves the whole launch: the largest any job or the
     // launch configuration asks for
     if (launch && launch->active_cap) cap = std::max(cap, launch->active_cap);
     if (cap > vp::kMaxActiveCap) return fail(VP_ERR_INVALID, "active_cap must be at most 65535");
-    vp_status st = vp_reset_counters(ctx, ctx->stream);
-    if (st != VP_OK) return st;
     double kms = 0.0;
-    st = vp_run_jobs(ctx, runs, launch, cap, 0, measure, ctx->stream, &kms, nullptr);
+    unsigned long long c[vp::kNumCounters];
+    const vp_status st = vp_run_jobs(ctx, runs, launch, cap, 0, measure, ctx->stream, &kms, nullptr, c);
     if (st != VP_OK) return st;
-    samples = 0;
-    for (uint32_t i = 0; i < njobs; ++i) {
-        const size_t bytes = static_cast<size_t>(jobs[i].params.width) * jobs[i].params.height * sizeof(float4);
-        VP_HIP_TRY(hipMemcpyAsync(jobs[i].out_rgba, means[i].p, bytes, hipMemcpyDeviceToHost, ctx->stream));
-        samples += runs[i].traced;
-    }
-    st = vp_read_stats(ctx, ctx->stream, stats);
-    if (st != VP_OK) return st;
+    uint64_t samples = 0;
+    for (const JobRun& r : runs) samples += r.traced;
+    vp_fill_stats(c, stats);
     if (stats) {
         stats->kernel_ms = kms;
         stats->launches = ctx->last_launches;

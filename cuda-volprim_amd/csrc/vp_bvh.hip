@@ -433,8 +433,9 @@ struct BuildTemps {
 
 // Builds scene sc (whose n is set): records, Morton codes and stored order,
 // the order from the radix sort or, with VP_SCENE_BVH_SAH / _MEDIAN in flags,
-// from the host tree, and the walk tree over it.  The temporaries are one
-// allocation and the scene owns two.
+// from the host tree, and the walk tree over it.  Temporaries are scratch;
+// the scene owns two allocations.  Returns VP_ERR_INVALID without a message
+// where a primitive is not valid.
 vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32_t n, uint32_t flags, vp_scene* sc) {
     using namespace vp;
     hipStream_t s = ctx->stream;
@@ -444,14 +445,11 @@ vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32
     const size_t records = w4_records(levels);
     Arena need;
     BuildTemps(need, n, nb_sort, nbounds, records);
+    ScratchLease scratch;
+    vp_status st = vp_lease_scratch(ctx, need.used, s, scratch);
+    if (st != VP_OK) return st;
     Arena arena;
-    struct Free {
-        char*& p;
-        ~Free() {
-            if (p) (void)hipFree(p);
-        }
-    } free_temps{arena.base};
-    VP_HIP_TRY(hipMalloc(reinterpret_cast<void**>(&arena.base), need.used));
+    arena.base = static_cast<char*>(scratch.p);
     const BuildTemps T(arena, n, nb_sort, nbounds, records);
     // the records are padded to a multiple of the leaf block with zero records
     // (zero inverse scales: no ray enters them), so a walk may hand every slot
@@ -466,7 +464,9 @@ vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32
         if (pass == 0) VP_HIP_TRY(hipMalloc(&sc->mem, a.used));
     }
     if (n_slots > n) VP_HIP_TRY(hipMemsetAsync(sc->prims + n, 0, sizeof(PrimRecord) * (n_slots - n), s));
-    VP_HIP_TRY(hipMemcpyAsync(T.in, host_prims, sizeof(vp_primitive) * n, hipMemcpyHostToDevice, s));
+    bool valid = false;
+    st = vp_copy_in(ctx, T.in, host_prims, sizeof(vp_primitive), n, vp_primitives_valid, &valid, s);
+    if (st != VP_OK || !valid) return st != VP_OK ? st : VP_ERR_INVALID;
     VP_HIP_TRY(hipMemsetAsync(T.depth, 0, sizeof(uint32_t), s));
     VP_HIP_TRY(hipMemsetAsync(T.sums, 0, 2 * sizeof(double), s));
 
@@ -501,7 +501,6 @@ vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32
             hipLaunchKernelGGL(k_depth, dim3(g), dim3(256), 0, s, (int)n, T.parent, T.depth);
         }
         VP_HIP_TRY(hipGetLastError());
-        VP_HIP_TRY(hipMemcpyAsync(&depth, T.depth, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
     }
     hipLaunchKernelGGL(k_gather, dim3(g), dim3(256), 0, s, sc->order, n, T.rec, T.box, sc->prims, T.sorted_box);
 
@@ -518,10 +517,11 @@ vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32
     if (!(flags & VP_SCENE_WALK_F32)) {
         hipLaunchKernelGGL(k_w4_half, dim3(cdiv(static_cast<uint32_t>(records), 256u)), dim3(256), 0, s, T.w4,
                            static_cast<uint32_t>(records), w4_level_base(levels - 1u), T.w4_half, T.sums);
-        VP_HIP_TRY(hipMemcpyAsync(sums, T.sums, sizeof(sums), hipMemcpyDeviceToHost, s));
     }
     VP_HIP_TRY(hipGetLastError());
-    VP_HIP_TRY(hipStreamSynchronize(s));
+    const HostCopy outs[2] = {{&depth, T.depth, sizeof(depth)}, {sums, T.sums, sizeof(sums)}};
+    st = vp_copy_out(ctx, outs, 2, s);
+    if (st != VP_OK) return st;
     if (!host_tree) sc->depth = depth;
     sc->w4_growth = sums[0] > 0.0 ? sums[1] / sums[0] - 1.0 : 0.0;
     const bool half = !(flags & VP_SCENE_WALK_F32) && ((flags & VP_SCENE_WALK_F16) || sc->w4_growth <= 1.0 / 16.0);
@@ -531,5 +531,6 @@ vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32
                               hipMemcpyDeviceToDevice, s));
     sc->w4_half = half ? 1u : 0u;
     VP_HIP_TRY(hipStreamSynchronize(s));
+    scratch.done = true;
     return VP_OK;
 }

@@ -1,9 +1,9 @@
 // vp_exec.cpp — execution of job lists on the persistent renderer.
 //
 // A step renders one slice of samples of every job in a table: the table,
-// the slice start offsets and a two-word launch descriptor are staged in
-// pinned host memory, copied to the device, and a fixed sequence (counter
-// reset, k_render, k_resolve_all) runs over them.  Finished paths add into
+// the slice start offsets and a launch descriptor are written to pinned host
+// memory, and a fixed sequence (k_begin, k_render, k_resolve_all) runs over
+// them.  Finished paths add into
 // per-pixel accumulators that live across the slices of a job, so slicing
 // (the reference's 16-spp batches) does not change the result.
 #include <algorithm>
@@ -31,9 +31,6 @@ vp_status vp_ensure_slab(vp_context* ctx, size_t words) {
 }
 
 void vp_drop_graph(vp_context* ctx) {
-    if (ctx->graph_exec) (void)hipGraphExecDestroy(ctx->graph_exec);
-    ctx->graph_exec = nullptr;
-    for (auto& k : ctx->graph_key) k = 0;
     if (ctx->wf_graph) (void)hipGraphExecDestroy(ctx->wf_graph);
     ctx->wf_graph = nullptr;
     for (auto& k : ctx->wf_graph_key) k = 0;
@@ -238,15 +235,11 @@ vp_status vp_wf_prepare(vp_context* ctx, const RenderLaunch& L, hipStream_t s) {
 // two-iteration graph until every path of the step has retired (checked one
 // replay behind, so the device never waits on the host), resolve the means.
 static vp_status vp_run_step_wf(vp_context* ctx, const RenderLaunch& L, uint64_t total_paths, uint32_t max_jobs,
-                                uint32_t max_npix, hipStream_t s) {
+                                uint32_t max_npix, bool first, unsigned long long* accum, size_t accum_words,
+                                hipStream_t s) {
     vp_status st = vp_wf_prepare(ctx, L, s);
     if (st != VP_OK) return st;
-    VP_HIP_TRY(hipMemcpyAsync(ctx->jobs_dev, ctx->jobs_pinned, sizeof(vp::JobDesc) * max_jobs, hipMemcpyHostToDevice,
-                              s));
-    VP_HIP_TRY(hipMemcpyAsync(ctx->job_begin_dev, ctx->begin_pinned, sizeof(uint64_t) * max_jobs,
-                              hipMemcpyHostToDevice, s));
-    VP_HIP_TRY(hipMemcpyAsync(ctx->launch_desc, ctx->desc_pinned, sizeof(uint64_t) * 3, hipMemcpyHostToDevice, s));
-    VP_HIP_TRY(vp_launch_fill_u64(ctx->path_counter, vp::kClaimWords, 0ull, s));
+    VP_HIP_TRY(vp_launch_begin(ctx, max_jobs, first, accum, accum_words, s));
     VP_HIP_TRY(vp_launch_fill_u64(ctx->job_done_dev, max_jobs, 0ull, s));
     VP_HIP_TRY(vp_wf_launch_init(ctx->wf, s));
     // Every replay advances each live path by two bounces or retires it, and
@@ -269,53 +262,21 @@ static vp_status vp_run_step_wf(vp_context* ctx, const RenderLaunch& L, uint64_t
 }
 
 vp_status vp_run_step(vp_context* ctx, const RenderLaunch& L, uint32_t nslices, uint64_t total_paths,
-                      uint32_t max_jobs, uint32_t max_npix, bool use_graph, hipStream_t s) {
+                      uint32_t max_jobs, uint32_t max_npix, bool first, unsigned long long* accum, size_t accum_words,
+                      hipStream_t s) {
     ctx->desc_pinned[0] = nslices;
     ctx->desc_pinned[1] = total_paths;
     ctx->desc_pinned[2] = 0;  // the launch's paths start at 0
-    if (L.pipeline == VP_PIPELINE_WAVEFRONT) return vp_run_step_wf(ctx, L, total_paths, max_jobs, max_npix, s);
-    auto enqueue = [&]() -> hipError_t {
-        hipError_t e = hipMemcpyAsync(ctx->jobs_dev, ctx->jobs_pinned, sizeof(vp::JobDesc) * max_jobs,
-                                      hipMemcpyHostToDevice, s);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(ctx->job_begin_dev, ctx->begin_pinned, sizeof(uint64_t) * max_jobs,
-                               hipMemcpyHostToDevice, s);
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(ctx->launch_desc, ctx->desc_pinned, sizeof(uint64_t) * 3, hipMemcpyHostToDevice, s);
-        if (e == hipSuccess) e = vp_launch_step(ctx, L, max_jobs, max_npix, s);
-        return e;
-    };
-    if (!use_graph) {
-        VP_HIP_TRY(enqueue());
-        return VP_OK;
-    }
-    const uint64_t key[6] = {L.block, L.grid, (uint64_t(L.active_cap) << 32) | (L.first_paths << 16) | (L.claim_step << 8) | L.regen_min,
-                             uint64_t(L.count_events) << 1 | uint64_t(L.measure), (uint64_t(max_jobs) << 32) | max_npix,
-                             reinterpret_cast<uint64_t>(s)};
-    if (!ctx->graph_exec || !std::equal(key, key + 6, ctx->graph_key)) {
-        vp_drop_graph(ctx);
-        VP_HIP_TRY(hipStreamBeginCapture(s, hipStreamCaptureModeThreadLocal));
-        const hipError_t e = enqueue();
-        hipGraph_t g = nullptr;
-        const hipError_t e2 = hipStreamEndCapture(s, &g);
-        if (e != hipSuccess || e2 != hipSuccess) {
-            if (g) (void)hipGraphDestroy(g);
-            return fail(VP_ERR_HIP, std::string("graph capture failed: ") + hipGetErrorString(e != hipSuccess ? e : e2));
-        }
-        const hipError_t e3 = hipGraphInstantiate(&ctx->graph_exec, g, nullptr, nullptr, 0);
-        (void)hipGraphDestroy(g);
-        if (e3 != hipSuccess) {
-            ctx->graph_exec = nullptr;
-            return fail(VP_ERR_HIP, std::string("graph instantiation failed: ") + hipGetErrorString(e3));
-        }
-        std::copy(key, key + 6, ctx->graph_key);
-    }
-    VP_HIP_TRY(hipGraphLaunch(ctx->graph_exec, s));
+    if (L.pipeline == VP_PIPELINE_WAVEFRONT)
+        return vp_run_step_wf(ctx, L, total_paths, max_jobs, max_npix, first, accum, accum_words, s);
+    VP_HIP_TRY(vp_launch_begin(ctx, max_jobs, first, accum, accum_words, s));
+    VP_HIP_TRY(vp_launch_step(ctx, L, max_jobs, max_npix, s));
     return VP_OK;
 }
 
 vp_status vp_run_jobs(vp_context* ctx, std::vector<JobRun>& runs, const vp_launch_config* cfg, uint32_t active_cap,
-                      int count, int measure, hipStream_t s, double* kernel_ms, uint64_t* paths) {
+                      int count, int measure, hipStream_t s, double* kernel_ms, uint64_t* paths,
+                      unsigned long long* counters) {
     RenderLaunch L = vp_resolve_launch(ctx, cfg, active_cap, count, measure);
     // per-sample output (and adaptive sampling, which folds the per-sample
     // radiance of each batch) is written by the megakernel only
@@ -341,83 +302,75 @@ vp_status vp_run_jobs(vp_context* ctx, std::vector<JobRun>& runs, const vp_launc
     st = vp_ensure_jobs(ctx, static_cast<uint32_t>(runs.size()));
     if (st != VP_OK) return st;
 
-    // per-pixel accumulators of every job, zeroed once: the slices of a job
-    // add into the same sums
+    // scratch, each part 256-byte aligned: the per-pixel accumulators of every
+    // job, zeroed once (the slices of a job add into the same sums); the
+    // images that no caller holds; and of every adaptive job, per pixel the
+    // Welford M2 (float4), the sample count / converged flag and the
+    // per-sample radiance of one batch (the reference's batch of 16 unless the
+    // launch sets batch_spp); its Welford mean lives in the output image
     size_t acc_words = 0;
     uint32_t max_npix = 1;
     for (auto& r : runs) {
         const size_t npix = static_cast<size_t>(r.desc.width) * r.desc.height;
         acc_words += npix * vp::kAccumWords;
         max_npix = std::max(max_npix, static_cast<uint32_t>(npix));
+        if (r.desc.adapt_threshold > 0.0f && r.slice_spp == 0) r.slice_spp = kAdaptiveBatch;
     }
-    void* acc_buf = nullptr;
-    if (hipMalloc(&acc_buf, acc_words * sizeof(unsigned long long)) != hipSuccess)
-        return fail(VP_ERR_OOM, "cannot allocate " + std::to_string(acc_words * 8) + " bytes of pixel accumulators");
-    struct Free {
-        void* p;
-        ~Free() {
-            if (p) (void)hipFree(p);
-        }
-    } free_acc{acc_buf};
-    // adaptive sampling state of every adaptive job, in one allocation: per
-    // pixel the Welford M2 (float4) and the sample count / converged flag,
-    // and the per-sample radiance of one batch (the reference's batch of 16
-    // unless the launch sets batch_spp); the Welford mean lives in the
-    // job's output image
-    size_t adapt_bytes = 0;
-    for (auto& r : runs) {
-        if (!(r.desc.adapt_threshold > 0.0f)) continue;
-        if (r.slice_spp == 0) r.slice_spp = kAdaptiveBatch;
-        const size_t npix = static_cast<size_t>(r.desc.width) * r.desc.height;
-        adapt_bytes += npix * (sizeof(float4) * (1 + std::min(r.slice_spp, r.desc.spp)) + sizeof(uint32_t));
-        adapt_bytes = (adapt_bytes + 255) & ~size_t(255);
-    }
-    void* adapt_buf = nullptr;
-    if (adapt_bytes && hipMalloc(&adapt_buf, adapt_bytes) != hipSuccess)
-        return fail(VP_ERR_OOM, "cannot allocate " + std::to_string(adapt_bytes) + " bytes of adaptive-sampling state");
-    Free free_adapt{adapt_buf};
-    {
-        size_t off = 0, aoff = 0;
+    ScratchLease scratch;
+    for (int pass = 0; pass < 2; ++pass) {
+        size_t off = 0, acc = 0;
+        auto take = [&](size_t bytes) {
+            char* p = static_cast<char*>(scratch.p) + off;
+            off += (bytes + 255) & ~size_t(255);
+            return p;
+        };
+        unsigned long long* sums = reinterpret_cast<unsigned long long*>(take(acc_words * sizeof(unsigned long long)));
         for (auto& r : runs) {
             const size_t npix = static_cast<size_t>(r.desc.width) * r.desc.height;
-            r.desc.accum = static_cast<unsigned long long*>(acc_buf) + off;
-            r.desc.mean = r.mean;
+            float4* image = r.mean ? r.mean : reinterpret_cast<float4*>(take(npix * sizeof(float4)));
+            const bool adaptive = r.desc.adapt_threshold > 0.0f;
+            float4* m2 = adaptive ? reinterpret_cast<float4*>(take(npix * sizeof(float4))) : nullptr;
+            float4* batch = adaptive ? reinterpret_cast<float4*>(
+                                           take(npix * sizeof(float4) * std::min(r.slice_spp, r.desc.spp)))
+                                     : nullptr;
+            uint32_t* state = adaptive ? reinterpret_cast<uint32_t*>(take(npix * sizeof(uint32_t))) : nullptr;
+            if (pass == 0) continue;
+            r.desc.accum = sums + acc;
+            acc += npix * vp::kAccumWords;
+            r.desc.mean = image;
             r.desc.samples = nullptr;
             r.desc.done = nullptr;
-            r.desc.adapt_m2 = nullptr;
-            r.desc.adapt_state = nullptr;
-            r.batch = nullptr;
+            r.desc.adapt_m2 = m2;
+            r.desc.adapt_state = state;
+            r.batch = batch;
             r.issued = 0;
-            off += npix * vp::kAccumWords;
-            if (r.desc.adapt_threshold > 0.0f) {
-                char* b = static_cast<char*>(adapt_buf) + aoff;
-                r.desc.adapt_m2 = reinterpret_cast<float4*>(b);
-                r.batch = r.desc.adapt_m2 + npix;
-                r.desc.adapt_state =
-                    reinterpret_cast<uint32_t*>(r.batch + npix * std::min(r.slice_spp, r.desc.spp));
-                aoff += npix * (sizeof(float4) * (1 + std::min(r.slice_spp, r.desc.spp)) + sizeof(uint32_t));
-                aoff = (aoff + 255) & ~size_t(255);
-                // Welford state from zero (raygen.cuh:30-36 reads zeroed buffers)
-                VP_HIP_TRY(vp_launch_fill_u64(reinterpret_cast<unsigned long long*>(r.desc.adapt_m2),
-                                              static_cast<uint32_t>(2 * npix), 0ull, s));
-                VP_HIP_TRY(vp_launch_fill_u64(reinterpret_cast<unsigned long long*>(r.mean),
-                                              static_cast<uint32_t>(2 * npix), 0ull, s));
-                VP_HIP_TRY(vp_launch_fill_u32(r.desc.adapt_state, static_cast<uint32_t>(npix), 0u, s));
-            }
         }
-        // fill kernels (not hipMemsetAsync): the launch sequences below may
-        // be captured into graphs by callers
-        for (size_t o = 0; o < acc_words; o += (size_t(1) << 30)) {
-            const uint32_t n = static_cast<uint32_t>(std::min<size_t>(acc_words - o, size_t(1) << 30));
-            VP_HIP_TRY(vp_launch_fill_u64(static_cast<unsigned long long*>(acc_buf) + o, n, 0ull, s));
-        }
+        if (pass == 0) st = vp_lease_scratch(ctx, off, s, scratch);
+        if (st != VP_OK) return st;
+    }
+    for (auto& r : runs) {
+        if (r.desc.adapt_state == nullptr) continue;
+        // Welford state from zero (raygen.cuh:30-36 reads zeroed buffers)
+        const uint32_t npix = r.desc.width * r.desc.height;
+        VP_HIP_TRY(vp_launch_fill_u64(reinterpret_cast<unsigned long long*>(r.desc.adapt_m2), 2 * npix, 0ull, s));
+        VP_HIP_TRY(vp_launch_fill_u64(reinterpret_cast<unsigned long long*>(r.desc.mean), 2 * npix, 0ull, s));
+        VP_HIP_TRY(vp_launch_fill_u32(r.desc.adapt_state, npix, 0u, s));
     }
 
     uint64_t total_paths_all = 0;
     double render_ms = 0.0;
     uint32_t launches = 0;
     const uint32_t max_jobs = static_cast<uint32_t>(runs.size());
-    while (true) {
+    // a step's kernels, waited for before the pinned tables are written again
+    auto wait_step = [&]() -> vp_status {
+        VP_HIP_TRY(hipEventSynchronize(ctx->ev1));
+        float ms = 0.0f;
+        VP_HIP_TRY(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
+        render_ms += ms;
+        return VP_OK;
+    };
+    while (std::any_of(runs.begin(), runs.end(), [](const JobRun& r) { return r.issued < r.desc.spp; })) {
+        if (launches > 0 && (st = wait_step()) != VP_OK) return st;
         uint64_t total = 0;
         uint32_t k = 0;
         for (auto& r : runs) {
@@ -437,53 +390,49 @@ vp_status vp_run_jobs(vp_context* ctx, std::vector<JobRun>& runs, const vp_launc
             r.issued += J.s_count;
             ++k;
         }
-        if (k == 0) break;
         VP_HIP_TRY(hipEventRecord(ctx->ev0, s));
-        st = vp_run_step(ctx, vp_size_launch(L, total), k, total, max_jobs, max_npix, false, s);
+        st = vp_run_step(ctx, vp_size_launch(L, total), k, total, max_jobs, max_npix, launches == 0,
+                         runs[0].desc.accum, acc_words, s);
         if (st != VP_OK) return st;
         VP_HIP_TRY(hipEventRecord(ctx->ev1, s));
-        // the pinned staging is rewritten next round (and the accumulators
-        // are freed on return): wait for this step
-        VP_HIP_TRY(hipEventSynchronize(ctx->ev1));
-        float ms = 0.0f;
-        VP_HIP_TRY(hipEventElapsedTime(&ms, ctx->ev0, ctx->ev1));
-        render_ms += ms;
         total_paths_all += total;
         ++launches;
     }
+    std::vector<HostCopy> outs;
+    if (counters) outs.push_back({counters, ctx->counters, sizeof(unsigned long long) * vp::kNumCounters});
+    std::vector<std::vector<uint32_t>> states(runs.size());
+    for (size_t i = 0; i < runs.size(); ++i) {
+        const JobRun& r = runs[i];
+        const size_t npix = static_cast<size_t>(r.desc.width) * r.desc.height;
+        if (r.host_out) outs.push_back({r.host_out, r.desc.mean, npix * sizeof(float4)});
+        if (r.desc.adapt_state == nullptr) continue;
+        states[i].resize(npix);
+        outs.push_back({states[i].data(), r.desc.adapt_state, npix * sizeof(uint32_t)});
+    }
+    if (!outs.empty()) st = vp_copy_out(ctx, outs.data(), outs.size(), s);
+    if (st == VP_OK) st = wait_step();
+    if (st != VP_OK) return st;
+    scratch.done = true;
     if (kernel_ms) *kernel_ms = render_ms;
     ctx->last_launches = launches;
     if (paths) *paths = total_paths_all;
     // samples traced per job: every sample, or under adaptive sampling the
     // per-pixel counts
-    for (auto& r : runs) {
-        const size_t npix = static_cast<size_t>(r.desc.width) * r.desc.height;
-        r.traced = static_cast<uint64_t>(npix) * r.desc.spp;
+    for (size_t i = 0; i < runs.size(); ++i) {
+        JobRun& r = runs[i];
+        r.traced = static_cast<uint64_t>(r.desc.width) * r.desc.height * r.desc.spp;
         if (r.desc.adapt_state == nullptr) continue;
-        std::vector<uint32_t> state(npix);
-        VP_HIP_TRY(hipMemcpyAsync(state.data(), r.desc.adapt_state, npix * sizeof(uint32_t), hipMemcpyDeviceToHost, s));
-        VP_HIP_TRY(hipStreamSynchronize(s));
         uint64_t t = 0;
-        for (uint32_t v : state) t += v & 0x7fffffffu;
+        for (uint32_t v : states[i]) t += v & 0x7fffffffu;
         r.traced = t;
     }
     return VP_OK;
 }
 
-vp_status vp_read_stats(vp_context* ctx, hipStream_t s, vp_render_stats* stats) {
-    unsigned long long c[vp::kNumCounters];
-    VP_HIP_TRY(hipMemcpyAsync(c, ctx->counters, sizeof(c), hipMemcpyDeviceToHost, s));
-    VP_HIP_TRY(hipStreamSynchronize(s));
-    if (stats) {
-        stats->active_overflow = c[vp::kCntActiveOverflow];
-        stats->hit_overflow = 0;
-        stats->max_hits_per_ray = static_cast<uint32_t>(c[vp::kCntMaxHits]);
-        stats->max_point_overlap = static_cast<uint32_t>(c[vp::kCntMaxOverlap]);
-    }
-    return VP_OK;
-}
-
-vp_status vp_reset_counters(vp_context* ctx, hipStream_t s) {
-    VP_HIP_TRY(vp_launch_fill_u64(ctx->counters, static_cast<uint32_t>(vp::kNumCounters), 0ull, s));
-    return VP_OK;
+void vp_fill_stats(const unsigned long long* c, vp_render_stats* stats) {
+    if (!stats) return;
+    stats->active_overflow = c[vp::kCntActiveOverflow];
+    stats->hit_overflow = 0;
+    stats->max_hits_per_ray = static_cast<uint32_t>(c[vp::kCntMaxHits]);
+    stats->max_point_overlap = static_cast<uint32_t>(c[vp::kCntMaxOverlap]);
 }

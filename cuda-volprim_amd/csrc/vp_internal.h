@@ -5,6 +5,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include <atomic>
 #include <mutex>
 #include <string>
 #include <vector>
@@ -183,6 +184,12 @@ enum CounterSlot : int {
 // ---------------------------------------------------------------------------
 // Host objects behind the opaque C handles.
 // ---------------------------------------------------------------------------
+// Pinned slots of a context: eight of 1 MiB, filled and emptied by up to four
+// host threads.
+constexpr size_t kStageSlot = size_t(1) << 20;
+constexpr uint32_t kStageSlots = 8;
+constexpr uint32_t kStageThreads = 4;
+
 struct vp_context {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -202,9 +209,13 @@ struct vp_context {
     uint64_t* begin_pinned = nullptr;
     uint64_t* desc_pinned = nullptr;
     uint32_t pinned_cap = 0;
-    // captured step graph and the shape it was captured for
-    hipGraphExec_t graph_exec = nullptr;
-    uint64_t graph_key[6] = {0, 0, 0, 0, 0, 0};
+    // scratch and pinned slots kept between calls (vp_transfer.cpp)
+    void* scratch = nullptr;
+    size_t scratch_bytes = 0;
+    std::atomic<bool> scratch_busy{false};
+    char* stage = nullptr;
+    uint32_t stage_slots = 0;
+    hipEvent_t stage_ev[kStageSlots] = {};
     hipEvent_t ev0 = nullptr, ev1 = nullptr;
     // wavefront pipeline: path pool, its allocation, the captured
     // two-iteration graph and the pinned completion counters
@@ -214,7 +225,7 @@ struct vp_context {
     uint64_t wf_graph_key[6] = {0, 0, 0, 0, 0, 0};
     unsigned long long* wf_done_pinned = nullptr;  // [2]
     hipEvent_t wf_ev[2] = {nullptr, nullptr};
-    std::mutex mu;
+    std::mutex mu;  // of the pinned slots
     uint32_t last_launches = 0;
     vp_launch_config tuned{};
     bool have_tuned = false;
@@ -273,7 +284,52 @@ vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32
 void vp_host_tree_order(const vp_primitive* in, uint32_t n, bool median, std::vector<uint32_t>& order,
                         uint32_t& depth);
 
+// Device scratch for the duration of one call.  Up to kScratchKeep bytes are
+// kept in the context between calls and freed with it; larger ones, and those
+// of a call that finds the kept block in use, are allocated for the call.  A
+// holder that has waited for its work on the stream sets done, otherwise the
+// release waits.
+constexpr size_t kScratchKeep = size_t(256) << 20;
+struct ScratchLease {
+    vp_context* ctx = nullptr;
+    hipStream_t stream = nullptr;
+    void* p = nullptr;
+    bool owned = false;
+    bool done = false;
+    ScratchLease() = default;
+    ScratchLease(const ScratchLease&) = delete;
+    ScratchLease& operator=(const ScratchLease&) = delete;
+    ~ScratchLease();
+};
+vp_status vp_lease_scratch(vp_context* ctx, size_t bytes, hipStream_t s, ScratchLease& lease);
+
+// Copies device memory (whole 4-byte words) to the host and waits for them
+// and for all earlier work of s.
+struct HostCopy {
+    void* dst;
+    const void* src;
+    size_t bytes;
+};
+vp_status vp_copy_out(vp_context* ctx, const HostCopy* copies, size_t n, hipStream_t s);
+// Copies count elements to the device and runs check over them on the way;
+// good says whether it held for all of them.
+vp_status vp_copy_in(vp_context* ctx, void* dst, const void* src, size_t elem, size_t count,
+                     bool (*check)(const void* rows, size_t count), bool* good, hipStream_t s);
+
 // launchers (vp_render.hip)
+// Up to kCopyParts runs of words, copied by one launch.
+constexpr uint32_t kCopyParts = 4;
+struct CopyParts {
+    const uint32_t* src[kCopyParts];
+    uint32_t* dst[kCopyParts];
+    uint32_t words[kCopyParts];
+};
+hipError_t vp_launch_copy_parts(const CopyParts& c, hipStream_t s);
+// Job table, slice begins and launch descriptor from ctx's pinned staging to
+// the device, the path counters to zero, and with first the event counters and
+// accum_words of accumulators.
+hipError_t vp_launch_begin(vp_context* ctx, uint32_t max_jobs, bool first, unsigned long long* accum,
+                           size_t accum_words, hipStream_t s);
 struct RenderLaunch {
     uint32_t block;
     uint32_t grid;
@@ -298,7 +354,8 @@ hipError_t vp_launch_render(const RenderLaunch& L, const vp::JobDesc* jobs, cons
 // execution of job lists (vp_exec.cpp)
 struct JobRun {
     vp::JobDesc desc;
-    float4* mean = nullptr;         // device W*H mean (output)
+    float4* mean = nullptr;         // device W*H mean (output); null: in scratch
+    void* host_out = nullptr;       // W*H mean for the host
     float4* samples_all = nullptr;  // optional caller buffer spp*W*H of per-sample radiance
     uint32_t issued = 0;            // samples launched so far
     uint32_t slice_spp = 0;         // samples per launch (0 = all at once)
@@ -317,13 +374,18 @@ RenderLaunch vp_resolve_launch(vp_context* ctx, const vp_launch_config* cfg, uin
 RenderLaunch vp_size_launch(RenderLaunch L, uint64_t paths);
 // One step over the first nslices entries of the pinned job table (capacity max_jobs).
 vp_status vp_run_step(vp_context* ctx, const RenderLaunch& L, uint32_t nslices, uint64_t total_paths,
-                      uint32_t max_jobs, uint32_t max_npix, bool use_graph, hipStream_t s);
+                      uint32_t max_jobs, uint32_t max_npix, bool first, unsigned long long* accum, size_t accum_words,
+                      hipStream_t s);
+// Runs the jobs to completion and waits; counters (kNumCounters words, may be
+// null) receives the event counters.
 vp_status vp_run_jobs(vp_context* ctx, std::vector<JobRun>& runs, const vp_launch_config* cfg, uint32_t active_cap,
-                      int count, int measure, hipStream_t s, double* kernel_ms, uint64_t* paths);
-vp_status vp_read_stats(vp_context* ctx, hipStream_t s, vp_render_stats* stats);
-vp_status vp_reset_counters(vp_context* ctx, hipStream_t s);
+                      int count, int measure, hipStream_t s, double* kernel_ms, uint64_t* paths,
+                      unsigned long long* counters);
+void vp_fill_stats(const unsigned long long* counters, vp_render_stats* stats);
 vp::JobDesc vp_make_job(const vp_scene* sc, const vp_env* env, const vp_camera* cam, const vp_render_params* p);
 vp_status vp_check_params(const vp_render_params* p);
+// Whether all count primitives pass the validation of vp_scene_create.
+bool vp_primitives_valid(const void* rows, size_t count);
 // Resolves ctx->noalloc_scratch on ctx's device (which must be current).
 vp_status vp_noalloc_attach(vp_context* ctx);
 hipError_t vp_launch_fill_u64(unsigned long long* p, uint32_t n, unsigned long long v, hipStream_t s);

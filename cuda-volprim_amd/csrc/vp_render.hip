@@ -1141,6 +1141,31 @@ __global__ void k_fill_u32(uint32_t* p, uint32_t n, uint32_t v) {
     if (i < n) p[i] = v;
 }
 
+// Start of a step.  The tables are read straight from pinned memory: one
+// launch instead of three copies and three fills, which with the image's
+// copies and the allocations took 100 of the 160 us of the smallest renders.
+__global__ void __launch_bounds__(256) k_begin(const uint32_t* __restrict__ jobs_from, uint32_t* __restrict__ jobs, uint32_t job_words,
+                        const uint64_t* __restrict__ begin_from, uint64_t* __restrict__ job_begin, uint32_t njobs,
+                        const uint64_t* __restrict__ desc_from, uint64_t* __restrict__ desc,
+                        unsigned long long* __restrict__ path_counter, unsigned long long* __restrict__ counters,
+                        uint32_t n_counters, uint4* __restrict__ accum, size_t accum_n) {
+    const size_t t = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x;
+    const size_t stride = static_cast<size_t>(gridDim.x) * blockDim.x;
+    for (size_t i = t; i < job_words; i += stride) jobs[i] = jobs_from[i];
+    for (size_t i = t; i < njobs; i += stride) job_begin[i] = begin_from[i];
+    if (t < 3) desc[t] = desc_from[t];
+    for (size_t i = t; i < kClaimWords; i += stride) path_counter[i] = 0ull;
+    if (t < n_counters) counters[t] = 0ull;
+    for (size_t i = t; i < accum_n; i += stride) accum[i] = make_uint4(0u, 0u, 0u, 0u);
+}
+
+__global__ void __launch_bounds__(256) k_copy_parts(CopyParts c) {
+    const uint32_t t = blockIdx.x * blockDim.x + threadIdx.x, stride = gridDim.x * blockDim.x;
+#pragma unroll
+    for (uint32_t k = 0; k < kCopyParts; ++k)
+        for (uint32_t i = t; i < c.words[k]; i += stride) c.dst[k][i] = c.src[k][i];
+}
+
 // normalize_accumulator_kernel (device/kernels/normalize_accumulator.cu:16-35)
 __global__ void k_normalize(float4* __restrict__ out, const float4* __restrict__ in, size_t n, float scale) {
     for (size_t i = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; i < n;
@@ -1309,10 +1334,10 @@ hipError_t vp_launch_render(const RenderLaunch& L, const JobDesc* jobs, const ui
 // One step of the persistent renderer over the job table in ctx->jobs_dev:
 // reset the path counter (a fill kernel, so the sequence can be captured in a
 // graph), trace every path of every job slice, resolve the means.  Job count
-// and path total come from ctx->launch_desc.
+// and path total come from ctx->launch_desc, the path counters from
+// vp_launch_begin.
 hipError_t vp_launch_step(vp_context* ctx, const RenderLaunch& L, uint32_t max_jobs, uint32_t max_npix,
                           hipStream_t s) {
-    hipLaunchKernelGGL(k_fill_u64, dim3(cdiv(kClaimWords, 64)), dim3(64), 0, s, ctx->path_counter, kClaimWords, 0ull);
     const hipError_t e = vp_launch_render(L, ctx->jobs_dev, ctx->job_begin_dev, ctx->launch_desc, ctx->path_counter,
                                           ctx->slab, ctx->counters, s);
     if (e != hipSuccess) return e;
@@ -1328,6 +1353,25 @@ hipError_t vp_launch_resolve(vp_context* ctx, uint32_t max_jobs, uint32_t max_np
 hipError_t vp_launch_resolve_job(const JobDesc* jobs, uint32_t j, uint32_t npix, hipStream_t s) {
     const uint32_t gx = std::max<uint32_t>(1u, std::min<uint32_t>(cdiv(npix, 256), 1024u));
     hipLaunchKernelGGL(k_resolve_job, dim3(gx), dim3(256), 0, s, jobs, j);
+    return hipGetLastError();
+}
+
+hipError_t vp_launch_begin(vp_context* ctx, uint32_t max_jobs, bool first, unsigned long long* accum,
+                           size_t accum_words, hipStream_t s) {
+    const uint32_t job_words = static_cast<uint32_t>(sizeof(JobDesc) / sizeof(uint32_t)) * max_jobs;
+    const size_t accum_n = first ? accum_words / 2 : 0;  // kAccumWords is even
+    const size_t most = std::max<size_t>(std::max<size_t>(job_words, kClaimWords), accum_n / 4);
+    const uint32_t grid = static_cast<uint32_t>(std::min<size_t>((most + 255) / 256, 2048u));
+    hipLaunchKernelGGL(k_begin, dim3(grid), dim3(256), 0, s, reinterpret_cast<const uint32_t*>(ctx->jobs_pinned),
+                       reinterpret_cast<uint32_t*>(ctx->jobs_dev), job_words, ctx->begin_pinned, ctx->job_begin_dev,
+                       max_jobs, ctx->desc_pinned, ctx->launch_desc, ctx->path_counter, ctx->counters,
+                       first ? static_cast<uint32_t>(kNumCounters) : 0u, reinterpret_cast<uint4*>(accum), accum_n);
+    return hipGetLastError();
+}
+hipError_t vp_launch_copy_parts(const CopyParts& c, hipStream_t s) {
+    uint32_t most = 1;
+    for (uint32_t w : c.words) most = std::max(most, w);
+    hipLaunchKernelGGL(k_copy_parts, dim3(std::min<uint32_t>(cdiv(most, 256), 256u)), dim3(256), 0, s, c);
     return hipGetLastError();
 }
 

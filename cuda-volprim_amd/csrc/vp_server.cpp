@@ -631,35 +631,20 @@ vp_status vp_autotune(vp_context* ctx, vp_job* jobs, uint32_t njobs, vp_launch_c
         }
         cams[i] = c;
     }
-    std::vector<void*> means(njobs, nullptr);
-    struct Free {
-        std::vector<void*>& v;
-        ~Free() {
-            for (void* p : v)
-                if (p) (void)hipFree(p);
-        }
-    } fr{means};
-    for (uint32_t i = 0; i < njobs; ++i)
-        if (hipMalloc(&means[i], sizeof(float4) * params[i].width * params[i].height) != hipSuccess)
-            return fail(VP_ERR_OOM, "autotune: cannot allocate images");
     auto make_runs = [&](std::vector<JobRun>& runs) {
         runs.assign(njobs, JobRun{});
-        for (uint32_t i = 0; i < njobs; ++i) {
+        for (uint32_t i = 0; i < njobs; ++i)
             runs[i].desc = vp_make_job(jobs[i].scene, jobs[i].env, &cams[i], &params[i]);
-            runs[i].mean = static_cast<float4*>(means[i]);
-        }
     };
     // active-set capacity from the measured maximum overlap
     uint32_t cap = 128;
     {
         std::vector<JobRun> runs;
         make_runs(runs);
-        vp_status st = vp_reset_counters(ctx, s);
-        if (st == VP_OK) st = vp_run_jobs(ctx, runs, nullptr, 1024, 0, 1, s, nullptr, nullptr);
-        vp_render_stats rs{};
-        if (st == VP_OK) st = vp_read_stats(ctx, s, &rs);
+        unsigned long long c[vp::kNumCounters];
+        const vp_status st = vp_run_jobs(ctx, runs, nullptr, 1024, 0, 1, s, nullptr, nullptr, c);
         if (st != VP_OK) return st;
-        const uint32_t v = rs.max_point_overlap;
+        const uint32_t v = static_cast<uint32_t>(c[vp::kCntMaxOverlap]);
         cap = std::max<uint32_t>(16u, ((v * 9 + 7) / 8 + 15) / 16 * 16);
         // the reduced mix sees fewer vertices than the full one: never go
         // below the capacities the jobs ask for
@@ -685,7 +670,7 @@ vp_status vp_autotune(vp_context* ctx, vp_job* jobs, uint32_t njobs, vp_launch_c
         make_runs(runs);
         uint64_t paths = 0;
         const auto t0 = clk::now();
-        vp_status st = vp_run_jobs(ctx, runs, &c, cap, 0, 0, s, nullptr, &paths);
+        vp_status st = vp_run_jobs(ctx, runs, &c, cap, 0, 0, s, nullptr, &paths, nullptr);
         if (st != VP_OK) return st;
         const double wall = std::chrono::duration<double, std::milli>(clk::now() - t0).count();
         const double rate = static_cast<double>(paths) / std::max(wall, 1e-3);
