@@ -188,7 +188,20 @@ RenderLaunch vp_resolve_launch(vp_context* ctx, const vp_launch_config* cfg, uin
 // wavefronts to the others.  Starting on 4 and claiming 4, 8 and 16: 192x128x2
 // cloud (12 paths per wavefront) 17, 24, 38 ms, 512x512x1 torus (64) 19.9, 20.2,
 // 21.9, 256x256x24 scattering (384) 27.0, 26.4, 26.1.
+// The wavefronts of a workgroup help each other at the end (help_walks in
+// vp_render.hip), so workgroups are as large as they can be, 16 wavefronts, once
+// there are 32 paths to a compute unit, and smaller below, where a launch's paths
+// would sit on few compute units (workgroups of 4, 8 and 16 wavefronts: 192x128x2
+// cloud 13.5, 12.6, 12.0 ms, 128x128 adaptive 18.6, 18.4, 18.0; 32x32x4 probe, 16
+// paths to a compute unit, 69, 69, 73 us).
 RenderLaunch vp_size_launch(RenderLaunch L, uint64_t paths) {
+    if (L.wide) {
+        const uint64_t total = static_cast<uint64_t>(L.grid) * L.block / 64u;
+        uint32_t w = L.block / 64u;
+        while (w < 16u && paths >= total / 16u * 4u * w) w *= 2u;
+        L.block = 64u * w;
+        L.grid = static_cast<uint32_t>(total / w);
+    }
     const uint64_t waves_per_block = L.block / 64u;
     L.grid = static_cast<uint32_t>(
         std::max<uint64_t>(1u, std::min<uint64_t>(L.grid, (paths + waves_per_block - 1) / waves_per_block)));
@@ -294,6 +307,10 @@ vp_status vp_run_jobs(vp_context* ctx, std::vector<JobRun>& runs, const vp_launc
         c.pipeline = VP_PIPELINE_MEGAKERNEL;
         L = vp_resolve_launch(ctx, &c, active_cap, count, measure);
     }
+    // larger workgroups where the caller leaves their size to the library and
+    // the launch fills the device with workgroups of 4 wavefronts
+    L.wide = L.pipeline == VP_PIPELINE_MEGAKERNEL && !count && !measure && !(cfg && cfg->block) &&
+             !(!cfg && ctx->have_tuned) && L.block == 256u && L.grid == 4u * ctx->prop.multiProcessorCount;
     const size_t lanes = static_cast<size_t>(L.grid) * L.block;
     vp_status st = VP_OK;
     if (L.pipeline == VP_PIPELINE_MEGAKERNEL)

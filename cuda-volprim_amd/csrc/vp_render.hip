@@ -47,106 +47,40 @@ struct PathState {
 #define VP_RENDER_WAVES_PER_EU 4
 #endif
 
-// Argmin free flight over the entered primitives (sampling.cuh:372-412) with
-// the wave-shared leaf queue.  All 64 lanes of the wavefront call it: a lane
-// with a path (alive) walks its own ray, and the origin-set members and queued
-// leaves of all rays are shared out among all lanes, so a wavefront with few
-// paths left still evaluates them 64 at a time.
-// Each ray's running minimum is an LDS atomic minimum over float bits (all
-// candidates are >= 0), so the result does not depend on which lane handles
-// which leaf.  Candidates for the rebuild are recorded while t_entry is at
-// most the running minimum at the time, which covers every primitive entered
-// before the final one; their order is fixed by the sort in the rebuild.  At
-// bounce 0 (direct) the walk also sums the direct term's optical depth into
-// dacc, and runs over the whole ray until that sum reaches dlimit (the
-// tau = 88 saturation or the direct term's roulette level, where T becomes
-// 0); from there on it prunes at the running minimum like any other ray.
-// ts_origin is the minimum over the origin set; the result keeps it unless a
-// walk candidate is strictly smaller.
-// Flights waiting to be inverted are taken up once there are kFlightMin of
-// them (few leaves have one, and the inversion's erf and erfinv cost as much
-// as the leaf round), or at the end of a run of leaves.  A flight ends inside
-// its chord, so until then its exit bounds the minimum (bound, which the walk
-// prunes by): without that bound, waiting for 16 flights cost the 10^6 cloud
-// 12 % and the 192x128 cloud 18 % against waiting for 4; with it, nothing.
+// How many free flights of an argmin walk wait to be inverted together (see
+// argmin_walk_shared).
 constexpr uint32_t kFlightMin = 16;
-__device__ __forceinline__ void argmin_walk_shared(bool alive, const WaveScene& ws, uint32_t job, f3 o, f3 d, uint64_t key,
-                                                   uint32_t b, bool direct, const uint32_t* act, uint32_t na_path,
-                                                   float* act_exit, float ts_set, uint32_t* __restrict__ slab,
-                                                   uint32_t cap, const MegaQueue& q, float& ts, uint32_t& nc,
-                                                   uint64_t dlimit, uint64_t& dacc,
-                                                   uint32_t& rounds) {
+
+// The path key and bounce of lane l's draws.
+__device__ __forceinline__ uint64_t draw_key(const MegaQueue& q, uint32_t l) {
+    return (static_cast<uint64_t>(q.draw(l)[1]) << 32) | q.draw(l)[0];
+}
+__device__ __forceinline__ uint32_t draw_bounce(const MegaQueue& q, uint32_t l) { return q.draw(l)[2] & 0x7fffffffu; }
+
+// The rounds of argmin walks, from nn items on, over the stack and leaf queue
+// of stack and the rays of rays (those of wavefront rays_of of the workgroup).
+// The rays' own wavefront (kOwn) keeps their ends: a ray is walked up to the
+// bound of its minimum, a direct one whole until its depth reaches the limit.
+template <bool kOwn>
+__device__ __forceinline__ void argmin_rounds(const WaveScene& ws, uint32_t* lds, const MegaQueue& stack,
+                                              const MegaQueue& rays, uint32_t rays_of, uint64_t lim,
+                                              uint32_t* __restrict__ slab, uint32_t cap, uint32_t nn,
+                                              uint32_t& rounds) {
     const uint32_t lane = __lane_id();
-    const uint32_t na = direct ? na_path : 0u;
-    lds_store3(q.ro + 3 * lane, o);
-    lds_store3(q.rd + 3 * (2 * lane), d);
-    lds_store3(q.inv + 3 * (2 * lane), safe_inv(d));
-    q.draw(lane)[0] = static_cast<uint32_t>(key);
-    q.draw(lane)[1] = static_cast<uint32_t>(key >> 32);
-    q.draw(lane)[2] = b | (direct ? 0x80000000u : 0u);
-    q.job[lane] = job;
-    q.acc[2 * lane] = 0ull;
-    q.ts(lane) = __float_as_uint(direct ? kTMax : ts_set);
-    q.nc(lane) = 0u;
-    // the path key and bounce of lane l's draws
-    auto key_of = [&](uint32_t l) {
-        return (static_cast<uint64_t>(q.draw(l)[1]) << 32) | q.draw(l)[0];
-    };
-    auto bounce_of = [&](uint32_t l) { return q.draw(l)[2] & 0x7fffffffu; };
-    // The origin set (sampling.cuh:356-370) of a path at bounce 0; from then
-    // on the last vertex's pass over the set has evaluated it (vertex_members)
-    // and ts_set is its minimum.  The wavefront's (member, lane) pairs are
-    // numbered through a prefix sum of the set sizes and shared out over the
-    // lanes.  Per member: its exit (kept in the owner's slab for the rebuild),
-    // its free flight into the owner's running minimum, and its chord into the
-    // owner's direct-term optical depth; minima and fixed-point sums do not
-    // depend on which lane adds what.  (Active sets of the megakernel are
-    // contiguous.)
-    if (__builtin_amdgcn_ballot_w64(na != 0u) != 0ull) {
-        const uint32_t** set_of = reinterpret_cast<const uint32_t**>(q.scratch);  // [64]
-        float** exit_of = reinterpret_cast<float**>(q.scratch) + 64;               // [64]
-        uint32_t* pre_of = q.scratch + 4 * 64;                                    // [64]
-        static_assert(kScratch >= 5 * 64, "the origin-set tables must fit in the queue");
-        uint32_t total;
-        pre_of[lane] = wave_prefix(na, total);
-        set_of[lane] = act;
-        exit_of[lane] = act_exit;
-        wave_sync();
-        for (uint32_t g = lane; g < total; g += 64u) {
-            const uint32_t ol = prefix_owner(pre_of, g), k = g - pre_of[ol];
-            const uint32_t i = set_of[ol][k];
-            const PrimRecord pr = load_prim(ws.jobs[q.job[ol]].scene.prims, i);
-            const f3 ro = lds_load3(q.ro + 3 * ol), rd = lds_load3(q.rd + 3 * (2 * ol));
-            const InsideChord x = inside_chord(pr, ro, rd);
-            exit_of[ol][k] = x.t1;
-            const float tau = free_flight_tau(prim_uniform(key_of(ol), bounce_of(ol), 0u, i));
-            if (tau <= x.tau) {
-                const float t = origin_flight(pr, ro, rd, x, tau);
-                atomicMin(&q.ts(ol), t == 0.0f ? 0u : __float_as_uint(t));
-            }
-            if (x.tau > 0.0f) atomicAdd(&q.acc[2 * ol], tau_fixed(x.tau));
-        }
-    }
-    wave_sync();
-    const float ts_origin = __uint_as_float(q.ts(lane));
-    // a ray is walked up to the bound of its minimum, a direct one whole until
-    // its depth reaches the limit
-    const uint64_t lim = direct ? dlimit : 0ull;
+    const MegaQueue q = rays_with_stack(rays, stack);
     auto set_tmax = [&]() { q.tmax[2 * lane] = q.acc[2 * lane] < lim ? kTMax : __uint_as_float(q.bound(lane)); };
-    q.bound(lane) = q.ts(lane);
-    set_tmax();
-    // the first thread of this wavefront, for the owners' candidate buffers
-    const uint32_t gbase = blockIdx.x * blockDim.x + (threadIdx.x & ~63u);
+    // the first thread of the rays' wavefront, for the owners' candidate buffers
+    const uint32_t gbase = blockIdx.x * blockDim.x + rays_of * 64u;
     const uint32_t bs = mega_slab_stride(cap);
-    uint32_t nn = 0, nl = 0, nf = 0;
-    const unsigned long long am = __builtin_amdgcn_ballot_w64(alive);
-    if (alive) q.list[lanes_below(am)] = static_cast<uint8_t>(2 * lane);
-    wave_sync();
-    push_rays(q, ws, q.list, static_cast<uint32_t>(__popcll(am)), nn);
+    uint32_t nl = 0, nf = 0;
+    if (kOwn) {
+        set_tmax();
+        wave_sync();
+    }
     static_assert(kLeafItems >= 64u + kFlightMin + 64 + 4, "room for a step's leaves and the flights");
-    wave_sync();
     while (true) {
         if (nl < 64u && nn != 0u) {
+            if (nn >= kHelpMin && (rounds & (kHelpEvery - 1u)) == 0u) give_items(lds, q, rays_of, ws.one, true, nn);
             walk_nodes<true>(q, ws, nn, nl, kLeafItems - nf);
             ++rounds;
             continue;
@@ -181,7 +115,7 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const WaveScene& 
                             mine[3 * bs + pos] = __float_as_uint(x.t0);
                             mine[4 * bs + pos] = __float_as_uint(x.t1);
                         }
-                        const float tau = free_flight_tau(prim_uniform(key_of(own), meta & 0x7fffffffu, 1u, prim));
+                        const float tau = free_flight_tau(prim_uniform(draw_key(q, own), meta & 0x7fffffffu, 1u, prim));
                         keep = tau <= x.tau;
                         if (keep) atomicMin(&q.bound(own), __float_as_uint(x.t1));
                     }
@@ -198,7 +132,7 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const WaveScene& 
             }
             nf += static_cast<uint32_t>(__popcll(km));
             wave_sync();
-            set_tmax();
+            if (kOwn) set_tmax();
             wave_sync();
         }
         if (nf >= kFlightMin || (nl == 0u && nf != 0u)) {
@@ -208,7 +142,7 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const WaveScene& 
                 const uint32_t own = ray >> 1;
                 const f3 ro = lds_load3(q.ro + 3 * own), rd = lds_load3(q.rd + 3 * ray);
                 const PrimRecord pr = load_prim(ws.jobs[q.job[own]].scene.prims, prim);
-                const float tau = free_flight_tau(prim_uniform(key_of(own), bounce_of(own), 1u, prim));
+                const float tau = free_flight_tau(prim_uniform(draw_key(q, own), draw_bounce(q, own), 1u, prim));
                 const float t = entered_flight(pr, ro, rd, crossing(pr, ro, rd), tau);
                 const uint32_t tb = t == 0.0f ? 0u : __float_as_uint(t);
                 atomicMin(&q.ts(own), tb);
@@ -216,16 +150,141 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const WaveScene& 
             }
             nf = 0;
             wave_sync();
-            set_tmax();
+            if (kOwn) set_tmax();
             wave_sync();
         }
         if (nl == 0u && nn == 0u) break;
     }
+    if (kOwn)
+        while (help_load(q.help + 1) != 0u) {
+            set_tmax();
+            __builtin_amdgcn_s_sleep(4);
+        }
+}
+
+// Argmin free flight over the entered primitives (sampling.cuh:372-412) with
+// the wave-shared leaf queue.  All 64 lanes of the wavefront call it: a lane
+// with a path (alive) walks its own ray, and the origin-set members and queued
+// leaves of all rays are shared out among all lanes, so a wavefront with few
+// paths left still evaluates them 64 at a time.
+// Each ray's running minimum is an LDS atomic minimum over float bits (all
+// candidates are >= 0), so the result does not depend on which lane handles
+// which leaf.  Candidates for the rebuild are recorded while t_entry is at
+// most the running minimum at the time, which covers every primitive entered
+// before the final one; their order is fixed by the sort in the rebuild.  At
+// bounce 0 (direct) the walk also sums the direct term's optical depth into
+// dacc, and runs over the whole ray until that sum reaches dlimit (the
+// tau = 88 saturation or the direct term's roulette level, where T becomes
+// 0); from there on it prunes at the running minimum like any other ray.
+// ts_origin is the minimum over the origin set; the result keeps it unless a
+// walk candidate is strictly smaller.
+// Flights waiting to be inverted are taken up once there are kFlightMin of
+// them (few leaves have one, and the inversion's erf and erfinv cost as much
+// as the leaf round), or at the end of a run of leaves.  A flight ends inside
+// its chord, so until then its exit bounds the minimum (bound, which the walk
+// prunes by): without that bound, waiting for 16 flights cost the 10^6 cloud
+// 12 % and the 192x128 cloud 18 % against waiting for 4; with it, nothing.
+__device__ __forceinline__ void argmin_walk_shared(bool alive, const WaveScene& ws, uint32_t job, f3 o, f3 d, uint64_t key,
+                                                   uint32_t b, bool direct, const uint32_t* act, uint32_t na_path,
+                                                   float* act_exit, float ts_set, uint32_t* __restrict__ slab,
+                                                   uint32_t cap, const MegaQueue& q, float& ts, uint32_t& nc,
+                                                   uint64_t dlimit, uint64_t& dacc, uint32_t& rounds,
+                                                   uint32_t* lds) {
+    const uint32_t lane = __lane_id();
+    const uint32_t na = direct ? na_path : 0u;
+    lds_store3(q.ro + 3 * lane, o);
+    lds_store3(q.rd + 3 * (2 * lane), d);
+    lds_store3(q.inv + 3 * (2 * lane), safe_inv(d));
+    q.draw(lane)[0] = static_cast<uint32_t>(key);
+    q.draw(lane)[1] = static_cast<uint32_t>(key >> 32);
+    q.draw(lane)[2] = b | (direct ? 0x80000000u : 0u);
+    q.job[lane] = job;
+    q.acc[2 * lane] = 0ull;
+    q.ts(lane) = __float_as_uint(direct ? kTMax : ts_set);
+    q.nc(lane) = 0u;
+    // The origin set (sampling.cuh:356-370) of a path at bounce 0; from then
+    // on the last vertex's pass over the set has evaluated it (vertex_members)
+    // and ts_set is its minimum.  The wavefront's (member, lane) pairs are
+    // numbered through a prefix sum of the set sizes and shared out over the
+    // lanes.  Per member: its exit (kept in the owner's slab for the rebuild),
+    // its free flight into the owner's running minimum, and its chord into the
+    // owner's direct-term optical depth; minima and fixed-point sums do not
+    // depend on which lane adds what.  (Active sets of the megakernel are
+    // contiguous.)
+    if (__builtin_amdgcn_ballot_w64(na != 0u) != 0ull) {
+        const uint32_t** set_of = reinterpret_cast<const uint32_t**>(q.scratch);  // [64]
+        float** exit_of = reinterpret_cast<float**>(q.scratch) + 64;               // [64]
+        uint32_t* pre_of = q.scratch + 4 * 64;                                    // [64]
+        static_assert(kScratch >= 5 * 64, "the origin-set tables must fit in the queue");
+        uint32_t total;
+        pre_of[lane] = wave_prefix(na, total);
+        set_of[lane] = act;
+        exit_of[lane] = act_exit;
+        wave_sync();
+        for (uint32_t g = lane; g < total; g += 64u) {
+            const uint32_t ol = prefix_owner(pre_of, g), k = g - pre_of[ol];
+            const uint32_t i = set_of[ol][k];
+            const PrimRecord pr = load_prim(ws.jobs[q.job[ol]].scene.prims, i);
+            const f3 ro = lds_load3(q.ro + 3 * ol), rd = lds_load3(q.rd + 3 * (2 * ol));
+            const InsideChord x = inside_chord(pr, ro, rd);
+            exit_of[ol][k] = x.t1;
+            const float tau = free_flight_tau(prim_uniform(draw_key(q, ol), draw_bounce(q, ol), 0u, i));
+            if (tau <= x.tau) {
+                const float t = origin_flight(pr, ro, rd, x, tau);
+                atomicMin(&q.ts(ol), t == 0.0f ? 0u : __float_as_uint(t));
+            }
+            if (x.tau > 0.0f) atomicAdd(&q.acc[2 * ol], tau_fixed(x.tau));
+        }
+    }
+    wave_sync();
+    const float ts_origin = __uint_as_float(q.ts(lane));
+    q.bound(lane) = q.ts(lane);
+    uint32_t nn = 0;
+    const unsigned long long am = __builtin_amdgcn_ballot_w64(alive);
+    if (alive) q.list[lanes_below(am)] = static_cast<uint8_t>(2 * lane);
+    wave_sync();
+    push_rays(q, ws, q.list, static_cast<uint32_t>(__popcll(am)), nn);
+    // a direct ray is walked until its depth reaches the limit
+    argmin_rounds<true>(ws, lds, q, q, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), direct ? dlimit : 0ull, slab,
+                        cap, nn, rounds);
     const float wmin = __uint_as_float(q.ts(lane));
     ts = wmin < ts_origin ? wmin : ts_origin;
     nc = q.nc(lane);
     dacc = q.acc[2 * lane];
     wave_sync();
+}
+
+// A wavefront without paths works for the others of its workgroup until none
+// of them has any.
+__device__ __forceinline__ void help_walks(uint32_t* lds, const JobDesc* jobs, uint32_t* __restrict__ slab,
+                                           uint32_t cap) {
+    const uint32_t lane = __lane_id();
+    const MegaQueue q = mega_queue(lds);
+    uint32_t* const active = mega_queue_of(lds, 0u).help + 2;
+    if (lane == 0u)
+        (void)__hip_atomic_fetch_sub(active, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    while (true) {
+        if (lane == 0u)
+            __hip_atomic_store(q.help, kHelpWait, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+        uint32_t given;
+        while (((given = help_load(q.help)) & kHelpWork) == 0u) {
+            if (help_load(active) == 0u) return;
+            __builtin_amdgcn_s_sleep(8);
+        }
+        const uint32_t rays_of = (given >> 8) & 0xffu, n = given >> 16;
+        const MegaQueue rq = mega_queue_of(lds, rays_of);
+        WaveScene ws = wave_scene(jobs[rq.job[q.node_ray[0] >> 1]].scene, true, jobs);
+        ws.one = ws.one && (given & 4u) != 0u;
+        uint32_t rounds = 0;
+        if ((given & 8u) != 0u)
+            argmin_rounds<false>(ws, lds, q, rq, rays_of, 0ull, slab, cap, n, rounds);
+        else
+            shadow_rounds<false>(ws, lds, q, rq, rays_of, 0u, 0ull, 0ull, n, rounds);
+        // the candidates as well as the sums and minima are there first
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
+        if (lane == 0u)
+            (void)__hip_atomic_fetch_sub(rq.help + 1, 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+    }
 }
 
 // ---- the vertex stage of the timed kernel, all lanes of a wavefront together ----
@@ -555,7 +614,8 @@ __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has
 constexpr uint32_t kRoundsTarget = 256;
 constexpr uint32_t kPathsMin = 4;
 template <bool kCount, bool kMeasure>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(VP_RENDER_WAVES_PER_EU)))
+__global__ void __launch_bounds__(kCount || kMeasure ? 256 : 1024)
+    __attribute__((amdgpu_waves_per_eu(VP_RENDER_WAVES_PER_EU)))
 k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begin,
          const uint64_t* __restrict__ launch_desc, unsigned long long* __restrict__ path_counter,
          uint32_t* __restrict__ slab, uint32_t cap, uint32_t regen_min, uint32_t first_paths,
@@ -576,6 +636,10 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
     uint32_t* my = slab + static_cast<size_t>(gl) * kMegaSlabBuffers * bs;  // entry k of buffer b at my[b * bs + k]
     const LeafQueue lq = mega_leaf_queue(s_leafq);
     const MegaQueue q = mega_queue(s_leafq);  // the same LDS, used by the wave-wide walks
+    if constexpr (kShared) {
+        help_begin(s_leafq);
+        __syncthreads();
+    }
     PathState st{};
     bool alive = false;
     bool exhausted = false;  // every part of the path range is used up (the same in all lanes)
@@ -583,9 +647,11 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
     ev.reset();
     uint32_t overflow = 0;
     // The launch's paths in kClaimParts parts.  The first paths of part k are
-    // handed out without a counter: wavefront i of the workgroups with
-    // blockIdx % kClaimParts = k starts on its first_paths paths from i * first_paths
-    // (workgroups are dealt out to the XCDs in turn), so a launch with no more
+    // handed out without a counter: the wavefronts of the workgroups with
+    // blockIdx % kClaimParts = k start on first_paths paths each (workgroups are
+    // dealt out to the XCDs in turn), a workgroup's wavefronts on paths far
+    // apart, since neighbouring ones cost alike (192x128x2 cloud 11.9 -> 10.3
+    // ms, others the same), so a launch with no more
     // paths than that needs no atomics (each wavefront's 8 on the way out took
     // 430 us of a 4096-path launch).  The rest of part k is claimed through
     // path_counter[k * kClaimStride]; a wavefront starts with the part of the
@@ -620,8 +686,9 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
                 const uint32_t k = blockIdx.x % kClaimParts;
                 const uint64_t lo_k = path_lo + k * part;
                 const uint64_t hi_k = lo_k + part < total_paths ? lo_k + part : total_paths;
-                base = lo_k + (static_cast<uint64_t>(blockIdx.x / kClaimParts) * waves_per_block +
-                               __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * first_paths;
+                const uint32_t blocks_k = (gridDim.x + kClaimParts - 1u - k) / kClaimParts;
+                base = lo_k + (static_cast<uint64_t>(__builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) * blocks_k +
+                               blockIdx.x / kClaimParts) * first_paths;
                 if (base < hi_k) got = hi_k - base < first_paths ? static_cast<uint32_t>(hi_k - base) : first_paths;
                 first = false;
             }
@@ -752,7 +819,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
                 dlimit = direct_rr(kd).limit();
             }
             argmin_walk_shared(alive, ws, st.job, o, d, st.key, b, direct, act, na, act_exit, st.ts_set, slab, cap, q, ts, nc,
-                               dlimit, dwalk, rounds);
+                               dlimit, dwalk, rounds, s_leafq);
         } else {
             for (uint32_t k = 0; k < na; ++k) {
                 const uint32_t i = act[k * stride];
@@ -1019,7 +1086,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         // them one by one, so the former's counts are per-ray work)
         uint64_t acc_a = 0, acc_b = 0;
         if constexpr (kShared) {
-            shadow_walks(ws, q, lim_a, lim_b, acc_a, acc_b, rounds);
+            shadow_walks(ws, s_leafq, q, lim_a, lim_b, acc_a, acc_b, rounds);
             // the bounce's rounds per path, smoothed over bounces, in sixteenths
             work = (3u * work + 16u * rounds / nalive) / 4u;
             limit = 16u * kRoundsTarget / (work + 1u);
@@ -1056,6 +1123,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         }
     }
     if (overflow) atomicAdd(&counters[kCntActiveOverflow], static_cast<unsigned long long>(overflow));
+    if constexpr (kShared) help_walks(s_leafq, jobs, slab, cap);
 }
 
 // Adaptive sampling, after a batch (the slice of J): the batch's samples of
