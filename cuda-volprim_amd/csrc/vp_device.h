@@ -345,11 +345,6 @@ constexpr uint32_t kWaveQ = VP_WAVE_Q;
 // A node phase of the shared-queue walks ends early, to share out the queued
 // leaves, once the queue holds kWaveQ / 4 entries and fewer than
 // VP_SHARED_STEP_MIN lanes still step.
-// Shadow leaf phases in two passes (entry tests, then the chords of the
-// entered leaves), each at full width: +2 % on the scattering workload.
-#ifndef VP_SHADOW_TWO_STAGE
-#define VP_SHADOW_TWO_STAGE 1
-#endif
 #ifndef VP_SHARED_STEP_MIN
 #define VP_SHARED_STEP_MIN VP_WALK_MIN
 #endif

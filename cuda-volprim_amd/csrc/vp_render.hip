@@ -5,7 +5,7 @@
 // enough of its lanes are idle, so lanes stay busy across uneven path
 // lengths.  Per bounce a lane
 //   1. takes the argmin of closed-form per-primitive free flights over the
-//      primitives containing its origin and, in one stackless walk of the
+//      primitives containing its origin and, in one walk of the
 //      BVH, over every primitive the ray enters (no hit buffer: each
 //      primitive's uniform is a counter hash, so the minimum can be taken in
 //      any order and the walk prunes boxes beyond the running minimum); at

@@ -8,7 +8,7 @@
 // table then starts on the second of two render streams.  Each launch
 // claims, with its own counter, the range of paths its table adds to the
 // previous launch's, so the new launch takes the new request's paths while
-// the older one finishes its own: as the older launch's wavefronts run out of
+// the older one finishes its own: as the older launch's workgroups run out of
 // paths and exit, the new launch's workgroups take their place, and no
 // request waits for a step barrier or another request's tail.  Each launch has its own
 // active-set slab, so two can run at once.  Finished paths add into their
