@@ -157,6 +157,7 @@ RenderLaunch vp_resolve_launch(vp_context* ctx, const vp_launch_config* cfg, uin
     L.regen_min = std::max<uint32_t>(1u, std::min<uint32_t>(64u, c.regen_min ? c.regen_min : 8u));
     L.first_paths = 4u;
     L.claim_step = 8u;
+    L.rounds_target = 256u;
     L.count_events = count;
     L.measure = measure;
     // the wavefront pipeline has no event-counting or measuring variant
@@ -188,6 +189,11 @@ RenderLaunch vp_resolve_launch(vp_context* ctx, const vp_launch_config* cfg, uin
 // wavefronts to the others.  Starting on 4 and claiming 4, 8 and 16: 192x128x2
 // cloud (12 paths per wavefront) 17, 24, 38 ms, 512x512x1 torus (64) 19.9, 20.2,
 // 21.9, 256x256x24 scattering (384) 27.0, 26.4, 26.1.
+// A wavefront's paths are held to 256 rounds a bounce, or to 128 where a launch
+// has up to 128 paths to a wavefront: fewer paths at a time leave more to the
+// others near the end, and cost width in the middle (128 against 256: 8 batched
+// requests 12.3 -> 11.8 ms, 128x128 adaptive 17.6 -> 16.9, torus the same, but
+// 256x256x24 scattering 22.9 -> 24.6, 10^6 cloud 163 -> 172; 384: batched 13.3).
 // The wavefronts of a workgroup help each other at the end (help_walks in
 // vp_render.hip), so workgroups are as large as they can be, 16 wavefronts, once
 // there are 32 paths to a compute unit, and smaller below, where a launch's paths
@@ -209,6 +215,7 @@ RenderLaunch vp_size_launch(RenderLaunch L, uint64_t paths) {
     const uint64_t share = (paths + waves - 1) / waves;
     L.first_paths = static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>(4u, share)));
     L.claim_step = static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>(8u, (share + 2u) / 3u)));
+    L.rounds_target = share <= 128u ? 128u : 256u;
     return L;
 }
 

@@ -594,7 +594,7 @@ __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has
 // costs when paths are short.
 //
 // How many of a wavefront's lanes hold a path: enough that a bounce's walks
-// take about kRoundsTarget rounds (node steps and leaf rounds), which its fixed
+// take about rounds_target rounds (node steps and leaf rounds), which its fixed
 // part (set-up, rebuild, sampling, the walks' ends) is small against, and not
 // more, since what a wavefront holds it has to finish by itself: a path of the
 // 10^6 cloud takes about 40 rounds a bounce and one of the scattering scene 5.
@@ -611,7 +611,6 @@ __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has
 // their members and leaves 64 at a time and shares out their walks.  Only the
 // timed build does so (kShared); the counting and the measuring build walk
 // each ray by its own lane.
-constexpr uint32_t kRoundsTarget = 256;
 constexpr uint32_t kPathsMin = 4;
 template <bool kCount, bool kMeasure>
 __global__ void __launch_bounds__(kCount || kMeasure ? 256 : 1024)
@@ -619,7 +618,7 @@ __global__ void __launch_bounds__(kCount || kMeasure ? 256 : 1024)
 k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begin,
          const uint64_t* __restrict__ launch_desc, unsigned long long* __restrict__ path_counter,
          uint32_t* __restrict__ slab, uint32_t cap, uint32_t regen_min, uint32_t first_paths,
-         uint32_t claim_step, unsigned long long* __restrict__ counters) {
+         uint32_t claim_step, uint32_t rounds_target, unsigned long long* __restrict__ counters) {
     constexpr bool kShared = !kCount && !kMeasure;
     extern __shared__ __align__(16) uint32_t s_leafq[];  // [blockDim.x][kLeafRow]
     const uint32_t njobs = static_cast<uint32_t>(launch_desc[0]);
@@ -1089,7 +1088,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
             shadow_walks(ws, s_leafq, q, lim_a, lim_b, acc_a, acc_b, rounds);
             // the bounce's rounds per path, smoothed over bounces, in sixteenths
             work = (3u * work + 16u * rounds / nalive) / 4u;
-            limit = 16u * kRoundsTarget / (work + 1u);
+            limit = 16u * rounds_target / (work + 1u);
             limit = limit < kPathsMin ? kPathsMin : (limit < 64u ? limit : 64u);
         } else {
             if (has_a) acc_a = shadow_depth(sc, x, da, act, nn, stride, lq, ev, lim_a);
@@ -1372,7 +1371,7 @@ __global__ void k_prim(int fn, const PrimRecord* __restrict__ rec, const float* 
 }
 
 using RenderKernel = void (*)(const JobDesc*, const uint64_t*, const uint64_t*, unsigned long long*, uint32_t*,
-                              uint32_t, uint32_t, uint32_t, uint32_t, unsigned long long*);
+                              uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, unsigned long long*);
 RenderKernel render_kernel(int count_events, int measure) {
     if (count_events) return measure ? k_render<true, true> : k_render<true, false>;
     return measure ? k_render<false, true> : k_render<false, false>;
@@ -1395,7 +1394,7 @@ hipError_t vp_launch_render(const RenderLaunch& L, const JobDesc* jobs, const ui
     const size_t lds = mega_queue_bytes(L.block);
     const auto k = render_kernel(L.count_events, L.measure);
     hipLaunchKernelGGL(k, dim3(L.grid), dim3(L.block), lds, s, jobs, job_begin, launch_desc, counter, slab,
-                       L.active_cap, L.regen_min, L.first_paths, L.claim_step, counters);
+                       L.active_cap, L.regen_min, L.first_paths, L.claim_step, L.rounds_target, counters);
     return hipGetLastError();
 }
 
