@@ -67,6 +67,17 @@ void on_threads(int device, size_t chunks, F&& work) {
     for (auto& t : pool) t.join();
 }
 
+// Waits for s where a function returns (an error, an exception) with copies
+// under way, before the lock of the slots is released: they are the next
+// call's then, and the caller's memory its own again.
+struct WaitOnFailure {
+    hipStream_t s;
+    bool armed = true;
+    ~WaitOnFailure() {
+        if (armed) (void)hipStreamSynchronize(s);
+    }
+};
+
 struct Slots {
     std::atomic<size_t> next{0};
     std::atomic<int> err{hipSuccess};
@@ -123,6 +134,7 @@ vp_status vp_lease_scratch(vp_context* ctx, size_t bytes, hipStream_t s, Scratch
 
 vp_status vp_copy_out(vp_context* ctx, const HostCopy* copies, size_t n, hipStream_t s) {
     std::lock_guard<std::mutex> lk(ctx->mu);
+    WaitOnFailure wait{s};
     struct Chunk {
         char* dst;
         const char* src;
@@ -143,6 +155,7 @@ vp_status vp_copy_out(vp_context* ctx, const HostCopy* copies, size_t n, hipStre
         (void)hipGetLastError();
         for (const Chunk& c : parts) VP_HIP_TRY(hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyDeviceToHost, s));
         VP_HIP_TRY(hipStreamSynchronize(s));
+        wait.armed = false;
         return VP_OK;
     }
     if (total <= kStageSlot) {
@@ -160,6 +173,7 @@ vp_status vp_copy_out(vp_context* ctx, const HostCopy* copies, size_t n, hipStre
             VP_HIP_TRY(vp_launch_copy_parts(cp, s));
         }
         VP_HIP_TRY(hipStreamSynchronize(s));
+        wait.armed = false;
         at = ctx->stage;
         for (const Chunk& c : parts) {
             std::memcpy(c.dst, at, c.bytes);
@@ -190,12 +204,14 @@ vp_status vp_copy_out(vp_context* ctx, const HostCopy* copies, size_t n, hipStre
     });
     VP_HIP_TRY(static_cast<hipError_t>(S.err.load()));
     VP_HIP_TRY(hipStreamSynchronize(s));
+    wait.armed = false;
     return VP_OK;
 }
 
 vp_status vp_copy_in(vp_context* ctx, void* dst, const void* src, size_t elem, size_t count,
                      bool (*check)(const void* rows, size_t count), bool* good, hipStream_t s) {
     std::lock_guard<std::mutex> lk(ctx->mu);
+    WaitOnFailure wait{s};
     const char* from = static_cast<const char*>(src);
     char* to = static_cast<char*>(dst);
     const size_t rows = kStageSlot / elem;
@@ -203,6 +219,7 @@ vp_status vp_copy_in(vp_context* ctx, void* dst, const void* src, size_t elem, s
         (void)hipGetLastError();
         *good = check(src, count);
         if (*good) VP_HIP_TRY(hipMemcpyAsync(dst, src, elem * count, hipMemcpyHostToDevice, s));
+        wait.armed = false;
         return VP_OK;
     }
     const size_t chunks = (count + rows - 1) / rows;
@@ -228,5 +245,6 @@ vp_status vp_copy_in(vp_context* ctx, void* dst, const void* src, size_t elem, s
     *good = ok.load();
     VP_HIP_TRY(static_cast<hipError_t>(S.err.load()));
     VP_HIP_TRY(hipStreamSynchronize(s));  // the slots are the next call's
+    wait.armed = false;
     return VP_OK;
 }

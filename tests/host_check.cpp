@@ -1,0 +1,105 @@
+// host_check.cpp — checks of the library's host side over hip_stub.h: what it
+// does when a call of the runtime fails, what memory it takes, which launches
+// it makes.  host_check NAME runs one check and prints "ok NAME".
+#include "hip_stub.h"
+
+#include <cmath>
+
+#include "../include/vp_api.h"
+
+using stub::check;
+
+namespace {
+
+std::vector<vp_primitive> primitives(uint32_t n) {
+    std::vector<vp_primitive> p(n);
+    for (uint32_t i = 0; i < n; ++i) {
+        std::memset(&p[i], 0, sizeof(p[i]));
+        for (int k = 0; k < 3; ++k) {
+            p[i].center[k] = float((i >> k) % 17u);
+            p[i].scale[k] = 0.1f;
+            p[i].albedo[k] = 0.5f;
+        }
+        p[i].quat_wxyz[0] = 1.0f;
+        p[i].mass = 1.0f;
+    }
+    return p;
+}
+
+struct Program {
+    vp_context* ctx = nullptr;
+    vp_scene* scene = nullptr;
+    explicit Program(uint32_t n, int device = 0) {
+        check(vp_context_create(device, &ctx) == VP_OK, "vp_context_create");
+        const auto p = primitives(n);
+        check(vp_scene_create(ctx, p.data(), n, &scene) == VP_OK, "vp_scene_create");
+    }
+    ~Program() {
+        vp_scene_destroy(scene);
+        vp_context_destroy(ctx);
+    }
+};
+
+// A call that fails in the middle of its copies returns only when none of
+// them is under way any more: the slots are the next call's, the destination
+// the caller's.
+void failed_copies() {
+    for (uint32_t n : {1000u, 300000u}) {  // one slot, several
+        Program prog(n);
+        std::vector<uint32_t> order(n), morton(n);
+        std::vector<float> records(16 * size_t(n));
+        for (int fail = 0; fail < 12; ++fail) {
+            // the copy, the event or the launch number `fail` of an export
+            // fails, with the records and without
+            for (int what = 0; what < 6; ++what) {
+                int left = fail;
+                bool failed = false;
+                const auto f = [&] { return left-- > 0 ? hipSuccess : (failed = true, hipErrorUnknown); };
+                if (what % 3 == 0) stub::on_copy = f;
+                if (what % 3 == 1) stub::on_record = f;
+                if (what % 3 == 2) stub::on_launch = [&](const std::string&, dim3) { return f(); };
+                const vp_status st = vp_scene_export(prog.scene, order.data(), morton.data(),
+                                                     what < 3 ? records.data() : nullptr, nullptr);
+                stub::on_copy = nullptr;
+                stub::on_record = nullptr;
+                stub::on_launch = nullptr;
+                check((st == VP_OK) == !failed, "the export reports the failure");
+                check(stub::queue.empty(), "no copy is under way after the call");
+                (void)hipGetLastError();
+            }
+        }
+        // a destination in pinned memory is copied to directly
+        uint32_t* pinned = nullptr;
+        (void)hipHostMalloc(reinterpret_cast<void**>(&pinned), 4 * size_t(n), 0);
+        int left = 1;
+        stub::on_copy = [&] { return left-- > 0 ? hipSuccess : hipErrorUnknown; };
+        if (n > 100000u) {
+            check(vp_scene_export(prog.scene, pinned, morton.data(), nullptr, nullptr) != VP_OK, "the copy fails");
+            check(stub::queue.empty(), "no direct copy is under way after the call");
+        }
+        stub::on_copy = nullptr;
+        (void)hipHostFree(pinned);
+        // the same for the primitives on their way in
+        const auto p = primitives(n);
+        for (int fail = 0; fail < 12; ++fail) {
+            left = fail;
+            stub::on_record = [&] { return left-- > 0 ? hipSuccess : hipErrorUnknown; };
+            vp_scene* sc = nullptr;
+            if (vp_scene_create(prog.ctx, p.data(), n, &sc) == VP_OK) vp_scene_destroy(sc);
+            else check(stub::queue.empty(), "no copy of the primitives is under way after the call");
+            stub::on_record = nullptr;
+            (void)hipGetLastError();
+        }
+    }
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+    const std::map<std::string, void (*)()> checks = {{"failed_copies", failed_copies}};
+    check(argc == 2 && checks.count(argv[1]) == 1, "usage: host_check NAME");
+    checks.at(argv[1])();
+    std::printf("ok %s\n", argv[1]);
+    std::fflush(stdout);
+    std::_Exit(0);
+}
