@@ -296,6 +296,7 @@ vp_status vp_scene_destroy(vp_scene* sc) {
 
 vp_status vp_scene_export(vp_scene* sc, uint32_t* order, uint32_t* morton, float* records16, uint32_t* depth) {
     if (!sc) return fail(VP_ERR_INVALID, "scene is null");
+    VP_HIP_TRY(hipSetDevice(sc->ctx->device));
     hipStream_t s = sc->ctx->stream;
     const size_t words = sizeof(uint32_t) * static_cast<size_t>(sc->n);
     HostCopy outs[3];

@@ -93,10 +93,20 @@ void failed_copies() {
     }
 }
 
+// A scene is exported on its own context's device, whichever is current.
+void export_device() {
+    Program first(1000, 0), second(1000, 1);
+    std::vector<uint32_t> order(1000);
+    std::vector<float> records(16 * 1000);
+    for (Program* p : {&first, &second, &first})
+        check(vp_scene_export(p->scene, order.data(), nullptr, records.data(), nullptr) == VP_OK, "vp_scene_export");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
-    const std::map<std::string, void (*)()> checks = {{"failed_copies", failed_copies}};
+    const std::map<std::string, void (*)()> checks = {{"failed_copies", failed_copies},
+                                                          {"export_device", export_device}};
     check(argc == 2 && checks.count(argv[1]) == 1, "usage: host_check NAME");
     checks.at(argv[1])();
     std::printf("ok %s\n", argv[1]);
