@@ -303,15 +303,19 @@ vp_status vp_scene_export(vp_scene* sc, uint32_t* order, uint32_t* morton, float
     size_t k = 0;
     if (order) outs[k++] = {order, sc->order, words};
     if (morton) outs[k++] = {morton, sc->morton, words};
-    ScratchLease rec;  // the records in the exported field order
+    // the records in the exported field order: rearranged on the device, or,
+    // where it has no memory left for that, after the copy
+    ScratchLease rec;
+    bool on_host = false;
     if (records16) {
-        const vp_status st = vp_lease_scratch(sc->ctx, 16 * words, s, rec);
-        if (st != VP_OK) return st;
-        VP_HIP_TRY(vp_launch_export_records(sc->prims, sc->n, static_cast<float4*>(rec.p), s));
-        outs[k++] = {records16, rec.p, 16 * words};
+        on_host = vp_lease_scratch(sc->ctx, 16 * words, s, rec) != VP_OK;
+        if (!on_host) VP_HIP_TRY(vp_launch_export_records(sc->prims, sc->n, static_cast<float4*>(rec.p), s));
+        outs[k++] = {records16, on_host ? static_cast<const void*>(sc->prims) : rec.p, 16 * words};
     }
     const vp_status st = vp_copy_out(sc->ctx, outs, k, s);
     if (st != VP_OK) return st;
+    if (on_host)
+        for (size_t i = 0; i < sc->n; ++i) records16[16 * i + 11] *= vp::kRootHalfPi;
     rec.done = true;
     if (depth) *depth = sc->depth;
     return VP_OK;

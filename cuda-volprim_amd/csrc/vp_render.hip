@@ -1334,7 +1334,7 @@ __global__ void k_math(int fn, const float* __restrict__ x, const float* __restr
 // order, the inverse-CDF factor M dnf sqrt(pi/2) in word 11.
 __global__ void k_export_records(const PrimRecord* __restrict__ in, uint32_t n, float4* __restrict__ out) {
     const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= 4u * n) return;
+    if ((i >> 2) >= n) return;
     float4 v = reinterpret_cast<const float4*>(in)[i];
     if ((i & 3u) == 2u) v.w *= kRootHalfPi;
     out[i] = v;

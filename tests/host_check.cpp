@@ -102,11 +102,29 @@ void export_device() {
         check(vp_scene_export(p->scene, order.data(), nullptr, records.data(), nullptr) == VP_OK, "vp_scene_export");
 }
 
+// The records of a scene are exported whatever device memory is left, in the
+// same order and with the same word 11 (the stored one times sqrt(pi / 2)).
+void export_without_memory() {
+    const uint32_t n = 1100000;  // a build whose scratch is not kept
+    Program prog(n);
+    float* stored = nullptr;
+    for (const auto& m : stub::device_mem)
+        if (m.second >= 72 * size_t(n) && m.second < 73 * size_t(n)) stored = static_cast<float*>(m.first);
+    check(stored != nullptr, "the scene's records");
+    for (size_t i = 0; i < 16 * size_t(n); ++i) stored[i] = 0.37f * float(i % 1013u);
+    stub::limit = stub::used;
+    std::vector<float> records(16 * size_t(n));
+    check(vp_scene_export(prog.scene, nullptr, nullptr, records.data(), nullptr) == VP_OK, "vp_scene_export");
+    for (size_t i = 0; i < records.size(); ++i)
+        check(records[i] == (i % 16 == 11 ? stored[i] * 1.2533141374f : stored[i]), "the exported record");
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {{"failed_copies", failed_copies},
-                                                          {"export_device", export_device}};
+                                                          {"export_device", export_device},
+                                                          {"export_without_memory", export_without_memory}};
     check(argc == 2 && checks.count(argv[1]) == 1, "usage: host_check NAME");
     checks.at(argv[1])();
     std::printf("ok %s\n", argv[1]);
