@@ -358,9 +358,9 @@ vp_status vp_env_create(vp_context* ctx, const float* rgba, uint32_t w, uint32_t
     env->total = total;
     build_alias(env->joint_host, env->alias_host);
     hipStream_t s = ctx->stream;
-    if (hipMalloc(&env->tex, n * 4 * sizeof(float)) != hipSuccess ||
-        hipMalloc(&env->joint, n * sizeof(float)) != hipSuccess ||
-        hipMalloc(&env->alias, n * sizeof(vp::AliasEntry)) != hipSuccess) {
+    if (vp_device_malloc(ctx, &env->tex, n * 4 * sizeof(float)) != hipSuccess ||
+        vp_device_malloc(ctx, &env->joint, n * sizeof(float)) != hipSuccess ||
+        vp_device_malloc(ctx, &env->alias, n * sizeof(vp::AliasEntry)) != hipSuccess) {
         vp_env_destroy(env);
         return fail(VP_ERR_OOM, "cannot allocate the environment");
     }
@@ -565,8 +565,8 @@ vp_status vp_transmittance_rays(vp_context* ctx, vp_scene* sc, const float* rays
     if (m == 0) return VP_OK;
     VP_HIP_TRY(hipSetDevice(ctx->device));
     Dev dr, dt;
-    VP_HIP_TRY(hipMalloc(&dr.p, sizeof(float) * 6 * m));
-    VP_HIP_TRY(hipMalloc(&dt.p, sizeof(float) * m));
+    VP_HIP_TRY(vp_device_malloc(ctx, &dr.p, sizeof(float) * 6 * m));
+    VP_HIP_TRY(vp_device_malloc(ctx, &dt.p, sizeof(float) * m));
     VP_HIP_TRY(hipMemcpyAsync(dr.p, rays, sizeof(float) * 6 * m, hipMemcpyHostToDevice, ctx->stream));
     VP_HIP_TRY(vp_launch_transmittance(sc->view(), static_cast<const float*>(dr.p), m, static_cast<float*>(dt.p),
                                        ctx->stream));
@@ -582,10 +582,10 @@ vp_status vp_collect_overlaps(vp_context* ctx, vp_scene* sc, const float* rays, 
     if (cap == 0) return fail(VP_ERR_INVALID, "cap must be positive");
     VP_HIP_TRY(hipSetDevice(ctx->device));
     Dev dr, dc, dt, di;
-    VP_HIP_TRY(hipMalloc(&dr.p, sizeof(float) * 6 * m));
-    VP_HIP_TRY(hipMalloc(&dc.p, sizeof(uint32_t) * m));
-    VP_HIP_TRY(hipMalloc(&dt.p, sizeof(float) * static_cast<size_t>(m) * cap));
-    VP_HIP_TRY(hipMalloc(&di.p, sizeof(uint32_t) * static_cast<size_t>(m) * cap));
+    VP_HIP_TRY(vp_device_malloc(ctx, &dr.p, sizeof(float) * 6 * m));
+    VP_HIP_TRY(vp_device_malloc(ctx, &dc.p, sizeof(uint32_t) * m));
+    VP_HIP_TRY(vp_device_malloc(ctx, &dt.p, sizeof(float) * static_cast<size_t>(m) * cap));
+    VP_HIP_TRY(vp_device_malloc(ctx, &di.p, sizeof(uint32_t) * static_cast<size_t>(m) * cap));
     VP_HIP_TRY(hipMemsetAsync(dt.p, 0, sizeof(float) * static_cast<size_t>(m) * cap, ctx->stream));
     VP_HIP_TRY(hipMemsetAsync(di.p, 0, sizeof(uint32_t) * static_cast<size_t>(m) * cap, ctx->stream));
     VP_HIP_TRY(hipMemcpyAsync(dr.p, rays, sizeof(float) * 6 * m, hipMemcpyHostToDevice, ctx->stream));
@@ -604,9 +604,9 @@ vp_status vp_math_eval(vp_context* ctx, int fn, const float* x, const float* y, 
     if (n == 0) return VP_OK;
     VP_HIP_TRY(hipSetDevice(ctx->device));
     Dev dx, dy, dout;
-    VP_HIP_TRY(hipMalloc(&dx.p, sizeof(float) * n));
-    VP_HIP_TRY(hipMalloc(&dy.p, sizeof(float) * n));
-    VP_HIP_TRY(hipMalloc(&dout.p, sizeof(float) * n));
+    VP_HIP_TRY(vp_device_malloc(ctx, &dx.p, sizeof(float) * n));
+    VP_HIP_TRY(vp_device_malloc(ctx, &dy.p, sizeof(float) * n));
+    VP_HIP_TRY(vp_device_malloc(ctx, &dout.p, sizeof(float) * n));
     VP_HIP_TRY(hipMemcpyAsync(dx.p, x, sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
     if (y) VP_HIP_TRY(hipMemcpyAsync(dy.p, y, sizeof(float) * n, hipMemcpyHostToDevice, ctx->stream));
     else VP_HIP_TRY(hipMemsetAsync(dy.p, 0, sizeof(float) * n, ctx->stream));
@@ -622,9 +622,9 @@ vp_status vp_prim_eval(vp_context* ctx, int fn, const float* record16, const flo
     if (m == 0) return VP_OK;
     VP_HIP_TRY(hipSetDevice(ctx->device));
     Dev drec, dargs, dout;
-    VP_HIP_TRY(hipMalloc(&drec.p, sizeof(vp::PrimRecord)));
-    VP_HIP_TRY(hipMalloc(&dargs.p, sizeof(float) * 9 * m));
-    VP_HIP_TRY(hipMalloc(&dout.p, sizeof(float) * m));
+    VP_HIP_TRY(vp_device_malloc(ctx, &drec.p, sizeof(vp::PrimRecord)));
+    VP_HIP_TRY(vp_device_malloc(ctx, &dargs.p, sizeof(float) * 9 * m));
+    VP_HIP_TRY(vp_device_malloc(ctx, &dout.p, sizeof(float) * m));
     VP_HIP_TRY(hipMemcpyAsync(drec.p, record16, sizeof(vp::PrimRecord), hipMemcpyHostToDevice, ctx->stream));
     VP_HIP_TRY(hipMemcpyAsync(dargs.p, args9, sizeof(float) * 9 * m, hipMemcpyHostToDevice, ctx->stream));
     VP_HIP_TRY(vp_launch_prim(fn, static_cast<const vp::PrimRecord*>(drec.p), static_cast<const float*>(dargs.p), m,

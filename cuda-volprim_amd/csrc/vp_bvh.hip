@@ -461,7 +461,7 @@ vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32
         sc->prims = a.take<PrimRecord>(n_slots);
         sc->order = a.take<uint32_t>(n);
         sc->morton = a.take<uint32_t>(n);
-        if (pass == 0) VP_HIP_TRY(hipMalloc(&sc->mem, a.used));
+        if (pass == 0) VP_HIP_TRY(vp_device_malloc(ctx, &sc->mem, a.used));
     }
     if (n_slots > n) VP_HIP_TRY(hipMemsetAsync(sc->prims + n, 0, sizeof(PrimRecord) * (n_slots - n), s));
     bool valid = false;
@@ -526,7 +526,7 @@ vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32
     sc->w4_growth = sums[0] > 0.0 ? sums[1] / sums[0] - 1.0 : 0.0;
     const bool half = !(flags & VP_SCENE_WALK_F32) && ((flags & VP_SCENE_WALK_F16) || sc->w4_growth <= 1.0 / 16.0);
     const size_t w4_bytes = (half ? static_cast<size_t>(kW4hRecordB) : sizeof(float4) * kW4RecordF4) * records;
-    VP_HIP_TRY(hipMalloc(&sc->w4, w4_bytes));
+    VP_HIP_TRY(vp_device_malloc(ctx, &sc->w4, w4_bytes));
     VP_HIP_TRY(hipMemcpyAsync(sc->w4, half ? static_cast<const void*>(T.w4_half) : T.w4, w4_bytes,
                               hipMemcpyDeviceToDevice, s));
     sc->w4_half = half ? 1u : 0u;

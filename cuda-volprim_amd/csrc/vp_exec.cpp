@@ -23,7 +23,7 @@ vp_status vp_ensure_slab(vp_context* ctx, size_t words) {
     if (ctx->slab) (void)hipFree(ctx->slab);
     ctx->slab = nullptr;
     ctx->slab_words = 0;
-    if (hipMalloc(&ctx->slab, words * sizeof(uint32_t)) != hipSuccess)
+    if (vp_device_malloc(ctx, &ctx->slab, words * sizeof(uint32_t)) != hipSuccess)
         return fail(VP_ERR_OOM, "cannot allocate the active-set slab (" + std::to_string(words * 4) + " bytes)");
     ctx->slab_words = words;
     vp_drop_graph(ctx);
@@ -71,7 +71,7 @@ vp_status vp_ensure_wf(vp_context* ctx, uint32_t P, uint32_t cap) {
     const size_t o_cb = carve(16), o_fin = carve(8);
     const size_t o_slab = carve(static_cast<size_t>(vp::kSlabBuffers) * cap * p * 4);
     const size_t o_ncand = carve(4 * p);
-    if (hipMalloc(&ctx->wf_mem, off) != hipSuccess) {
+    if (vp_device_malloc(ctx, &ctx->wf_mem, off) != hipSuccess) {
         ctx->wf_mem = nullptr;
         return fail(VP_ERR_OOM, "cannot allocate the wavefront path pool (" + std::to_string(off) + " bytes)");
     }
@@ -128,9 +128,9 @@ vp_status vp_ensure_jobs(vp_context* ctx, uint32_t n) {
     ctx->jobs_pinned = nullptr;
     ctx->begin_pinned = nullptr;
     ctx->jobs_cap = ctx->pinned_cap = 0;
-    VP_HIP_TRY(hipMalloc(&ctx->jobs_dev, sizeof(vp::JobDesc) * n));
-    VP_HIP_TRY(hipMalloc(&ctx->job_begin_dev, sizeof(uint64_t) * n));
-    VP_HIP_TRY(hipMalloc(&ctx->job_done_dev, sizeof(unsigned long long) * n));
+    VP_HIP_TRY(vp_device_malloc(ctx, &ctx->jobs_dev, sizeof(vp::JobDesc) * n));
+    VP_HIP_TRY(vp_device_malloc(ctx, &ctx->job_begin_dev, sizeof(uint64_t) * n));
+    VP_HIP_TRY(vp_device_malloc(ctx, &ctx->job_done_dev, sizeof(unsigned long long) * n));
     VP_HIP_TRY(hipHostMalloc(&ctx->jobs_pinned, sizeof(vp::JobDesc) * n, hipHostMallocDefault));
     VP_HIP_TRY(hipHostMalloc(&ctx->begin_pinned, sizeof(uint64_t) * n, hipHostMallocDefault));
     ctx->jobs_cap = ctx->pinned_cap = n;

@@ -284,6 +284,15 @@ vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32
 void vp_host_tree_order(const vp_primitive* in, uint32_t n, bool median, std::vector<uint32_t>& order,
                         uint32_t& depth);
 
+// Device memory on ctx's device (which must be current); where none is left,
+// the context's kept scratch is given back for it, if no call has it.
+hipError_t vp_device_malloc(vp_context* ctx, void** p, size_t bytes);
+template <typename T>
+hipError_t vp_device_malloc(vp_context* ctx, T** p, size_t bytes) {
+    return vp_device_malloc(ctx, reinterpret_cast<void**>(p), bytes);
+}
+bool vp_give_back_scratch(vp_context* ctx);  // whether there was any
+
 // Device scratch for the duration of one call.  Up to kScratchKeep bytes are
 // kept in the context between calls and freed with it; larger ones, and those
 // of a call that finds the kept block in use, are allocated for the call.  A

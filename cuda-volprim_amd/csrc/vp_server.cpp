@@ -160,7 +160,9 @@ bool streams_idle(vp_server* S) {
 vp_status install_request(vp_server* S, Request* r) {
     const size_t npix = static_cast<size_t>(r->job.params.width) * r->job.params.height;
     const size_t acc_bytes = npix * vp::kAccumWords * sizeof(unsigned long long);
-    if (hipMallocAsync(reinterpret_cast<void**>(&r->accum), acc_bytes, S->side) != hipSuccess) {
+    void** accum = reinterpret_cast<void**>(&r->accum);
+    if (hipMallocAsync(accum, acc_bytes, S->side) != hipSuccess &&
+        !(vp_give_back_scratch(S->ctx) && hipMallocAsync(accum, acc_bytes, S->side) == hipSuccess)) {
         (void)hipGetLastError();
         r->accum = nullptr;
         return fail(VP_ERR_OOM, "server: cannot allocate a request's accumulator");
@@ -453,13 +455,13 @@ vp_status vp_server_create(vp_context* ctx, const vp_server_config* cfg, vp_serv
     }
     if (free_cus > 0 && S->L.grid >= cus) S->L.grid = S->L.grid / cus * (cus - free_cus);
     const size_t slab_words = vp::kMegaSlabBuffers * static_cast<size_t>(vp::mega_slab_stride(cap)) * S->L.grid * S->L.block;
-    bool ok = hipMalloc(&S->jobs_dev, sizeof(vp::JobDesc) * kServerTable) == hipSuccess &&
-              hipMalloc(&S->begin_dev, sizeof(uint64_t) * kServerTable) == hipSuccess &&
-              hipMalloc(&S->done_dev, sizeof(unsigned long long) * kServerTable) == hipSuccess &&
-              hipMalloc(&S->counter, 2 * vp::kClaimWords * sizeof(unsigned long long)) == hipSuccess &&
-              hipMalloc(&S->desc_dev, 8 * sizeof(uint64_t)) == hipSuccess &&
-              hipMalloc(&S->slab[0], slab_words * sizeof(uint32_t)) == hipSuccess &&
-              hipMalloc(&S->slab[1], slab_words * sizeof(uint32_t)) == hipSuccess;
+    bool ok = vp_device_malloc(ctx, &S->jobs_dev, sizeof(vp::JobDesc) * kServerTable) == hipSuccess &&
+              vp_device_malloc(ctx, &S->begin_dev, sizeof(uint64_t) * kServerTable) == hipSuccess &&
+              vp_device_malloc(ctx, &S->done_dev, sizeof(unsigned long long) * kServerTable) == hipSuccess &&
+              vp_device_malloc(ctx, &S->counter, 2 * vp::kClaimWords * sizeof(unsigned long long)) == hipSuccess &&
+              vp_device_malloc(ctx, &S->desc_dev, 8 * sizeof(uint64_t)) == hipSuccess &&
+              vp_device_malloc(ctx, &S->slab[0], slab_words * sizeof(uint32_t)) == hipSuccess &&
+              vp_device_malloc(ctx, &S->slab[1], slab_words * sizeof(uint32_t)) == hipSuccess;
     if (!ok) return fail(VP_ERR_OOM, "server: cannot allocate its tables and active-set slabs");
     ok = hipHostMalloc(&S->jobs_pinned, sizeof(vp::JobDesc) * kServerTable, hipHostMallocDefault) == hipSuccess &&
          hipHostMalloc(&S->begin_pinned, sizeof(uint64_t) * kServerTable, hipHostMallocDefault) == hipSuccess &&

@@ -99,6 +99,23 @@ struct Slots {
 
 }  // namespace
 
+bool vp_give_back_scratch(vp_context* ctx) {
+    if (ctx->scratch_busy.exchange(true, std::memory_order_acquire)) return false;
+    const bool any = ctx->scratch != nullptr;
+    if (any) (void)hipFree(ctx->scratch);
+    ctx->scratch = nullptr;
+    ctx->scratch_bytes = 0;
+    ctx->scratch_busy.store(false, std::memory_order_release);
+    return any;
+}
+
+hipError_t vp_device_malloc(vp_context* ctx, void** p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e == hipSuccess || !vp_give_back_scratch(ctx)) return e;
+    (void)hipGetLastError();
+    return hipMalloc(p, bytes);
+}
+
 ScratchLease::~ScratchLease() {
     if (!p) return;
     if (!done) (void)hipStreamSynchronize(stream);
@@ -124,7 +141,7 @@ vp_status vp_lease_scratch(vp_context* ctx, size_t bytes, hipStream_t s, Scratch
         lease.p = ctx->scratch;
         if (!lease.p) ctx->scratch_busy.store(false, std::memory_order_release);
     } else {
-        lease.owned = hipMalloc(&lease.p, bytes) == hipSuccess;
+        lease.owned = vp_device_malloc(ctx, &lease.p, bytes) == hipSuccess;
         if (!lease.owned) lease.p = nullptr;
     }
     if (lease.p) return VP_OK;

@@ -119,12 +119,55 @@ void export_without_memory() {
         check(records[i] == (i % 16 == 11 ? stored[i] * 1.2533141374f : stored[i]), "the exported record");
 }
 
+// The largest allocation: after a build of 300000 primitives, its scratch,
+// which the context keeps.
+size_t largest() {
+    size_t m = 0;
+    for (const auto& a : stub::device_mem) m = std::max(m, a.second);
+    return m;
+}
+
+// The scratch that a context keeps is given back to a call that finds no other
+// memory: what fits without it still fits.
+void kept_scratch() {
+    const size_t mib = size_t(1) << 20;
+    {
+        Program prog(300000);
+        vp_env* env = nullptr;
+        std::vector<float> texels(4 * 16);
+        check(vp_env_create(prog.ctx, texels.data(), 4, 4, &env) == VP_OK, "vp_env_create");
+        vp_camera cam{};
+        vp_render_params p{};
+        vp_default_params(&p);
+        p.width = p.height = 8;
+        p.spp = 1;
+        const size_t kept = largest(), slab = size_t(4096) * 64 * 6 * 128 * 4;
+        check(kept > 100 * mib, "the build's scratch");
+        stub::limit = stub::used - kept + slab + mib;
+        std::vector<float> image(4 * 64);
+        check(vp_render(prog.ctx, prog.scene, env, &cam, &p, image.data(), nullptr) == VP_OK, "vp_render");
+        stub::limit = ~size_t(0);
+        vp_env_destroy(env);
+    }
+    {
+        Program prog(300000);
+        vp_env* env = nullptr;
+        const uint32_t w = 2048, h = 1024;
+        std::vector<float> texels(4 * size_t(w) * h, 1.0f);
+        stub::limit = stub::used - largest() + 28 * size_t(w) * h + mib;
+        check(vp_env_create(prog.ctx, texels.data(), w, h, &env) == VP_OK, "vp_env_create");
+        stub::limit = ~size_t(0);
+        vp_env_destroy(env);
+    }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {{"failed_copies", failed_copies},
                                                           {"export_device", export_device},
-                                                          {"export_without_memory", export_without_memory}};
+                                                          {"export_without_memory", export_without_memory},
+                                                          {"kept_scratch", kept_scratch}};
     check(argc == 2 && checks.count(argv[1]) == 1, "usage: host_check NAME");
     checks.at(argv[1])();
     std::printf("ok %s\n", argv[1]);
