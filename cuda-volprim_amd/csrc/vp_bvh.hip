@@ -397,22 +397,18 @@ struct Arena {
     }
 };
 
-// Device temporaries of a scene build.
-struct BuildTemps {
+// Device temporaries of a scene build: of the order,
+struct OrderTemps {
     vp_primitive* in;
     PrimRecord* rec;                // input order
-    float *centers, *box, *sorted_box, *partial, *bounds;
+    float *centers, *box, *partial, *bounds;
     uint32_t *codes, *idx, *codes2, *idx2, *hist, *depth;
     int* parent;
-    float4* w4;                     // 32-bit records
-    uint4* w4_half;
-    double* sums;
-    BuildTemps(Arena& a, uint32_t n, uint32_t nb_sort, uint32_t nbounds, size_t records) {
+    OrderTemps(Arena& a, uint32_t n, uint32_t nb_sort, uint32_t nbounds) {
         in = a.take<vp_primitive>(n);
         rec = a.take<PrimRecord>(n);
         centers = a.take<float>(3 * static_cast<size_t>(n));
         box = a.take<float>(6 * static_cast<size_t>(n));
-        sorted_box = a.take<float>(6 * static_cast<size_t>(n));
         partial = a.take<float>(6 * nbounds);
         bounds = a.take<float>(6);
         codes = a.take<uint32_t>(n);
@@ -422,35 +418,77 @@ struct BuildTemps {
         hist = a.take<uint32_t>(256 * static_cast<size_t>(nb_sort));
         depth = a.take<uint32_t>(1);
         parent = a.take<int>(2 * static_cast<size_t>(n));
-        w4 = a.take<float4>(kW4RecordF4 * records);
-        w4_half = a.take<uint4>(kW4hRecordB / sizeof(uint4) * records);
+    }
+};
+// between the order and the tree,
+struct BoxTemps {
+    float* sorted_box;
+    double* sums;
+    BoxTemps(Arena& a, uint32_t n) {
+        sorted_box = a.take<float>(6 * static_cast<size_t>(n));
         sums = a.take<double>(2);
     }
 };
+// and of the tree.
+struct TreeTemps {
+    float4* w4;                     // 32-bit records
+    uint4* w4_half;
+    TreeTemps() = default;
+    TreeTemps(Arena& a, size_t records) {
+        w4 = a.take<float4>(kW4RecordF4 * records);
+        w4_half = a.take<uint4>(kW4hRecordB / sizeof(uint4) * records);
+    }
+};
+
+struct DevMem {
+    void* p = nullptr;
+    DevMem() = default;
+    DevMem(const DevMem&) = delete;
+    DevMem& operator=(const DevMem&) = delete;
+    ~DevMem() {
+        if (p) (void)hipFree(p);
+    }
+};
+
+vp_status scene_malloc(vp_context* ctx, void** p, size_t bytes) {
+    if (vp_device_malloc(ctx, p, bytes) == hipSuccess) return VP_OK;
+    *p = nullptr;
+    (void)hipGetLastError();
+    vp_set_error("cannot allocate " + std::to_string(bytes) + " bytes of device memory");
+    return VP_ERR_OOM;
+}
 
 }  // namespace
 }  // namespace vp
 
-// Builds scene sc (whose n is set): records, Morton codes and stored order,
-// the order from the radix sort or, with VP_SCENE_BVH_SAH / _MEDIAN in flags,
-// from the host tree, and the walk tree over it.  Temporaries are scratch;
-// the scene owns two allocations.  Returns VP_ERR_INVALID without a message
-// where a primitive is not valid.
-vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32_t n, uint32_t flags, vp_scene* sc) {
+// The build of scene sc (see vp_build_scene).  Its temporaries are one block
+// of scratch, or (staged) one of each stage's own, the order's released before
+// the tree's are taken: 2 more allocations and a wait, but 276 bytes a
+// primitive, then 104 and 192 a node, at once, scene included, against 276
+// and 320.
+static vp_status build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32_t n, uint32_t flags, vp_scene* sc,
+                             bool staged) {
     using namespace vp;
     hipStream_t s = ctx->stream;
     const uint32_t nb_sort = cdiv(n, kSortTile);
     const uint32_t nbounds = min(cdiv(n, 256u), 1024u);
     const uint32_t levels = w4_levels(n);
     const size_t records = w4_records(levels);
-    Arena need;
-    BuildTemps(need, n, nb_sort, nbounds, records);
-    ScratchLease scratch;
-    vp_status st = vp_lease_scratch(ctx, need.used, s, scratch);
+    Arena order_need, box_need, tree_need;
+    OrderTemps(order_need, n, nb_sort, nbounds);
+    BoxTemps(box_need, n);
+    TreeTemps(tree_need, records);
+    ScratchLease boxes, first;
+    DevMem w4_32, w4_16;  // of the staged form
+    vp_status st = vp_lease_scratch(ctx, staged ? order_need.used : order_need.used + box_need.used + tree_need.used,
+                                    s, first);
+    if (st == VP_OK && staged) st = vp_lease_scratch(ctx, box_need.used, s, boxes);
     if (st != VP_OK) return st;
-    Arena arena;
-    arena.base = static_cast<char*>(scratch.p);
-    const BuildTemps T(arena, n, nb_sort, nbounds, records);
+    Arena arena, box_arena;
+    arena.base = static_cast<char*>(first.p);
+    box_arena.base = static_cast<char*>(boxes.p);
+    const OrderTemps T(arena, n, nb_sort, nbounds);
+    const BoxTemps B(staged ? box_arena : arena, n);
     // the records are padded to a multiple of the leaf block with zero records
     // (zero inverse scales: no ray enters them), so a walk may hand every slot
     // of a leaf block to the leaf tests
@@ -461,14 +499,14 @@ vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32
         sc->prims = a.take<PrimRecord>(n_slots);
         sc->order = a.take<uint32_t>(n);
         sc->morton = a.take<uint32_t>(n);
-        if (pass == 0) VP_HIP_TRY(vp_device_malloc(ctx, &sc->mem, a.used));
+        if (pass == 0 && (st = scene_malloc(ctx, &sc->mem, a.used)) != VP_OK) return st;
     }
     if (n_slots > n) VP_HIP_TRY(hipMemsetAsync(sc->prims + n, 0, sizeof(PrimRecord) * (n_slots - n), s));
     bool valid = false;
     st = vp_copy_in(ctx, T.in, host_prims, sizeof(vp_primitive), n, vp_primitives_valid, &valid, s);
     if (st != VP_OK || !valid) return st != VP_OK ? st : VP_ERR_INVALID;
     VP_HIP_TRY(hipMemsetAsync(T.depth, 0, sizeof(uint32_t), s));
-    VP_HIP_TRY(hipMemsetAsync(T.sums, 0, 2 * sizeof(double), s));
+    VP_HIP_TRY(hipMemsetAsync(B.sums, 0, 2 * sizeof(double), s));
 
     const uint32_t g = cdiv(n, 256u);
     hipLaunchKernelGGL(k_setup, dim3(g), dim3(256), 0, s, T.in, n, T.rec, T.centers, T.box);
@@ -502,35 +540,68 @@ vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32
         }
         VP_HIP_TRY(hipGetLastError());
     }
-    hipLaunchKernelGGL(k_gather, dim3(g), dim3(256), 0, s, sc->order, n, T.rec, T.box, sc->prims, T.sorted_box);
+    hipLaunchKernelGGL(k_gather, dim3(g), dim3(256), 0, s, sc->order, n, T.rec, T.box, sc->prims, B.sorted_box);
+    TreeTemps R = staged ? TreeTemps{} : TreeTemps(arena, records);
+    if (staged) {
+        const HostCopy out{&depth, T.depth, sizeof(depth)};
+        if ((st = vp_copy_out(ctx, &out, 1, s)) != VP_OK) return st;
+        first.release();
+        st = scene_malloc(ctx, &w4_32.p, sizeof(float4) * kW4RecordF4 * records);
+        if (st == VP_OK && !(flags & VP_SCENE_WALK_F32))
+            st = scene_malloc(ctx, &w4_16.p, static_cast<size_t>(kW4hRecordB) * records);
+        if (st != VP_OK) return st;
+        R.w4 = static_cast<float4*>(w4_32.p);
+        R.w4_half = static_cast<uint4*>(w4_16.p);
+    }
 
     // the walk tree in 32-bit records, bottom up
     const uint32_t bottom = 1u << (2u * (levels - 1u));
-    hipLaunchKernelGGL(k_w4_bottom, dim3(cdiv(bottom, 256u)), dim3(256), 0, s, T.sorted_box, n, levels, T.w4);
+    hipLaunchKernelGGL(k_w4_bottom, dim3(cdiv(bottom, 256u)), dim3(256), 0, s, B.sorted_box, n, levels, R.w4);
     for (uint32_t l = levels - 1u; l-- > 0;)
-        hipLaunchKernelGGL(k_w4_level, dim3(cdiv(1u << (2u * l), 256u)), dim3(256), 0, s, l, T.w4);
+        hipLaunchKernelGGL(k_w4_level, dim3(cdiv(1u << (2u * l), 256u)), dim3(256), 0, s, l, R.w4);
     sc->w4_levels = levels;
     // the 16-bit records, kept when forced or when the leaf boxes' summed
     // surface grows by at most 1/16 (more leaf tests and node visits, against
     // half the bytes per node visit)
     double sums[2] = {0.0, 0.0};
     if (!(flags & VP_SCENE_WALK_F32)) {
-        hipLaunchKernelGGL(k_w4_half, dim3(cdiv(static_cast<uint32_t>(records), 256u)), dim3(256), 0, s, T.w4,
-                           static_cast<uint32_t>(records), w4_level_base(levels - 1u), T.w4_half, T.sums);
+        hipLaunchKernelGGL(k_w4_half, dim3(cdiv(static_cast<uint32_t>(records), 256u)), dim3(256), 0, s, R.w4,
+                           static_cast<uint32_t>(records), w4_level_base(levels - 1u), R.w4_half, B.sums);
     }
     VP_HIP_TRY(hipGetLastError());
-    const HostCopy outs[2] = {{&depth, T.depth, sizeof(depth)}, {sums, T.sums, sizeof(sums)}};
-    st = vp_copy_out(ctx, outs, 2, s);
+    const HostCopy outs[2] = {{sums, B.sums, sizeof(sums)}, {&depth, T.depth, sizeof(depth)}};
+    st = vp_copy_out(ctx, outs, staged ? 1 : 2, s);
     if (st != VP_OK) return st;
     if (!host_tree) sc->depth = depth;
     sc->w4_growth = sums[0] > 0.0 ? sums[1] / sums[0] - 1.0 : 0.0;
     const bool half = !(flags & VP_SCENE_WALK_F32) && ((flags & VP_SCENE_WALK_F16) || sc->w4_growth <= 1.0 / 16.0);
-    const size_t w4_bytes = (half ? static_cast<size_t>(kW4hRecordB) : sizeof(float4) * kW4RecordF4) * records;
-    VP_HIP_TRY(vp_device_malloc(ctx, &sc->w4, w4_bytes));
-    VP_HIP_TRY(hipMemcpyAsync(sc->w4, half ? static_cast<const void*>(T.w4_half) : T.w4, w4_bytes,
-                              hipMemcpyDeviceToDevice, s));
     sc->w4_half = half ? 1u : 0u;
+    if (staged) {
+        DevMem& kept = half ? w4_16 : w4_32;
+        sc->w4 = static_cast<float4*>(kept.p);
+        kept.p = nullptr;
+    } else {
+        const size_t w4_bytes = (half ? static_cast<size_t>(kW4hRecordB) : sizeof(float4) * kW4RecordF4) * records;
+        void* w4 = nullptr;
+        if ((st = scene_malloc(ctx, &w4, w4_bytes)) != VP_OK) return st;
+        sc->w4 = static_cast<float4*>(w4);
+        VP_HIP_TRY(hipMemcpyAsync(w4, half ? static_cast<const void*>(R.w4_half) : R.w4, w4_bytes,
+                                  hipMemcpyDeviceToDevice, s));
+    }
     VP_HIP_TRY(hipStreamSynchronize(s));
-    scratch.done = true;
+    first.done = boxes.done = true;
     return VP_OK;
+}
+
+// Builds scene sc (whose n is set): records, Morton codes and stored order,
+// the order from the radix sort or, with VP_SCENE_BVH_SAH / _MEDIAN in flags,
+// from the host tree, and the walk tree over it.  Temporaries are scratch;
+// the scene owns two allocations.  Returns VP_ERR_INVALID without a message
+// where a primitive is not valid.
+vp_status vp_build_scene(vp_context* ctx, const vp_primitive* host_prims, uint32_t n, uint32_t flags, vp_scene* sc) {
+    const vp_status st = build_scene(ctx, host_prims, n, flags, sc, false);
+    if (st != VP_ERR_OOM) return st;
+    if (sc->mem) (void)hipFree(sc->mem);
+    sc->mem = nullptr;
+    return build_scene(ctx, host_prims, n, flags, sc, true);
 }

@@ -308,7 +308,8 @@ struct ScratchLease {
     ScratchLease() = default;
     ScratchLease(const ScratchLease&) = delete;
     ScratchLease& operator=(const ScratchLease&) = delete;
-    ~ScratchLease();
+    ~ScratchLease() { release(); }
+    void release();
 };
 vp_status vp_lease_scratch(vp_context* ctx, size_t bytes, hipStream_t s, ScratchLease& lease);
 

@@ -116,13 +116,14 @@ hipError_t vp_device_malloc(vp_context* ctx, void** p, size_t bytes) {
     return hipMalloc(p, bytes);
 }
 
-ScratchLease::~ScratchLease() {
+void ScratchLease::release() {
     if (!p) return;
     if (!done) (void)hipStreamSynchronize(stream);
     if (owned)
         (void)hipFree(p);
     else
         ctx->scratch_busy.store(false, std::memory_order_release);
+    p = nullptr;
 }
 
 vp_status vp_lease_scratch(vp_context* ctx, size_t bytes, hipStream_t s, ScratchLease& lease) {

@@ -161,13 +161,36 @@ void kept_scratch() {
     }
 }
 
+// What a scene build takes of the device's memory at once, its scene included,
+// where there is no more: 384 bytes a primitive for the order, then 160 bytes
+// a primitive and 192 a node for the tree.
+void build_memory() {
+    Program prog(1);
+    for (uint32_t n : {65537u, 262144u, 1048577u})
+        for (uint32_t flags : {0u, VP_SCENE_WALK_F32, VP_SCENE_WALK_F16}) {
+            size_t nodes = 0;
+            for (size_t level = 1; 3 * nodes + 1 < n; level *= 4) nodes += level;
+            const size_t order = 384 * size_t(n), tree = 160 * size_t(n) + 192 * nodes;
+            const auto p = primitives(n);
+            vp_scene* sc = nullptr;
+            stub::limit = stub::used + std::max(order, tree) + (size_t(1) << 20);
+            check(vp_scene_create_ex(prog.ctx, p.data(), n, flags, &sc) == VP_OK, "vp_scene_create_ex");
+            uint32_t half = 0;
+            check(vp_scene_walk_info(sc, &half, nullptr) == VP_OK && half == (flags == VP_SCENE_WALK_F32 ? 0u : 1u),
+                  "the tree's form");
+            stub::limit = ~size_t(0);
+            vp_scene_destroy(sc);
+        }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
     const std::map<std::string, void (*)()> checks = {{"failed_copies", failed_copies},
                                                           {"export_device", export_device},
                                                           {"export_without_memory", export_without_memory},
-                                                          {"kept_scratch", kept_scratch}};
+                                                          {"kept_scratch", kept_scratch},
+                                                          {"build_memory", build_memory}};
     check(argc == 2 && checks.count(argv[1]) == 1, "usage: host_check NAME");
     checks.at(argv[1])();
     std::printf("ok %s\n", argv[1]);
