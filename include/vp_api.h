@@ -112,7 +112,8 @@ typedef struct {
 
 /* Launch configuration chosen by the autotuner or forced by the caller. */
 typedef struct {
-    uint32_t block;        /* threads per workgroup (64..1024, multiple of 64) */
+    uint32_t block;        /* threads per workgroup (64, 128, 192 or 256, 0 = 256); where workgroups of 256
+                              fill the device, the megakernel may join up to four of them into one */
     uint32_t blocks_per_cu;/* persistent workgroups per CU (0 = occupancy max) */
     uint32_t active_cap;   /* active-set capacity (entries per path) */
     uint32_t batch_spp;    /* samples per pixel per launch (0 = all) */

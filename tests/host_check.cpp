@@ -183,6 +183,60 @@ void build_memory() {
         }
 }
 
+// Workgroups of 256 threads at the occupancy limit are joined to larger ones
+// where a launch has the paths for it, whether the library, a launch
+// configuration or the autotuner chose them; other shapes are kept.
+void launch_shapes() {
+    Program prog(1000);
+    vp_env* env = nullptr;
+    std::vector<float> texels(4 * 16);
+    check(vp_env_create(prog.ctx, texels.data(), 4, 4, &env) == VP_OK, "vp_env_create");
+    std::vector<float> image(4 * 128 * 128);
+    vp_job job{};
+    job.scene = prog.scene;
+    job.env = env;
+    vp_default_params(&job.params);
+    job.params.width = job.params.height = 128;
+    job.params.spp = 1;
+    job.out_rgba = image.data();
+    unsigned threads = 0, most = 0;  // of the last render kernel, and of any
+    bool slow_256 = false;           // which shapes the autotuner finds slow
+    stub::on_launch = [&](const std::string& name, dim3 block) {
+        if (name.find("k_renderILb0ELb0E") != std::string::npos) {
+            threads = block.x;
+            most = std::max(most, threads);
+        }
+        if (name == "graph" || (name.find("k_renderILb0ELb0E") != std::string::npos && (block.x != 128) == slow_256))
+            std::this_thread::sleep_for(std::chrono::milliseconds(30));
+        return hipSuccess;
+    };
+    const auto rendered = [&](const vp_launch_config* cfg) {
+        check(vp_render_jobs(prog.ctx, &job, 1, cfg, nullptr) == VP_OK, "vp_render_jobs");
+        return threads;
+    };
+    check(rendered(nullptr) == 1024, "the library's shape");
+    for (uint32_t blocks : {0u, 4u, 2u, 1u}) {
+        vp_launch_config cfg{};
+        cfg.block = 256;
+        cfg.blocks_per_cu = blocks;
+        check(rendered(&cfg) == (blocks == 0 || blocks == 4 ? 1024u : 256u), "256 threads");
+        cfg.block = 128;
+        check(rendered(&cfg) == 128, "128 threads");
+        cfg.block = 64;
+        check(rendered(&cfg) == 64, "64 threads");
+    }
+    vp_launch_config best{};
+    most = 0;
+    check(vp_autotune(prog.ctx, &job, 1, &best) == VP_OK && best.block == 256, "the autotuner finds 256 threads");
+    check(most == 1024, "and timed them as they are launched");
+    check(rendered(nullptr) == 1024 && rendered(&best) == 1024, "the tuned shape");
+    slow_256 = true;
+    check(vp_autotune(prog.ctx, &job, 1, &best) == VP_OK && best.block == 128, "the autotuner finds 128 threads");
+    check(rendered(nullptr) == 128 && rendered(&best) == 128, "the tuned shape");
+    stub::on_launch = nullptr;
+    vp_env_destroy(env);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -190,7 +244,8 @@ int main(int argc, char** argv) {
                                                           {"export_device", export_device},
                                                           {"export_without_memory", export_without_memory},
                                                           {"kept_scratch", kept_scratch},
-                                                          {"build_memory", build_memory}};
+                                                          {"build_memory", build_memory},
+                                                          {"launch_shapes", launch_shapes}};
     check(argc == 2 && checks.count(argv[1]) == 1, "usage: host_check NAME");
     checks.at(argv[1])();
     std::printf("ok %s\n", argv[1]);
