@@ -704,6 +704,9 @@ struct MegaQueue {
     __device__ __forceinline__ uint32_t& nc(uint32_t l) const {  // candidates recorded
         return reinterpret_cast<uint32_t*>(acc + 2 * l + 1)[1];
     }
+    __device__ __forceinline__ uint32_t& hits(uint32_t l) const {  // entries counted (measuring build)
+        return reinterpret_cast<uint32_t*>(inv + 3 * (2 * l + 1))[0];
+    }
     __device__ __forceinline__ uint32_t* draw(uint32_t l) const {  // [3] path key (2 words), bounce | direct << 31
         return reinterpret_cast<uint32_t*>(rd + 3 * (2 * l + 1));
     }

@@ -318,7 +318,7 @@ vp_status vp_run_jobs(vp_context* ctx, std::vector<JobRun>& runs, const vp_launc
     // ones, whoever chose them: left out for a tuned context's, its 192x128x2
     // cloud took 4.5 ms against an untuned one's 4.1, a mix of three jobs 7.0
     // against 6.5
-    L.wide = L.pipeline == VP_PIPELINE_MEGAKERNEL && !count && !measure && L.block == 256u &&
+    L.wide = L.pipeline == VP_PIPELINE_MEGAKERNEL && !count && L.block == 256u &&
              L.grid == 4u * ctx->prop.multiProcessorCount;
     const size_t lanes = static_cast<size_t>(L.grid) * L.block;
     vp_status st = VP_OK;

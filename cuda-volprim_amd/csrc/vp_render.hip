@@ -60,15 +60,18 @@ __device__ __forceinline__ uint32_t draw_bounce(const MegaQueue& q, uint32_t l) 
 // The rounds of argmin walks, from nn items on, over the stack and leaf queue
 // of stack and the rays of rays (those of wavefront rays_of of the workgroup).
 // The rays' own wavefront (kOwn) keeps their ends: a ray is walked up to the
-// bound of its minimum, a direct one whole until its depth reaches the limit.
-template <bool kOwn>
+// bound of its minimum, a direct one whole until its depth reaches the limit,
+// and with kMeasure every ray whole, its entries counted.
+template <bool kOwn, bool kMeasure>
 __device__ __forceinline__ void argmin_rounds(const WaveScene& ws, uint32_t* lds, const MegaQueue& stack,
                                               const MegaQueue& rays, uint32_t rays_of, uint64_t lim,
                                               uint32_t* __restrict__ slab, uint32_t cap, uint32_t nn,
                                               uint32_t& rounds) {
     const uint32_t lane = __lane_id();
     const MegaQueue q = rays_with_stack(rays, stack);
-    auto set_tmax = [&]() { q.tmax[2 * lane] = q.acc[2 * lane] < lim ? kTMax : __uint_as_float(q.bound(lane)); };
+    auto set_tmax = [&]() {
+        q.tmax[2 * lane] = kMeasure || q.acc[2 * lane] < lim ? kTMax : __uint_as_float(q.bound(lane));
+    };
     // the first thread of the rays' wavefront, for the owners' candidate buffers
     const uint32_t gbase = blockIdx.x * blockDim.x + rays_of * 64u;
     const uint32_t bs = mega_slab_stride(cap);
@@ -105,6 +108,7 @@ __device__ __forceinline__ void argmin_rounds(const WaveScene& ws, uint32_t* lds
                 const f3 ro = lds_load3(q.ro + 3 * own), rd = lds_load3(q.rd + 3 * ray);
                 const Crossing x = crossing(load_wave_leaf(q, ws, own, prim), ro, rd);
                 if (x.t0 >= 0.0f) {
+                    if (kMeasure) atomicAdd(&q.hits(own), 1u);
                     const uint32_t meta = q.draw(own)[2];
                     if ((meta >> 31) != 0u && x.tau > 0.0f) atomicAdd(&q.acc[ray], tau_fixed(x.tau));
                     if (x.t0 <= __uint_as_float(q.bound(own))) {
@@ -184,12 +188,14 @@ __device__ __forceinline__ void argmin_rounds(const WaveScene& ws, uint32_t* lds
 // its chord, so until then its exit bounds the minimum (bound, which the walk
 // prunes by): without that bound, waiting for 16 flights cost the 10^6 cloud
 // 12 % and the 192x128 cloud 18 % against waiting for 4; with it, nothing.
+// hits receives the ray's entries (kMeasure).
+template <bool kMeasure>
 __device__ __forceinline__ void argmin_walk_shared(bool alive, const WaveScene& ws, uint32_t job, f3 o, f3 d, uint64_t key,
                                                    uint32_t b, bool direct, const uint32_t* act, uint32_t na_path,
                                                    float* act_exit, float ts_set, uint32_t* __restrict__ slab,
                                                    uint32_t cap, const MegaQueue& q, float& ts, uint32_t& nc,
                                                    uint64_t dlimit, uint64_t& dacc, uint32_t& rounds,
-                                                   uint32_t* lds) {
+                                                   uint32_t* lds, uint32_t& hits) {
     const uint32_t lane = __lane_id();
     const uint32_t na = direct ? na_path : 0u;
     lds_store3(q.ro + 3 * lane, o);
@@ -202,6 +208,7 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const WaveScene& 
     q.acc[2 * lane] = 0ull;
     q.ts(lane) = __float_as_uint(direct ? kTMax : ts_set);
     q.nc(lane) = 0u;
+    if (kMeasure) q.hits(lane) = 0u;
     // The origin set (sampling.cuh:356-370) of a path at bounce 0; from then
     // on the last vertex's pass over the set has evaluated it (vertex_members)
     // and ts_set is its minimum.  The wavefront's (member, lane) pairs are
@@ -245,17 +252,19 @@ __device__ __forceinline__ void argmin_walk_shared(bool alive, const WaveScene& 
     wave_sync();
     push_rays(q, ws, q.list, static_cast<uint32_t>(__popcll(am)), nn);
     // a direct ray is walked until its depth reaches the limit
-    argmin_rounds<true>(ws, lds, q, q, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), direct ? dlimit : 0ull, slab,
+    argmin_rounds<true, kMeasure>(ws, lds, q, q, __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), direct ? dlimit : 0ull, slab,
                         cap, nn, rounds);
     const float wmin = __uint_as_float(q.ts(lane));
     ts = wmin < ts_origin ? wmin : ts_origin;
     nc = q.nc(lane);
     dacc = q.acc[2 * lane];
+    if (kMeasure) hits = q.hits(lane);
     wave_sync();
 }
 
 // A wavefront without paths works for the others of its workgroup until none
 // of them has any.
+template <bool kMeasure>
 __device__ __forceinline__ void help_walks(uint32_t* lds, const JobDesc* jobs, uint32_t* __restrict__ slab,
                                            uint32_t cap) {
     const uint32_t lane = __lane_id();
@@ -277,7 +286,7 @@ __device__ __forceinline__ void help_walks(uint32_t* lds, const JobDesc* jobs, u
         ws.one = ws.one && (given & 4u) != 0u;
         uint32_t rounds = 0;
         if ((given & 8u) != 0u)
-            argmin_rounds<false>(ws, lds, q, rq, rays_of, 0ull, slab, cap, n, rounds);
+            argmin_rounds<false, kMeasure>(ws, lds, q, rq, rays_of, 0ull, slab, cap, n, rounds);
         else
             shadow_rounds<false>(ws, lds, q, rq, rays_of, 0u, 0ull, 0ull, n, rounds);
         // the candidates as well as the sums and minima are there first
@@ -608,18 +617,17 @@ __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has
 // The argmin and shadow walks are run by all 64 lanes of a wavefront together,
 // so lanes without a path work on
 // the rays of those that have one: a wavefront with two paths left evaluates
-// their members and leaves 64 at a time and shares out their walks.  Only the
-// timed build does so (kShared); the counting and the measuring build walk
-// each ray by its own lane.
+// their members and leaves 64 at a time and shares out their walks.  The
+// counting build does not (kShared): it walks each ray by its own lane.
 constexpr uint32_t kPathsMin = 4;
 template <bool kCount, bool kMeasure>
-__global__ void __launch_bounds__(kCount || kMeasure ? 256 : 1024)
+__global__ void __launch_bounds__(kCount ? 256 : 1024)
     __attribute__((amdgpu_waves_per_eu(VP_RENDER_WAVES_PER_EU)))
 k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begin,
          const uint64_t* __restrict__ launch_desc, unsigned long long* __restrict__ path_counter,
          uint32_t* __restrict__ slab, uint32_t cap, uint32_t regen_min, uint32_t first_paths,
          uint32_t claim_step, uint32_t rounds_target, unsigned long long* __restrict__ counters) {
-    constexpr bool kShared = !kCount && !kMeasure;
+    constexpr bool kShared = !kCount;
     extern __shared__ __align__(16) uint32_t s_leafq[];  // [blockDim.x][kLeafRow]
     const uint32_t njobs = static_cast<uint32_t>(launch_desc[0]);
     const uint64_t total_paths = launch_desc[1];
@@ -777,14 +785,12 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         bool finish = false;
 
         // At bounce 0 the analytic direct term needs the transmittance of the
-        // camera ray itself, so the timed and the measuring kernel integrate
-        // it during the argmin (the walk then runs over the whole ray instead
-        // of stopping at the running minimum): the same chords, summed in the
-        // same fixed point as transmittance() does.  The counting build
-        // keeps the separate shadow walk, so its counts are per-ray work.
-        const bool direct = !kCount && alive && b == 0;
-        uint64_t dacc = 0;
-        bool dfull = false;
+        // camera ray itself, so it is integrated during the argmin (the walk
+        // then runs over the whole ray instead of stopping at the running
+        // minimum): the same chords, summed in the same fixed point as a
+        // shadow ray's.  The counting build keeps the separate shadow walk, so
+        // its counts are per-ray work.
+        const bool direct = kShared && alive && b == 0;
 
         float ts = kTMax;
         // the origin-set members' exits, kept for the rebuild
@@ -817,8 +823,11 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
                 f3 kd;
                 dlimit = direct_rr(kd).limit();
             }
-            argmin_walk_shared(alive, ws, st.job, o, d, st.key, b, direct, act, na, act_exit, st.ts_set, slab, cap, q, ts, nc,
-                               dlimit, dwalk, rounds, s_leafq);
+            uint32_t hits = 0;
+            argmin_walk_shared<kMeasure>(alive, ws, st.job, o, d, st.key, b, direct, act, na, act_exit, st.ts_set, slab,
+                                         cap, q, ts, nc, dlimit, dwalk, rounds, s_leafq, hits);
+            if constexpr (kMeasure)
+                if (alive) atomicMax(&counters[kCntMaxHits], static_cast<unsigned long long>(hits));
         } else {
             for (uint32_t k = 0; k < na; ++k) {
                 const uint32_t i = act[k * stride];
@@ -827,7 +836,6 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
                 act_exit[k * stride] = x.t1;
                 const float tau = free_flight_tau(prim_uniform(st.key, b, 0u, i));
                 if (tau <= x.tau) ts = minf(ts, origin_flight(pr, o, d, x, tau));
-                if (direct && !dfull) dfull = tau_add(dacc, x.tau);
             }
             const f3 inv = safe_inv(d);
             const bool prune = !kMeasure;
@@ -839,7 +847,6 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
                 const Crossing x = crossing(pr, o, d);
                 if (x.t0 < 0.0f) return true;
                 ++hits;
-                if (direct && !dfull) dfull = tau_add(dacc, x.tau);
                 // beyond the running minimum nothing below can change
                 // (t >= entry > ts)
                 if (x.t0 > ts) return true;
@@ -875,7 +882,6 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
             const ShadowRr drr = direct_rr(kd);
             uint64_t a;
             if constexpr (kCount) a = shadow_depth(sc, o, d, act, na, stride, lq, ev, drr.limit());
-            else if constexpr (kMeasure) a = dfull ? kTauLimitFixed : dacc;
             else a = dwalk;
             const float T = shadow_rr_T(a, drr, depth_T(a));
             st.L = st.L + kd * T;
@@ -900,7 +906,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         auto nee_rr = [&](f3 k, uint32_t ray) { return shadow_rr(max3(k), J.shadow_rr, st.key, b, ray); };
         // rebuild the active set at the scatter point (sampling.cuh:422-458):
         // from the candidates of the argmin walk, or, if they were more than
-        // fit (and in the other builds), by a point query
+        // fit (and in the counting build), by a point query
         const bool listed = kShared && nc <= cap;
         if constexpr (kShared)
             nn = rebuild_shared(vertex && listed, na, nc, st.cur, ts, slab, cap, q, overflow);
@@ -1081,8 +1087,8 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
             if (has_b) lim_b = nee_rr(kb, 1u).limit();
         }
 
-        // the shadow rays' depths (the counting and the measuring build walk
-        // them one by one, so the former's counts are per-ray work)
+        // the shadow rays' depths (the counting build walks them one by one,
+        // so its counts are per-ray work)
         uint64_t acc_a = 0, acc_b = 0;
         if constexpr (kShared) {
             shadow_walks(ws, s_leafq, q, lim_a, lim_b, acc_a, acc_b, rounds);
@@ -1122,7 +1128,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         }
     }
     if (overflow) atomicAdd(&counters[kCntActiveOverflow], static_cast<unsigned long long>(overflow));
-    if constexpr (kShared) help_walks(s_leafq, jobs, slab, cap);
+    if constexpr (kShared) help_walks<kMeasure>(s_leafq, jobs, slab, cap);
 }
 
 // Adaptive sampling, after a batch (the slice of J): the batch's samples of

@@ -185,7 +185,8 @@ void build_memory() {
 
 // Workgroups of 256 threads at the occupancy limit are joined to larger ones
 // where a launch has the paths for it, whether the library, a launch
-// configuration or the autotuner chose them; other shapes are kept.
+// configuration or the autotuner chose them, in measuring launches as well;
+// other shapes are kept.
 void launch_shapes() {
     Program prog(1000);
     vp_env* env = nullptr;
@@ -202,7 +203,7 @@ void launch_shapes() {
     unsigned threads = 0, most = 0;  // of the last render kernel, and of any
     bool slow_256 = false;           // which shapes the autotuner finds slow
     stub::on_launch = [&](const std::string& name, dim3 block) {
-        if (name.find("k_renderILb0ELb0E") != std::string::npos) {
+        if (name.find("k_renderILb0E") != std::string::npos) {
             threads = block.x;
             most = std::max(most, threads);
         }
@@ -215,6 +216,9 @@ void launch_shapes() {
         return threads;
     };
     check(rendered(nullptr) == 1024, "the library's shape");
+    job.params.measure_caps = 1;
+    check(rendered(nullptr) == 1024, "a measuring launch's shape");
+    job.params.measure_caps = 0;
     for (uint32_t blocks : {0u, 4u, 2u, 1u}) {
         vp_launch_config cfg{};
         cfg.block = 256;
