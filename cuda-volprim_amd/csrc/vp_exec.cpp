@@ -430,7 +430,8 @@ vp_status vp_run_jobs(vp_context* ctx, std::vector<JobRun>& runs, const vp_launc
     for (size_t i = 0; i < runs.size(); ++i) {
         const JobRun& r = runs[i];
         const size_t npix = static_cast<size_t>(r.desc.width) * r.desc.height;
-        if (r.host_out) outs.push_back({r.host_out, r.desc.mean, npix * sizeof(float4)});
+        const bool joins = i > 0 && runs[i - 1].host_out && !runs[i - 1].mean && !r.mean;  // both images in scratch
+        if (r.host_out) outs.push_back({r.host_out, r.desc.mean, npix * sizeof(float4), joins});
         if (r.desc.adapt_state == nullptr) continue;
         states[i].resize(npix);
         outs.push_back({states[i].data(), r.desc.adapt_state, npix * sizeof(uint32_t)});

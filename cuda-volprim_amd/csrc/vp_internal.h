@@ -319,6 +319,8 @@ struct HostCopy {
     void* dst;
     const void* src;
     size_t bytes;
+    bool joins = false;  // src lies in the allocation of the copy before: one within 256 bytes of that
+                         // copy's end may leave the device in one copy with it
 };
 vp_status vp_copy_out(vp_context* ctx, const HostCopy* copies, size_t n, hipStream_t s);
 // Copies count elements to the device and runs check over them on the way;

@@ -53,7 +53,7 @@ bool ordinary(const void* p) {
 template <typename F>
 void on_threads(int device, size_t chunks, F&& work) {
     std::vector<std::thread> pool;
-    const size_t extra = std::min<size_t>(kStageThreads, chunks / 2) - 1;
+    const size_t extra = std::max<size_t>(1, std::min<size_t>(kStageThreads, chunks / 2)) - 1;
     try {
         pool.reserve(extra);
         for (size_t k = 0; k < extra; ++k)
@@ -153,71 +153,89 @@ vp_status vp_lease_scratch(vp_context* ctx, size_t bytes, hipStream_t s, Scratch
 vp_status vp_copy_out(vp_context* ctx, const HostCopy* copies, size_t n, hipStream_t s) {
     std::lock_guard<std::mutex> lk(ctx->mu);
     WaitOnFailure wait{s};
-    struct Chunk {
+    // what leaves the device in one copy: a part, a slot's worth of a longer
+    // one, or several short ones that lie one after the other
+    struct Piece {
         char* dst;
-        const char* src;
-        size_t bytes;
+        size_t offset, bytes;  // in its run
     };
-    std::vector<Chunk> parts;
-    size_t total = 0;
+    struct Run {
+        const char* src;
+        size_t bytes, first, end;  // pieces
+    };
+    std::vector<Piece> pieces;
+    std::vector<Run> runs;
     for (size_t i = 0; i < n; ++i) {
+        const char* src = static_cast<const char*>(copies[i].src);
         if (copies[i].bytes == 0) continue;
         if (!ordinary(copies[i].dst)) {
-            VP_HIP_TRY(hipMemcpyAsync(copies[i].dst, copies[i].src, copies[i].bytes, hipMemcpyDeviceToHost, s));
+            VP_HIP_TRY(hipMemcpyAsync(copies[i].dst, src, copies[i].bytes, hipMemcpyDeviceToHost, s));
             continue;
         }
-        parts.push_back({static_cast<char*>(copies[i].dst), static_cast<const char*>(copies[i].src), copies[i].bytes});
-        total += (copies[i].bytes + 15) / 16 * 16;
+        for (size_t o = 0; o < copies[i].bytes; o += kStageSlot) {
+            const size_t bytes = std::min(kStageSlot, copies[i].bytes - o);
+            const bool joins = o == 0 && copies[i].joins && !runs.empty() && src >= runs.back().src + runs.back().bytes &&
+                               src < runs.back().src + runs.back().bytes + 256 &&
+                               src + bytes <= runs.back().src + kStageSlot;
+            if (!joins) runs.push_back({src + o, 0, pieces.size(), pieces.size()});
+            Run& r = runs.back();
+            pieces.push_back({static_cast<char*>(copies[i].dst) + o, static_cast<size_t>(src + o - r.src), bytes});
+            r.bytes = pieces.back().offset + bytes;
+            ++r.end;
+        }
     }
+    size_t total = 0;
+    for (const Run& r : runs) total += (r.bytes + 15) / 16 * 16;
     if (!ensure_stage(ctx, total <= kStageSlot ? 1u : kStageSlots)) {
         (void)hipGetLastError();
-        for (const Chunk& c : parts) VP_HIP_TRY(hipMemcpyAsync(c.dst, c.src, c.bytes, hipMemcpyDeviceToHost, s));
+        for (const Run& r : runs)
+            for (size_t k = r.first; k < r.end; ++k)
+                VP_HIP_TRY(hipMemcpyAsync(pieces[k].dst, r.src + pieces[k].offset, pieces[k].bytes, hipMemcpyDeviceToHost,
+                                          s));
         VP_HIP_TRY(hipStreamSynchronize(s));
         wait.armed = false;
         return VP_OK;
     }
+    const auto deliver = [&](const Run& r, const char* from) {
+        for (size_t k = r.first; k < r.end; ++k) std::memcpy(pieces[k].dst, from + pieces[k].offset, pieces[k].bytes);
+    };
     if (total <= kStageSlot) {
         // everything in one slot, written there by a kernel: one launch and
         // one wait (a copy through the runtime takes two of its launches)
         char* at = ctx->stage;
-        for (size_t i = 0; i < parts.size(); i += kCopyParts) {
+        for (size_t i = 0; i < runs.size(); i += kCopyParts) {
             CopyParts cp{};
-            for (uint32_t k = 0; k < kCopyParts && i + k < parts.size(); ++k) {
-                cp.src[k] = reinterpret_cast<const uint32_t*>(parts[i + k].src);
+            for (uint32_t k = 0; k < kCopyParts && i + k < runs.size(); ++k) {
+                cp.src[k] = reinterpret_cast<const uint32_t*>(runs[i + k].src);
                 cp.dst[k] = reinterpret_cast<uint32_t*>(at);
-                cp.words[k] = static_cast<uint32_t>(parts[i + k].bytes / 4);
-                at += (parts[i + k].bytes + 15) / 16 * 16;
+                cp.words[k] = static_cast<uint32_t>(runs[i + k].bytes / 4);
+                at += (runs[i + k].bytes + 15) / 16 * 16;
             }
             VP_HIP_TRY(vp_launch_copy_parts(cp, s));
         }
         VP_HIP_TRY(hipStreamSynchronize(s));
         wait.armed = false;
         at = ctx->stage;
-        for (const Chunk& c : parts) {
-            std::memcpy(c.dst, at, c.bytes);
-            at += (c.bytes + 15) / 16 * 16;
+        for (const Run& r : runs) {
+            deliver(r, at);
+            at += (r.bytes + 15) / 16 * 16;
         }
         return VP_OK;
     }
-    std::vector<Chunk> chunks;
-    for (const Chunk& c : parts)
-        for (size_t o = 0; o < c.bytes; o += kStageSlot)
-            chunks.push_back({c.dst + o, c.src + o, std::min(kStageSlot, c.bytes - o)});
     Slots S;
     auto queue = [&](size_t c) {
         char* slot = ctx->stage + (c % kStageSlots) * kStageSlot;
-        if (S.good()) S.note(hipMemcpyAsync(slot, chunks[c].src, chunks[c].bytes, hipMemcpyDeviceToHost, s));
+        if (S.good()) S.note(hipMemcpyAsync(slot, runs[c].src, runs[c].bytes, hipMemcpyDeviceToHost, s));
         if (S.good()) S.note(hipEventRecord(ctx->stage_ev[c % kStageSlots], s));
         S.set_queued(c);
     };
-    for (size_t c = 0; c < kStageSlots && c < chunks.size(); ++c) queue(c);
-    on_threads(ctx->device, chunks.size(), [&] {
-        for (size_t c; (c = S.next.fetch_add(1)) < chunks.size();) {
+    for (size_t c = 0; c < kStageSlots && c < runs.size(); ++c) queue(c);
+    on_threads(ctx->device, runs.size(), [&] {
+        for (size_t c; (c = S.next.fetch_add(1)) < runs.size();) {
             S.wait_queued(c);
             if (S.good()) S.note(hipEventSynchronize(ctx->stage_ev[c % kStageSlots]));
-            if (S.good())
-                std::memcpy(chunks[c].dst, ctx->stage + (c % kStageSlots) * kStageSlot, chunks[c].bytes);
-            if (c + kStageSlots < chunks.size()) queue(c + kStageSlots);
+            if (S.good()) deliver(runs[c], ctx->stage + (c % kStageSlots) * kStageSlot);
+            if (c + kStageSlots < runs.size()) queue(c + kStageSlots);
         }
     });
     VP_HIP_TRY(static_cast<hipError_t>(S.err.load()));

@@ -241,6 +241,59 @@ void launch_shapes() {
     vp_env_destroy(env);
 }
 
+// The images of a batch leave the device in copies of a slot each, not one by
+// one, and arrive where they belong, whatever their sizes and whether one slot
+// holds them all.
+void batch_images() {
+    Program prog(1000);
+    vp_env* env = nullptr;
+    std::vector<float> texels(4 * 16);
+    check(vp_env_create(prog.ctx, texels.data(), 4, 4, &env) == VP_OK, "vp_env_create");
+    const struct {
+        uint32_t jobs, w, h, most_copies;
+    } batches[] = {{200, 63, 65, 14}, {200, 64, 64, 14}, {300, 16, 16, 3}, {3, 300, 300, 8}, {100, 17, 19, 3},
+                   {1, 1024, 256, 6}, {5, 256, 256, 6}};
+    for (const auto& b : batches) {
+        const size_t pixels = size_t(b.w) * b.h;
+        std::vector<std::vector<float>> images(b.jobs, std::vector<float>(4 * pixels));
+        std::vector<vp_job> jobs(b.jobs);
+        for (uint32_t i = 0; i < b.jobs; ++i) {
+            jobs[i] = vp_job{};
+            jobs[i].scene = prog.scene;
+            jobs[i].env = env;
+            vp_default_params(&jobs[i].params);
+            jobs[i].params.width = b.w;
+            jobs[i].params.height = b.h;
+            jobs[i].params.spp = 1;
+            jobs[i].out_rgba = images[i].data();
+        }
+        // the scratch of a batch of this size is the context's largest block
+        // from its first call on, or an earlier batch's
+        size_t copies = 0;
+        stub::on_copy = [&] { return ++copies, hipSuccess; };
+        stub::on_launch = [&](const std::string& name, dim3) {
+            copies += name.find("k_copy_parts") != std::string::npos ? 1 : 0;
+            return hipSuccess;
+        };
+        check(vp_render_jobs(prog.ctx, jobs.data(), b.jobs, nullptr, nullptr) == VP_OK, "vp_render_jobs");
+        check(copies <= b.most_copies, "the copies of a batch");
+        stub::on_copy = nullptr;
+        stub::on_launch = nullptr;
+        // scratch: 64 bytes a pixel of sums, then the images, parts of 256 bytes
+        const size_t sums = (64 * pixels * b.jobs + 255) / 256 * 256, image = (16 * pixels + 255) / 256 * 256;
+        char* scratch = nullptr;
+        for (const auto& m : stub::device_mem)
+            if (m.second >= sums + image * b.jobs && m.second < (size_t(256) << 20)) scratch = static_cast<char*>(m.first);
+        check(scratch != nullptr, "the scratch");
+        float* words = reinterpret_cast<float*>(scratch + sums);
+        for (size_t i = 0; i < image / 4 * b.jobs; ++i) words[i] = float(i % 16777213u);
+        check(vp_render_jobs(prog.ctx, jobs.data(), b.jobs, nullptr, nullptr) == VP_OK, "vp_render_jobs");
+        for (uint32_t i = 0; i < b.jobs; ++i)
+            check(std::memcmp(images[i].data(), words + image / 4 * i, 16 * pixels) == 0, "an image of the batch");
+    }
+    vp_env_destroy(env);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -249,7 +302,8 @@ int main(int argc, char** argv) {
                                                           {"export_without_memory", export_without_memory},
                                                           {"kept_scratch", kept_scratch},
                                                           {"build_memory", build_memory},
-                                                          {"launch_shapes", launch_shapes}};
+                                                          {"launch_shapes", launch_shapes},
+                                                          {"batch_images", batch_images}};
     check(argc == 2 && checks.count(argv[1]) == 1, "usage: host_check NAME");
     checks.at(argv[1])();
     std::printf("ok %s\n", argv[1]);
