@@ -1,6 +1,7 @@
 // vp_device.h — device building blocks shared by the render kernels:
-// record loads, the stackless BVH walks (plain and with the LDS leaf queue),
-// fixed-point optical depth, shadow-ray transmittance, event counters and
+// record loads, the stackless walks of single lanes (plain and with a leaf
+// queue in LDS), the wave-wide walks of the megakernel (a node stack in LDS) and
+// the help between wavefronts, fixed-point optical depth, event counters and
 // the job lookup.  Included by vp_render.hip (megakernel, test kernels) and
 // vp_wavefront.hip (wavefront pipeline).
 #pragma once
@@ -330,10 +331,10 @@ __device__ __forceinline__ void walk_point(const SceneView& s, f3 x, uint32_t& v
 constexpr uint32_t kLeafQ = VP_LEAF_Q;
 constexpr uint32_t kLeafRow = kLeafQ + 1;
 
-// Wave-shared leaf queue.  The LDS of a wavefront holds either its threads'
-// queue rows or one queue for the whole wavefront (the two are used at
-// different times): node phases append crossed leaves with their owner lane,
-// and in the leaf phase every active lane takes the next entry, whichever
+// Wave-shared leaf queue of the wavefront pipeline.  The LDS of a wavefront
+// holds either its threads' queue rows or one queue for the whole wavefront
+// (in different kernels): node phases append crossed leaves with their owner
+// lane, and in the leaf phase every active lane takes the next entry, whichever
 // lane's ray it belongs to.  Leaf work then runs at full width however
 // unevenly the lanes' walks found leaves.  Per-ray results are combined with
 // LDS atomics whose outcome does not depend on order (fixed-point sums, and
@@ -352,32 +353,23 @@ constexpr uint32_t kWaveQ = VP_WAVE_Q;
 #ifndef VP_SHARED_END_DIV
 #define VP_SHARED_END_DIV 4u
 #endif
-// Rays are numbered per wavefront: ray k of a one-ray-per-lane walk belongs
-// to lane k; the MIS shadow rays of lane l are rays 2l and 2l + 1.
+// A lane walks one ray; queued leaves belong to the lane of their ray.
 struct WaveQueue {
     uint32_t* prim;                // [kWaveQ] queued leaf
-    float* tj;                     // [kWaveQ] entry distances of the leaves that passed the entry test
-    uint8_t* owner;                // [kWaveQ] the ray each leaf belongs to
+    uint8_t* owner;                // [kWaveQ] the lane each leaf belongs to
     float* ro;                     // [64 * 3] ray origin of each lane
     const PrimRecord** prims;      // [64] primitive array of each lane's scene (lanes of one
                                    //      wavefront may run jobs over different scenes)
-    float* rd;                     // [128 * 3] ray directions
-    unsigned long long* acc;       // [128] fixed-point optical depth of each ray
-    // MIS shadow-ray pool
-    const float4** nodes;          // [64] walk-tree records of each lane's scene
-    uint32_t* nn;                  // [64] its level count (or, in the wavefront argmin
-                                   //      kernel, the pool slot of each lane's path)
-    uint8_t* list;                 // [128] the rays still to be walked
-    uint32_t* lim;                 // [128] depth at which each ray's walk may stop, >> 16 (shadow roulette)
-    // argmin walks (one ray per lane); they lie over rd[64..128) and acc[64..128)
-    unsigned long long* key;       // [64] path key of each lane
+    float* rd;                     // [64 * 3] ray directions
+    unsigned long long* acc;       // [64] fixed-point optical depth of each ray (shadow walks), or
+    unsigned long long* key;       // [64] path key of each lane (argmin walks, as the rest)
     uint32_t* ts;                  // [64] running minimum of each lane's argmin, as float bits
     uint32_t* nc;                  // [64] candidates recorded for each lane's argmin
-    uint32_t* meta;                // [64] bounce | direct-term flag << 31
+    uint32_t* meta;                // [64] bounce
+    uint32_t* slot;                // [64] pool slot of each lane's path
 };
-constexpr uint32_t kWaveQueueBytes = kWaveQ * 9 + 64 * 12 + 64 * 8 + 128 * 12 + 128 * 8 + 64 * 8 + 64 * 4 + 128 + 128 * 4;
+constexpr uint32_t kWaveQueueBytes = kWaveQ * 5 + 64 * (12 + 8 + 12 + 8 + 4 * 4);
 static_assert(kWaveQ % 8 == 0, "queue arrays keep the per-lane arrays 8-byte aligned");
-static_assert(64 * (8 + 4) <= 64 * 12 && 64 * (4 + 4) <= 64 * 8, "argmin arrays fit over the upper rays");
 // LDS bytes per wavefront: the larger of the two uses, in 16-byte units
 constexpr uint32_t kWaveBytes =
     ((64 * kLeafRow * 4 > kWaveQueueBytes ? 64 * kLeafRow * 4 : kWaveQueueBytes) + 15) / 16 * 16;
@@ -387,20 +379,15 @@ __device__ __forceinline__ WaveQueue wave_queue(uint32_t* lds) {
     uint8_t* base = reinterpret_cast<uint8_t*>(lds) + (threadIdx.x >> 6) * kWaveBytes;
     WaveQueue q;
     q.prim = reinterpret_cast<uint32_t*>(base);
-    q.tj = reinterpret_cast<float*>(base + 4 * kWaveQ);
-    q.owner = base + 8 * kWaveQ;
-    q.ro = reinterpret_cast<float*>(base + 9 * kWaveQ);
+    q.owner = base + 4 * kWaveQ;
+    q.ro = reinterpret_cast<float*>(base + 5 * kWaveQ);
     q.prims = reinterpret_cast<const PrimRecord**>(q.ro + 64 * 3);
     q.rd = reinterpret_cast<float*>(q.prims + 64);
-    q.acc = reinterpret_cast<unsigned long long*>(q.rd + 128 * 3);
-    q.nodes = reinterpret_cast<const float4**>(q.acc + 128);
-    q.nn = reinterpret_cast<uint32_t*>(q.nodes + 64);
-    q.list = reinterpret_cast<uint8_t*>(q.nn + 64);
-    q.lim = reinterpret_cast<uint32_t*>(q.list + 128);
-    q.key = reinterpret_cast<unsigned long long*>(q.rd + 64 * 3);
+    q.acc = q.key = reinterpret_cast<unsigned long long*>(q.rd + 64 * 3);
     q.ts = reinterpret_cast<uint32_t*>(q.key + 64);
-    q.nc = reinterpret_cast<uint32_t*>(q.acc + 64);
+    q.nc = q.ts + 64;
     q.meta = q.nc + 64;
+    q.slot = q.meta + 64;
     return q;
 }
 
@@ -624,12 +611,6 @@ __device__ uint64_t shadow_depth(const SceneView& s, f3 o, f3 d, const uint32_t*
     ev.add(kCntLeafTests, leaves);
     ev.add(kCntShHit, sh);
     return acc;
-}
-
-template <bool kCount>
-__device__ float transmittance(const SceneView& s, f3 o, f3 d, const uint32_t* act, uint32_t na, uint32_t stride,
-                               const LeafQueue& lq, Ev<kCount>& ev) {
-    return depth_T(shadow_depth(s, o, d, act, na, stride, lq, ev, kTauLimitFixed));
 }
 
 // one chord in fixed point, as tau_add adds it; a chord of tau >= 88 alone
@@ -1080,7 +1061,7 @@ __device__ __forceinline__ void shadow_rounds(const WaveScene& ws, uint32_t* lds
 // q.rd and q.acc hold the rays' origins, jobs, directions and the depths of
 // their origin sets.  Each ray's chords are summed in fixed point in LDS (a
 // ray is saturated once its sum reaches the tau = 88 limit, in whatever order
-// the chords arrive), so Ta and Tb equal two transmittance() calls bit for
+// the chords arrive), so the depths equal those of shadow_depth() bit for
 // bit.
 // Each ray's walk may stop once its depth reaches its limit (lim_a, lim_b:
 // the tau = 88 saturation, or a shadow-roulette threshold); a limit of 0 is a

@@ -628,7 +628,7 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
          uint32_t* __restrict__ slab, uint32_t cap, uint32_t regen_min, uint32_t first_paths,
          uint32_t claim_step, uint32_t rounds_target, unsigned long long* __restrict__ counters) {
     constexpr bool kShared = !kCount;
-    extern __shared__ __align__(16) uint32_t s_leafq[];  // [blockDim.x][kLeafRow]
+    extern __shared__ __align__(16) uint32_t s_leafq[];  // a queue of kMegaBytes to a wavefront
     const uint32_t njobs = static_cast<uint32_t>(launch_desc[0]);
     const uint64_t total_paths = launch_desc[1];
     const uint64_t path_lo = launch_desc[2];
@@ -1405,10 +1405,9 @@ hipError_t vp_launch_render(const RenderLaunch& L, const JobDesc* jobs, const ui
 }
 
 // One step of the persistent renderer over the job table in ctx->jobs_dev:
-// reset the path counter (a fill kernel, so the sequence can be captured in a
-// graph), trace every path of every job slice, resolve the means.  Job count
-// and path total come from ctx->launch_desc, the path counters from
-// vp_launch_begin.
+// trace every path of every job slice, resolve the means.  The table, its job
+// count and path total (ctx->launch_desc) and the zeroed path counters are
+// vp_launch_begin's.
 hipError_t vp_launch_step(vp_context* ctx, const RenderLaunch& L, uint32_t max_jobs, uint32_t max_npix,
                           hipStream_t s) {
     const hipError_t e = vp_launch_render(L, ctx->jobs_dev, ctx->job_begin_dev, ctx->launch_desc, ctx->path_counter,

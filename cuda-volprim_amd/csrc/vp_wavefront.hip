@@ -242,7 +242,7 @@ __device__ __forceinline__ uint32_t wave_fetch(unsigned int* head, bool want, ui
 __global__ void VP_WF_LB k_wf_extend(const JobDesc* __restrict__ jobs, WfPool w, uint32_t par, uint32_t fetch_min) {
     extern __shared__ __align__(16) uint32_t s_leafq[];
     const WaveQueue wq = wave_queue(s_leafq);
-    uint32_t* slot = wq.nn;  // the pool slot of each lane's path
+    uint32_t* slot = wq.slot;  // the pool slot of each lane's path
     const uint32_t lane = __lane_id();
     unsigned int* qc = qcs(w, par);
     const uint32_t n = qc[0];
