@@ -416,8 +416,14 @@ vp_status vp_run_jobs(vp_context* ctx, std::vector<JobRun>& runs, const vp_launc
             r.issued += J.s_count;
             ++k;
         }
+        // a joined workgroup of 16 wavefronts needs a compute unit to itself,
+        // and a busy server's launches leave none: beside requests that arrived
+        // at 1.2 times what the device renders, a 64x64x2 image waited for the
+        // end of all 40 of them (920 ms), in workgroups of 4 wavefronts 106 ms
+        RenderLaunch step = L;
+        step.wide = L.wide && !vp_device_serves(ctx->device);
         VP_HIP_TRY(hipEventRecord(ctx->ev0, s));
-        st = vp_run_step(ctx, vp_size_launch(L, total), k, total, max_jobs, max_npix, launches == 0,
+        st = vp_run_step(ctx, vp_size_launch(step, total), k, total, max_jobs, max_npix, launches == 0,
                          runs[0].desc.accum, acc_words, s);
         if (st != VP_OK) return st;
         VP_HIP_TRY(hipEventRecord(ctx->ev1, s));

@@ -396,6 +396,8 @@ vp_status vp_run_jobs(vp_context* ctx, std::vector<JobRun>& runs, const vp_launc
                       int count, int measure, hipStream_t s, double* kernel_ms, uint64_t* paths,
                       unsigned long long* counters);
 void vp_fill_stats(const unsigned long long* counters, vp_render_stats* stats);
+// Whether a server has requests in flight on the device (vp_server.cpp).
+bool vp_device_serves(int device);
 vp::JobDesc vp_make_job(const vp_scene* sc, const vp_env* env, const vp_camera* cam, const vp_render_params* p);
 vp_status vp_check_params(const vp_render_params* p);
 // Whether all count primitives pass the validation of vp_scene_create.

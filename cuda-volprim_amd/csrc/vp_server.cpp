@@ -125,6 +125,11 @@ struct vp_server {
 
 namespace {
 
+// Requests submitted and not finished on each device, over all its servers
+// (devices that share an entry only see more of them).
+std::atomic<uint32_t> g_requests[64];
+std::atomic<uint32_t>& requests_on(int device) { return g_requests[static_cast<uint32_t>(device) % 64u]; }
+
 void release_request(vp_server* S, Request* r) {
     if (r->accum) (void)hipFreeAsync(r->accum, S->side);
     r->accum = nullptr;
@@ -145,6 +150,7 @@ void finish_request(vp_server* S, Request* r, vp_status st) {
         S->samples += r->paths;
     }
     S->inflight.erase(std::find(S->inflight.begin(), S->inflight.end(), r));
+    requests_on(S->ctx->device).fetch_sub(1u, std::memory_order_relaxed);
     S->cv_done.notify_all();
 }
 
@@ -412,6 +418,8 @@ void free_server(vp_server* S) {
 
 }  // namespace
 
+bool vp_device_serves(int device) { return requests_on(device).load(std::memory_order_relaxed) != 0u; }
+
 extern "C" {
 
 vp_status vp_server_create(vp_context* ctx, const vp_server_config* cfg, vp_server** out) {
@@ -522,6 +530,7 @@ vp_status vp_server_submit(vp_server* S, const vp_job* job, uint64_t* ticket) {
         r->ticket = S->next_ticket++;
         S->by_ticket[r->ticket] = r;
         S->pending.push_back(r);
+        requests_on(S->ctx->device).fetch_add(1u, std::memory_order_relaxed);
     }
     S->cv.notify_one();
     *ticket = r->ticket;
@@ -576,6 +585,7 @@ vp_status vp_server_destroy(vp_server* S) {
         for (Request* r : S->pending) {
             r->status = VP_ERR_STATE;
             r->done = true;
+            requests_on(S->ctx->device).fetch_sub(1u, std::memory_order_relaxed);
         }
         S->pending.clear();
     }

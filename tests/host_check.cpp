@@ -241,6 +241,63 @@ void launch_shapes() {
     vp_env_destroy(env);
 }
 
+// A workgroup of 1024 threads needs a compute unit to itself, and those of
+// 256 that a busy server launches one after the other leave none: beside
+// requests in flight on its device, a render's workgroups are not joined.
+void render_beside_server() {
+    Program prog(1000), other(1000);
+    vp_env* env = nullptr;
+    std::vector<float> texels(4 * 16);
+    check(vp_env_create(prog.ctx, texels.data(), 4, 4, &env) == VP_OK, "vp_env_create");
+    std::vector<float> image(4 * 128 * 128), served(4 * 128 * 128);
+    vp_job job{};
+    job.scene = prog.scene;
+    job.env = env;
+    vp_default_params(&job.params);
+    job.params.width = job.params.height = 128;
+    job.params.spp = 1;
+    job.out_rgba = image.data();
+    const auto here = std::this_thread::get_id();
+    unsigned threads = 0;       // of this thread's last render kernel
+    bool server_runs = false;
+    stub::on_launch = [&](const std::string& name, dim3 block) {
+        if (name.find("k_renderILb0E") != std::string::npos) {
+            if (std::this_thread::get_id() == here) threads = block.x;
+            else server_runs = true;
+        }
+        return hipSuccess;
+    };
+    const auto rendered = [&](vp_context* ctx) {
+        check(vp_render_jobs(ctx, &job, 1, nullptr, nullptr) == VP_OK, "vp_render_jobs");
+        return threads;
+    };
+    vp_server* srv = nullptr;
+    check(vp_server_create(prog.ctx, nullptr, &srv) == VP_OK, "vp_server_create");
+    check(rendered(prog.ctx) == 1024 && rendered(other.ctx) == 1024, "beside an idle server");
+    vp_job request = job;
+    request.out_rgba = served.data();
+    uint64_t ticket = 0;
+    check(vp_server_submit(srv, &request, &ticket) == VP_OK, "vp_server_submit");
+    check(rendered(prog.ctx) == 256 && rendered(other.ctx) == 256, "beside a request");
+    for (bool ready = false; !ready; std::this_thread::yield()) {
+        STUB_LOCK;
+        ready = server_runs;
+    }
+    check(rendered(prog.ctx) == 256 && rendered(other.ctx) == 256, "beside a running request");
+    // its paths finish: the table of finished paths (16384 entries)
+    {
+        STUB_LOCK;
+        stub::drain();
+        for (const auto& m : stub::device_mem)
+            if (m.second == 16384 * sizeof(uint64_t)) std::memset(m.first, 0x7f, m.second);
+    }
+    check(vp_server_drain(srv) == VP_OK, "vp_server_drain");
+    check(rendered(prog.ctx) == 1024 && rendered(other.ctx) == 1024, "after the request");
+    stub::on_launch = nullptr;
+    check(vp_server_destroy(srv) == VP_OK, "vp_server_destroy");
+    vp_env_destroy(env);
+}
+
 // The images of a batch leave the device in copies of a slot each, not one by
 // one, and arrive where they belong, whatever their sizes and whether one slot
 // holds them all.
@@ -303,7 +360,8 @@ int main(int argc, char** argv) {
                                                           {"kept_scratch", kept_scratch},
                                                           {"build_memory", build_memory},
                                                           {"launch_shapes", launch_shapes},
-                                                          {"batch_images", batch_images}};
+                                                          {"batch_images", batch_images},
+                                                          {"render_beside_server", render_beside_server}};
     check(argc == 2 && checks.count(argv[1]) == 1, "usage: host_check NAME");
     checks.at(argv[1])();
     std::printf("ok %s\n", argv[1]);
