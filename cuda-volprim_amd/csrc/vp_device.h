@@ -897,8 +897,13 @@ __device__ __forceinline__ void walk_nodes(const MegaQueue& q, const WaveScene& 
 // instead of its root, a lane per node: the top of the tree is a chain of
 // steps with little in them, two of the six or seven that such a walk takes
 // (64x64x2 scattering 1.92 -> 1.77 ms, 157x83x3 of 97 Gaussians 0.58 -> 0.54).
-// In deeper trees the top is less of the chain, and a walk that prunes or
-// saturates loses by opening all of it at once (torus +2 %, clouds +4 %).
+// In deeper trees the top is less of the chain, and in larger images a walk that
+// prunes or saturates loses by opening all of it at once (512x512 torus +2 %,
+// 192x128x2 cloud of 200000 and 10^6 cloud +4 %).  With against without, at 64x64x2:
+// scattering of 100, 1000, 4096 (4 to 6 levels) 0.88, 0.87, 0.89, of 8000 and
+// 16384 (7) 0.91 and 0.92, and it would be 0.94, 0.97 and 0.96 for 30000, 65536 (8)
+// and 150000 (9); at 96x96x1 torus and cloud of 10000 (7) 0.89 and 0.91, and 0.93
+// to 0.95 for 40000 and 100000 (8 and 9).
 __device__ __forceinline__ void push_rays(const MegaQueue& q, const WaveScene& ws, const uint8_t* list, uint32_t k,
                                           uint32_t& nn) {
     const uint32_t lane = __lane_id();

@@ -194,6 +194,12 @@ RenderLaunch vp_resolve_launch(vp_context* ctx, const vp_launch_config* cfg, uin
 // others near the end, and cost width in the middle (128 against 256: 8 batched
 // requests 12.3 -> 11.8 ms, 128x128 adaptive 17.6 -> 16.9, torus the same, but
 // 256x256x24 scattering 22.9 -> 24.6, 10^6 cloud 163 -> 172; 384: batched 13.3).
+// Where the line lies, 128 against 256 rounds at that many paths to a wavefront:
+// batches of small jobs 0.90, 0.93, 0.95 and 0.95 of the time at 66, 88, 116 and
+// 125, but 1.05, 1.02 and 1.04 at 381, 431 and 499; one 256x256 image of the
+// scattering scene 0.99, 1.0, 1.02, 1.04 and 1.05 at 32, 64, 96, 128 and 160, of
+// the torus 0.97, 1.01, 1.03, 1.05 and 1.04, of a cloud 0.88, 1.02 and 1.09 at 32,
+// 64 and 128.  So below 128 batches gain more than single images lose.
 // The wavefronts of a workgroup help each other at the end (help_walks in
 // vp_render.hip), so workgroups are as large as they can be, 16 wavefronts, once
 // there are 32 paths to a compute unit, and smaller below, where a launch's paths

@@ -116,7 +116,8 @@ extern "C" vp_status vp_render_device_noalloc(vp_context* ctx, vp_scene* sc, vp_
     if (ctx->noalloc_scratch == nullptr) return fail(VP_ERR_HIP, "vp_render_device_noalloc: no scratch address");
     const uint32_t cap = params->active_cap ? params->active_cap : 128u;
     // the megakernel, at the context's tuned (or default) shape, with no
-    // more lanes than the slab holds at this capacity
+    // more lanes than the slab holds at this capacity (its workgroups are not
+    // joined to larger ones: the lanes would sit on a few compute units)
     vp_launch_config c{};
     if (ctx->have_tuned) c = ctx->tuned;
     c.pipeline = VP_PIPELINE_MEGAKERNEL;

@@ -439,6 +439,8 @@ vp_status vp_server_create(vp_context* ctx, const vp_server_config* cfg, vp_serv
     uint32_t cap = c.active_cap ? c.active_cap : 128u;
     if (S->cfg.active_cap > cap) cap = S->cfg.active_cap;
     c.active_cap = cap;
+    // (workgroups are not joined to larger ones: one of 16 wavefronts holds its
+    // compute unit until its last path ends, and the next launch waits for it)
     S->L = vp_resolve_launch(ctx, &c, cap, 0, 0);
     // With cfg.reserve_cus the render streams leave one CU of each of the 8
     // XCDs free, and their launches are sized for the rest: the side stream's

@@ -125,6 +125,11 @@ typedef struct {
 #define VP_PIPELINE_WAVEFRONT 1u
 
 /* ---- context ---------------------------------------------------------- */
+/* A context keeps memory between calls, until it is destroyed: its largest
+ * active-set slab and wavefront pool, up to 256 MiB of device scratch (sums,
+ * images for the host, scene-build temporaries; given back to any call of the
+ * context that finds no other device memory), and 1 or 8 MiB of pinned memory
+ * for copies to and from ordinary host memory. */
 vp_status vp_context_create(int device, vp_context** out);
 vp_status vp_context_destroy(vp_context* ctx);
 const char* vp_last_error(void);
