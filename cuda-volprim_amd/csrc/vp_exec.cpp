@@ -157,6 +157,7 @@ RenderLaunch vp_resolve_launch(vp_context* ctx, const vp_launch_config* cfg, uin
     L.regen_min = std::max<uint32_t>(1u, std::min<uint32_t>(64u, c.regen_min ? c.regen_min : 8u));
     L.first_paths = 4u;
     L.claim_step = 8u;
+    L.claim_cheap = 8u;
     L.rounds_target = 256u;
     L.count_events = count;
     L.measure = measure;
@@ -189,6 +190,10 @@ RenderLaunch vp_resolve_launch(vp_context* ctx, const vp_launch_config* cfg, uin
 // wavefronts to the others.  Starting on 4 and claiming 4, 8 and 16: 192x128x2
 // cloud (12 paths per wavefront) 17, 24, 38 ms, 512x512x1 torus (64) 19.9, 20.2,
 // 21.9, 256x256x24 scattering (384) 27.0, 26.4, 26.1.
+// Cheap paths in small scenes are claimed in sixteenths of the share, up to 64
+// (eighths: far views of 300 and 3000 Gaussians at 512x512x4 1.9 -> 2.6 and 1.1 ->
+// 1.2 ms, sixteenths the same as 8 a claim; quarters: 10^6 cloud +15 % without the
+// limit on the scene).
 // A wavefront's paths are held to 256 rounds a bounce, or to 128 where a launch
 // has up to 128 paths to a wavefront: fewer paths at a time leave more to the
 // others near the end, and cost width in the middle (128 against 256: 8 batched
@@ -221,6 +226,7 @@ RenderLaunch vp_size_launch(RenderLaunch L, uint64_t paths) {
     const uint64_t share = (paths + waves - 1) / waves;
     L.first_paths = static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>(4u, share)));
     L.claim_step = static_cast<uint32_t>(std::max<uint64_t>(1u, std::min<uint64_t>(8u, (share + 2u) / 3u)));
+    L.claim_cheap = static_cast<uint32_t>(std::max<uint64_t>(L.claim_step, std::min<uint64_t>(64u, share / 16u)));
     L.rounds_target = share <= 128u ? 128u : 256u;
     return L;
 }

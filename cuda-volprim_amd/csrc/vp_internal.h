@@ -348,7 +348,8 @@ struct RenderLaunch {
     uint32_t active_cap;
     uint32_t regen_min;
     uint32_t first_paths;  // megakernel: paths a wavefront starts on, and the most it claims at
-    uint32_t claim_step;   // a time from then on (vp_size_launch)
+    uint32_t claim_step;   // a time from then on, or, in small scenes and while its paths are
+    uint32_t claim_cheap;  // so cheap that it may hold 64 of them, this many (vp_size_launch)
     uint32_t rounds_target;  // rounds a bounce of a wavefront is held to (vp_size_launch)
     bool wide;             // workgroups may be made larger (vp_size_launch)
     int count_events;

@@ -381,7 +381,6 @@ __device__ __forceinline__ uint32_t rebuild_shared(bool part, uint32_t na, uint3
         total_c += static_cast<uint32_t>(__popcll(kc_m));
         wave_sync();
     }
-    const uint32_t mm = kept_of[lane], mc = kept_of[64 + lane];
     bool serial = false;
     if (total != 0u) {
         // items were met path by path, so the kept candidates lie in LDS path
@@ -390,8 +389,8 @@ __device__ __forceinline__ uint32_t rebuild_shared(bool part, uint32_t na, uint3
         uint32_t* c_of = reinterpret_cast<uint32_t*>(ts_of);
         uint32_t total_m;
         wave_sync();
-        pre_of[lane] = wave_prefix(mm, total_m);
-        c_of[lane] = wave_prefix(mc, total_c);
+        pre_of[lane] = wave_prefix(kept_of[lane], total_m);
+        c_of[lane] = wave_prefix(kept_of[64 + lane], total_c);
         wave_sync();
         // kept candidates of path own below id
         auto below = [&](uint32_t own, uint32_t id) {
@@ -439,6 +438,8 @@ __device__ __forceinline__ uint32_t rebuild_shared(bool part, uint32_t na, uint3
             if (pos < cap) mine[bs - set + pos] = id;
         }
     }
+    wave_sync();
+    const uint32_t mm = kept_of[lane], mc = kept_of[64 + lane];
     uint32_t nn = mm + mc;
     if (__builtin_amdgcn_ballot_w64(serial) != 0ull) {
         // each lane sorts its kept candidates and merges them with its kept
@@ -614,6 +615,15 @@ __device__ __forceinline__ f3 vertex_members(uint32_t nn, uint32_t cur, bool has
 // the 192x128 cloud 9 times the mean).  At least 4 paths, target 128, 192 and
 // 256 rounds, scattering 27.3, 26.4, 25.9 ms, torus 19.9, 20.2, 20.6, 10^6 cloud
 // 202, 199, 197; 64 lanes always: 25.9, 41.3, 243.
+// A wavefront that may hold 64 paths, in a scene of at most 4096 primitives
+// (6 levels), claims claim_cheap at a time: where paths end after a bounce or
+// two, 8 a claim are all it ever holds (1 Gaussian at 1024x1024x16 12.4 -> 7.6
+// ms, 10 at 1024x1024x8 6.5 -> 2.7, 97 at 1024x1024x8 18.3 -> 13.5; 8.7, 3.7
+// and 26.6 with one path per lane and no limits).  In larger scenes the cheap
+// paths are those beside the object and the next ones may cost hundreds of
+// times as much: 10^6 cloud 1024x1024x4 856 -> 904 ms, a far view of it 20 -> 49.
+// hand_out: first_paths | claim_step << 8 | claim_cheap << 16 | regen_min << 24
+// (one scalar register, where four were spilled to a vector register's lanes).
 // The argmin and shadow walks are run by all 64 lanes of a wavefront together,
 // so lanes without a path work on
 // the rays of those that have one: a wavefront with two paths left evaluates
@@ -625,10 +635,11 @@ __global__ void __launch_bounds__(kCount ? 256 : 1024)
     __attribute__((amdgpu_waves_per_eu(VP_RENDER_WAVES_PER_EU)))
 k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begin,
          const uint64_t* __restrict__ launch_desc, unsigned long long* __restrict__ path_counter,
-         uint32_t* __restrict__ slab, uint32_t cap, uint32_t regen_min, uint32_t first_paths,
-         uint32_t claim_step, uint32_t rounds_target, unsigned long long* __restrict__ counters) {
+         uint32_t* __restrict__ slab, uint32_t cap, uint32_t hand_out, uint32_t rounds_target,
+         unsigned long long* __restrict__ counters) {
     constexpr bool kShared = !kCount;
     extern __shared__ __align__(16) uint32_t s_leafq[];  // a queue of kMegaBytes to a wavefront
+    const uint32_t first_paths = hand_out & 0xffu;
     const uint32_t njobs = static_cast<uint32_t>(launch_desc[0]);
     const uint64_t total_paths = launch_desc[1];
     const uint64_t path_lo = launch_desc[2];
@@ -682,10 +693,13 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
         // ---- claim new paths for idle lanes: one atomic per wavefront and part tried ----
         const unsigned long long idle = __builtin_amdgcn_ballot_w64(!alive);
         const uint32_t busy = 64u - static_cast<uint32_t>(__popcll(idle));
-        uint32_t room = limit > busy ? limit - busy : 0u;
+        const uint32_t lanes = limit < 64u ? limit : 64u;
+        uint32_t room = lanes > busy ? lanes - busy : 0u;
+        const uint32_t regen_min = hand_out >> 24;
         const uint32_t claim_min = regen_min < (limit + 1u) / 2u ? regen_min : (limit + 1u) / 2u;
         if (!exhausted && room != 0u && (room >= claim_min || busy == 0u)) {
-            if (kShared && room > claim_step) room = claim_step;
+            const uint32_t most = (limit > 64u ? hand_out >> 16 : hand_out >> 8) & 0xffu;
+            if (kShared && room > most) room = most;
             const uint32_t leader = static_cast<uint32_t>(__builtin_ctzll(idle));
             unsigned long long base = 0;
             uint32_t got = 0;
@@ -1095,7 +1109,8 @@ k_render(const JobDesc* __restrict__ jobs, const uint64_t* __restrict__ job_begi
             // the bounce's rounds per path, smoothed over bounces, in sixteenths
             work = (3u * work + 16u * rounds / nalive) / 4u;
             limit = 16u * rounds_target / (work + 1u);
-            limit = limit < kPathsMin ? kPathsMin : (limit < 64u ? limit : 64u);
+            const uint32_t all = ws.leaf_base <= w4_level_base(5u) ? 65u : 64u;
+            limit = limit < kPathsMin ? kPathsMin : (limit < 64u ? limit : all);
         } else {
             if (has_a) acc_a = shadow_depth(sc, x, da, act, nn, stride, lq, ev, lim_a);
             if (has_b) acc_b = shadow_depth(sc, x, db, act, nn, stride, lq, ev, lim_b);
@@ -1377,7 +1392,7 @@ __global__ void k_prim(int fn, const PrimRecord* __restrict__ rec, const float* 
 }
 
 using RenderKernel = void (*)(const JobDesc*, const uint64_t*, const uint64_t*, unsigned long long*, uint32_t*,
-                              uint32_t, uint32_t, uint32_t, uint32_t, uint32_t, unsigned long long*);
+                              uint32_t, uint32_t, uint32_t, unsigned long long*);
 RenderKernel render_kernel(int count_events, int measure) {
     if (count_events) return measure ? k_render<true, true> : k_render<true, false>;
     return measure ? k_render<false, true> : k_render<false, false>;
@@ -1400,7 +1415,8 @@ hipError_t vp_launch_render(const RenderLaunch& L, const JobDesc* jobs, const ui
     const size_t lds = mega_queue_bytes(L.block);
     const auto k = render_kernel(L.count_events, L.measure);
     hipLaunchKernelGGL(k, dim3(L.grid), dim3(L.block), lds, s, jobs, job_begin, launch_desc, counter, slab,
-                       L.active_cap, L.regen_min, L.first_paths, L.claim_step, L.rounds_target, counters);
+                       L.active_cap, L.first_paths | L.claim_step << 8 | L.claim_cheap << 16 | L.regen_min << 24,
+                       L.rounds_target, counters);
     return hipGetLastError();
 }
 

@@ -31,7 +31,9 @@ inline std::map<const void*, std::string>& kernels() {
     static auto* m = new std::map<const void*, std::string>();
     return *m;
 }
-// called for every launch (kernel, workgroup); an error is its result
+// called for every launch (kernel, workgroup; its arguments are in launch_args);
+// an error is its result
+inline void** launch_args = nullptr;
 inline std::function<hipError_t(const std::string&, dim3)> on_launch;
 // called for every queued copy and recorded event; an error is its result
 inline std::function<hipError_t()> on_copy, on_record;
@@ -214,6 +216,7 @@ hipError_t hipLaunchKernel(const void* host, dim3, dim3 block, void** args, size
     STUB_LOCK;
     const std::string& name = stub::kernels()[host];
     if (s && reinterpret_cast<stub::Stream*>(s)->device != stub::device) return stub::keep(hipErrorInvalidHandle);
+    stub::launch_args = args;
     if (stub::on_launch) {
         const hipError_t e = stub::on_launch(name, block);
         if (e != hipSuccess) return stub::keep(e);

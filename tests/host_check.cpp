@@ -298,6 +298,39 @@ void render_beside_server() {
     vp_env_destroy(env);
 }
 
+// How many paths the wavefronts of a launch start on, claim at a time, and claim
+// while they are cheap: by the launch's paths to each of its 4096 wavefronts.
+void path_claims() {
+    Program prog(1000);
+    vp_env* env = nullptr;
+    std::vector<float> texels(4 * 16);
+    check(vp_env_create(prog.ctx, texels.data(), 4, 4, &env) == VP_OK, "vp_env_create");
+    const struct {
+        uint32_t side, spp, first, step, cheap;
+    } launches[] = {{32, 4, 1, 1, 1},   {64, 2, 2, 1, 1},    {64, 8, 4, 3, 3},     {128, 4, 4, 6, 6},
+                    {256, 8, 4, 8, 8},  {256, 16, 4, 8, 16}, {256, 24, 4, 8, 24},  {512, 8, 4, 8, 32},
+                    {512, 16, 4, 8, 64}, {1024, 16, 4, 8, 64}};
+    uint32_t hand_out = 0;
+    stub::on_launch = [&](const std::string& name, dim3) {
+        if (name.find("k_renderILb0E") != std::string::npos)
+            hand_out = *static_cast<const uint32_t*>(stub::launch_args[6]);
+        return hipSuccess;
+    };
+    for (const auto& l : launches) {
+        std::vector<float> image(4 * size_t(l.side) * l.side);
+        vp_camera cam{};
+        vp_render_params p{};
+        vp_default_params(&p);
+        p.width = p.height = l.side;
+        p.spp = l.spp;
+        check(vp_render(prog.ctx, prog.scene, env, &cam, &p, image.data(), nullptr) == VP_OK, "vp_render");
+        check((hand_out & 0xffffffu) == (l.first | l.step << 8 | l.cheap << 16), "the hand-out");
+        check(hand_out >> 24 == 8, "the idle lanes a wavefront waits for");
+    }
+    stub::on_launch = nullptr;
+    vp_env_destroy(env);
+}
+
 // The images of a batch leave the device in copies of a slot each, not one by
 // one, and arrive where they belong, whatever their sizes and whether one slot
 // holds them all.
@@ -361,7 +394,8 @@ int main(int argc, char** argv) {
                                                           {"build_memory", build_memory},
                                                           {"launch_shapes", launch_shapes},
                                                           {"batch_images", batch_images},
-                                                          {"render_beside_server", render_beside_server}};
+                                                          {"render_beside_server", render_beside_server},
+                                                          {"path_claims", path_claims}};
     check(argc == 2 && checks.count(argv[1]) == 1, "usage: host_check NAME");
     checks.at(argv[1])();
     std::printf("ok %s\n", argv[1]);

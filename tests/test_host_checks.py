@@ -26,7 +26,7 @@ def host_check(tmp_path_factory):
 
 @pytest.mark.parametrize("name", ["failed_copies", "export_device", "export_without_memory", "kept_scratch",
                                   "build_memory", "launch_shapes", "batch_images",
-                                  "render_beside_server"])
+                                  "render_beside_server", "path_claims"])
 def test_host_check(host_check, name):
     r = subprocess.run([host_check, name], capture_output=True, text=True, timeout=100)
     assert r.returncode == 0 and r.stdout.startswith(f"ok {name}"), r.stdout + r.stderr
