@@ -293,7 +293,7 @@ VP_HD InsideChord inside_chord_from(const PrimRecord& pr, f3 p, float pp, f3 d, 
     const float tau = maxf(pr.md * (far - near), 0.0f);
     InsideChord r;
     r.t1 = (-b + sq) * a_inv;
-    r.tau = (r.t1 > kSegMin) & (r.t1 < kTMax) ? tau : 0.0f;
+    r.tau = ((r.t1 > kSegMin) & (r.t1 < kTMax)) ? tau : 0.0f;
     return r;
 }
 VP_HD InsideChord inside_chord(const PrimRecord& pr, f3 o, f3 d) {
