@@ -208,7 +208,7 @@ void launch_shapes() {
             most = std::max(most, threads);
         }
         if (name == "graph" || (name.find("k_renderILb0ELb0E") != std::string::npos && (block.x != 128) == slow_256))
-            std::this_thread::sleep_for(std::chrono::milliseconds(30));
+            std::this_thread::sleep_for(std::chrono::milliseconds(150));
         return hipSuccess;
     };
     const auto rendered = [&](const vp_launch_config* cfg) {
